@@ -130,6 +130,7 @@ struct ScoreArgs {
   int head_off;     //   this launch serves (it serves REP of them; other ratios take several launches)
   int head_split;   // scores_kernel: head_split blocks share a tile, each owns n_kv_heads/head_split heads
   int row_slabs;    // scores_mfma_i4_gqa_kernel<SPLIT>: 128-dimension slabs of a whole cached row (n_kv_heads of them per block)
+  int tiles_per_block;   // scores_mfma_i8_kernel: consecutive tiles of a block, 1 to kI8TilesPerBlock
 };
 
 template <int SCHEME, int REP, int Q_DT>
@@ -810,7 +811,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NKV * NSET 
 // A wavefront owns kv heads {w, w+4, ...} and keeps their A operands in registers (8
 // k-steps of 16 dimensions per head); per 16-token slice a lane loads the two 16-byte
 // halves of its token's head row, so one load instruction fetches whole 128-byte lines.
-constexpr int kI8TilesPerBlock = 4;
+constexpr int kI8TilesPerBlock = 4;   // the most; launch_i8_mfma_q says when a block takes fewer
 constexpr int kI8QsFloats = 4 * 4 * 4 * 16;   // query sums in LDS: 4 wavefronts x up to 4 kv head slots x up to 4 parts x 16
 
 // Heads narrower than 128 (HPS = 128 / head_dim = 2 or 4): a.n_kv_heads counts 128-dimension slabs of
@@ -830,7 +831,7 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
 
   const int c = blockIdx.y;
   const int len = a.fill[c] < a.max_len ? a.fill[c] : a.max_len;
-  const int64_t tile0 = (int64_t)blockIdx.x * kI8TilesPerBlock;
+  const int64_t tile0 = (int64_t)blockIdx.x * a.tiles_per_block;
   if (tile0 * kTile >= len) return;  // uniform for the block
   // a launch serves heads a.head_off .. a.head_off + rep - 1 of every kv head (more than 16 per kv head: several
   // launches, heads of 128 only); the staged rows are those heads, rep per kv head
@@ -1008,7 +1009,7 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (spread) {
     const int tpr = kI8TilesPerBlock / spread;   // tiles per round, each with a staging area of its own
-    for (int round = 0; round < spread; ++round) {
+    for (int round = 0; round * tpr < a.tiles_per_block; ++round) {
       const int item = wave + 4 * round;
       const int tt = item / spread;
       if ((tile0 + tt) * kTile < len) head_tile(0, item % spread, (tile0 + tt) * kTile, stage + (tt % tpr) * a.n_q_heads * kTile);
@@ -1024,7 +1025,7 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
     }
     return;
   }
-  for (int tt = 0; tt < kI8TilesPerBlock; ++tt) {
+  for (int tt = 0; tt < a.tiles_per_block; ++tt) {
     const int64_t tile = tile0 + tt;
     const int64_t n0 = tile * kTile;
     if (n0 >= len) break;  // uniform
@@ -1051,9 +1052,18 @@ static size_t i8_mfma_lds_bytes(int n_slabs, int n_q_heads) {
 constexpr size_t kI8MfmaMaxLds = 64 * 1024;   // beyond it the vector form serves the cache (one block per compute unit otherwise)
 
 template <int SCHEME, int HPS, bool QF32>
-static void launch_i8_mfma_q(const ScoreArgs& a, int n_caches, int64_t n_tiles, hipStream_t st) {
+static void launch_i8_mfma_q(const ScoreArgs& a0, int n_caches, int64_t n_tiles, hipStream_t st) {
+  ScoreArgs a = a0;
   const size_t lds = i8_mfma_lds_bytes(a.n_kv_heads, a.n_q_heads);
-  const dim3 grid((unsigned)((n_tiles + kI8TilesPerBlock - 1) / kI8TilesPerBlock), (unsigned)n_caches);
+  // Four tiles per block share the load of the queries, but a call whose blocks would not cover the chip's 256
+  // compute units twice is a chain of tile latencies: there a block takes as few tiles as its wavefronts can be
+  // dealt (one; 4 / heads on rows of 1 or 2 kv heads): 8 caches x 433 of 1024 tokens, 8 kv heads x 32 q heads,
+  // 32 blocks of 4 tiles 39.8 us, 128 blocks of one 13.3 us
+  const int fewest = a.n_kv_heads <= 2 ? kI8TilesPerBlock / a.n_kv_heads : 1;
+  a.tiles_per_block = kI8TilesPerBlock;
+  while (a.tiles_per_block > fewest && (n_tiles + a.tiles_per_block - 1) / a.tiles_per_block * n_caches < 512)
+    a.tiles_per_block >>= 1;
+  const dim3 grid((unsigned)((n_tiles + a.tiles_per_block - 1) / a.tiles_per_block), (unsigned)n_caches);
   if (a.n_kv_heads <= 4)
     hipLaunchKernelGGL((scores_mfma_i8_kernel<SCHEME, 1, HPS, QF32>), grid, dim3(256), lds, st, a);
   else if (a.n_kv_heads <= 8)
