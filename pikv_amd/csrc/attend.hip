@@ -1462,13 +1462,16 @@ static DecodeWs decode_ws(int n_caches, int n_q_heads, int head_dim, int64_t max
   w.stride = w.n_tiles * PIKV_SCORE_TILE;
   w.scores = 0;  // float scores [cache][head][stride], or the exchange rows [cache][tile][head][64] (same size)
   // (the two tile tables have room for one tile more than max_len holds: the one-pass form keeps a spare
-  // record per cache there, and its ranges' statistics - 8 bytes per head and range of at least 128 tokens -
-  // fit the second table)
+  // record per cache there, and its ranges' statistics - 8 bytes per head and range of at least 64 tokens -
+  // lie in the second table)
   w.tmax = align256((int64_t)n_caches * n_q_heads * w.stride * 4);
   w.tsum = w.tmax + align256((int64_t)n_caches * (w.n_tiles + 1) * n_q_heads * 4);
-  w.stats = w.tsum + align256((int64_t)n_caches * (w.n_tiles + 1) * n_q_heads * 4);
+  w.stats = w.tsum + align256((int64_t)n_caches * (w.n_tiles + 1) * n_q_heads * 8);
   w.partial = w.stats + align256((int64_t)n_caches * n_q_heads * 2 * 4);
-  w.total = w.partial + align256(pikv_attend_workspace_bytes(n_caches, n_q_heads, head_dim, max_len));
+  const int64_t fused_tpb = fused_min_tokens_per_block(n_caches, max_len);
+  const int64_t fused = (max_len + fused_tpb - 1) / fused_tpb * n_caches * (int64_t)n_q_heads * head_dim * (int64_t)sizeof(float);
+  const int64_t two_kernel = pikv_attend_workspace_bytes(n_caches, n_q_heads, head_dim, max_len);
+  w.total = w.partial + align256(fused > two_kernel ? fused : two_kernel);
   return w;
 }
 
@@ -1514,7 +1517,7 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
   // in the tile-sum table.
   if (decode_fused_serves(scheme, group, n_kv_heads, n_q_heads, head_dim, q_dtype, row_acc != nullptr) && (!any_asym || (k_zero && v_zero)) &&
       n_caches <= 65535) {
-    const int tpb = fused_tokens_per_block(n_caches, n_kv_heads, max_len, attend_tokens_per_block(n_caches, max_len));
+    const int tpb = fused_tokens_per_block(n_caches, n_kv_heads, n_q_heads, scheme, q_dtype, max_len);
     return decode_fused_launch(k_codes, k_scale, k_zero, v_codes, v_scale, v_zero, scheme, group, n_kv_heads, n_q_heads, q,
                                q_dtype, scale_qk, cache_row_base, cache_fill, n_caches, max_len, tpb, decay, now, row_acc, row_ts,
                                out, ws + w.scores, tmax, tsum, reinterpret_cast<float*>(partial), stats, st);

@@ -455,7 +455,8 @@ int scores_exchange_launch(const void* k_codes, const void* k_scale, const void*
 // kv heads; 4-bit codes in groups of 32 with up to 4 bf16 or float32 query heads per kv head, or 5 to 8 bf16
 // ones; 8-bit codes with a scale per kv head or coarser and up to 8 bf16 or float32 ones).
 bool decode_fused_serves(int scheme, int group, int n_kv_heads, int n_q_heads, int head_dim, int q_dtype, bool bookkeeping);
-int fused_tokens_per_block(int n_caches, int n_kv_heads, int64_t max_len, int min_tpb);
+int fused_min_tokens_per_block(int n_caches, int64_t max_len);   // what the workspace has room for
+int fused_tokens_per_block(int n_caches, int n_kv_heads, int n_q_heads, int scheme, int q_dtype, int64_t max_len);
 int decode_fused_launch(const void* k_codes, const void* k_scale, const void* k_zero, const void* v_codes,
                         const void* v_scale, const void* v_zero, int scheme, int group, int n_kv_heads, int n_q_heads,
                         const void* q, int q_dtype, float scale_qk, const int64_t* cache_row_base, const int32_t* cache_fill,

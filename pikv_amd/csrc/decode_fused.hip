@@ -88,7 +88,7 @@ struct FusedArgs {
   int n_caches;
   int n_kv_heads;
   int n_q_heads;
-  int tokens_per_block;     // a multiple of 128
+  int tokens_per_block;     // a multiple of 64 (of 128 for the one-set kernel, which walks tiles in pairs)
   float scale_qk;
   int groups;               // blocks per token range: each takes n_kv_heads / groups neighbouring kv heads
 };
@@ -1244,35 +1244,86 @@ __global__ __launch_bounds__(512) void decode_fused_i8_kernel(Fused8Args a) {
 }
 
 // out[c,h,:] = sum over ranges of partial * exp(m_range - M) / Z,  M = max of the ranges' maxima,
-// Z = sum of their sums scaled alike.  One thread per output element; caches without a token give 0.
+// Z = sum of their sums scaled alike.  W wavefronts per (cache, q head), two dimensions per lane; caches
+// without a token give 0.  Bound by the latency of its loads: a lane holds the statistics of one range (64 at
+// a time), so that the factors of all ranges come from one round trip, the partial outputs are asked for
+// eight ranges at a time, and from 32 ranges on four wavefronts take a quarter of them each.  (One thread per
+// output element, the ranges' statistics and partials one after the other, had taken 10.6 us for 24 caches x
+// 28 heads x 16 ranges; W = 1 at 256 ranges 11 us.)
+template <int W>
 __global__ __launch_bounds__(256) void decode_finish_kernel(const float* __restrict__ partial,
                                                            const float* __restrict__ pstats,
                                                            const int32_t* __restrict__ fill, int64_t max_len,
                                                            int n_caches, int n_q_heads, int n_splits,
                                                            int tokens_per_block, float* __restrict__ out,
                                                            float* __restrict__ head_stats) {
-  const int64_t per_cache = (int64_t)n_q_heads * 128;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= per_cache * n_caches) return;
-  const int c = (int)(idx / per_cache);
-  const int h = (int)((idx - (int64_t)c * per_cache) >> 7);
+  __shared__ float2 part_s[W > 1 ? W : 1][64];
+  __shared__ float part_z[W > 1 ? W : 1];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t items = (int64_t)n_caches * n_q_heads;
+  const int64_t item = W > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wv;   // (cache, head)
+  if (item >= items) return;   // (W > 1: the grid is one block per item)
+  const int c = (int)(item / n_q_heads);
   const int64_t len = fill[c] < max_len ? (int64_t)fill[c] : max_len;
   const int64_t used = (len + tokens_per_block - 1) / tokens_per_block;
   const int lim = used < n_splits ? (int)used : n_splits;
+  const float2* const ps = reinterpret_cast<const float2*>(pstats) + item;   // (maximum, sum) of range sp at sp * items
+  const float2* const po = reinterpret_cast<const float2*>(partial) + item * 64 + lane;
   float M = -__builtin_inff();
-  for (int sp = 0; sp < lim; ++sp) M = fmaxf(M, pstats[(((int64_t)sp * n_caches + c) * n_q_heads + h) * 2]);
-  float Z = 0.f, s = 0.f;
-  for (int sp = 0; sp < lim; ++sp) {
-    const int64_t pi = ((int64_t)sp * n_caches + c) * n_q_heads + h;
-    const float f = __builtin_amdgcn_exp2f((pstats[pi * 2] - M) * kLog2e);
-    Z = fmaf(pstats[pi * 2 + 1], f, Z);
-    s = fmaf(partial[(int64_t)sp * per_cache * n_caches + idx], f, s);
+  for (int s0 = 0; s0 < lim; s0 += 64)
+    M = fmaxf(M, group_max_dpp(s0 + lane < lim ? ps[(s0 + lane) * items].x : -__builtin_inff(), 64));
+  const int share = (lim + W - 1) / W;                     // ranges of this wavefront: [first, last)
+  const int first = W > 1 ? wv * share : 0;
+  const int last = W > 1 ? (first + share < lim ? first + share : lim) : lim;
+  float Z = 0.f;
+  float2 s = make_float2(0.f, 0.f);
+  for (int s0 = first; s0 < last; s0 += 64) {
+    float f = 0.f, z = 0.f;
+    if (s0 + lane < last) {
+      const float2 mz = ps[(s0 + lane) * items];
+      f = __builtin_amdgcn_exp2f((mz.x - M) * kLog2e);
+      z = mz.y * f;
+    }
+    Z += group_sum_dpp(z, 64);
+    const int n = last - s0 < 64 ? last - s0 : 64;
+    for (int j0 = 0; j0 < n; j0 += 8) {
+      float2 p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = po[(s0 + (j0 + j < n ? j0 + j : n - 1)) * items * 64];   // (past the end: a copy, factor 0)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float fj = j0 + j < n ? read_lane_f(f, j0 + j) : 0.f;
+        s.x = fmaf(p[j].x, fj, s.x);
+        s.y = fmaf(p[j].y, fj, s.y);
+      }
+    }
   }
-  out[idx] = lim > 0 ? s / Z : 0.f;
-  if (head_stats != nullptr && (idx & 127) == 0) {
-    head_stats[((int64_t)c * n_q_heads + h) * 2] = M;
-    head_stats[((int64_t)c * n_q_heads + h) * 2 + 1] = Z;
+  if constexpr (W > 1) {
+    part_s[wv][lane] = s;
+    if (lane == 0) part_z[wv] = Z;
+    __syncthreads();
+    if (wv != 0) return;
+#pragma unroll
+    for (int k = 1; k < W; ++k) {
+      s.x += part_s[k][lane].x;
+      s.y += part_s[k][lane].y;
+      Z += part_z[k];
+    }
   }
+  reinterpret_cast<float2*>(out)[item * 64 + lane] = lim > 0 ? make_float2(s.x / Z, s.y / Z) : make_float2(0.f, 0.f);
+  if (head_stats != nullptr && lane == 0) reinterpret_cast<float2*>(head_stats)[item] = make_float2(M, Z);
+}
+
+static void launch_finish(const float* partial, const float* pstats, const int32_t* fill, int64_t max_len, int n_caches,
+                          int n_q_heads, int n_splits, int tokens_per_block, float* out, float* head_stats, hipStream_t st) {
+  const int64_t items = (int64_t)n_caches * n_q_heads;
+  if (n_splits >= 32)
+    hipLaunchKernelGGL(decode_finish_kernel<4>, dim3((unsigned)items), dim3(256), 0, st, partial, pstats, fill, max_len,
+                       n_caches, n_q_heads, n_splits, tokens_per_block, out, head_stats);
+  else
+    hipLaunchKernelGGL(decode_finish_kernel<1>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, st, partial, pstats, fill,
+                       max_len, n_caches, n_q_heads, n_splits, tokens_per_block, out, head_stats);
 }
 
 // H2O bookkeeping from the halves the fused pass left: one wavefront per tile of 64 cached tokens.
@@ -1433,34 +1484,50 @@ using namespace pikv;
 
 namespace pikv {
 
-// Cached tokens per block of the fused pass: a block is n_kv_heads wavefronts and as many pieces of
-// LDS, so a compute unit holds 8 / n_kv_heads of them (at most 8 wavefronts' pieces fit); the longest
-// range that still fills the chip wins, and it is never shorter than `min_tpb` (the workspace is
-// laid out for that many ranges).
 // (4-bit rows as two blocks of half the kv heads per token range measured slower - 662 vs 632 us at 8 kv
 // heads: the halves of a 128-byte line then belong to different blocks and the metadata is fetched 1.75 x.)
 static int fused_groups(int n_kv_heads) { (void)n_kv_heads; return 1; }
 // the 8-bit pass: its wavefronts share no code lines (a kv head's 128 bytes of a row are a line of their own)
 static int fused8_blocks_per_range(int n_kv_heads) { return (n_kv_heads == 8 || n_kv_heads == 6) ? 2 : 1; }
 
-int fused_tokens_per_block(int n_caches, int n_kv_heads, int64_t max_len, int min_tpb) {
-  const int groups = fused_groups(n_kv_heads);
-  int per_cu = 8 / (n_kv_heads / groups);
-  if (per_cu < 1) per_cu = 1;
-  const int64_t resident = 256 * (int64_t)per_cu / groups;
-  int best = 0;
-  double best_eff = -1.0;
-  for (int tpb = 8192; tpb >= 128 && tpb >= min_tpb; tpb >>= 1) {
-    const int64_t blocks = (int64_t)n_caches * ((max_len + tpb - 1) / tpb);
-    const int64_t rounds = (blocks + resident - 1) / resident;
-    const double eff = rounds > 0 ? (double)blocks / (double)(rounds * resident) : 0.0;
-    if (eff >= 0.85) return tpb;
-    if (eff > best_eff) {
-      best_eff = eff;
+// the finest cut the workspace is laid out for: at most 1024 ranges, of at least one tile
+int fused_min_tokens_per_block(int n_caches, int64_t max_len) {
+  int tpb = kFTile;
+  while (tpb < 8192 && (max_len + tpb - 1) / tpb * n_caches > 1024) tpb <<= 1;
+  return tpb;
+}
+
+// Cached tokens per block of the fused pass.  A block costs its start and end (about 6 us: the fill, the queries,
+// the first tile on its way, the partial output) and about 3 us per 64-token tile whatever else runs, until the
+// memory system is what it waits for; the merge costs some 0.03 us per range.  The cut with the least of that sum
+// over the rounds the chip needs is taken.  Blocks of more than four wavefronts sit alone on a compute unit, so
+// their rounds are whole; smaller ones overlap, and their rounds count in parts - which also favours the finer
+// cut when caches of different lengths share a call (the lengths are not known on the host).
+// Measured, one call with bookkeeping, bf16 queries, coarsest / chosen / finest cut, us: 4-bit 8 kv x 32 q heads,
+// 1 cache x 700: 48 (1024 tokens) / 18.0 (128); 1 x 32768: 426 / 35 (256) / 41 (128); 24 x <= 4000: 222 / 44 (512) /
+// 51; 64 x 4096: 250 / 93 (1024) / 120 (256); 8-bit 4 x 28: 1 x 700 39 / 13.2 (64); 24 x <= 4000: 173 / 33 (256) / 34.
+int fused_tokens_per_block(int n_caches, int n_kv_heads, int n_q_heads, int scheme, int q_dtype, int64_t max_len) {
+  const bool eight = scheme == PIKV_Q_I8_SYM || scheme == PIKV_Q_I8_ASYM;
+  const bool pairs = !eight && q_dtype == PIKV_BF16 && n_q_heads <= 4 * n_kv_heads;   // walks tiles two at a time
+  const int finest = fused_min_tokens_per_block(n_caches, max_len);
+  const int min_tpb = pairs && finest < 2 * kFTile ? 2 * kFTile : finest;
+  const int wave_blocks = eight ? fused8_blocks_per_range(n_kv_heads) : fused_groups(n_kv_heads);   // blocks per range
+  const int per_cu = 8 / (n_kv_heads / wave_blocks) > 0 ? 8 / (n_kv_heads / wave_blocks) : 1;
+  int best = 8192;
+  double best_us = 1e30;
+  for (int tpb = 8192; tpb >= min_tpb; tpb >>= 1) {
+    const int64_t splits = (max_len + tpb - 1) / tpb;
+    double rounds = (double)(n_caches * splits * wave_blocks) / (256.0 * per_cu);
+    if (rounds < 1.0) rounds = 1.0;
+    if (per_cu == 1) rounds = (double)(int64_t)(rounds + 0.999999);
+    const int64_t tiles = max_len < tpb ? (max_len + kFTile - 1) / kFTile : tpb / kFTile;
+    const double us = rounds * (6.0 + 3.0 * (double)tiles) + 0.03 * (double)splits;
+    if (us < best_us * 0.999) {
+      best_us = us;
       best = tpb;
     }
   }
-  return best > 0 ? best : (min_tpb > 128 ? min_tpb : 128);
+  return best;
 }
 
 // Which calls take the one-pass form (measured against the two-kernel forms at 64 caches x 32768 tokens,
@@ -1513,7 +1580,7 @@ int decode_fused_launch(const void* k_codes, const void* k_scale, const void* k_
   // one spare record per cache for the one-set 4-bit kernel (it walks tiles in pairs); the others touch no tile past a range's end
   const int64_t n_tiles = (max_len + kFTile - 1) / kFTile + ((q_dtype == PIKV_F32 || n_q_heads > 4 * n_kv_heads) ? 0 : 1);
   const int64_t splits = (max_len + tokens_per_block - 1) / tokens_per_block;
-  if (splits > 65535 || (tokens_per_block & 127) != 0) return PIKV_ERR_SHAPE;
+  if (splits > 65535 || (tokens_per_block & 63) != 0) return PIKV_ERR_SHAPE;
   const bool book = row_acc != nullptr || row_ts != nullptr;
   if (q_dtype != PIKV_BF16 && q_dtype != PIKV_F32) return PIKV_ERR_UNSUPPORTED;
   if (scheme == PIKV_Q_I8_SYM || scheme == PIKV_Q_I8_ASYM) {
@@ -1541,9 +1608,7 @@ int decode_fused_launch(const void* k_codes, const void* k_scale, const void* k_
     }
 #undef PIKV_FUSED8
     PIKV_CHECK_LAUNCH();
-    const int64_t total8 = (int64_t)n_caches * n_q_heads * 128;
-    hipLaunchKernelGGL(decode_finish_kernel, dim3((unsigned)((total8 + 255) / 256)), dim3(256), 0, st, partial, pstats,
-                       cache_fill, max_len, n_caches, n_q_heads, (int)splits, tokens_per_block, out, head_stats);
+    launch_finish(partial, pstats, cache_fill, max_len, n_caches, n_q_heads, (int)splits, tokens_per_block, out, head_stats, st);
     if (book)
       hipLaunchKernelGGL(decode_importance8_kernel, dim3((unsigned)((n_tiles8 + 3) / 4), (unsigned)n_caches), dim3(256), 0,
                          st, reinterpret_cast<const uint4*>(e16), tref, head_stats, cache_row_base, cache_fill, max_len,
@@ -1575,9 +1640,7 @@ int decode_fused_launch(const void* k_codes, const void* k_scale, const void* k_
   else PIKV_FUSED(PIKV_Q_I4_SYM);
 #undef PIKV_FUSED
   PIKV_CHECK_LAUNCH();
-  const int64_t total = (int64_t)n_caches * n_q_heads * 128;
-  hipLaunchKernelGGL(decode_finish_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, partial, pstats,
-                     cache_fill, max_len, n_caches, n_q_heads, (int)splits, tokens_per_block, out, head_stats);
+  launch_finish(partial, pstats, cache_fill, max_len, n_caches, n_q_heads, (int)splits, tokens_per_block, out, head_stats, st);
   if (book)
     hipLaunchKernelGGL(decode_importance_kernel, dim3((unsigned)((n_tiles + 3) / 4), (unsigned)n_caches), dim3(256), 0,
                        st, reinterpret_cast<const uint2*>(e16), tref, head_stats, cache_row_base, cache_fill, max_len,
