@@ -81,6 +81,7 @@ extern "C" {
 /* ---- eviction policies (core/single/cache_scheduling.py:9-17) ----------- */
 #define PIKV_EVICT_H2O   0
 #define PIKV_EVICT_LRU   1
+#define PIKV_EVICT_ALL   2   /* pikv_cache_make_room only: an overflowing cache is emptied */
 
 const char* pikv_status_string(int status);
 
@@ -266,6 +267,20 @@ int pikv_quant_gather(const void* k_src, const void* v_src, int src_dtype,
                       const int64_t* src_row_base, const int32_t* src_index,
                       const int32_t* n_take, int64_t max_take, const float* src_score,
                       const int64_t* cache_row_base, const int32_t* cache_fill,
+                      const int32_t* cache_cap, int n_caches,
+                      void* k_codes, void* v_codes,
+                      void* k_scale, void* v_scale,
+                      void* k_zero, void* v_zero,
+                      float* row_acc, float* row_ts, float now,
+                      void* stream);
+
+/* The same for rows that go to the caches in order: source row c*rows_per_cache + i
+ * becomes row first_row[c] + i of cache c (dropped at cache_cap[c]).  first_row is the
+ * cache_fill before the rows came, e.g. the new_len of pikv_cache_make_room.
+ * Replaces: PiKVAttention._update_cache's write (core/single/pikv_attention.py:92-100). */
+int pikv_quant_append(const void* k_src, const void* v_src, int src_dtype,
+                      int64_t rows_per_cache, int D, int group, int scheme,
+                      const int64_t* cache_row_base, const int32_t* first_row,
                       const int32_t* cache_cap, int n_caches,
                       void* k_codes, void* v_codes,
                       void* k_scale, void* v_scale,
@@ -484,6 +499,30 @@ int pikv_compact_rows(void* const* plane_ptrs_host,
                       const int64_t* cache_row_base, const int32_t* keep_index,
                       const int32_t* new_len, int32_t* cache_fill,
                       int n_caches, void* stream);
+
+/* Room for new rows: every cache that would overflow evicts and is compacted, the others
+ * keep all their rows; no host read of cache_fill.
+ * Replaces: the overflow handling of CacheSchedulingManager.update_cache
+ *   (core/single/cache_scheduling.py:404-427) and PiKVAttention._update_cache's wipe
+ *   (core/single/pikv_attention.py:85-90).
+ *   Cache c takes n_new = min(count[c] (count_all when count == NULL), per_call_limit (< 0:
+ *   none), cache_cap[c]) rows; it evicts when cache_fill[c] + n_new > cache_cap[c]:
+ *     PIKV_EVICT_H2O  keep the max(1, int(fill*heavy_ratio)) rows of largest row_acc and the
+ *                     max(1, int(fill*recent_ratio)) of largest row_ts; leave_room != 0 cuts
+ *                     the two so that together they leave n_new rows of space
+ *     PIKV_EVICT_LRU  drop the fill + n_new - cap rows of smallest row_ts
+ *     PIKV_EVICT_ALL  drop every row
+ *   Planes as in pikv_compact_rows; new_len [n_caches] = rows kept (cache_fill for a cache
+ *   that did not evict); cache_fill = new_len, or min(new_len + n_new, cap) with append != 0.
+ *   keep_flag, keep_index [rows_total] and budgets int32 [3*n_caches] are scratch;
+ *   max_len >= max_c cache_fill[c]; workspace as in pikv_evict_select. */
+int pikv_cache_make_room(int policy, const int32_t* count, int64_t count_all, int64_t per_call_limit,
+                         double heavy_ratio, double recent_ratio, int leave_room, int append,
+                         const float* row_acc, const float* row_ts, const int64_t* cache_row_base,
+                         int32_t* cache_fill, const int32_t* cache_cap, int n_caches, int64_t max_len,
+                         void* const* plane_ptrs_host, const int64_t* plane_row_bytes_host, int n_planes,
+                         uint8_t* keep_flag, int32_t* keep_index, int32_t* new_len, int32_t* budgets,
+                         void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * API-compatible fake quantisation of QuantizedCompressor.forward

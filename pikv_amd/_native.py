@@ -19,7 +19,7 @@ LIB_PATH = os.environ.get("PIKV_HIP_LIB", os.path.join(_HERE, "libpikv_hip.so"))
 # element types / schemes / policies (mirrors include/pikv_hip.h)
 F32, BF16 = 0, 1
 Q_I8_SYM, Q_I8_ASYM, Q_I4_ASYM, Q_I4_SYM = 0, 1, 2, 3
-EVICT_H2O, EVICT_LRU = 0, 1
+EVICT_H2O, EVICT_LRU, EVICT_ALL = 0, 1, 2
 SCORE_TILE = 64
 MAX_PLANES = 10
 
@@ -43,6 +43,8 @@ SIGNATURES = {
     "pikv_cache_advance": (_i, [_p, _p, _p, _i, _l, _p]),
     "pikv_quant_gather": (_i, [_p, _p, _i, _i, _i, _i, _p, _p, _p, _l, _p, _p, _p, _p, _i,
                                _p, _p, _p, _p, _p, _p, _p, _p, _f, _p]),
+    "pikv_quant_append": (_i, [_p, _p, _i, _l, _i, _i, _i, _p, _p, _p, _i,
+                               _p, _p, _p, _p, _p, _p, _p, _p, _f, _p]),
     "pikv_quantize_rows": (_i, [_p, _i, _l, _i, _i, _i, _l, _p, _p, _p, _p]),
     "pikv_quant8_minshift": (_i, [_p, _i, _l, _i, _p, _p, _p, _p, _p]),
     "pikv_gather_dequant": (_i, [_p, _p, _p, _i, _i, _i, _p, _l, _l, _p, _i, _p]),
@@ -59,6 +61,8 @@ SIGNATURES = {
     "pikv_evict_select": (_i, [_i, _p, _p, _p, _p, _p, _p, _i, _l, _p, _p, _p, _p, _l, _p]),
     "pikv_evict_workspace_bytes": (_l, [_i, _l]),
     "pikv_h2o_budget": (_i, [_p, _i, _d, _d, _p, _p, _p]),
+    "pikv_cache_make_room": (_i, [_i, _p, _l, _l, _d, _d, _i, _i, _p, _p, _p, _p, _p, _i, _l,
+                                  C.POINTER(_p), C.POINTER(_l), _i, _p, _p, _p, _p, _p, _l, _p]),
     "pikv_compact_rows": (_i, [C.POINTER(_p), C.POINTER(_l), _i, _p, _p, _p, _p, _i, _p]),
     "pikv_fakequant_colblocks": (_i, [_p, _l, _i, _i, _i, _i, _p, _p, _p, _p, _l, _p]),
     "pikv_fakequant_workspace_bytes": (_l, [_l, _i, _i]),

@@ -127,30 +127,15 @@ class PiKVAttention(nn.Module):
         pikv_attention.py:74-102), making room first when a cache would overflow."""
         B, S = k.shape[0], k.shape[1]
         pool = self._ensure_pool(B, k.device)
-        dev = pool.device
-        n_new = torch.full((B,), min(S, self.cache_size), dtype=torch.int32, device=dev)
-        over = (pool.fill + n_new - pool.cap).clamp_min(0)
-        if self.on_overflow == "reset":
-            pool.fill.copy_(torch.where(over > 0, torch.zeros_like(pool.fill), pool.fill))
-        else:
-            f = pool.fill.double()
-            nh = (f * self.heavy_ratio).floor().clamp_min(1).to(torch.int32)
-            nr = (f * self.recent_ratio).floor().clamp_min(1).to(torch.int32)
-            # never keep more than what leaves room for the new rows
-            room = (pool.cap - n_new).clamp_min(0)
-            nh = torch.minimum(nh, room)
-            nr = torch.minimum(nr, (room - nh).clamp_min(0))
-            keep_all = over == 0
-            pool.evict(ops.EVICT_H2O, n_heavy=torch.where(keep_all, pool.fill, nh).contiguous(),
-                       n_recent=torch.where(keep_all, torch.zeros_like(nr), nr).contiguous())
+        # a cache that would overflow keeps its heavy and recent rows, as many as leave room for the new
+        # ones, or (on_overflow="reset") none
+        policy = ops.EVICT_ALL if self.on_overflow == "reset" else ops.EVICT_H2O
+        pool.make_room(policy, count_all=S, heavy_ratio=self.heavy_ratio, recent_ratio=self.recent_ratio,
+                       leave_room=True, append=True)
         self.clock += 1
-        D = self.num_kv_heads * self.head_dim
-        dt = k.dtype if k.dtype in (torch.float32, torch.bfloat16) else torch.float32
-        cid = torch.arange(B, dtype=torch.int32, device=dev).repeat_interleave(S)
-        slot = torch.arange(S, dtype=torch.int32, device=dev).repeat(B)
-        pool.quant_scatter(k.reshape(B * S, D).to(dt).contiguous(), v.reshape(B * S, D).to(dt).contiguous(),
-                           cid, slot, 1, now=float(self.clock))
-        pool.advance(n_new)
+        if k.dtype not in (torch.float32, torch.bfloat16):
+            k = k.float()
+        pool.append_rows(k.contiguous(), v.to(k.dtype).contiguous(), now=float(self.clock))
 
     def _split_past(self, past_key_values, layer_idx: Optional[int]):
         """(k, v) tensors of one layer out of what callers carry: a (k, v) pair, a tuple of

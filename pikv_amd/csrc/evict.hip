@@ -618,8 +618,10 @@ template <bool TAIL>
 __global__ __launch_bounds__(256) void compact_rows_kernel(CompactPlanes pl,
                                                            const int64_t* __restrict__ row_base,
                                                            const int32_t* __restrict__ keep_index,
-                                                           const int32_t* __restrict__ new_len) {
+                                                           const int32_t* __restrict__ new_len,
+                                                           const int32_t* __restrict__ active) {
   const int c = blockIdx.y;
+  if (active != nullptr && active[c] == 0) return;   // every row of this cache stays where it is
   const int slab = blockIdx.x;
   int p = 0;
   while (p + 1 < pl.n_planes && slab >= pl.slab_begin[p + 1]) ++p;
@@ -656,6 +658,176 @@ __global__ __launch_bounds__(256) void compact_rows_kernel(CompactPlanes pl,
 __global__ void set_fill_kernel(int32_t* __restrict__ fill, const int32_t* __restrict__ new_len, int n) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < n) fill[c] = new_len[c];
+}
+
+// ---- making room: budgets, selection, compaction and fill of every cache that would overflow ------------------
+//
+// A cache takes n_new = min(count[c] (count_all), limit, cap[c]) rows.  One that has the space keeps all its rows:
+// its block writes the fill and ends - what almost every decode step finds, so the call costs one launch.
+// Caches of up to kRoomMaxLen rows are selected by one block each, flags and survivor list in LDS, and - unless the
+// survivors are many bytes - compacted by the same block: the launches between the steps (3 to 5 us each, and as
+// much on the host) cost more than the other compute units would give back.  Longer caches take the multi-block
+// selection.
+// One decode step of 8 caches x 3000 rows that all have the space: 24 launches (budgets as elementwise torch
+// operations, selection, two compactions, fill), 105 us of GPU time, before; now one of 2.5 us.
+constexpr int kRoomMaxLen = 8192;
+
+struct RoomArgs {
+  int policy;              // PIKV_EVICT_H2O, PIKV_EVICT_LRU or PIKV_EVICT_ALL
+  const int32_t* count;    // rows every cache takes, or nullptr: count_all for each
+  int64_t count_all;
+  int64_t limit;           // < 0: none
+  double heavy_ratio, recent_ratio;
+  int leave_room;          // H2O: never keep more rows than leave room for the new ones
+  int append;              // fill = min(survivors + n_new, cap); otherwise fill = survivors
+  const float* acc;
+  const float* ts;
+  const int64_t* row_base;
+  int32_t* fill;
+  const int32_t* cap;
+  int32_t* keep_index;
+  int32_t* new_len;        // survivors: where the new rows begin
+  int32_t* n_heavy;        // multi-block path: budgets
+  int32_t* n_recent;
+  int32_t* active;         // [n_caches] 1: the survivors have to be moved
+  int n_caches;
+};
+
+// Returns whether cache c has to evict, with its budgets (LRU: n_heavy = rows to evict) and the rows it takes.
+__device__ __forceinline__ bool room_budget(const RoomArgs& a, int c, int len, int& n_heavy, int& n_recent, int& n_new) {
+  const int cap = a.cap[c];
+  int64_t n = a.count ? (int64_t)a.count[c] : a.count_all;
+  if (a.limit >= 0 && n > a.limit) n = a.limit;
+  if (n > cap) n = cap;
+  if (n < 0) n = 0;
+  n_new = (int)n;
+  const int64_t over = (int64_t)len + n - cap;
+  n_heavy = len;
+  n_recent = 0;
+  if (a.policy == PIKV_EVICT_LRU) {
+    n_heavy = over <= 0 ? 0 : (over < len ? (int)over : len);
+    return n_heavy > 0;
+  }
+  if (over <= 0) return false;
+  if (a.policy == PIKV_EVICT_ALL) {
+    n_heavy = 0;
+    return true;
+  }
+  int h = (int)floor((double)len * a.heavy_ratio), r = (int)floor((double)len * a.recent_ratio);
+  h = h < 1 ? 1 : h;
+  r = r < 1 ? 1 : r;
+  if (a.leave_room) {
+    const int room = cap - n_new > 0 ? cap - n_new : 0;
+    h = h < room ? h : room;
+    r = r < room - h ? r : room - h;
+  }
+  n_heavy = h;
+  n_recent = r;
+  return true;
+}
+
+__device__ __forceinline__ int room_fill(const RoomArgs& a, int c, int kept, int n_new) {
+  if (!a.append) return kept;
+  return kept + n_new < a.cap[c] ? kept + n_new : a.cap[c];
+}
+
+// Rows list[j] -> j of one plane, ascending passes of the whole block: every pass reads all its pieces before it
+// writes any, and a later one reads only rows beyond those (list[j] >= j).
+template <typename V>
+__device__ __forceinline__ void room_move(char* plane, int64_t base_row, int64_t row_bytes, const int32_t* list, int m) {
+  constexpr int U = 4;
+  const int per_row = (int)(row_bytes / (int64_t)sizeof(V));
+  char* const p0 = plane + base_row * row_bytes;
+  const int64_t total = (int64_t)m * per_row;
+  for (int64_t u0 = 0; u0 < total; u0 += (int64_t)kSelThreads * U) {
+    V val[U];
+    int64_t dst[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int64_t u = u0 + k * kSelThreads + threadIdx.x;
+      dst[k] = -1;
+      val[k] = V{};
+      if (u < total) {
+        const int j = (int)((uint32_t)u / (uint32_t)per_row);   // (total < 2^31: kRoomMaxLen rows of at most 2^17 pieces)
+        const int col = (int)(u - (int64_t)j * per_row);
+        const int src = list[j];
+        if (src != j) {
+          val[k] = *reinterpret_cast<const V*>(p0 + (int64_t)src * row_bytes + (int64_t)col * (int)sizeof(V));
+          dst[k] = (int64_t)j * row_bytes + (int64_t)col * (int)sizeof(V);
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (dst[k] >= 0) *reinterpret_cast<V*>(p0 + dst[k]) = val[k];
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(kSelThreads) void room_small_kernel(RoomArgs a, CompactPlanes pl) {
+  __shared__ SelShared s;
+  __shared__ uint8_t flag[kRoomMaxLen];
+  __shared__ int32_t list[kRoomMaxLen];
+  __shared__ int32_t kept_s;
+  const int c = blockIdx.x;
+  // (a fill beyond max_len must not leave the LDS arrays; PIKV_EVICT_ALL selects nothing and takes any length)
+  const int len = a.fill[c] < kRoomMaxLen || a.policy == PIKV_EVICT_ALL ? a.fill[c] : kRoomMaxLen;
+  int nh, nr, n_new;
+  const bool evict = room_budget(a, c, len, nh, nr, n_new);   // uniform
+  if (!evict || len <= 0 || a.policy == PIKV_EVICT_ALL) {
+    const int kept = evict ? 0 : len;
+    __syncthreads();                                           // everybody has read the fill
+    if (threadIdx.x == 0) {
+      a.new_len[c] = kept;
+      a.active[c] = 0;
+      a.fill[c] = room_fill(a, c, kept, n_new);
+    }
+    return;
+  }
+  const int64_t base = a.row_base[c];
+  SelGeom g;
+  g.len = len;
+  g.items = (len + kSelThreads - 1) / kSelThreads;
+  g.lane = threadIdx.x & 63;
+  g.wave = threadIdx.x >> 6;
+  g.seg0 = g.wave * g.items * 64;
+  evict_select_body<true>(a.policy, a.acc ? a.acc + base : nullptr, a.ts + base, nh, nr, flag, list, &kept_s, g, s);
+  __syncthreads();
+  const int kept = kept_s;
+  if (pl.n_planes == 0)                                        // the move is a launch of its own: it needs the list
+    for (int j = threadIdx.x; j < kept; j += kSelThreads) a.keep_index[base + j] = list[j];
+  for (int p = 0; p < pl.n_planes; ++p) {
+    char* const plane = reinterpret_cast<char*>(pl.ptr[p]);
+    const int64_t rb = pl.row_bytes[p];
+    if (rb % 16 == 0) room_move<uint4>(plane, base, rb, list, kept);
+    else if (rb % 4 == 0) room_move<uint32_t>(plane, base, rb, list, kept);
+    else if (rb % 2 == 0) room_move<uint16_t>(plane, base, rb, list, kept);
+    else room_move<uint8_t>(plane, base, rb, list, kept);
+  }
+  if (threadIdx.x == 0) {
+    a.new_len[c] = kept;
+    a.active[c] = 1;
+    a.fill[c] = room_fill(a, c, kept, n_new);
+  }
+}
+
+__global__ void room_budget_kernel(RoomArgs a) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= a.n_caches) return;
+  int nh, nr, n_new;
+  a.active[c] = room_budget(a, c, a.fill[c], nh, nr, n_new) ? 1 : 0;
+  a.n_heavy[c] = nh;
+  a.n_recent[c] = nr;
+}
+
+__global__ void room_fill_kernel(RoomArgs a) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= a.n_caches) return;
+  int nh, nr, n_new;
+  room_budget(a, c, a.fill[c], nh, nr, n_new);
+  if (!a.active[c]) a.new_len[c] = a.fill[c];
+  a.fill[c] = room_fill(a, c, a.new_len[c], n_new);
 }
 
 }  // namespace pikv
@@ -724,6 +896,39 @@ extern "C" int pikv_h2o_budget(const int32_t* cache_fill, int n_caches, double h
   return PIKV_OK;
 }
 
+static int make_planes(void* const* plane_ptrs_host, const int64_t* plane_row_bytes_host, int n_planes, CompactPlanes& pl) {
+  if (n_planes < 0 || n_planes > PIKV_MAX_PLANES) return PIKV_ERR_SHAPE;
+  pl = CompactPlanes{};
+  pl.n_planes = n_planes;
+  int slabs = 0;
+  for (int p = 0; p < n_planes; ++p) {
+    if (!plane_ptrs_host[p]) return PIKV_ERR_NULL;
+    const int64_t rb = plane_row_bytes_host[p];
+    if (rb <= 0 || rb > (1 << 24)) return PIKV_ERR_SHAPE;
+    pl.ptr[p] = plane_ptrs_host[p];
+    pl.row_bytes[p] = rb;
+    pl.slab_begin[p] = slabs;
+    slabs += (int)((rb + kSlabBytes - 1) / kSlabBytes);
+  }
+  pl.slab_begin[n_planes] = slabs;
+  return PIKV_OK;
+}
+
+// active [n_caches] or nullptr: caches with active[c] == 0 are left alone
+static void launch_compact(const CompactPlanes& pl, const int64_t* cache_row_base, const int32_t* keep_index,
+                           const int32_t* new_len, const int32_t* active, int n_caches, hipStream_t st) {
+  const int slabs = pl.slab_begin[pl.n_planes];
+  if (slabs > 0) {
+    // ordered head first, then the free-moving tail spread over enough blocks to fill the chip
+    hipLaunchKernelGGL(compact_rows_kernel<false>, dim3((unsigned)slabs, (unsigned)n_caches), dim3(256), 0,
+                       st, pl, cache_row_base, keep_index, new_len, active);
+    int64_t chunks = 4096 / ((int64_t)slabs * n_caches);
+    chunks = chunks < 1 ? 1 : (chunks > 64 ? 64 : chunks);
+    hipLaunchKernelGGL(compact_rows_kernel<true>, dim3((unsigned)slabs, (unsigned)n_caches, (unsigned)chunks),
+                       dim3(256), 0, st, pl, cache_row_base, keep_index, new_len, active);
+  }
+}
+
 extern "C" int pikv_compact_rows(void* const* plane_ptrs_host, const int64_t* plane_row_bytes_host,
                                  int n_planes, const int64_t* cache_row_base,
                                  const int32_t* keep_index, const int32_t* new_len,
@@ -733,31 +938,57 @@ extern "C" int pikv_compact_rows(void* const* plane_ptrs_host, const int64_t* pl
   if (n_planes < 0 || n_planes > PIKV_MAX_PLANES || n_caches < 1 || n_caches > 65535)
     return PIKV_ERR_SHAPE;
   hipStream_t st = (hipStream_t)stream;
-  if (n_planes > 0) {
-    CompactPlanes pl{};
-    pl.n_planes = n_planes;
-    int slabs = 0;
-    for (int p = 0; p < n_planes; ++p) {
-      if (!plane_ptrs_host[p]) return PIKV_ERR_NULL;
-      const int64_t rb = plane_row_bytes_host[p];
-      if (rb <= 0 || rb > (1 << 24)) return PIKV_ERR_SHAPE;
-      pl.ptr[p] = plane_ptrs_host[p];
-      pl.row_bytes[p] = rb;
-      pl.slab_begin[p] = slabs;
-      slabs += (int)((rb + kSlabBytes - 1) / kSlabBytes);
-    }
-    pl.slab_begin[n_planes] = slabs;
-    // ordered head first, then the free-moving tail spread over enough blocks to fill the chip
-    hipLaunchKernelGGL(compact_rows_kernel<false>, dim3((unsigned)slabs, (unsigned)n_caches), dim3(256), 0,
-                       st, pl, cache_row_base, keep_index, new_len);
-    int64_t chunks = 4096 / ((int64_t)slabs * n_caches);
-    chunks = chunks < 1 ? 1 : (chunks > 64 ? 64 : chunks);
-    hipLaunchKernelGGL(compact_rows_kernel<true>, dim3((unsigned)slabs, (unsigned)n_caches, (unsigned)chunks),
-                       dim3(256), 0, st, pl, cache_row_base, keep_index, new_len);
-  }
+  CompactPlanes pl;
+  const int rc = make_planes(plane_ptrs_host, plane_row_bytes_host, n_planes, pl);
+  if (rc != PIKV_OK) return rc;
+  launch_compact(pl, cache_row_base, keep_index, new_len, nullptr, n_caches, st);
   if (cache_fill)
     hipLaunchKernelGGL(set_fill_kernel, dim3((n_caches + 63) / 64), dim3(64), 0, st, cache_fill,
                        new_len, n_caches);
+  PIKV_CHECK_LAUNCH();
+  return PIKV_OK;
+}
+
+extern "C" int pikv_cache_make_room(int policy, const int32_t* count, int64_t count_all, int64_t per_call_limit,
+                                    double heavy_ratio, double recent_ratio, int leave_room, int append,
+                                    const float* row_acc, const float* row_ts, const int64_t* cache_row_base,
+                                    int32_t* cache_fill, const int32_t* cache_cap, int n_caches, int64_t max_len,
+                                    void* const* plane_ptrs_host, const int64_t* plane_row_bytes_host, int n_planes,
+                                    uint8_t* keep_flag, int32_t* keep_index, int32_t* new_len, int32_t* budgets,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!row_ts || !cache_row_base || !cache_fill || !cache_cap || !keep_flag || !keep_index || !new_len || !budgets)
+    return PIKV_ERR_NULL;
+  if (n_planes > 0 && (!plane_ptrs_host || !plane_row_bytes_host)) return PIKV_ERR_NULL;
+  if (policy != PIKV_EVICT_H2O && policy != PIKV_EVICT_LRU && policy != PIKV_EVICT_ALL) return PIKV_ERR_UNSUPPORTED;
+  if (policy == PIKV_EVICT_H2O && !row_acc) return PIKV_ERR_NULL;
+  if (n_caches < 1 || n_caches > 65535 || max_len < 0 || count_all < 0) return PIKV_ERR_SHAPE;
+  hipStream_t st = (hipStream_t)stream;
+  CompactPlanes pl;
+  int rc = make_planes(plane_ptrs_host, plane_row_bytes_host, n_planes, pl);
+  if (rc != PIKV_OK) return rc;
+  RoomArgs a{policy, count, count_all, per_call_limit, heavy_ratio, recent_ratio, leave_room, append, row_acc, row_ts,
+             cache_row_base, cache_fill, cache_cap, keep_index, new_len, budgets, budgets + n_caches,
+             budgets + 2 * (int64_t)n_caches, n_caches};
+  if (policy == PIKV_EVICT_ALL || max_len <= kRoomMaxLen) {
+    // the block that selects a cache also moves its survivors while those are at most a megabyte
+    int64_t row = 0;
+    for (int p = 0; p < n_planes; ++p) row += pl.row_bytes[p];
+    double kept = (double)max_len;
+    if (policy == PIKV_EVICT_H2O) kept *= heavy_ratio + recent_ratio < 1.0 ? heavy_ratio + recent_ratio : 1.0;
+    const bool here = policy == PIKV_EVICT_ALL || kept * (double)row <= (double)(1 << 20);
+    CompactPlanes none{};
+    hipLaunchKernelGGL(room_small_kernel, dim3((unsigned)n_caches), dim3(kSelThreads), 0, st, a, here ? pl : none);
+    if (!here) launch_compact(pl, cache_row_base, keep_index, new_len, a.active, n_caches, st);
+    PIKV_CHECK_LAUNCH();
+    return PIKV_OK;
+  }
+  const dim3 cgrid((unsigned)((n_caches + 63) / 64));
+  hipLaunchKernelGGL(room_budget_kernel, cgrid, dim3(64), 0, st, a);
+  rc = pikv_evict_select(policy, row_acc, row_ts, cache_row_base, cache_fill, a.n_heavy, a.n_recent, n_caches, max_len,
+                         keep_flag, keep_index, new_len, workspace, workspace_bytes, stream);
+  if (rc != PIKV_OK) return rc;
+  launch_compact(pl, cache_row_base, keep_index, new_len, a.active, n_caches, st);
+  hipLaunchKernelGGL(room_fill_kernel, cgrid, dim3(64), 0, st, a);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
 }

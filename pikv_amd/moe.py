@@ -125,7 +125,7 @@ class KVCache(nn.Module):
         # this cache takes n rows, the other caches of a shared pool none: they keep every row
         n_new = torch.zeros(pool.n_caches, dtype=torch.int32, device=dev)
         n_new[self.index] = min(n, self.size)
-        _evict_for(pool, n_new, self._policy())
+        pool.make_room(self._policy(), count=n_new)
         self._time = max(self._time + 1, int(idx) + 1)
         pool.quant_scatter(k2, v2, torch.full((n,), self.index, dtype=torch.int32, device=dev),
                            torch.arange(n, dtype=torch.int32, device=dev), 1, now=float(self._time))
@@ -156,24 +156,6 @@ class KVCache(nn.Module):
 
     def change_scheduling_policy(self, new_policy: SchedulingPolicy):
         self.scheduling_policy = new_policy
-
-
-def _evict_for(pool: ops.CachePool, n_new: torch.Tensor, policy: int, heavy_ratio=0.1,
-               recent_ratio=0.1):
-    """Make room for n_new[c] rows in every cache (core/single/cache_scheduling.py:
-    404-427): caches that would overflow evict first - the fill+n_new-cap least
-    recently used rows, or everything outside H2O's heavy and recent sets - and are
-    compacted in place; the others keep all their rows.  No host synchronisation."""
-    over = (pool.fill + n_new - pool.cap).clamp_min(0)
-    if policy == ops.EVICT_LRU:
-        pool.evict(ops.EVICT_LRU, n_evict=torch.minimum(over, pool.fill).to(torch.int32))
-        return
-    f = pool.fill.double()
-    nh = (f * heavy_ratio).floor().clamp_min(1).to(torch.int32)
-    nr = (f * recent_ratio).floor().clamp_min(1).to(torch.int32)
-    keep_all = over == 0
-    pool.evict(ops.EVICT_H2O, n_heavy=torch.where(keep_all, pool.fill, nh).contiguous(),
-               n_recent=torch.where(keep_all, torch.zeros_like(nr), nr).contiguous())
 
 
 class PiKVMoE(nn.Module):
@@ -288,14 +270,16 @@ class PiKVMoE(nn.Module):
             capacity = int(B * S * config.get('capacity_factor', 1.5) * k / E)
             slot, count = ops.capacity_slots(idx32, E, capacity)
             values = stacked[idx32.long(), tok].contiguous()
-            n_new = torch.minimum(torch.minimum(count, torch.full_like(count, capacity)), pool.cap)
             policy = (ops.EVICT_H2O if self.use_cache_scheduling and
                       self.cache_scheduling_policy == SchedulingPolicy.H2O else ops.EVICT_LRU)
-            _evict_for(pool, n_new, policy)
+            # caches that the kept assignments would overflow evict first (core/single/cache_scheduling.py:
+            # 404-427), the others keep all their rows
+            pool.make_room(policy, count=count, limit=capacity)
             self.clock += 1
             if self.debug_capture:
                 self.captured = dict(keys=keys, values=values, idx=idx32.view(T, k), slot=slot.view(T, k),
-                                     count=count, capacity=capacity, n_new=n_new, cached=cached,
+                                     count=count, capacity=capacity, cached=cached,
+                                     n_new=count.clamp_max(capacity).minimum(pool.cap),
                                      fill_before=pool.fill.clone(), routing_weights=routing_weights,
                                      top_k_weights=top_k_weights, importance=importance)
             pool.quant_scatter(keys, values, idx32, slot, 1, now=float(self.clock))

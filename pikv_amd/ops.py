@@ -22,7 +22,7 @@ from typing import Optional, Sequence
 import torch
 
 from . import _native as N
-from ._native import (BF16, EVICT_H2O, EVICT_LRU, F32, Q_I4_ASYM, Q_I4_SYM,
+from ._native import (BF16, EVICT_ALL, EVICT_H2O, EVICT_LRU, F32, Q_I4_ASYM, Q_I4_SYM,
                       Q_I8_ASYM, Q_I8_SYM, SCORE_TILE)
 
 __all__ = [
@@ -446,6 +446,7 @@ class CachePool:
         self.new_len = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
         self.n_heavy = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
         self.n_recent = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
+        self._budgets = torch.empty(3 * self.n_caches, dtype=torch.int32, device=dev)
 
     # ---- checkpoint ----
     _STATE_PLANES = ("k_codes", "k_scale", "k_zero", "v_codes", "v_scale", "v_zero", "acc", "ts")
@@ -752,6 +753,49 @@ class CachePool:
         rbs = (C.c_int64 * len(ps))(*[math.prod(p.shape[1:]) * p.element_size() for p in ps])
         N.call("pikv_compact_rows", ptrs, rbs, len(ps), _ptr(self.row_base), _ptr(self.keep_index),
                _ptr(self.new_len), _ptr(self.fill), self.n_caches, _stream())
+
+    def make_room(self, policy: int, *, count: Optional[torch.Tensor] = None, count_all: int = 0,
+                  limit: int = -1, heavy_ratio: float = 0.1, recent_ratio: float = 0.1,
+                  leave_room: bool = False, append: bool = False):
+        """Caches that min(count[c] or count_all, limit, cap[c]) new rows would overflow evict by
+        `policy` (EVICT_H2O, EVICT_LRU, EVICT_ALL) and are compacted; the others keep their rows.
+        new_len = the rows kept; fill = new_len, or the fill after the new rows with append=True
+        (for an append_rows call that follows)."""
+        if count is not None:
+            count = _need(count, "count", dtype=torch.int32, ndim=1)
+            if count.numel() != self.n_caches:
+                raise ValueError("count must have one entry per cache")
+        if policy not in (EVICT_H2O, EVICT_LRU, EVICT_ALL):
+            raise ValueError(f"unknown eviction policy {policy}")
+        ps = self.planes()
+        ptrs = (C.c_void_p * len(ps))(*[p.data_ptr() for p in ps])
+        rbs = (C.c_int64 * len(ps))(*[math.prod(p.shape[1:]) * p.element_size() for p in ps])
+        if getattr(self, "_evict_ws", None) is None:
+            self._evict_ws = _evict_workspace(self.n_caches, self.max_cap, self.device)
+        ws, ws_bytes = self._evict_ws
+        N.call("pikv_cache_make_room", policy, _ptr(count), int(count_all), int(limit), float(heavy_ratio),
+               float(recent_ratio), int(leave_room), int(append), _ptr(self.acc), _ptr(self.ts), _ptr(self.row_base),
+               _ptr(self.fill), _ptr(self.cap), self.n_caches, self.max_cap, ptrs, rbs, len(ps), _ptr(self.keep_flag),
+               _ptr(self.keep_index), _ptr(self.new_len), _ptr(self._budgets), _ptr(ws), ws_bytes, _stream())
+
+    def append_rows(self, k_src, v_src, now: float = 0.0):
+        """Quantise k_src / v_src [n_caches * rows, D] (cache-major) behind the new_len rows of every
+        cache, as make_room(append=True) has left them; rows past the capacity are dropped."""
+        k_src = _need(k_src, "k_src")
+        dt = _dt(k_src, "k_src")
+        rows = k_src.numel() // (self.D * self.n_caches)
+        if k_src.numel() != rows * self.D * self.n_caches:
+            raise ValueError("k_src must hold the same number of rows for every cache")
+        if self.with_v:
+            v_src = _need(v_src, "v_src", dtype=k_src.dtype)
+            if v_src.numel() != k_src.numel():
+                raise ValueError("v_src must match k_src")
+        if rows == 0:
+            return
+        N.call("pikv_quant_append", _ptr(k_src), _ptr(v_src) if self.with_v else None, dt, rows, self.D, self.group,
+               self.scheme, _ptr(self.row_base), _ptr(self.new_len), _ptr(self.cap), self.n_caches,
+               _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero),
+               _ptr(self.v_zero), _ptr(self.acc), _ptr(self.ts), float(now), _stream())
 
     def evict(self, policy: int, **kw):
         self.evict_select(policy, **kw)

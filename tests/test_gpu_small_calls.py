@@ -56,3 +56,57 @@ def test_decode_attend_few_ranges(dev, scheme, qdtype, length):
         rms = np.sqrt((want[c].astype(np.float64) ** 2).mean()) + 1e-12
         assert np.abs(out[c] - want[c]).max() <= 1e-3 * rms
     np.testing.assert_allclose(np_of(pool.acc), acc, rtol=1e-3, atol=1e-5)
+
+
+@pytest.mark.parametrize("policy", ["h2o", "h2o_leave_room", "lru", "all"])
+@pytest.mark.parametrize("caps,D,heavy,recent", [
+    ([128, 118, 1, 90], 64, 0.1, 0.1),          # selected and compacted by one block per cache
+    ([1024, 1500, 1025], 2048, 0.5, 0.3),       # selected by one block, more than a megabyte of survivors
+    ([8192, 8000], 32, 0.06, 0.01),             # the longest caches of the one-block form
+    ([9000, 5000], 32, 0.1, 0.05),              # several blocks per cache
+])
+def test_make_room_and_append(dev, policy, caps, D, heavy, recent):
+    """make_room(append=True) + append_rows: survivors of every overflowing cache and their order against the
+    restatement's selections, exact; caches with the space keep every row; then the new rows behind them."""
+    import torch
+    from pikv_amd import ops
+    r = rng(len(caps) + D)
+    n_add = 7
+    fills = [max(1, c - (3 if i % 2 == 0 else 40)) for i, c in enumerate(caps)]   # every other cache overflows
+    pool = ops.CachePool(caps, 1, D, min(D, 1024), ops.Q_I8_SYM, dev)
+    pool.k_codes.random_(-127, 127), pool.v_codes.random_(-127, 127)
+    acc = np.round(r.random(pool.rows) * 50).astype(np.float32)                   # many ties
+    ts = r.permutation(pool.rows).astype(np.float32)
+    pool.acc.copy_(to_dev(acc, dev)), pool.ts.copy_(to_dev(ts, dev))
+    pool.fill.copy_(to_dev(np.array(fills, np.int32), dev))
+    before_k, before_v = np_of(pool.k_codes), np_of(pool.v_codes)
+    code = {"lru": ops.EVICT_LRU, "all": ops.EVICT_ALL}.get(policy, ops.EVICT_H2O)
+    pool.make_room(code, count_all=n_add, heavy_ratio=heavy, recent_ratio=recent, leave_room=policy == "h2o_leave_room",
+                   append=True)
+    kn, vn = r.standard_normal((len(caps) * n_add, D)).astype(np.float32), r.standard_normal((len(caps) * n_add, D)).astype(np.float32)
+    pool.append_rows(to_dev(kn, dev), to_dev(vn, dev), now=9.0)
+    k, v, acc2, ts2 = (np_of(t) for t in (pool.k_codes, pool.v_codes, pool.acc, pool.ts))
+    new_codes = O.quantize_groups(kn, min(D, 1024), O.Q_I8_SYM)[0]
+    for c, (cap, L) in enumerate(zip(caps, fills)):
+        base, n = int(pool.row_base[c]), min(n_add, cap)
+        over = L + n - cap
+        a, t = acc[base:base + L], ts[base:base + L]
+        keep = np.ones(L, bool)
+        if over > 0 and policy == "lru":
+            keep = O.lru_keep(t, min(over, L))
+        elif over > 0 and policy == "all":
+            keep[:] = False
+        elif over > 0:
+            nh, nr = O.h2o_budget(L, heavy, recent)
+            if policy == "h2o_leave_room":
+                nh = min(nh, cap - n)
+                nr = min(nr, cap - n - nh)
+            keep = O.h2o_keep(a, t, nh, nr)
+        rows = base + np.nonzero(keep)[0]
+        m = len(rows)
+        assert int(pool.new_len[c]) == m and int(pool.fill[c]) == min(m + n, cap), c
+        assert np.array_equal(k[base:base + m], before_k[rows]) and np.array_equal(v[base:base + m], before_v[rows]), c
+        assert np.array_equal(acc2[base:base + m], acc[rows]) and np.array_equal(ts2[base:base + m], ts[rows]), c
+        w = min(n_add, cap - m)
+        assert np.array_equal(k[base + m:base + m + w].astype(np.int16), new_codes[c * n_add:c * n_add + w]), c
+        assert (ts2[base + m:base + m + w] == 9.0).all() and (acc2[base + m:base + m + w] == 0.0).all()
