@@ -447,6 +447,27 @@ int pikv_decode_attend(const void* k_codes, const void* k_scale, const void* k_z
 int64_t pikv_decode_attend_workspace_bytes(int n_caches, int n_q_heads, int head_dim,
                                            int64_t max_len);
 
+/* Attention of a prompt chunk, in float32: the chunk's queries over the cached rows of their
+ * sequence (dequantised on the way) followed by the chunk's own, exact rows.
+ * Replaces: PiKVAttention's dense attention over [past ; current]
+ *   (core/single/pikv_attention.py:104-191, :240-244) where no mask, dropout or gradient is
+ *   asked for.
+ *   q [n_seqs][S][n_q_heads][head_dim], k / v [n_seqs][S][n_kv_heads][head_dim], out as q, all
+ *   float and contiguous; head_dim 64 or 128; sequence b attends to cache b's
+ *   min(cache_fill[b], max_cached) rows (k_codes == NULL: no cached rows) and to the own rows
+ *   0 .. i of query i (all S with causal == 0).
+ *   workspace: pikv_prefill_attend_workspace_bytes(...) bytes (0 for most shapes), 256-byte
+ *   aligned. */
+int pikv_prefill_attend(const float* q, const float* k, const float* v, int n_seqs, int S,
+                        int n_kv_heads, int n_q_heads, int head_dim, int causal, float scale_qk,
+                        const void* k_codes, const void* k_scale, const void* k_zero,
+                        const void* v_codes, const void* v_scale, const void* v_zero,
+                        int scheme, int group, const int64_t* cache_row_base,
+                        const int32_t* cache_fill, int64_t max_cached, float* out,
+                        void* workspace, int64_t workspace_bytes, void* stream);
+int64_t pikv_prefill_attend_workspace_bytes(int n_seqs, int S, int n_kv_heads, int n_q_heads,
+                                            int head_dim, int64_t max_cached);
+
 /* ------------------------------------------------------------------------
  * K4  eviction top-k + stable in-place compaction
  * Replaces: H2OScheduler.select_eviction_candidates

@@ -13,9 +13,10 @@ context natively:
     context  = pikv_attend_values           (probabilities x compressed V rows, :188; the same
                                              pass adds the probabilities to the H2O importance)
 
-Multi-token or masked calls compute their attention in torch as the reference does, over
-the dequantised cached rows followed by their own K/V (the reference concatenates
-`past_key_values` and the current K/V, :240-244), and write their K/V rows into the cache.  When a cache would overflow, the
+Multi-token or masked calls attend to the dequantised cached rows followed by their own K/V (the
+reference concatenates `past_key_values` and the current K/V, :240-244), in one native kernel
+(ops.prefill_attend) where they need no mask, dropout or gradient and in torch as the reference
+does otherwise, and write their K/V rows into the cache.  When a cache would overflow, the
 reference wipes it (:85-90); here H2O eviction keeps the heavy and the recent rows
 (`on_overflow="reset"` restores the wipe).
 
@@ -239,6 +240,20 @@ class PiKVAttention(nn.Module):
         return pool.decode_attend(qq.contiguous(), self.num_heads, now=float(self.clock),
                                   scale_qk=1.0 / math.sqrt(self.head_dim))
 
+    def _native_prefill(self, q, k, v, attention_mask) -> bool:
+        """Whether a chunk goes through ops.prefill_attend: float32 without a mask, dropout or gradient, and a head
+        width that kernel has.  Everything else keeps the torch path below, whose score matrix, masks and copies
+        of the cached rows cost more than the products: 2 x 500 tokens x 16 heads over 500 cached rows."""
+        if attention_mask is not None or self.head_dim not in (64, 128) or not q.is_cuda:
+            return False
+        if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+            return False
+        if not (q.dtype == k.dtype == v.dtype == torch.float32):
+            return False
+        if type(self.attn_dropout) is not nn.Dropout or (self.attn_dropout.training and self.attn_dropout.p > 0):
+            return False
+        return q.shape[1] > 0 and q.shape[0] * self.num_kv_heads <= 65535
+
     def _dense_attention(self, q, k, v, attention_mask, causal_mask, past=None):
         """core/single/pikv_attention.py:104-191 over [cached rows ; rows of this call]
         (:240-244 concatenates past and current K/V along the sequence axis)."""
@@ -284,8 +299,9 @@ class PiKVAttention(nn.Module):
                 stream_position: Optional[int] = None):
         """The context of a call is everything cached (after `past_key_values`, if given, has
         replaced the caches' contents) followed by the call's own tokens.  A single new token
-        without a mask takes the native read path over the compressed rows; any other call
-        attends in torch over the dequantised cached rows plus its own exact K/V.  Call
+        without a mask takes the native read path over the compressed rows.  Any other call
+        attends to the dequantised cached rows plus its own exact K/V: in one kernel where it
+        needs no mask, dropout or gradient (_native_prefill), in torch otherwise.  Call
         reset_cache() to start a new sequence."""
         B, S, _ = hidden_states.shape
         q = self.q_proj(hidden_states).view(B, S, self.num_heads, self.head_dim)
@@ -303,10 +319,16 @@ class PiKVAttention(nn.Module):
                 self._update_cache(k.detach(), v.detach())
             context = self._decode_attention(q[:, 0]).unsqueeze(1)  # over everything cached
         else:
-            with torch.no_grad():
-                past = self._cached_rows()                          # before this call's rows go in
-                self._update_cache(k.detach(), v.detach())
-            context = self._dense_attention(q, k, v, attention_mask, causal_mask, past)
+            if self._native_prefill(q, k, v, attention_mask):
+                pool = self.pool if self.pool is not None and self.pool.n_caches == B else None
+                context = ops.prefill_attend(q.contiguous(), k.contiguous(), v.contiguous(), pool, causal_mask)
+                with torch.no_grad():
+                    self._update_cache(k.detach(), v.detach())
+            else:
+                with torch.no_grad():
+                    past = self._cached_rows()                      # before this call's rows go in
+                    self._update_cache(k.detach(), v.detach())
+                context = self._dense_attention(q, k, v, attention_mask, causal_mask, past)
         output = self.o_proj(context.reshape(B, S, self.num_heads * self.head_dim).to(hidden_states.dtype))
         # `present` in the module's past_layout: [B,S,kv_heads,head_dim] as the reference returns it
         # (core/single/pikv_attention.py:240-247), or [B,kv_heads,S,head_dim] for past_layout="hf"

@@ -27,7 +27,7 @@ from ._native import (BF16, EVICT_ALL, EVICT_H2O, EVICT_LRU, F32, Q_I4_ASYM, Q_I
 
 __all__ = [
     "router_fused", "router_tail", "capacity_slots", "quantize_rows", "quant8_minshift",
-    "dequantize_rows", "fakequant_colblocks", "fakequant_preset", "CachePool", "scheme_bits",
+    "dequantize_rows", "prefill_attend", "fakequant_colblocks", "fakequant_preset", "CachePool", "scheme_bits",
     "Q_I8_SYM", "Q_I8_ASYM", "Q_I4_ASYM", "Q_I4_SYM", "EVICT_H2O", "EVICT_LRU",
 ]
 
@@ -396,6 +396,40 @@ def select_top_rows(score, seg_base, seg_len, n_keep, max_len: Optional[int] = N
            _ptr(n_keep), _ptr(zero), n, int(max_len), _ptr(flag), _ptr(index), _ptr(kept), _ptr(ws),
            ws_bytes, _stream())
     return flag, index, kept
+
+
+def prefill_attend(q, k, v, pool: Optional["CachePool"] = None, causal: bool = True,
+                   scale_qk: Optional[float] = None):
+    """softmax(q.k) v of a prompt chunk in float32: q [B, S, n_q_heads, head_dim] over the rows that
+    cache b of `pool` holds (None: nothing cached) and the chunk's own k, v [B, S, n_kv_heads,
+    head_dim], query i seeing own rows 0..i (all of them with causal=False).  head_dim 64 or 128.
+    Returns out like q."""
+    q = _need(q, "q", dtype=torch.float32, ndim=4)
+    k = _need(k, "k", dtype=torch.float32, ndim=4)
+    v = _need(v, "v", dtype=torch.float32, ndim=4)
+    B, S, hq, dh = q.shape
+    hkv = k.shape[2]
+    if k.shape != (B, S, hkv, dh) or v.shape != k.shape:
+        raise ValueError(f"k and v must be [{B}, {S}, kv_heads, {dh}], got {tuple(k.shape)} and {tuple(v.shape)}")
+    if hkv == 0 or hq % hkv:
+        raise ValueError("the query heads must be a multiple of the kv heads")
+    if dh not in (64, 128):
+        raise ValueError(f"head_dim must be 64 or 128, got {dh}")
+    if pool is not None and (pool.n_caches != B or pool.n_heads != hkv or pool.head_dim != dh or not pool.with_v):
+        raise ValueError("the pool's caches do not match k and v")
+    out = torch.empty_like(q)
+    if out.numel() == 0:
+        return out
+    max_cached = pool.max_cap if pool is not None and pool.rows > 0 else 0
+    planes = [None] * 6 if max_cached == 0 else [_ptr(p) for p in (*pool._planes("k"), *pool._planes("v"))]
+    nb = int(N.lib().pikv_prefill_attend_workspace_bytes(B, S, hkv, hq, dh, max_cached))
+    ws = torch.empty(nb, dtype=torch.uint8, device=q.device) if nb else None
+    N.call("pikv_prefill_attend", _ptr(q), _ptr(k), _ptr(v), B, S, hkv, hq, dh, int(bool(causal)),
+           float(1.0 / math.sqrt(dh) if scale_qk is None else scale_qk), *planes,
+           pool.scheme if max_cached else Q_I8_SYM, pool.group if max_cached else 0,
+           _ptr(pool.row_base) if max_cached else None, _ptr(pool.fill) if max_cached else None, max_cached,
+           _ptr(out), _ptr(ws), nb, _stream())
+    return out
 
 
 class CachePool:

@@ -110,3 +110,39 @@ def test_make_room_and_append(dev, policy, caps, D, heavy, recent):
         w = min(n_add, cap - m)
         assert np.array_equal(k[base + m:base + m + w].astype(np.int16), new_codes[c * n_add:c * n_add + w]), c
         assert (ts2[base + m:base + m + w] == 9.0).all() and (acc2[base + m:base + m + w] == 0.0).all()
+
+
+@pytest.mark.parametrize("scheme,heads,hq,dh,group", [
+    (O.Q_I8_SYM, 2, 4, 128, 128), (O.Q_I8_ASYM, 4, 4, 64, 32), (O.Q_I4_ASYM, 2, 6, 64, 32), (O.Q_I4_SYM, 1, 7, 128, 64)])
+@pytest.mark.parametrize("S,lens", [(1, [5]), (2, [0, 33]), (31, [1, 64]), (33, None), (70, [32, 300]), (5, [1500])])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_attend(dev, scheme, heads, hq, dh, group, S, lens, causal):
+    """Chunks around the 32-row and 32-key tiles, over no cached rows, a few, and enough for several blocks a row,
+    against float64.  Bound: a score is a float32 sum of d products, off by some 2^-24 sqrt(d) of the largest score
+    (the cached rows have channels 20 times the others), which is the relative error of its probability; the output
+    averages n values by them.  4 * 2^-24 * sqrt(d + n) * (1 + largest score) of the largest value covers both."""
+    from pikv_amd import ops
+    r = rng(S * 131 + dh + hq)
+    B = 2 if lens is None else len(lens)
+    D = heads * dh
+    q, k, v = (r.standard_normal((B, S, h, dh)).astype(np.float32) for h in (hq, heads, heads))
+    pool = ref = None
+    if lens is not None:
+        pool, ref = _fill_pool(dev, r, [max(lens) + 3] * B, lens, heads, dh, group, scheme)
+    got = np_of(ops.prefill_attend(*(to_dev(t, dev, "f32") for t in (q, k, v)), pool, causal)).astype(np.float64)
+    for b in range(B):
+        n = 0 if lens is None else lens[b]
+        kk, vv = k[b].astype(np.float64), v[b].astype(np.float64)
+        if n:
+            rows = ref.valid_rows(b)[:n]
+            past = [O.dequantize_groups(c[rows], s[rows], z[rows], group).reshape(n, heads, dh)
+                    for c, s, z in ((ref.k_codes, ref.k_scale, ref.k_zero), (ref.v_codes, ref.v_scale, ref.v_zero))]
+            kk, vv = np.concatenate([past[0], kk]), np.concatenate([past[1], vv])
+        for h in range(hq):
+            s = q[b, :, h].astype(np.float64) @ kk[:, h // (hq // heads)].T / np.sqrt(dh)
+            size = (1.0 + np.abs(s).max()) * np.abs(vv).max()
+            if causal:
+                s[np.arange(n + S)[None, :] > n + np.arange(S)[:, None]] = -np.inf
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            want = (p / p.sum(axis=1, keepdims=True)) @ vv[:, h // (hq // heads)]
+            assert np.abs(got[b, :, h] - want).max() <= 4 * 2.0 ** -24 * np.sqrt(dh + n + S) * size
