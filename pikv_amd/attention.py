@@ -252,7 +252,7 @@ class PiKVAttention(nn.Module):
             return False
         if type(self.attn_dropout) is not nn.Dropout or (self.attn_dropout.training and self.attn_dropout.p > 0):
             return False
-        return q.shape[1] > 0 and q.shape[0] * self.num_kv_heads <= 65535
+        return 0 < q.shape[1] * (self.num_heads // self.num_kv_heads) <= 65535 * 32
 
     def _dense_attention(self, q, k, v, attention_mask, causal_mask, past=None):
         """core/single/pikv_attention.py:104-191 over [cached rows ; rows of this call]
