@@ -546,6 +546,69 @@ int pikv_cache_make_room(int policy, const int32_t* count, int64_t count_all, in
                          void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
+ * Mixture-of-experts layer (core/single/pikv_moe.py:139-336), float32.
+ * ---------------------------------------------------------------------- */
+
+/* Linear layers over one input, in one launch (a second one before it where a layer has LoRA):
+ *   out[g][t][n] = act(x[t] . w[g][n] + bias[g][n] + ((x[t] lora_a[g]) lora_b[g])[n] * scaling[g])
+ *                  + add[g][n]
+ *   x [T][K]; host arrays of n_layers (at most 20) entries: w [n_out][K], bias [n_out],
+ *   lora_a [K][rank] / lora_b [rank][n_out] (rank at most 8; rank 0, NULL array or entry: none),
+ *   add [n_out] (NULL array or entry: none), relu (0 / 1), out [T][n_out].  K a multiple of 128,
+ *   n_out of 32; x and w 16-byte aligned.  Other sizes: PIKV_ERR_UNSUPPORTED.
+ *   workspace: pikv_linear_group_workspace_bytes(...) bytes, needed only with LoRA. */
+int pikv_linear_group(const float* x, int64_t T, int K, int n_layers, const float* const* w,
+                      const float* const* bias, const int32_t* n_out, const int32_t* relu, int rank,
+                      const float* const* lora_a, const float* const* lora_b, const float* scaling,
+                      const float* const* add, float* const* out, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+int64_t pikv_linear_group_workspace_bytes(int64_t T, int n_layers, int rank);
+
+/* out [n_caches][D] = mean of every cache's dequantised rows (zero for an empty cache).
+ * max_len >= max_c cache_fill[c]; workspace: pikv_cache_mean_workspace_bytes(...) bytes. */
+int pikv_cache_mean(const void* codes, const void* scale, const void* zero, int scheme, int group,
+                    int D, const int64_t* cache_row_base, const int32_t* cache_fill, int n_caches,
+                    int64_t max_len, float* out, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t pikv_cache_mean_workspace_bytes(int n_caches, int D, int64_t max_len);
+
+/* out[e] = mean[e] + ((mean[e] lora_a[e]) lora_b[e]) * scaling[e], mean and out [n_experts][H],
+ * host arrays of n_experts (at most 20) entries, lora_a [H][rank], lora_b [rank][H], rank at most 8. */
+int pikv_value_lora(const float* mean, int n_experts, int H, int rank, const float* const* lora_a,
+                    const float* const* lora_b, const float* scaling, float* out, void* stream);
+
+/* mix[t] = sum over e, in order, of outs[e][t] * weights[t][e]; outs [E][T][H], weights [T][E]. */
+int pikv_expert_mix(const float* outs, const float* weights, int64_t T, int E, int H, float* mix,
+                    void* stream);
+
+/* AdaptiveRouter (core/single/routing_strategy.py:100-150) behind its hidden layers, T = n_seqs * S:
+ *   blend [n_seqs][2] = softmax(relu(x_mean sel_w1^T + sel_b1) sel_w2^T + sel_b2)
+ *   lb_probs [T][E]   = softmax((h_lb w_lb^T + b_lb) / temp_lb + mask), the other router likewise,
+ *                       times importance [T] = sigmoid(h_pred w_pred + b_pred) and renormalised
+ *   weights [T][E]    = blend of the two; topk_idx / topk_w [T][top_k] their largest, renormalised
+ *                       (ties to the lower expert, NaN last)
+ *   balance_loss [1]  = balance_weight * std / mean of the experts' mean lb_probs
+ *   h_lb, h_imp [T][H], h_pred [T][H2] hold the hidden layers after ReLU; mask [E] or NULL. */
+int pikv_adaptive_router(const float* x_mean, int n_seqs, int S, int H, int H2, int E, int top_k,
+                         const float* sel_w1, const float* sel_b1, const float* sel_w2, const float* sel_b2,
+                         const float* h_lb, const float* w_lb, const float* b_lb, float temp_lb,
+                         const float* h_imp, const float* w_imp, const float* b_imp, float temp_imp,
+                         const float* h_pred, const float* w_pred, const float* b_pred, const float* mask,
+                         float balance_weight, float* blend, float* lb_probs, float* weights,
+                         int64_t* topk_idx, float* topk_w, float* importance, float* balance_loss,
+                         void* stream);
+
+/* pikv_quant_scatter for rows that differ per cache: token t's per_token assignments
+ * (cache_id / slot [n_tokens * per_token]) take its K row k_src[t] and the V row
+ * v_src[cache_id][t] of k_src [n_tokens][D], v_src [n_caches][n_tokens][D], float.
+ * Replaces: the repeated keys and gathered expert outputs of core/single/pikv_moe.py:249-336. */
+int pikv_quant_scatter_routed(const float* k_src, const float* v_src, int64_t n_tokens, int per_token,
+                              int D, int group, int scheme, const int32_t* cache_id, const int32_t* slot,
+                              const int64_t* cache_row_base, const int32_t* cache_fill,
+                              const int32_t* cache_cap, int n_caches, void* k_codes, void* v_codes,
+                              void* k_scale, void* v_scale, void* k_zero, void* v_zero, float* row_acc,
+                              float* row_ts, float now, void* stream);
+
+/* ------------------------------------------------------------------------
  * API-compatible fake quantisation of QuantizedCompressor.forward
  * Replaces: core/single/pikv_compression.py:474-506 - min/max over ALL rows
  *   of each block of `group` columns, asymmetric, output = dequantised floats.

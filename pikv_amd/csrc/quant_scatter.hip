@@ -47,6 +47,8 @@ struct QuantScatterArgs {
   int group;
   int n_tensors;        // 1 (K only) or 2 (K and V)
   int n_caches;
+  int src_div;          // routed mode: assignment s belongs to token s / src_div, its K row ...
+  int64_t v_rows;       //   and its V row is that token's of the slab of v_rows rows of its cache
   int lpr_shift;        // log2(lanes per row) or -1 when it is not a power of two
   int lpg_shift;        // log2(lanes per group)
 };
@@ -90,7 +92,8 @@ struct RawRow {
 // ROW_UNIFORM: lanes_per_row is a power of two >= 64, so a wavefront never spans two
 // source rows; the row index, its destinations and every address base are then
 // wave-uniform and live in scalar registers.
-template <int SCHEME, int SRC_DT, int FANOUT, bool ROW_UNIFORM>
+// ROUTED (FANOUT 1): a K row per token, a V row per token and cache, one assignment per s.
+template <int SCHEME, int SRC_DT, int FANOUT, bool ROW_UNIFORM, bool ROUTED = false>
 __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) {
   using Q = QScheme<SCHEME>;
   constexpr int EPL = Q::epl;
@@ -117,6 +120,11 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) 
   }
   bool valid = s < a.n_src;
   int64_t srow = s;  // row of src[] this lane reads
+  int64_t vrow = s;
+  if constexpr (ROUTED) {
+    srow = s / a.src_div;
+    vrow = valid ? (int64_t)a.cache_id[s] * a.v_rows + srow : 0;   // not read where the id is outside the pool
+  }
   int64_t gather_dst = -1;
   if (a.seg_index != nullptr) {
     const int c = blockIdx.y;
@@ -181,7 +189,7 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) 
     // The V row is fetched only now: holding both raw rows across the K arithmetic cost
     // the registers of one to two resident wavefronts per SIMD (4-bit: 86 -> 68 registers,
     // 150 -> 125 us at 131072 rows x 1024), and the other wavefronts cover the wait.
-    if (t == 1 && live) raw[1].load(a.src[1], srow * a.D + (int64_t)part * EPL);
+    if (t == 1 && live) raw[1].load(a.src[1], (ROUTED ? vrow : srow) * a.D + (int64_t)part * EPL);
     float x[EPL];
     raw[t].to_float(x);
     float mn = x[0], mx = x[0];
@@ -257,6 +265,28 @@ static int launch_quant(QuantScatterArgs a, int src_dtype, hipStream_t st) {
   return PIKV_OK;
 }
 
+template <int SCHEME>
+static int launch_routed(QuantScatterArgs a, hipStream_t st) {
+  using Q = QScheme<SCHEME>;
+  const int lanes_per_row = a.D / Q::epl;
+  a.lpr_shift = -1;
+  if (is_pow2(lanes_per_row)) {
+    a.lpr_shift = 0;
+    while ((1 << a.lpr_shift) < lanes_per_row) ++a.lpr_shift;
+  }
+  a.lpg_shift = 0;
+  while ((Q::epl << a.lpg_shift) < a.group) ++a.lpg_shift;
+  const int64_t blocks = (a.n_src * lanes_per_row + 255) / 256;
+  if (blocks == 0) return PIKV_OK;
+  if (blocks > 0x7fffffffLL) return PIKV_ERR_SHAPE;
+  if (a.lpr_shift >= 6)
+    hipLaunchKernelGGL((quant_scatter_kernel<SCHEME, PIKV_F32, 1, true, true>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((quant_scatter_kernel<SCHEME, PIKV_F32, 1, false, true>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+  PIKV_CHECK_LAUNCH();
+  return PIKV_OK;
+}
+
 static int check_quant_shape(int D, int group, int scheme) {
   if (scheme < 0 || scheme > 3) return PIKV_ERR_UNSUPPORTED;
   const bool eight = (scheme == PIKV_Q_I8_SYM || scheme == PIKV_Q_I8_ASYM);
@@ -321,6 +351,41 @@ extern "C" int pikv_quant_scatter(const void* k_src, const void* v_src, int src_
   a.n_tensors = v_src ? 2 : 1;
   a.n_caches = n_caches;
   return dispatch_quant(a, scheme, src_dtype, (hipStream_t)stream);
+}
+
+extern "C" int pikv_quant_scatter_routed(const float* k_src, const float* v_src, int64_t n_tokens, int per_token, int D,
+                                         int group, int scheme, const int32_t* cache_id, const int32_t* slot,
+                                         const int64_t* cache_row_base, const int32_t* cache_fill,
+                                         const int32_t* cache_cap, int n_caches, void* k_codes, void* v_codes,
+                                         void* k_scale, void* v_scale, void* k_zero, void* v_zero, float* row_acc,
+                                         float* row_ts, float now, void* stream) {
+  if (!k_src || !v_src || !k_codes || !k_scale || !v_codes || !v_scale || !cache_id || !slot || !cache_row_base ||
+      !cache_fill || !cache_cap)
+    return PIKV_ERR_NULL;
+  if (n_tokens < 1 || per_token < 1 || per_token > 64 || n_caches < 1) return PIKV_ERR_SHAPE;
+  int rc = check_quant_shape(D, group, scheme);
+  if (rc != PIKV_OK) return rc;
+  const bool asym = (scheme == PIKV_Q_I8_ASYM || scheme == PIKV_Q_I4_ASYM);
+  if (asym && (!k_zero || !v_zero)) return PIKV_ERR_NULL;
+  QuantScatterArgs a{};
+  a.src[0] = k_src; a.src[1] = v_src;
+  a.codes[0] = k_codes; a.codes[1] = v_codes;
+  a.scale[0] = k_scale; a.scale[1] = v_scale;
+  a.zero[0] = k_zero; a.zero[1] = v_zero;
+  a.cache_id = cache_id; a.slot = slot; a.row_base = cache_row_base;
+  a.fill = cache_fill; a.cap = cache_cap;
+  a.row_acc = row_acc; a.row_ts = row_ts; a.now = now;
+  a.n_src = n_tokens * per_token; a.fanout = 1; a.D = D; a.group = group;
+  a.src_div = per_token; a.v_rows = n_tokens;
+  a.n_tensors = 2;
+  a.n_caches = n_caches;
+  hipStream_t st = (hipStream_t)stream;
+  switch (scheme) {
+    case PIKV_Q_I8_SYM: return launch_routed<PIKV_Q_I8_SYM>(a, st);
+    case PIKV_Q_I8_ASYM: return launch_routed<PIKV_Q_I8_ASYM>(a, st);
+    case PIKV_Q_I4_ASYM: return launch_routed<PIKV_Q_I4_ASYM>(a, st);
+    default: return launch_routed<PIKV_Q_I4_SYM>(a, st);
+  }
 }
 
 extern "C" int pikv_quant_append(const void* k_src, const void* v_src, int src_dtype, int64_t rows_per_cache, int D,

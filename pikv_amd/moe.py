@@ -1,9 +1,9 @@
 """PiKVMoE and KVCache with the reference's interface (core/single/pikv_moe.py),
 their cache traffic routed through the HIP library.
 
-What stays in torch: the embedding, the dense experts (LoRAExpert,
-core/single/lora.py:31-52), the query/key projections and the vocabulary
-projection - dense GEMMs of the caller, not part of the cache data path.
+What stays in torch: the embedding, the query projection and the vocabulary projection, and
+with gradients the dense experts (LoRAExpert, core/single/lora.py:31-52) and the key projection;
+without gradients experts, key projection and their weighted sum are native too.
 
 The router is the reference's routing_strategy.AdaptiveRouter (routing_strategy.py in this
 package: same parameter names, a reference state_dict loads), and the expert outputs are
@@ -16,8 +16,9 @@ What runs natively, once per forward and for all experts together:
   * every softmax + top-k + renormalise of the router, and the capacity slots of its top-k;
   * eviction of the rows that have to make room (LRU by default, H2O on request)
     and in-place compaction of every per-expert cache;
+  * the means of the cached values that every expert adds to its output;
   * quantisation of the routed tokens' K/V rows and their scatter into the
-    per-expert caches;
+    per-expert caches, straight from the key rows and the stacked expert outputs;
   * with H2O scheduling, the scores of a per-expert query over the compressed
     cache and the importance accumulation that H2O selects on.
 
@@ -39,7 +40,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import dense, ops
 from .config import config
 from .routing_strategy import AdaptiveRouter
 from .scheduling import SchedulingPolicy
@@ -209,14 +210,48 @@ class PiKVMoE(nn.Module):
         return F.softmax(scores, dim=-1).sum(dim=1)
 
     def _cached_means(self, pool):
-        """Mean dequantised cached value of every expert, [E, H] (zeros when empty).  Plain
-        masked sums per cache: the result does not depend on scheduling."""
-        v = pool.gather_dequant("v")                                   # [rows, H]
-        means = []
-        for c, (b, cap) in enumerate(zip(pool.base_host, pool.caps_host)):
-            live = (torch.arange(cap, device=pool.device) < pool.fill[c]).unsqueeze(1)
-            means.append((v[b:b + cap] * live).sum(dim=0))
-        return torch.stack(means) / pool.fill.clamp_min(1).unsqueeze(1).float()
+        """Mean dequantised cached value of every expert, [E, H] (zeros when empty)."""
+        return pool.mean_rows("v")
+
+    def _lora_ok(self, m, rank, device):
+        H = config['hidden_size']
+        return (dense.plain(m, LoRALayer) and type(m.scaling) in (int, float) and m.lora_A.shape == (H, rank) and m.lora_B.shape == (rank, H)
+                and dense._ordinary_tensor(m.lora_A, device) and dense._ordinary_tensor(m.lora_B, device)
+                and dense.plain(m.dropout, nn.Dropout) and not (m.dropout.training and m.dropout.p > 0))
+
+    def _native_experts(self, x, routing_weights) -> bool:
+        """Whether the experts, the key projection and the weighted sum run in linear_group's one launch: a float32
+        forward without autograd over unmodified layers of widths the kernel has (128 tokens x 4 experts of
+        256 x 256: 33 us a library product, 13 launches an expert)."""
+        E, H = len(self.experts), x.shape[-1]
+        if not (dense.forward_only(x) and x.numel() > 0 and H % 128 == 0 and H == config['hidden_size']
+                and E == config['num_experts'] <= dense.MAX_LAYERS - 1 and len(self.kv_caches) == E):
+            return False
+        if not (dense._ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)
+                and x.shape[0] * x.shape[1] <= 65535 * 32):
+            return False
+        rank = self.key_lora.lora_A.shape[1]
+        if not (1 <= rank <= dense.MAX_LORA_RANK and self._lora_ok(self.key_lora, rank, x.device)
+                and dense.linear_ok(self.key_proj, H, H, x.device)):
+            return False
+        return all(dense.plain(e, LoRAExpert) and dense.linear_ok(e.dense, H, H, x.device)
+                   and self._lora_ok(e.lora, rank, x.device) and self._lora_ok(c.value_lora, rank, x.device)
+                   for e, c in zip(self.experts, self.kv_caches))
+
+    def _experts_forward(self, x2, cached, routing_weights):
+        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]) in five launches."""
+        T, H = x2.shape
+        E = len(self.experts)
+        lora = [c.value_lora for c in self.kv_caches]
+        add = ops.value_lora(cached, [m.lora_A for m in lora], [m.lora_B for m in lora], [m.scaling for m in lora])
+        outs = torch.empty(E, T, H, dtype=torch.float32, device=x2.device)
+        keys = torch.empty(T, H, dtype=torch.float32, device=x2.device)
+        layers = [dict(weight=e.dense.weight, bias=e.dense.bias, lora_a=e.lora.lora_A, lora_b=e.lora.lora_B,
+                       scaling=e.lora.scaling, relu=True, add=add[i], out=outs[i]) for i, e in enumerate(self.experts)]
+        layers.append(dict(weight=self.key_proj.weight, bias=self.key_proj.bias, lora_a=self.key_lora.lora_A,
+                           lora_b=self.key_lora.lora_B, scaling=self.key_lora.scaling, out=keys))
+        ops.linear_group(x2, layers, rank=self.key_lora.lora_A.shape[1])
+        return outs, keys, ops.expert_mix(outs, routing_weights.view(T, E))
 
     def update_cache(self, expert_idx, key, value, importance):
         """Update one expert's cache with new key / value rows (core/single/pikv_moe.py:249-261).
@@ -249,27 +284,31 @@ class PiKVMoE(nn.Module):
             importance = self.compute_token_importance(query.to(torch.float32), x)
 
         cached = self._cached_means(pool)                              # [E, H]
-        expert_output = torch.zeros(B, S, H, device=x.device)
-        outs = []
-        for i, expert in enumerate(self.experts):
-            c = cached[i] + self.kv_caches[i].value_lora(cached[i])
-            out_i = expert(x) + c.view(1, 1, H)
-            outs.append(out_i)
-            expert_output = expert_output + out_i * routing_weights[:, :, i].unsqueeze(-1)
+        x2 = x.reshape(T, H)
+        keys = None
+        if self._native_experts(x, routing_weights):
+            stacked, keys, expert_output = self._experts_forward(x2, cached, routing_weights)
+            expert_output = expert_output.view(B, S, H)
+        else:
+            expert_output = torch.zeros(B, S, H, device=x.device)
+            outs = []
+            for i, expert in enumerate(self.experts):
+                c = cached[i] + self.kv_caches[i].value_lora(cached[i])
+                out_i = expert(x) + c.view(1, 1, H)
+                outs.append(out_i)
+                expert_output = expert_output + out_i * routing_weights[:, :, i].unsqueeze(-1)
 
         # cache update: K = projected token, V = its expert's output, one row per assignment
         with torch.no_grad():
-            x2 = x.reshape(T, H)
-            keys = (self.key_proj(x2) + self.key_lora(x2)).repeat_interleave(k, dim=0).contiguous()
-            stacked = torch.stack([o.reshape(T, H) for o in outs])     # [E, T, H]
-            tok = torch.arange(T, device=x.device).repeat_interleave(k)
+            if keys is None:
+                keys = (self.key_proj(x2) + self.key_lora(x2)).contiguous()    # [T, H]
+                stacked = torch.stack([o.reshape(T, H) for o in outs])     # [E, T, H]
             # which token rows go to which expert's cache: the router's top-k, at most `capacity` per
             # expert and forward in token order (core/single/pikv_routing.py:40-42,
             # core/single/module/pikv_routing.py:93-104)
             idx32 = expert_indices.reshape(T * k).to(torch.int32).contiguous()
             capacity = int(B * S * config.get('capacity_factor', 1.5) * k / E)
             slot, count = ops.capacity_slots(idx32, E, capacity)
-            values = stacked[idx32.long(), tok].contiguous()
             policy = (ops.EVICT_H2O if self.use_cache_scheduling and
                       self.cache_scheduling_policy == SchedulingPolicy.H2O else ops.EVICT_LRU)
             # caches that the kept assignments would overflow evict first (core/single/cache_scheduling.py:
@@ -277,12 +316,13 @@ class PiKVMoE(nn.Module):
             pool.make_room(policy, count=count, limit=capacity)
             self.clock += 1
             if self.debug_capture:
-                self.captured = dict(keys=keys, values=values, idx=idx32.view(T, k), slot=slot.view(T, k),
+                tok = torch.arange(T, device=x.device).repeat_interleave(k)
+                self.captured = dict(keys=keys[tok], values=stacked[idx32.long(), tok], idx=idx32.view(T, k), slot=slot.view(T, k),
                                      count=count, capacity=capacity, cached=cached,
                                      n_new=count.clamp_max(capacity).minimum(pool.cap),
                                      fill_before=pool.fill.clone(), routing_weights=routing_weights,
                                      top_k_weights=top_k_weights, importance=importance)
-            pool.quant_scatter(keys, values, idx32, slot, 1, now=float(self.clock))
+            pool.quant_scatter_routed(keys, stacked, idx32, slot, k, now=float(self.clock))
             pool.advance(count, capacity)
             self.cache_ptrs = pool.fill.long()
             if policy == ops.EVICT_H2O:

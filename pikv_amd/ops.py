@@ -398,6 +398,102 @@ def select_top_rows(score, seg_base, seg_len, n_keep, max_len: Optional[int] = N
     return flag, index, kept
 
 
+def _ptr_array(ts):
+    return (C.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
+
+
+def linear_group(x, layers, rank: int = 0):
+    """Linear layers over one input x [T, K] float32 in one launch.  `layers`: dicts of weight [N, K], bias [N],
+    out [T, N] and optionally relu, add [N], lora_a [K, rank], lora_b [rank, N], scaling.  K a multiple of 128, N of
+    32, at most 20 layers, rank at most 8."""
+    x = _need(x, "x", dtype=torch.float32, ndim=2)
+    T, K = x.shape
+    for l in layers:
+        N_ = l["weight"].shape[0]
+        w, b, o = (_need(l[n], n, dtype=torch.float32) for n in ("weight", "bias", "out"))
+        if w.shape != (N_, K) or b.shape != (N_,) or o.shape != (T, N_):
+            raise ValueError("a layer's weight, bias or out does not match x")
+        if l.get("add") is not None and _need(l["add"], "add", dtype=torch.float32).shape != (N_,):
+            raise ValueError("add must have one value per output")
+        if l.get("lora_a") is not None:
+            a, bb = _need(l["lora_a"], "lora_a", dtype=torch.float32), _need(l["lora_b"], "lora_b", dtype=torch.float32)
+            if a.shape != (K, rank) or bb.shape != (rank, N_):
+                raise ValueError("a layer's LoRA does not match its weight and the rank")
+        if w.data_ptr() % 16 or x.data_ptr() % 16:
+            raise ValueError("x and the weights must be 16-byte aligned")
+    if T == 0:
+        return
+    n = len(layers)
+    nb = int(N.lib().pikv_linear_group_workspace_bytes(T, n, rank))
+    ws = torch.empty(nb, dtype=torch.uint8, device=x.device) if nb else None
+    N.call("pikv_linear_group", _ptr(x), T, K, n, _ptr_array([l["weight"] for l in layers]),
+           _ptr_array([l["bias"] for l in layers]), (C.c_int32 * n)(*[l["weight"].shape[0] for l in layers]),
+           (C.c_int32 * n)(*[int(bool(l.get("relu"))) for l in layers]), rank,
+           _ptr_array([l.get("lora_a") for l in layers]), _ptr_array([l.get("lora_b") for l in layers]),
+           (C.c_float * n)(*[float(l.get("scaling", 0.0)) for l in layers]), _ptr_array([l.get("add") for l in layers]),
+           _ptr_array([l["out"] for l in layers]), _ptr(ws), nb, _stream())
+
+
+def value_lora(mean, lora_a, lora_b, scaling):
+    """mean[e] + ((mean[e] lora_a[e]) lora_b[e]) * scaling[e] for mean [E, H] float32 and lists of E."""
+    mean = _need(mean, "mean", dtype=torch.float32, ndim=2)
+    E, H = mean.shape
+    rank = lora_a[0].shape[1]
+    if not len(lora_a) == len(lora_b) == len(scaling) == E:
+        raise ValueError("one lora_a, lora_b and scaling per row of mean")
+    for a, b in zip(lora_a, lora_b):
+        if (_need(a, "lora_a", dtype=torch.float32).shape != (H, rank)
+                or _need(b, "lora_b", dtype=torch.float32).shape != (rank, H)):
+            raise ValueError("lora_a must be [H, rank], lora_b [rank, H]")
+    out = torch.empty_like(mean)
+    N.call("pikv_value_lora", _ptr(mean), E, H, rank, _ptr_array(lora_a), _ptr_array(lora_b),
+           (C.c_float * E)(*[float(v) for v in scaling]), _ptr(out), _stream())
+    return out
+
+
+def expert_mix(outs, weights):
+    """Sum over e of outs[e][t] * weights[t][e]: outs [E, T, H], weights [T, E] float32 -> [T, H]."""
+    outs = _need(outs, "outs", dtype=torch.float32, ndim=3)
+    E, T, H = outs.shape
+    weights = _need(weights, "weights", dtype=torch.float32, ndim=2)
+    if weights.shape != (T, E) or H % 4:
+        raise ValueError(f"weights must be [{T}, {E}] and the width a multiple of 4")
+    mix = torch.empty(T, H, dtype=torch.float32, device=outs.device)
+    if mix.numel():
+        N.call("pikv_expert_mix", _ptr(outs), _ptr(weights), T, E, H, _ptr(mix), _stream())
+    return mix
+
+
+def adaptive_router(x_mean, selector, lb, imp, predictor, seq_len: int, top_k: int, mask=None, temp_lb: float = 1.0,
+                    temp_imp: float = 1.0, balance_weight: float = 0.01):
+    """AdaptiveRouter behind its hidden layers (pikv_adaptive_router).  x_mean [B, H]; selector (w1, b1, w2, b2);
+    lb, imp, predictor: (hidden after ReLU [T, .], w, b).  Returns (weights [T, E], idx int64 [T, k], topk_w [T, k],
+    balance loss [], importance [T])."""
+    x_mean = _need(x_mean, "x_mean", dtype=torch.float32, ndim=2)
+    B, H = x_mean.shape
+    T, E, H2 = B * seq_len, lb[1].shape[0], predictor[0].shape[1]
+    for t, shape in zip((*selector, *lb, *imp, *predictor),
+                        ((H2, H), (H2,), (2, H2), (2,), (T, H), (E, H), (E,), (T, H), (E, H), (E,), (T, H2), (1, H2), (1,))):
+        if _need(t, "a router tensor", dtype=torch.float32).shape != shape:
+            raise ValueError(f"a router tensor has shape {tuple(t.shape)}, expected {shape}")
+    if mask is not None and _need(mask, "mask", dtype=torch.float32).shape != (E,):
+        raise ValueError("mask must have one value per expert")
+    if not (1 <= E <= 64 and 1 <= top_k <= min(E, 8) and T >= 1):
+        raise ValueError("num_experts must be in [1,64], top_k in [1,min(E,8)], with at least one token")
+    dev = x_mean.device
+    blend = torch.empty(B, 2, dtype=torch.float32, device=dev)
+    probs = torch.empty(2, T, E, dtype=torch.float32, device=dev)
+    idx = torch.empty(T, top_k, dtype=torch.int64, device=dev)
+    topk_w = torch.empty(T, top_k, dtype=torch.float32, device=dev)
+    importance = torch.empty(T, dtype=torch.float32, device=dev)
+    loss = torch.empty((), dtype=torch.float32, device=dev)
+    N.call("pikv_adaptive_router", _ptr(x_mean), B, seq_len, H, H2, E, top_k, *[_ptr(t) for t in selector],
+           *[_ptr(t) for t in lb], float(temp_lb), *[_ptr(t) for t in imp], float(temp_imp),
+           *[_ptr(t) for t in predictor], _ptr(mask), float(balance_weight), _ptr(blend), _ptr(probs[0]), _ptr(probs[1]),
+           _ptr(idx), _ptr(topk_w), _ptr(importance), _ptr(loss), _stream())
+    return probs[1], idx, topk_w, loss, importance
+
+
 def prefill_attend(q, k, v, pool: Optional["CachePool"] = None, causal: bool = True,
                    scale_qk: Optional[float] = None):
     """softmax(q.k) v of a prompt chunk in float32: q [B, S, n_q_heads, head_dim] over the rows that
@@ -569,6 +665,28 @@ class CachePool:
                _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero), _ptr(self.v_zero),
                _ptr(self.acc), _ptr(self.ts), float(now), _stream())
 
+    def quant_scatter_routed(self, k_src, v_src, cache_id, slot, per_token: int, now: float = 0.0):
+        """quant_scatter for rows that differ per cache: assignment j of token t (cache_id / slot
+        [n_tokens * per_token]) takes the K row k_src[t] and the V row v_src[cache_id][t] of k_src
+        [n_tokens, D] and v_src [n_caches, n_tokens, D], float32.  fill is not advanced."""
+        if not self.with_v:
+            raise ValueError("this pool stores no V rows")
+        k_src = _need(k_src, "k_src", dtype=torch.float32, ndim=2)
+        n = k_src.shape[0]
+        v_src = _need(v_src, "v_src", dtype=torch.float32, ndim=3)
+        if k_src.shape[1] != self.D or v_src.shape != (self.n_caches, n, self.D):
+            raise ValueError(f"k_src must be [n, {self.D}], v_src [{self.n_caches}, n, {self.D}]")
+        cache_id = _need(cache_id, "cache_id", dtype=torch.int32)
+        slot = _need(slot, "slot", dtype=torch.int32)
+        if not 1 <= per_token <= 64 or cache_id.numel() != n * per_token or slot.numel() != n * per_token:
+            raise ValueError("cache_id and slot must have n * per_token elements")
+        if n == 0:
+            return
+        N.call("pikv_quant_scatter_routed", _ptr(k_src), _ptr(v_src), n, per_token, self.D, self.group, self.scheme,
+               _ptr(cache_id), _ptr(slot), _ptr(self.row_base), _ptr(self.fill), _ptr(self.cap), self.n_caches,
+               _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero),
+               _ptr(self.v_zero), _ptr(self.acc), _ptr(self.ts), float(now), _stream())
+
     def quant_gather(self, k_src, v_src, src_row_base, src_index, n_take, max_take: int,
                      src_score=None, now: float = 0.0):
         """Quantise the listed source rows into the caches in list order: for
@@ -624,6 +742,18 @@ class CachePool:
         codes, scale, zero = self._planes(which)
         return dequantize_rows(codes, scale, zero, self.group, self.scheme, out_dtype,
                                rows=rows, row0=row0, n=n)
+
+    def mean_rows(self, which="v"):
+        """Mean dequantised row of every cache, [n_caches, D] float32 (zero for an empty cache)."""
+        codes, scale, zero = self._planes(which)
+        out = torch.empty(self.n_caches, self.D, dtype=torch.float32, device=self.device)
+        if self.rows == 0:
+            return out.zero_()
+        nb = int(N.lib().pikv_cache_mean_workspace_bytes(self.n_caches, self.D, self.max_cap))
+        ws = torch.empty(nb, dtype=torch.uint8, device=self.device)
+        N.call("pikv_cache_mean", _ptr(codes), _ptr(scale), _ptr(zero), self.scheme, self.group, self.D,
+               _ptr(self.row_base), _ptr(self.fill), self.n_caches, self.max_cap, _ptr(out), _ptr(ws), nb, _stream())
+        return out
 
     def scores(self, q, n_q_heads: int, scale_qk: Optional[float] = None,
                max_len: Optional[int] = None):

@@ -2,8 +2,9 @@
 LoadBalancingRouter, ImportanceAwareRouter and their blend, AdaptiveRouter - same
 constructors, parameter names (a reference state_dict loads) and return tuples.
 
-What stays in torch: the small MLPs (gate, importance predictor, router selector) and the
-losses built on their outputs.  What runs natively: every softmax + top-k + renormalise
+AdaptiveRouter without autograd runs natively as a whole (_forward_native).  Otherwise the small
+MLPs (gate, importance predictor, router selector) and the losses built on their outputs stay in
+torch.  What runs natively in every case: every softmax + top-k + renormalise
 (`pikv_router_tail`, one wavefront per token), with this build's total order - value
 descending, lower expert first among equal float32 values - where torch.topk leaves ties
 unspecified.  Values come from the kernel; when gradients are wanted, the same quantities
@@ -15,7 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import dense, ops
 
 
 def _with_grad(value: torch.Tensor, differentiable: torch.Tensor) -> torch.Tensor:
@@ -123,12 +124,52 @@ class AdaptiveRouter(nn.Module):
             nn.Softmax(dim=-1),
         )
 
+    def _native(self, x, expert_mask) -> bool:
+        """Whether the three hidden layers run in one launch and everything behind them in three: a float32 forward
+        without autograd over unmodified layers (35 launches otherwise, 128 tokens as well as 2048)."""
+        H, E = self.hidden_size, self.num_experts
+        lb, imp = self.load_balancing_router, self.importance_router
+        if not (dense.forward_only(x) and x.dim() == 3 and x.numel() > 0 and x.shape[-1] == H and H % 128 == 0
+                and 1 <= E <= 64 and 1 <= min(self.top_k, E) <= 8 and x.shape[0] * x.shape[1] <= 65535 * 32):
+            return False
+        if expert_mask is not None and not (dense._ordinary_tensor(expert_mask, x.device) and expert_mask.shape == (E,)):
+            return False
+        if not (dense.plain(lb, LoadBalancingRouter) and dense.plain(imp, ImportanceAwareRouter)
+                and all(type(v) in (int, float) for v in (lb.temperature, imp.temperature, lb.balance_weight))
+                and lb.top_k >= 1 and imp.top_k >= 1 and max(min(lb.top_k, E), min(imp.top_k, E)) <= 8):
+            return False
+        dev = x.device
+        return (lb.num_experts == imp.num_experts == E
+                and dense.mlp_ok(lb.router, (nn.ReLU,), (H, H, E), dev)
+                and dense.mlp_ok(imp.router, (nn.ReLU,), (H, H, E), dev)
+                and dense.mlp_ok(imp.importance_predictor, (nn.ReLU, nn.Sigmoid), (H, H // 2, 1), dev)
+                and dense.mlp_ok(self.router_selector, (nn.ReLU, nn.Softmax), (H, H // 2, 2), dev)
+                and self.router_selector[3].dim in (-1, 1))
+
+    def _forward_native(self, x, x_mean, expert_mask):
+        B, S, H = x.shape
+        lb, imp = self.load_balancing_router, self.importance_router
+        x2, dev = x.reshape(B * S, H), x.device
+        hidden = [torch.empty(B * S, n, dtype=torch.float32, device=dev) for n in (H, H, H // 2)]
+        first = [lb.router[0], imp.router[0], imp.importance_predictor[0]]
+        ops.linear_group(x2, [dict(weight=m.weight, bias=m.bias, relu=True, out=h) for m, h in zip(first, hidden)])
+        last = [lb.router[2], imp.router[2], imp.importance_predictor[2]]
+        sel = self.router_selector
+        k = min(self.top_k, self.num_experts)
+        weights, idx, topk_w, loss, importance = ops.adaptive_router(
+            x_mean, (sel[0].weight, sel[0].bias, sel[2].weight, sel[2].bias),
+            *[(h, m.weight, m.bias) for h, m in zip(hidden, last)], seq_len=S, top_k=k, mask=expert_mask,
+            temp_lb=lb.temperature, temp_imp=imp.temperature, balance_weight=lb.balance_weight)
+        return (weights.view(B, S, -1), idx.view(B, S, k), topk_w.view(B, S, k), loss, importance.view(B, S, 1))
+
     def forward(self, x, expert_mask=None):
         if x.dim() == 2:
             x = x.unsqueeze(-1).expand(-1, -1, self.hidden_size)
         elif x.dim() == 1:
             x = x.unsqueeze(0).unsqueeze(-1).expand(-1, -1, self.hidden_size)
         x_mean = x.mean(dim=1)
+        if self._native(x, expert_mask):
+            return self._forward_native(x, x_mean, expert_mask)
         router_weights = self.router_selector(x_mean)
         lb_weights, _, _, lb_loss = self.load_balancing_router(x, expert_mask)
         imp_weights, _, _, importance = self.importance_router(x, expert_mask)

@@ -1,0 +1,139 @@
+"""GPU parity of the float32 dense kernels of the mixture-of-experts layer, against float64 or the torch path."""
+import numpy as np
+import pytest
+
+import pikv_oracle as O
+from test_gpu_read_evict import _fill_pool
+from util import np_of, rng, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _near(got, want, n, size):
+    """A float32 sum of n products of values up to `size`: 2^-24 a step, random signs, four times that."""
+    assert np.abs(np_of(got).astype(np.float64) - want).max() <= 4 * 2.0 ** -24 * np.sqrt(n) * size * size
+
+
+@pytest.mark.parametrize("T,K,widths,rank", [(1, 128, [32], 0), (33, 256, [256, 64, 96], 4), (64, 640, [32, 512], 8),
+                                             (500, 128, [64] * 20, 1)])
+def test_linear_group(dev, T, K, widths, rank):
+    from pikv_amd import ops
+    import torch
+    r = rng(T + K)
+    x = r.standard_normal((T, K)).astype(np.float32)
+    layers, want = [], []
+    for i, n in enumerate(widths):
+        w, b, c = (r.standard_normal(s).astype(np.float32) for s in ((n, K), (n,), (n,)))
+        y = x.astype(np.float64) @ w.T.astype(np.float64) + b
+        l = dict(weight=to_dev(w, dev), bias=to_dev(b, dev), relu=i % 2 == 0, out=torch.empty(T, n, device=dev))
+        if rank and i != 1:
+            la, lb = (r.standard_normal(s).astype(np.float32) for s in ((K, rank), (rank, n)))
+            y = y + x.astype(np.float64) @ la @ lb.astype(np.float64) * 0.25
+            l.update(lora_a=to_dev(la, dev), lora_b=to_dev(lb, dev), scaling=0.25)
+        y = np.maximum(y, 0) if l["relu"] else y
+        if i % 3 == 0:
+            y = y + c
+            l["add"] = to_dev(c, dev)
+        layers.append(l)
+        want.append(y)
+    ops.linear_group(to_dev(x, dev), layers, rank=rank)
+    for l, y in zip(layers, want):
+        _near(l["out"], y, K * max(rank, 1), 4.5)
+
+
+@pytest.mark.parametrize("scheme,D,group", [(O.Q_I8_SYM, 272, 16), (O.Q_I8_ASYM, 256, 256), (O.Q_I4_ASYM, 1088, 32),
+                                            (O.Q_I4_SYM, 64, 64)])
+@pytest.mark.parametrize("lens", [[0, 1, 63], [65, 64, 130], [5000, 4097, 2]])
+def test_mean_rows(dev, scheme, D, group, lens):
+    pool, ref = _fill_pool(dev, rng(D + lens[0]), [max(lens)] * 3, lens, 1, D, group, scheme)
+    got = np_of(pool.mean_rows("v")).astype(np.float64)
+    for c, n in enumerate(lens):
+        rows = ref.valid_rows(c)[:n]
+        v = O.dequantize_groups(ref.v_codes[rows], ref.v_scale[rows], ref.v_zero[rows], group).astype(np.float64)
+        want = v.mean(axis=0) if n else np.zeros(D)
+        assert np.abs(got[c] - want).max() <= 4 * 2.0 ** -24 * np.sqrt(max(n, 1)) * (np.abs(v).max() if n else 1)
+
+
+@pytest.mark.parametrize("scheme,D,group", [(O.Q_I8_SYM, 1024, 64), (O.Q_I8_ASYM, 272, 16), (O.Q_I4_SYM, 256, 32)])
+def test_quant_scatter_routed(dev, scheme, D, group):
+    """The same planes as quant_scatter leaves for the repeated K rows and the gathered V rows, dropped slots and
+    caches outside the pool among them."""
+    import torch
+    from pikv_amd import ops
+    r = rng(D)
+    E, T, k = 3, 45, 2
+    keys, vals = (to_dev(r.standard_normal(s).astype(np.float32), dev) for s in ((T, D), (E, T, D)))
+    cid = r.integers(0, E, T * k).astype(np.int32)
+    slot = np.array([np.count_nonzero(cid[:i] == c) for i, c in enumerate(cid)], dtype=np.int32)
+    slot[::7] = -1
+    pools = [ops.CachePool([20, 25, 9], 1, D, group, scheme, dev) for _ in range(2)]
+    odd = cid.copy()
+    odd[5], slot[5] = E + 4, 3
+    idx, sl = to_dev(odd, dev), to_dev(slot, dev)
+    pools[0].quant_scatter_routed(keys, vals, idx, sl, k, now=3.0)
+    tok = torch.arange(T, device=dev).repeat_interleave(k)
+    pools[1].quant_scatter(keys[tok].contiguous(), vals[to_dev(cid, dev).long(), tok].contiguous(), idx, sl, 1, now=3.0)
+    for a, b in zip(pools[0].planes(), pools[1].planes()):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,S,H,E,k,mask", [(1, 1, 128, 1, 1, False), (2, 33, 256, 4, 2, True), (3, 70, 384, 13, 8, False)])
+def test_adaptive_router_native(dev, B, S, H, E, k, mask):
+    """The native pass against the module's torch path (taken with autograd on): same selection, values to the
+    rounding of float32 sums of H products."""
+    import torch
+    from pikv_amd.routing_strategy import AdaptiveRouter
+    torch.manual_seed(H + E)
+    m = AdaptiveRouter(H, E, top_k=k).to(dev)
+    x = torch.randn(B, S, H, device=dev)
+    em = torch.randn(E, device=dev) if mask else None
+    ref = m(x, em)
+    with torch.no_grad():
+        assert m._native(x, em)
+        got = m(x, em)
+        handle = m.load_balancing_router.router[0].register_forward_hook(lambda *a: None)
+        assert not m._native(x, em)
+        handle.remove()
+        assert not m._native(x.double(), em) and not m._native(x[:, :, ::2], em)
+    for a, b in zip(got, ref):
+        assert a.shape == b.shape and a.dtype == b.dtype
+    assert (got[1] == ref[1]).float().mean() > 0.99
+    for i in (0, 3, 4):
+        if E > 1 or i != 3:                              # one expert: the spread of one value, NaN on both sides
+            assert torch.allclose(got[i], ref[i], rtol=0, atol=64 * 2.0 ** -24 * np.sqrt(H))
+    same = (got[1] == ref[1]).all(-1)
+    assert torch.allclose(got[2][same], ref[2][same], atol=64 * 2.0 ** -24 * np.sqrt(H))
+
+
+@pytest.mark.parametrize("H,policy", [(128, "lru"), (256, "h2o")])
+def test_moe_native_forward_equals_module_path(dev, H, policy):
+    """PiKVMoE without autograd through the native experts and through the modules (a hook on one expert)."""
+    import torch
+    from pikv_amd import moe
+    from pikv_amd.config import config
+    from pikv_amd.scheduling import SchedulingPolicy
+    saved = dict(config)
+    try:
+        config.update(hidden_size=H, num_experts=3, kv_cache_size=60, kv_heads=2, kv_quant="int8", kv_group=None,
+                      vocab_size=512, cache_decrement=5, top_k=2, capacity_factor=1.5)
+        pol = SchedulingPolicy.H2O if policy == "h2o" else SchedulingPolicy.LRU
+        models = []
+        for _ in range(2):
+            torch.manual_seed(1)
+            m = moe.PiKVMoE(use_cache_scheduling=True, cache_scheduling_policy=pol).to(dev)
+            with torch.no_grad():
+                for e in m.experts:
+                    e.lora.lora_B.normal_(0.0, 0.05)
+                for c in m.kv_caches:
+                    c.value_lora.lora_B.normal_(0.0, 0.05)
+            models.append(m)
+        models[1].experts[0].register_forward_hook(lambda *a: None)
+        ids = torch.randint(512, (2, 37), device=dev)
+        with torch.no_grad():
+            for _ in range(3):
+                a, b = (m(ids) for m in models)
+                assert torch.allclose(a, b, rtol=0, atol=1e-5 * float(b.abs().max()))
+        assert torch.equal(models[0].pool.fill, models[1].pool.fill)
+    finally:
+        config.clear()
+        config.update(saved)
