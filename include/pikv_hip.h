@@ -551,17 +551,15 @@ int pikv_cache_make_room(int policy, const int32_t* count, int64_t count_all, in
 
 /* Linear layers over one input, in one launch (a second one before it where a layer has LoRA):
  *   out[g][t][n] = act(x[t] . w[g][n] + bias[g][n] + ((x[t] lora_a[g]) lora_b[g])[n] * scaling[g])
- *                  + add[g][n]
  *   x [T][K]; host arrays of n_layers (at most 20) entries: w [n_out][K], bias [n_out],
  *   lora_a [K][rank] / lora_b [rank][n_out] (rank at most 8; rank 0, NULL array or entry: none),
- *   add [n_out] (NULL array or entry: none), relu (0 / 1), out [T][n_out].  K a multiple of 128,
+ *   relu (0 / 1), out [T][n_out].  K a multiple of 128,
  *   n_out of 32; x and w 16-byte aligned.  Other sizes: PIKV_ERR_UNSUPPORTED.
  *   workspace: pikv_linear_group_workspace_bytes(...) bytes, needed only with LoRA. */
 int pikv_linear_group(const float* x, int64_t T, int K, int n_layers, const float* const* w,
                       const float* const* bias, const int32_t* n_out, const int32_t* relu, int rank,
                       const float* const* lora_a, const float* const* lora_b, const float* scaling,
-                      const float* const* add, float* const* out, void* workspace,
-                      int64_t workspace_bytes, void* stream);
+                      float* const* out, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t pikv_linear_group_workspace_bytes(int64_t T, int n_layers, int rank);
 
 /* out [n_caches][D] = mean of every cache's dequantised rows (zero for an empty cache).
@@ -576,9 +574,13 @@ int64_t pikv_cache_mean_workspace_bytes(int n_caches, int D, int64_t max_len);
 int pikv_value_lora(const float* mean, int n_experts, int H, int rank, const float* const* lora_a,
                     const float* const* lora_b, const float* scaling, float* out, void* stream);
 
-/* mix[t] = sum over e, in order, of outs[e][t] * weights[t][e]; outs [E][T][H], weights [T][E]. */
-int pikv_expert_mix(const float* outs, const float* weights, int64_t T, int E, int H, float* mix,
-                    void* stream);
+/* outs[e] = relu(dense[e] + lora[e] * scaling[e]) + add[e] and
+ * mix[t] = sum over e, in order, of outs[e][t] * weights[t][e], each step rounded on its own;
+ * dense, lora, scaling: host arrays of E (at most 20) entries, dense / lora [T][H] 16-byte aligned,
+ * add [E][H], weights [T][E], outs [E][T][H], mix [T][H], H a multiple of 4. */
+int pikv_expert_combine(const float* const* dense, const float* const* lora, const float* scaling,
+                        const float* add, const float* weights, int64_t T, int E, int H, float* outs,
+                        float* mix, void* stream);
 
 /* AdaptiveRouter (core/single/routing_strategy.py:100-150) behind its hidden layers, T = n_seqs * S:
  *   blend [n_seqs][2] = softmax(relu(x_mean sel_w1^T + sel_b1) sel_w2^T + sel_b2)

@@ -68,12 +68,12 @@ SIGNATURES = {
                                   C.POINTER(_p), C.POINTER(_l), _i, _p, _p, _p, _p, _p, _l, _p]),
     "pikv_compact_rows": (_i, [C.POINTER(_p), C.POINTER(_l), _i, _p, _p, _p, _p, _i, _p]),
     "pikv_linear_group": (_i, [_p, _l, _i, _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(C.c_int32), C.POINTER(C.c_int32),
-                               _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), C.POINTER(_p), C.POINTER(_p), _p, _l, _p]),
+                               _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), C.POINTER(_p), _p, _l, _p]),
     "pikv_linear_group_workspace_bytes": (_l, [_l, _i, _i]),
     "pikv_cache_mean": (_i, [_p, _p, _p, _i, _i, _i, _p, _p, _i, _l, _p, _p, _l, _p]),
     "pikv_cache_mean_workspace_bytes": (_l, [_i, _i, _l]),
     "pikv_value_lora": (_i, [_p, _i, _i, _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), _p, _p]),
-    "pikv_expert_mix": (_i, [_p, _p, _l, _i, _i, _p, _p]),
+    "pikv_expert_combine": (_i, [C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), _p, _p, _l, _i, _i, _p, _p, _p]),
     "pikv_adaptive_router": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _f, _p, _p, _p,
                                   _p, _f, _p, _p, _p, _p, _p, _p, _p, _p]),
     "pikv_quant_scatter_routed": (_i, [_p, _p, _l, _i, _i, _i, _i, _p, _p, _p, _p, _p, _i,

@@ -1,15 +1,16 @@
-// Dense float32 pieces of the mixture-of-experts layer: the small linear layers that share one input (experts, key
-// projection, router hidden layers) in one launch, the rest of the adaptive router, the means of the cached values and
-// the weighted sum of the experts.
+// Float32 pieces of the mixture-of-experts layer around its library products: small linear layers that share one input
+// (key projection, router hidden layers) in one launch, the rest of the adaptive router, the means of the cached values,
+// and everything behind the experts' products.
 //
-// Bound: launches and latency.  A [128 x 256] x [256 x 256] product is 17 MFLOP; as one library call per expert
-// it ran on a single compute unit (one 256 x 128 tile, 33 us).  Here a tile is 32 x 32 and the contraction is split
-// over the wavefronts of its block, so that one launch of all layers covers the chip and no chain is longer than a
-// quarter of the contraction.  Everything is float32 (v_mfma_f32_32x32x2_f32): products, sums and results.
-// Measured, 128 tokens, 4 experts of 256 x 256: the model's forward 1725 -> 461 us with 20 launches instead of 133;
-// the five experts' layers 9.8 us (four library products 133), 768 tokens 34 us for 96; 2048 tokens x 7 layers of
-// 512 x 512 are even (141 and 134 us) before the launches around the products.  Error against float64 2.1e-7 where the
-// library's is 4.1e-7.
+// Bound: launches and latency.  A [128 x 256] x [256 x 256] product is 17 MFLOP; as a library call it runs on a
+// single compute unit (one 256 x 128 tile, 33 us).  Here a tile is 32 x 32 and the contraction is split over the
+// wavefronts of its block, so that one launch of all layers covers the chip and no chain is longer than a quarter of
+// the contraction.  Everything is float32 (v_mfma_f32_32x32x2_f32): products, sums and results; error against
+// float64 2.1e-7 where the library's is 4.1e-7.  The experts' own products stay with the library: their outputs are
+// quantised into the caches and come back as means in the next call, where another order of their sums - 2e-7, a code
+// in 10^4 - grew to 1e-4 of a cached row's scale.
+// Measured: linear_group, three layers of 2048 x 2048 over 8 rows 26 us (59 as three library calls), over 128 rows 55
+// and 59; adaptive router with 128 tokens, 4 experts 7.6 + 5.1 + 7.1 + 2.9 us for 35 launches.
 #include "common.hpp"
 
 namespace pikv {
@@ -27,7 +28,6 @@ struct LinearLayer {
   const float* bias;     // [N]
   const float* lora_a;   // [K][rank] or null
   const float* lora_b;   // [rank][N]
-  const float* add;      // [N] or null: added last
   float* out;            // [T][N]
   float scaling;
   int N, relu;
@@ -119,7 +119,6 @@ __global__ __launch_bounds__(256) void linear_group_kernel(LinearArgs a) {
       y = y + s * L.scaling;
     }
     if (L.relu) y = y < 0.f ? 0.f : y;   // a NaN stays
-    if (L.add != nullptr) y = y + L.add[n0 + n];
     L.out[(m0 + m) * L.N + n0 + n] = y;
   }
 }
@@ -233,20 +232,43 @@ __global__ __launch_bounds__(256) void value_lora_kernel(ValueLoraArgs a) {
   }
 }
 
-// ---- weighted sum of the experts ----------------------------------------------------------------
-// mix[t] = sum over e, in order, of outs[e][t] * w[t][e].
-__global__ __launch_bounds__(256) void expert_mix_kernel(const float* outs, const float* w, int64_t T, int E, int H4,
-                                                         float* mix) {
+// ---- experts behind their products ----------------------------------------------------------------
+struct ExpertArgs {
+  const float* dense[kMaxGroups];   // [T][H]
+  const float* lora[kMaxGroups];    // [T][H]
+  float scaling[kMaxGroups];
+  const float* add;                 // [E][H]
+  const float* w;                   // [T][E]
+  float* outs;                      // [E][T][H]
+  float* mix;                       // [T][H]
+  int64_t T;
+  int E, H4;
+};
+
+// outs[e] = relu(dense[e] + lora[e] * scaling[e]) + add[e]; mix[t] = sum over e, in order, of outs[e][t] * w[t][e].
+__global__ __launch_bounds__(256) void expert_combine_kernel(ExpertArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= T * H4) return;
-  const int64_t t = i / H4;
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int e = 0; e < E; ++e) {
-    const float4 o = reinterpret_cast<const float4*>(outs)[e * T * H4 + i];
-    const float we = w[t * E + e];
-    s.x = s.x + o.x * we; s.y = s.y + o.y * we; s.z = s.z + o.z * we; s.w = s.w + o.w * we;
+  if (i >= a.T * a.H4) return;
+  const int64_t t = i / a.H4;
+  const int h = (int)(i - t * a.H4);
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int e = 0; e < a.E; ++e) {
+    const float4 d = reinterpret_cast<const float4*>(a.dense[e])[i];
+    const float4 l = reinterpret_cast<const float4*>(a.lora[e])[i];
+    const float4 c = reinterpret_cast<const float4*>(a.add)[(int64_t)e * a.H4 + h];
+    const float dv[4] = {d.x, d.y, d.z, d.w}, lv[4] = {l.x, l.y, l.z, l.w}, cv[4] = {c.x, c.y, c.z, c.w};
+    const float we = a.w[t * a.E + e];
+    float o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float y = dv[j] + lv[j] * a.scaling[e];
+      y = y < 0.f ? 0.f : y;             // a NaN stays
+      o[j] = y + cv[j];
+      s[j] = s[j] + o[j] * we;
+    }
+    reinterpret_cast<float4*>(a.outs)[e * a.T * a.H4 + i] = make_float4(o[0], o[1], o[2], o[3]);
   }
-  reinterpret_cast<float4*>(mix)[i] = s;
+  reinterpret_cast<float4*>(a.mix)[i] = make_float4(s[0], s[1], s[2], s[3]);
 }
 
 // ---- adaptive router behind its hidden layers -------------------------------------------------------
@@ -422,8 +444,7 @@ extern "C" int64_t pikv_linear_group_workspace_bytes(int64_t T, int n_layers, in
 extern "C" int pikv_linear_group(const float* x, int64_t T, int K, int n_layers, const float* const* w,
                                  const float* const* bias, const int32_t* n_out, const int32_t* relu, int rank,
                                  const float* const* lora_a, const float* const* lora_b, const float* scaling,
-                                 const float* const* add, float* const* out, void* workspace, int64_t workspace_bytes,
-                                 void* stream) {
+                                 float* const* out, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!x || !w || !bias || !n_out || !relu || !out) return PIKV_ERR_NULL;
   if (T < 1 || K < 1 || n_layers < 1 || rank < 0) return PIKV_ERR_SHAPE;
   if (K % 128 != 0 || n_layers > kMaxGroups || rank > kMaxRank || (T + kTileMN - 1) / kTileMN > 65535)
@@ -435,7 +456,6 @@ extern "C" int pikv_linear_group(const float* x, int64_t T, int K, int n_layers,
   for (int g = 0; g < n_layers; ++g) {
     LinearLayer& l = a.l[g];
     l.w = w[g]; l.bias = bias[g]; l.out = out[g]; l.N = n_out[g]; l.relu = relu[g];
-    l.add = add ? add[g] : nullptr;
     if (!l.w || !l.bias || !l.out) return PIKV_ERR_NULL;
     if (l.N < 1) return PIKV_ERR_SHAPE;
     if (l.N % kTileMN != 0) return PIKV_ERR_UNSUPPORTED;
@@ -512,11 +532,20 @@ extern "C" int pikv_value_lora(const float* mean, int n_experts, int H, int rank
   return PIKV_OK;
 }
 
-extern "C" int pikv_expert_mix(const float* outs, const float* weights, int64_t T, int E, int H, float* mix, void* stream) {
-  if (!outs || !weights || !mix) return PIKV_ERR_NULL;
+extern "C" int pikv_expert_combine(const float* const* dense, const float* const* lora, const float* scaling,
+                                   const float* add, const float* weights, int64_t T, int E, int H, float* outs,
+                                   float* mix, void* stream) {
+  if (!dense || !lora || !scaling || !add || !weights || !outs || !mix) return PIKV_ERR_NULL;
   if (T < 1 || E < 1 || H < 4 || H % 4 != 0 || (T * (H / 4) + 255) / 256 > 0x7fffffffLL) return PIKV_ERR_SHAPE;
-  hipLaunchKernelGGL(expert_mix_kernel, dim3((unsigned)((T * (H / 4) + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     outs, weights, T, E, H / 4, mix);
+  if (E > kMaxGroups) return PIKV_ERR_UNSUPPORTED;
+  ExpertArgs a{};
+  for (int e = 0; e < E; ++e) {
+    if (!dense[e] || !lora[e]) return PIKV_ERR_NULL;
+    a.dense[e] = dense[e]; a.lora[e] = lora[e]; a.scaling[e] = scaling[e];
+  }
+  a.add = add; a.w = weights; a.outs = outs; a.mix = mix; a.T = T; a.E = E; a.H4 = H / 4;
+  hipLaunchKernelGGL(expert_combine_kernel, dim3((unsigned)((T * (H / 4) + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, a);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
 }

@@ -1,6 +1,6 @@
 """Where the float32 dense layers of the mixture-of-experts model take native kernels.
 
-linear_group / adaptive_router / expert_mix (csrc/moe.hip) serve forward passes without autograd,
+linear_group / adaptive_router / expert_combine (csrc/moe.hip) serve forward passes without autograd,
 over modules that are what their class says: a subclass, a hook, an instance-level forward, autocast,
 a functorch transform or forward-mode differentiation all go through the module's own call.
 """
@@ -12,7 +12,7 @@ from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
 MAX_LORA_RANK = 8
-MAX_LAYERS = 20          # of one linear_group launch
+MAX_LAYERS = 20          # of one linear_group or expert_combine launch
 
 
 def _no_hooks(m: nn.Module) -> bool:

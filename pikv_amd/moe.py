@@ -3,7 +3,8 @@ their cache traffic routed through the HIP library.
 
 What stays in torch: the embedding, the query projection and the vocabulary projection, and
 with gradients the dense experts (LoRAExpert, core/single/lora.py:31-52) and the key projection;
-without gradients experts, key projection and their weighted sum are native too.
+without gradients, in evaluation mode, the key projection and all of an expert but its two products
+are native too.
 
 The router is the reference's routing_strategy.AdaptiveRouter (routing_strategy.py in this
 package: same parameter names, a reference state_dict loads), and the expert outputs are
@@ -210,8 +211,17 @@ class PiKVMoE(nn.Module):
         return F.softmax(scores, dim=-1).sum(dim=1)
 
     def _cached_means(self, pool):
-        """Mean dequantised cached value of every expert, [E, H] (zeros when empty)."""
-        return pool.mean_rows("v")
+        """Mean dequantised cached value of every expert, [E, H] (zeros when empty).  A model in training mode sums
+        in torch's order, with and without autograd: the router selector's gradients are small differences of large
+        sums and follow the last bit of these means."""
+        if not self.training:
+            return pool.mean_rows("v")
+        v = pool.gather_dequant("v")                                   # [rows, H]
+        means = []
+        for c, (b, cap) in enumerate(zip(pool.base_host, pool.caps_host)):
+            live = (torch.arange(cap, device=pool.device) < pool.fill[c]).unsqueeze(1)
+            means.append((v[b:b + cap] * live).sum(dim=0))
+        return torch.stack(means) / pool.fill.clamp_min(1).unsqueeze(1).float()
 
     def _lora_ok(self, m, rank, device):
         H = config['hidden_size']
@@ -220,12 +230,12 @@ class PiKVMoE(nn.Module):
                 and dense.plain(m.dropout, nn.Dropout) and not (m.dropout.training and m.dropout.p > 0))
 
     def _native_experts(self, x, routing_weights) -> bool:
-        """Whether the experts, the key projection and the weighted sum run in linear_group's one launch: a float32
-        forward without autograd over unmodified layers of widths the kernel has (128 tokens x 4 experts of
-        256 x 256: 33 us a library product, 13 launches an expert)."""
+        """Whether the key projection, the value terms and everything behind the experts' products run natively
+        (_experts_forward): a float32 forward in evaluation mode, without autograd, over unmodified layers of widths
+        the kernels have (13 launches an expert otherwise)."""
         E, H = len(self.experts), x.shape[-1]
-        if not (dense.forward_only(x) and x.numel() > 0 and H % 128 == 0 and H == config['hidden_size']
-                and E == config['num_experts'] <= dense.MAX_LAYERS - 1 and len(self.kv_caches) == E):
+        if not (not self.training and dense.forward_only(x) and x.numel() > 0 and H % 128 == 0 and H == config['hidden_size']
+                and E == config['num_experts'] <= dense.MAX_LAYERS and len(self.kv_caches) == E):
             return False
         if not (dense._ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)
                 and x.shape[0] * x.shape[1] <= 65535 * 32):
@@ -238,20 +248,25 @@ class PiKVMoE(nn.Module):
                    and self._lora_ok(e.lora, rank, x.device) and self._lora_ok(c.value_lora, rank, x.device)
                    for e, c in zip(self.experts, self.kv_caches))
 
-    def _experts_forward(self, x2, cached, routing_weights):
-        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]) in five launches."""
-        T, H = x2.shape
-        E = len(self.experts)
+    def _experts_forward(self, x, cached, routing_weights):
+        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]): the experts' products by the
+        library, bit for bit those of LoRAExpert.forward, the rest in four launches."""
+        H = x.shape[-1]
+        x2 = x.reshape(-1, H)
+        T, E = x2.shape[0], len(self.experts)
         lora = [c.value_lora for c in self.kv_caches]
         add = ops.value_lora(cached, [m.lora_A for m in lora], [m.lora_B for m in lora], [m.scaling for m in lora])
-        outs = torch.empty(E, T, H, dtype=torch.float32, device=x2.device)
-        keys = torch.empty(T, H, dtype=torch.float32, device=x2.device)
-        layers = [dict(weight=e.dense.weight, bias=e.dense.bias, lora_a=e.lora.lora_A, lora_b=e.lora.lora_B,
-                       scaling=e.lora.scaling, relu=True, add=add[i], out=outs[i]) for i, e in enumerate(self.experts)]
-        layers.append(dict(weight=self.key_proj.weight, bias=self.key_proj.bias, lora_a=self.key_lora.lora_A,
-                           lora_b=self.key_lora.lora_B, scaling=self.key_lora.scaling, out=keys))
-        ops.linear_group(x2, layers, rank=self.key_lora.lora_A.shape[1])
-        return outs, keys, ops.expert_mix(outs, routing_weights.view(T, E))
+        keys = torch.empty(T, H, dtype=torch.float32, device=x.device)
+        ops.linear_group(x2, [dict(weight=self.key_proj.weight, bias=self.key_proj.bias, lora_a=self.key_lora.lora_A,
+                                   lora_b=self.key_lora.lora_B, scaling=self.key_lora.scaling, out=keys)],
+                         rank=self.key_lora.lora_A.shape[1])
+        products, terms = [], []
+        for e in self.experts:
+            products.append(F.linear(x2, e.dense.weight, e.dense.bias))
+            terms.append(torch.mm(torch.mm(x2, e.lora.lora_A), e.lora.lora_B))
+        outs, mix = ops.expert_combine(products, terms, [e.lora.scaling for e in self.experts], add,
+                                       routing_weights.view(T, E))
+        return outs, keys, mix
 
     def update_cache(self, expert_idx, key, value, importance):
         """Update one expert's cache with new key / value rows (core/single/pikv_moe.py:249-261).
@@ -287,7 +302,7 @@ class PiKVMoE(nn.Module):
         x2 = x.reshape(T, H)
         keys = None
         if self._native_experts(x, routing_weights):
-            stacked, keys, expert_output = self._experts_forward(x2, cached, routing_weights)
+            stacked, keys, expert_output = self._experts_forward(x, cached, routing_weights)
             expert_output = expert_output.view(B, S, H)
         else:
             expert_output = torch.zeros(B, S, H, device=x.device)

@@ -404,7 +404,7 @@ def _ptr_array(ts):
 
 def linear_group(x, layers, rank: int = 0):
     """Linear layers over one input x [T, K] float32 in one launch.  `layers`: dicts of weight [N, K], bias [N],
-    out [T, N] and optionally relu, add [N], lora_a [K, rank], lora_b [rank, N], scaling.  K a multiple of 128, N of
+    out [T, N] and optionally relu, lora_a [K, rank], lora_b [rank, N], scaling.  K a multiple of 128, N of
     32, at most 20 layers, rank at most 8."""
     x = _need(x, "x", dtype=torch.float32, ndim=2)
     T, K = x.shape
@@ -413,8 +413,6 @@ def linear_group(x, layers, rank: int = 0):
         w, b, o = (_need(l[n], n, dtype=torch.float32) for n in ("weight", "bias", "out"))
         if w.shape != (N_, K) or b.shape != (N_,) or o.shape != (T, N_):
             raise ValueError("a layer's weight, bias or out does not match x")
-        if l.get("add") is not None and _need(l["add"], "add", dtype=torch.float32).shape != (N_,):
-            raise ValueError("add must have one value per output")
         if l.get("lora_a") is not None:
             a, bb = _need(l["lora_a"], "lora_a", dtype=torch.float32), _need(l["lora_b"], "lora_b", dtype=torch.float32)
             if a.shape != (K, rank) or bb.shape != (rank, N_):
@@ -430,7 +428,7 @@ def linear_group(x, layers, rank: int = 0):
            _ptr_array([l["bias"] for l in layers]), (C.c_int32 * n)(*[l["weight"].shape[0] for l in layers]),
            (C.c_int32 * n)(*[int(bool(l.get("relu"))) for l in layers]), rank,
            _ptr_array([l.get("lora_a") for l in layers]), _ptr_array([l.get("lora_b") for l in layers]),
-           (C.c_float * n)(*[float(l.get("scaling", 0.0)) for l in layers]), _ptr_array([l.get("add") for l in layers]),
+           (C.c_float * n)(*[float(l.get("scaling", 0.0)) for l in layers]),
            _ptr_array([l["out"] for l in layers]), _ptr(ws), nb, _stream())
 
 
@@ -451,17 +449,26 @@ def value_lora(mean, lora_a, lora_b, scaling):
     return out
 
 
-def expert_mix(outs, weights):
-    """Sum over e of outs[e][t] * weights[t][e]: outs [E, T, H], weights [T, E] float32 -> [T, H]."""
-    outs = _need(outs, "outs", dtype=torch.float32, ndim=3)
-    E, T, H = outs.shape
+def expert_combine(dense, lora, scaling, add, weights):
+    """(outs [E, T, H], mix [T, H]): outs[e] = relu(dense[e] + lora[e] * scaling[e]) + add[e], mix the sum over e, in
+    order, of outs[e][t] * weights[t][e].  dense, lora: lists of E (at most 20) tensors [T, H]; add [E, H]; weights
+    [T, E]; float32."""
+    E, (T, H) = len(dense), dense[0].shape
+    if not 1 <= E == len(lora) == len(scaling) or H % 4:
+        raise ValueError("one lora and scaling per expert, and a width that is a multiple of 4")
+    for t in (*dense, *lora):
+        if _need(t, "an expert's product", dtype=torch.float32).shape != (T, H) or t.data_ptr() % 16:
+            raise ValueError(f"the experts' products must be [{T}, {H}] and 16-byte aligned")
+    add = _need(add, "add", dtype=torch.float32, ndim=2)
     weights = _need(weights, "weights", dtype=torch.float32, ndim=2)
-    if weights.shape != (T, E) or H % 4:
-        raise ValueError(f"weights must be [{T}, {E}] and the width a multiple of 4")
-    mix = torch.empty(T, H, dtype=torch.float32, device=outs.device)
+    if add.shape != (E, H) or weights.shape != (T, E) or add.data_ptr() % 16:
+        raise ValueError(f"add must be [{E}, {H}], weights [{T}, {E}]")
+    outs = torch.empty(E, T, H, dtype=torch.float32, device=add.device)
+    mix = torch.empty(T, H, dtype=torch.float32, device=add.device)
     if mix.numel():
-        N.call("pikv_expert_mix", _ptr(outs), _ptr(weights), T, E, H, _ptr(mix), _stream())
-    return mix
+        N.call("pikv_expert_combine", _ptr_array(dense), _ptr_array(lora), (C.c_float * E)(*[float(v) for v in scaling]),
+               _ptr(add), _ptr(weights), T, E, H, _ptr(outs), _ptr(mix), _stream())
+    return outs, mix
 
 
 def adaptive_router(x_mean, selector, lb, imp, predictor, seq_len: int, top_k: int, mask=None, temp_lb: float = 1.0,

@@ -2,7 +2,7 @@
 LoadBalancingRouter, ImportanceAwareRouter and their blend, AdaptiveRouter - same
 constructors, parameter names (a reference state_dict loads) and return tuples.
 
-AdaptiveRouter without autograd runs natively as a whole (_forward_native).  Otherwise the small
+AdaptiveRouter in evaluation mode and without autograd runs natively as a whole (_forward_native).  Otherwise the small
 MLPs (gate, importance predictor, router selector) and the losses built on their outputs stay in
 torch.  What runs natively in every case: every softmax + top-k + renormalise
 (`pikv_router_tail`, one wavefront per token), with this build's total order - value
@@ -126,10 +126,10 @@ class AdaptiveRouter(nn.Module):
 
     def _native(self, x, expert_mask) -> bool:
         """Whether the three hidden layers run in one launch and everything behind them in three: a float32 forward
-        without autograd over unmodified layers (35 launches otherwise, 128 tokens as well as 2048)."""
+        in evaluation mode, without autograd, over unmodified layers (35 launches otherwise, 128 tokens as well as 2048)."""
         H, E = self.hidden_size, self.num_experts
         lb, imp = self.load_balancing_router, self.importance_router
-        if not (dense.forward_only(x) and x.dim() == 3 and x.numel() > 0 and x.shape[-1] == H and H % 128 == 0
+        if not (not self.training and dense.forward_only(x) and x.dim() == 3 and x.numel() > 0 and x.shape[-1] == H and H % 128 == 0
                 and 1 <= E <= 64 and 1 <= min(self.top_k, E) <= 8 and x.shape[0] * x.shape[1] <= 65535 * 32):
             return False
         if expert_mask is not None and not (dense._ordinary_tensor(expert_mask, x.device) and expert_mask.shape == (E,)):

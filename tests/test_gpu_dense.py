@@ -23,7 +23,7 @@ def test_linear_group(dev, T, K, widths, rank):
     x = r.standard_normal((T, K)).astype(np.float32)
     layers, want = [], []
     for i, n in enumerate(widths):
-        w, b, c = (r.standard_normal(s).astype(np.float32) for s in ((n, K), (n,), (n,)))
+        w, b = (r.standard_normal(s).astype(np.float32) for s in ((n, K), (n,)))
         y = x.astype(np.float64) @ w.T.astype(np.float64) + b
         l = dict(weight=to_dev(w, dev), bias=to_dev(b, dev), relu=i % 2 == 0, out=torch.empty(T, n, device=dev))
         if rank and i != 1:
@@ -31,14 +31,28 @@ def test_linear_group(dev, T, K, widths, rank):
             y = y + x.astype(np.float64) @ la @ lb.astype(np.float64) * 0.25
             l.update(lora_a=to_dev(la, dev), lora_b=to_dev(lb, dev), scaling=0.25)
         y = np.maximum(y, 0) if l["relu"] else y
-        if i % 3 == 0:
-            y = y + c
-            l["add"] = to_dev(c, dev)
         layers.append(l)
         want.append(y)
     ops.linear_group(to_dev(x, dev), layers, rank=rank)
     for l, y in zip(layers, want):
         _near(l["out"], y, K * max(rank, 1), 4.5)
+
+
+@pytest.mark.parametrize("E,T,H", [(1, 1, 4), (3, 37, 132), (20, 5, 64)])
+def test_expert_combine(dev, E, T, H):
+    """Bit for bit what the torch operations give, a NaN and infinities among the products."""
+    import torch
+    from pikv_amd import ops
+    torch.manual_seed(E)
+    d, l, c, w = (torch.randn(*s, device=dev) for s in ((E, T, H), (E, T, H), (E, H), (T, E)))
+    d[0, 0, 0], d[E - 1, T - 1, 1], l[0, 0, 2] = float("nan"), float("inf"), float("-inf")
+    outs, mix = ops.expert_combine(list(d), list(l), [0.25] * E, c, w)
+    want = torch.zeros(T, H, device=dev)
+    for e in range(E):
+        o = torch.relu(d[e] + l[e] * 0.25) + c[e]
+        assert torch.equal(o.nan_to_num(7.0), outs[e].nan_to_num(7.0))
+        want = want + o * w[:, e:e + 1]
+    assert torch.equal(want.nan_to_num(7.0), mix.nan_to_num(7.0))
 
 
 @pytest.mark.parametrize("scheme,D,group", [(O.Q_I8_SYM, 272, 16), (O.Q_I8_ASYM, 256, 256), (O.Q_I4_ASYM, 1088, 32),
@@ -84,7 +98,7 @@ def test_adaptive_router_native(dev, B, S, H, E, k, mask):
     import torch
     from pikv_amd.routing_strategy import AdaptiveRouter
     torch.manual_seed(H + E)
-    m = AdaptiveRouter(H, E, top_k=k).to(dev)
+    m = AdaptiveRouter(H, E, top_k=k).to(dev).eval()
     x = torch.randn(B, S, H, device=dev)
     em = torch.randn(E, device=dev) if mask else None
     ref = m(x, em)
@@ -120,7 +134,7 @@ def test_moe_native_forward_equals_module_path(dev, H, policy):
         models = []
         for _ in range(2):
             torch.manual_seed(1)
-            m = moe.PiKVMoE(use_cache_scheduling=True, cache_scheduling_policy=pol).to(dev)
+            m = moe.PiKVMoE(use_cache_scheduling=True, cache_scheduling_policy=pol).to(dev).eval()
             with torch.no_grad():
                 for e in m.experts:
                     e.lora.lora_B.normal_(0.0, 0.05)
