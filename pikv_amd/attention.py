@@ -34,7 +34,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import dense, ops
 
 _SCHEMES = {"int8": ops.Q_I8_SYM, "int8_asym": ops.Q_I8_ASYM, "int4": ops.Q_I4_ASYM,
             "int4_sym": ops.Q_I4_SYM}
@@ -240,6 +240,20 @@ class PiKVAttention(nn.Module):
         return pool.decode_attend(qq.contiguous(), self.num_heads, now=float(self.clock),
                                   scale_qk=1.0 / math.sqrt(self.head_dim))
 
+    def _project(self, x: torch.Tensor):
+        """q, k, v of x [B, S, hidden]: in one launch for up to 64 tokens without autograd - 8 tokens, 1024 -> 1024: 25 us
+        for the three, 58 as library calls, 64 tokens of 2048: 37 and 59 - and by the library otherwise (128 tokens:
+        55 and 59)."""
+        layers = (self.q_proj, self.k_proj, self.v_proj)
+        T, H = x.shape[0] * x.shape[1], x.shape[2]
+        dq, dkv = self.num_heads * self.head_dim, self.num_kv_heads * self.head_dim
+        if not (0 < T <= 64 and H % 128 == 0 and dq % 32 == 0 and dkv % 32 == 0 and dense.forward_only(x)
+                and all(dense.linear_ok(m, H, n, x.device) for m, n in zip(layers, (dq, dkv, dkv)))):
+            return tuple(m(x) for m in layers)
+        out = [torch.empty(T, n, dtype=torch.float32, device=x.device) for n in (dq, dkv, dkv)]
+        ops.linear_group(x.view(T, H), [dict(weight=m.weight, bias=m.bias, out=o) for m, o in zip(layers, out)])
+        return out
+
     def _native_prefill(self, q, k, v, attention_mask) -> bool:
         """Whether a chunk goes through ops.prefill_attend: float32 without a mask, dropout or gradient, and a head
         width that kernel has.  Everything else keeps the torch path below, whose score matrix, masks and copies
@@ -304,9 +318,10 @@ class PiKVAttention(nn.Module):
         needs no mask, dropout or gradient (_native_prefill), in torch otherwise.  Call
         reset_cache() to start a new sequence."""
         B, S, _ = hidden_states.shape
-        q = self.q_proj(hidden_states).view(B, S, self.num_heads, self.head_dim)
-        k = self.k_proj(hidden_states).view(B, S, self.num_kv_heads, self.head_dim)
-        v = self.v_proj(hidden_states).view(B, S, self.num_kv_heads, self.head_dim)
+        q, k, v = self._project(hidden_states)
+        q = q.view(B, S, self.num_heads, self.head_dim)
+        k = k.view(B, S, self.num_kv_heads, self.head_dim)
+        v = v.view(B, S, self.num_kv_heads, self.head_dim)
         if self.use_rotary and position_ids is not None:
             q, k = self.rotary_emb(q, k, position_ids)
         if past_key_values is not None:
