@@ -1251,21 +1251,9 @@ __global__ __launch_bounds__(512) void decode_fused_i8_kernel(Fused8Args a) {
 // output element, the ranges' statistics and partials one after the other, had taken 10.6 us for 24 caches x
 // 28 heads x 16 ranges; W = 1 at 256 ranges 11 us.)
 template <int W>
-__global__ __launch_bounds__(256) void decode_finish_kernel(const float* __restrict__ partial,
-                                                           const float* __restrict__ pstats,
-                                                           const int32_t* __restrict__ fill, int64_t max_len,
-                                                           int n_caches, int n_q_heads, int n_splits,
-                                                           int tokens_per_block, float* __restrict__ out,
-                                                           float* __restrict__ head_stats) {
-  __shared__ float2 part_s[W > 1 ? W : 1][64];
-  __shared__ float part_z[W > 1 ? W : 1];
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t items = (int64_t)n_caches * n_q_heads;
-  const int64_t item = W > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wv;   // (cache, head)
-  if (item >= items) return;   // (W > 1: the grid is one block per item)
-  const int c = (int)(item / n_q_heads);
-  const int64_t len = fill[c] < max_len ? (int64_t)fill[c] : max_len;
+__device__ __forceinline__ void finish_item(const float* partial, const float* pstats, int64_t len, int64_t items, int64_t item,
+                                            int n_splits, int tokens_per_block, int wv, int lane, float* out,
+                                            float* head_stats, float2 (*part_s)[64], float* part_z) {
   const int64_t used = (len + tokens_per_block - 1) / tokens_per_block;
   const int lim = used < n_splits ? (int)used : n_splits;
   const float2* const ps = reinterpret_cast<const float2*>(pstats) + item;   // (maximum, sum) of range sp at sp * items
@@ -1315,6 +1303,69 @@ __global__ __launch_bounds__(256) void decode_finish_kernel(const float* __restr
   if (head_stats != nullptr && lane == 0) reinterpret_cast<float2*>(head_stats)[item] = make_float2(M, Z);
 }
 
+template <int W>
+__global__ __launch_bounds__(256) void decode_finish_kernel(const float* __restrict__ partial,
+                                                           const float* __restrict__ pstats,
+                                                           const int32_t* __restrict__ fill, int64_t max_len,
+                                                           int n_caches, int n_q_heads, int n_splits,
+                                                           int tokens_per_block, float* __restrict__ out,
+                                                           float* __restrict__ head_stats) {
+  __shared__ float2 part_s[W > 1 ? W : 1][64];
+  __shared__ float part_z[W > 1 ? W : 1];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t items = (int64_t)n_caches * n_q_heads;
+  const int64_t item = W > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wv;   // (cache, head)
+  if (item >= items) return;   // (W > 1: the grid is one block per item)
+  const int c = (int)(item / n_q_heads);
+  const int64_t len = fill[c] < max_len ? (int64_t)fill[c] : max_len;
+  finish_item<W>(partial, pstats, len, items, item, n_splits, tokens_per_block, wv, lane, out, head_stats, part_s, part_z);
+}
+
+// The importance kernels need every head's final (maximum, sum).  MERGE: they take them from the ranges' statistics
+// themselves, and the blocks behind the first n_imp of a cache merge its heads' outputs in the same launch; otherwise
+// decode_finish_kernel has run before and left them in head_stats.  A tile reads 8 bytes per head and range for it:
+// taken up to kMergeRanges ranges (half of what the tile's own records are) and kMergeTiles tiles, where the launch
+// and its tail are what a kernel of 4 us costs: the call 41.2 -> 36.9 us for 1 x 700 tokens (4-bit, 8 x 32 heads),
+// 41.4 -> 39.1 us for 24 x <= 4000 tokens (8-bit, 4 x 28 heads); 64 x 32768 stay with two launches (656 us either way).
+constexpr int kMergeRanges = 16;
+constexpr int64_t kMergeTiles = 8192;
+struct MergeArgs {
+  const float* partial;
+  const float* pstats;
+  float* out;
+  int n_splits, tokens_per_block, n_imp;
+};
+
+static bool merge_in_importance(int64_t splits, int64_t n_tiles, int n_caches) {
+  return splits <= kMergeRanges && n_tiles * n_caches <= kMergeTiles;
+}
+
+// Blocks n_imp ..: four heads of cache c each.
+__device__ __forceinline__ void merge_heads(const MergeArgs& m, int c, int64_t len, int n_q_heads, int64_t items, int lane) {
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = ((int)blockIdx.x - m.n_imp) * 4 + wv;
+  if (h < n_q_heads)
+    finish_item<1>(m.partial, m.pstats, len, items, (int64_t)c * n_q_heads + h, m.n_splits, m.tokens_per_block, wv, lane, m.out,
+                   nullptr, nullptr, nullptr);
+}
+
+// (maximum, sum) of head `lane` of cache c over its ranges.
+__device__ __forceinline__ float2 merged_stats(const MergeArgs& m, int c, int64_t len, int n_q_heads, int64_t items, int lane) {
+  const int64_t used = (len + m.tokens_per_block - 1) / m.tokens_per_block;
+  const int lim = used < m.n_splits ? (int)used : m.n_splits;
+  const float2* const ps = reinterpret_cast<const float2*>(m.pstats) + (int64_t)c * n_q_heads + lane;
+  float2 mz[kMergeRanges];
+#pragma unroll
+  for (int s = 0; s < kMergeRanges; ++s) mz[s] = ps[(s < lim ? s : 0) * items];
+  float M = -__builtin_inff(), Z = 0.f;
+#pragma unroll
+  for (int s = 0; s < kMergeRanges; ++s) M = fmaxf(M, s < lim ? mz[s].x : -__builtin_inff());
+#pragma unroll
+  for (int s = 0; s < kMergeRanges; ++s) Z += s < lim ? mz[s].y * __builtin_amdgcn_exp2f((mz[s].x - M) * kLog2e) : 0.f;
+  return make_float2(M, Z);
+}
+
 static void launch_finish(const float* partial, const float* pstats, const int32_t* fill, int64_t max_len, int n_caches,
                           int n_q_heads, int n_splits, int tokens_per_block, float* out, float* head_stats, hipStream_t st) {
   const int64_t items = (int64_t)n_caches * n_q_heads;
@@ -1329,6 +1380,7 @@ static void launch_finish(const float* partial, const float* pstats, const int32
 // H2O bookkeeping from the halves the fused pass left: one wavefront per tile of 64 cached tokens.
 //   acc[n] = acc[n] * decay + sum_h e[h,n] * exp(m_tile[h] - M[h]) / Z[h];  ts[n] = now
 // with (M, Z) of every head as decode_finish_kernel merged them into head_stats [cache][q head][2].
+template <bool MERGE>
 __global__ __launch_bounds__(256) void decode_importance_kernel(const uint2* __restrict__ e16,
                                                                const float* __restrict__ tref,
                                                                const float* __restrict__ head_stats,
@@ -1336,13 +1388,18 @@ __global__ __launch_bounds__(256) void decode_importance_kernel(const uint2* __r
                                                                const int32_t* __restrict__ fill, int64_t max_len,
                                                                int64_t n_tiles, int n_kv_heads, int n_q_heads,
                                                                float decay, float now, float* __restrict__ row_acc,
-                                                               float* __restrict__ row_ts, int sets) {
+                                                               float* __restrict__ row_ts, int sets, MergeArgs merge) {
   // sets = 1: one record of rep * 16 lanes per kv head (heads 0 .. rep - 1); sets = 2 (the two-set kernel with
   // 5 to 8 heads per kv head): two records of 64 lanes, heads 0..3 and 4..7
   const int lane = threadIdx.x & 63;
   const int c = blockIdx.y;
   const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t len = fill[c] < max_len ? (int64_t)fill[c] : max_len;
+  const int64_t items = (int64_t)gridDim.y * n_q_heads;
+  if (MERGE && (int)blockIdx.x >= merge.n_imp) {
+    merge_heads(merge, c, len, n_q_heads, items, lane);
+    return;
+  }
   if (tile * kFTile >= len) return;
   const int rep = n_q_heads / n_kv_heads;
   const int r = lane >> 4;
@@ -1366,7 +1423,8 @@ __global__ __launch_bounds__(256) void decode_importance_kernel(const uint2* __r
     }
     float fac = 0.f;   // lane h: what turns a stored half of head h in this tile into a probability
     if (lane < n_q_heads) {
-      const float2 mz = *reinterpret_cast<const float2*>(head_stats + ((int64_t)c * n_q_heads + lane) * 2);
+      const float2 mz = MERGE ? merged_stats(merge, c, len, n_q_heads, items, lane)
+                              : *reinterpret_cast<const float2*>(head_stats + ((int64_t)c * n_q_heads + lane) * 2);
       const float mt = tref[((int64_t)c * n_tiles + tile) * n_q_heads + lane];
       fac = __builtin_amdgcn_exp2f((mt - mz.x) * kLog2e) / (mz.y * kHalfScale);
     }
@@ -1402,6 +1460,7 @@ __global__ __launch_bounds__(256) void decode_importance_kernel(const uint2* __r
 // The same for the records of the 8-bit pass: lane (nl, rg) of a record holds heads 4 (rg % 2) .. + 3 of
 // tokens 4 nl + 2 (rg / 2) and the next one, two tokens x four heads as halves {token, token + 1} per
 // head; with up to four query heads per kv head a record is the 32 lanes of heads 0..3 only.
+template <bool MERGE>
 __global__ __launch_bounds__(256) void decode_importance8_kernel(const uint4* __restrict__ e16,
                                                                 const float* __restrict__ tref,
                                                                 const float* __restrict__ head_stats,
@@ -1409,11 +1468,16 @@ __global__ __launch_bounds__(256) void decode_importance8_kernel(const uint4* __
                                                                 const int32_t* __restrict__ fill, int64_t max_len,
                                                                 int64_t n_tiles, int n_kv_heads, int n_q_heads,
                                                                 float decay, float now, float* __restrict__ row_acc,
-                                                                float* __restrict__ row_ts) {
+                                                                float* __restrict__ row_ts, MergeArgs merge) {
   const int lane = threadIdx.x & 63;
   const int c = blockIdx.y;
   const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t len = fill[c] < max_len ? (int64_t)fill[c] : max_len;
+  const int64_t items = (int64_t)gridDim.y * n_q_heads;
+  if (MERGE && (int)blockIdx.x >= merge.n_imp) {
+    merge_heads(merge, c, len, n_q_heads, items, lane);
+    return;
+  }
   if (tile * kFTile >= len) return;
   const int rep = n_q_heads / n_kv_heads;
   const int nl = lane & 15, rg = lane >> 4;
@@ -1439,7 +1503,8 @@ __global__ __launch_bounds__(256) void decode_importance8_kernel(const uint4* __
     }
     float fac = 0.f;   // lane h: what turns a stored half of head h in this tile into a probability
     if (lane < n_q_heads) {
-      const float2 mz = *reinterpret_cast<const float2*>(head_stats + ((int64_t)c * n_q_heads + lane) * 2);
+      const float2 mz = MERGE ? merged_stats(merge, c, len, n_q_heads, items, lane)
+                              : *reinterpret_cast<const float2*>(head_stats + ((int64_t)c * n_q_heads + lane) * 2);
       const float mt = tref[((int64_t)c * n_tiles + tile) * n_q_heads + lane];
       fac = __builtin_amdgcn_exp2f((mt - mz.x) * kLog2e) / (mz.y * kHalfScale);
     }
@@ -1608,11 +1673,20 @@ int decode_fused_launch(const void* k_codes, const void* k_scale, const void* k_
     }
 #undef PIKV_FUSED8
     PIKV_CHECK_LAUNCH();
+    MergeArgs merge{partial, pstats, out, (int)splits, tokens_per_block, (int)((n_tiles8 + 3) / 4)};
+    if (book && merge_in_importance(splits, n_tiles8, n_caches)) {
+      hipLaunchKernelGGL(decode_importance8_kernel<true>,
+                         dim3((unsigned)(merge.n_imp + (n_q_heads + 3) / 4), (unsigned)n_caches), dim3(256), 0, st,
+                         reinterpret_cast<const uint4*>(e16), tref, head_stats, cache_row_base, cache_fill, max_len, n_tiles8,
+                         n_kv_heads, n_q_heads, decay, now, row_acc, row_ts, merge);
+      PIKV_CHECK_LAUNCH();
+      return PIKV_OK;
+    }
     launch_finish(partial, pstats, cache_fill, max_len, n_caches, n_q_heads, (int)splits, tokens_per_block, out, head_stats, st);
     if (book)
-      hipLaunchKernelGGL(decode_importance8_kernel, dim3((unsigned)((n_tiles8 + 3) / 4), (unsigned)n_caches), dim3(256), 0,
+      hipLaunchKernelGGL(decode_importance8_kernel<false>, dim3((unsigned)((n_tiles8 + 3) / 4), (unsigned)n_caches), dim3(256), 0,
                          st, reinterpret_cast<const uint4*>(e16), tref, head_stats, cache_row_base, cache_fill, max_len,
-                         n_tiles8, n_kv_heads, n_q_heads, decay, now, row_acc, row_ts);
+                         n_tiles8, n_kv_heads, n_q_heads, decay, now, row_acc, row_ts, merge);
     PIKV_CHECK_LAUNCH();
     return PIKV_OK;
   }
@@ -1640,11 +1714,21 @@ int decode_fused_launch(const void* k_codes, const void* k_scale, const void* k_
   else PIKV_FUSED(PIKV_Q_I4_SYM);
 #undef PIKV_FUSED
   PIKV_CHECK_LAUNCH();
+  MergeArgs merge{partial, pstats, out, (int)splits, tokens_per_block, (int)((n_tiles + 3) / 4)};
+  const int sets = (wide && !qf) ? 2 : 1;
+  if (book && merge_in_importance(splits, n_tiles, n_caches)) {
+    hipLaunchKernelGGL(decode_importance_kernel<true>,
+                       dim3((unsigned)(merge.n_imp + (n_q_heads + 3) / 4), (unsigned)n_caches), dim3(256), 0, st,
+                       reinterpret_cast<const uint2*>(e16), tref, head_stats, cache_row_base, cache_fill, max_len, n_tiles,
+                       n_kv_heads, n_q_heads, decay, now, row_acc, row_ts, sets, merge);
+    PIKV_CHECK_LAUNCH();
+    return PIKV_OK;
+  }
   launch_finish(partial, pstats, cache_fill, max_len, n_caches, n_q_heads, (int)splits, tokens_per_block, out, head_stats, st);
   if (book)
-    hipLaunchKernelGGL(decode_importance_kernel, dim3((unsigned)((n_tiles + 3) / 4), (unsigned)n_caches), dim3(256), 0,
+    hipLaunchKernelGGL(decode_importance_kernel<false>, dim3((unsigned)((n_tiles + 3) / 4), (unsigned)n_caches), dim3(256), 0,
                        st, reinterpret_cast<const uint2*>(e16), tref, head_stats, cache_row_base, cache_fill, max_len,
-                       n_tiles, n_kv_heads, n_q_heads, decay, now, row_acc, row_ts, (wide && !qf) ? 2 : 1);
+                       n_tiles, n_kv_heads, n_q_heads, decay, now, row_acc, row_ts, sets, merge);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
 }
