@@ -121,4 +121,6 @@ def check(code: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call an int-status entry point and raise on a non-zero status."""
-    check(getattr(lib(), name)(*args), name)
+    code = getattr(_lib or lib(), name)(*args)
+    if code:
+        check(code, name)

@@ -41,7 +41,9 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle of torch.cuda.current_stream(), without building the stream object (every caller holds a GPU
+    # tensor, so the runtime is up)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dt(t: torch.Tensor, name: str) -> int:
