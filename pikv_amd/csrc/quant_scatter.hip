@@ -40,7 +40,7 @@ struct QuantScatterArgs {
   const float* seg_score;  // optional: initial accumulator of a gathered row, by source row
   int64_t n_src;
   int64_t dst_row0;     // used when cache_id == nullptr
-  int64_t rows_per_cache;  // append mode (> 0, cache_id == nullptr): source row s goes to cache s / rows_per_cache
+  int64_t rows_per_cache;  // append mode: source row s goes to cache s / rows_per_cache
                            // as its new row s % rows_per_cache
   int fanout;
   int D;
@@ -92,8 +92,10 @@ struct RawRow {
 // ROW_UNIFORM: lanes_per_row is a power of two >= 64, so a wavefront never spans two
 // source rows; the row index, its destinations and every address base are then
 // wave-uniform and live in scalar registers.
-// ROUTED (FANOUT 1): a K row per token, a V row per token and cache, one assignment per s.
-template <int SCHEME, int SRC_DT, int FANOUT, bool ROW_UNIFORM, bool ROUTED = false>
+// MODE, both with FANOUT 1 and instantiations of their own (as run-time branches they cost the prefill scatter 0.8 %):
+// ROUTED: a K row per token, a V row per token and cache, one assignment per s; APPEND: rows in cache order.
+enum QuantMode { PLAIN, ROUTED, APPEND };
+template <int SCHEME, int SRC_DT, int FANOUT, bool ROW_UNIFORM, QuantMode MODE = PLAIN>
 __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) {
   using Q = QScheme<SCHEME>;
   constexpr int EPL = Q::epl;
@@ -121,7 +123,7 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) 
   bool valid = s < a.n_src;
   int64_t srow = s;  // row of src[] this lane reads
   int64_t vrow = s;
-  if constexpr (ROUTED) {
+  if constexpr (MODE == ROUTED) {
     srow = s / a.src_div;
     vrow = valid ? (int64_t)a.cache_id[s] * a.v_rows + srow : 0;   // not read where the id is outside the pool
   }
@@ -144,12 +146,12 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) 
   for (int j = 0; j < FANOUT; ++j) {
     dst[j] = -1;
     if (valid && j < a.fanout) {
-      if (a.seg_index != nullptr) {
-        dst[j] = gather_dst;
-      } else if (a.cache_id == nullptr && a.rows_per_cache > 0) {
+      if constexpr (MODE == APPEND) {
         const int c = (int)(s / a.rows_per_cache);
         const int64_t r = (int64_t)a.fill[c] + (s - (int64_t)c * a.rows_per_cache);
         if (r < a.cap[c]) dst[j] = a.row_base[c] + r;
+      } else if (a.seg_index != nullptr) {
+        dst[j] = gather_dst;
       } else if (a.cache_id == nullptr) {
         dst[j] = a.dst_row0 + s;
       } else {
@@ -189,7 +191,7 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) 
     // The V row is fetched only now: holding both raw rows across the K arithmetic cost
     // the registers of one to two resident wavefronts per SIMD (4-bit: 86 -> 68 registers,
     // 150 -> 125 us at 131072 rows x 1024), and the other wavefronts cover the wait.
-    if (t == 1 && live) raw[1].load(a.src[1], (ROUTED ? vrow : srow) * a.D + (int64_t)part * EPL);
+    if (t == 1 && live) raw[1].load(a.src[1], (MODE == ROUTED ? vrow : srow) * a.D + (int64_t)part * EPL);
     float x[EPL];
     raw[t].to_float(x);
     float mn = x[0], mx = x[0];
@@ -265,8 +267,9 @@ static int launch_quant(QuantScatterArgs a, int src_dtype, hipStream_t st) {
   return PIKV_OK;
 }
 
-template <int SCHEME>
-static int launch_routed(QuantScatterArgs a, hipStream_t st) {
+// The modes with an instantiation of their own: one destination per source row.
+template <int SCHEME, int SRC_DT, QuantMode MODE>
+static int launch_mode(QuantScatterArgs a, hipStream_t st) {
   using Q = QScheme<SCHEME>;
   const int lanes_per_row = a.D / Q::epl;
   a.lpr_shift = -1;
@@ -280,11 +283,21 @@ static int launch_routed(QuantScatterArgs a, hipStream_t st) {
   if (blocks == 0) return PIKV_OK;
   if (blocks > 0x7fffffffLL) return PIKV_ERR_SHAPE;
   if (a.lpr_shift >= 6)
-    hipLaunchKernelGGL((quant_scatter_kernel<SCHEME, PIKV_F32, 1, true, true>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((quant_scatter_kernel<SCHEME, SRC_DT, 1, true, MODE>), dim3((unsigned)blocks), dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((quant_scatter_kernel<SCHEME, PIKV_F32, 1, false, true>), dim3((unsigned)blocks), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((quant_scatter_kernel<SCHEME, SRC_DT, 1, false, MODE>), dim3((unsigned)blocks), dim3(256), 0, st, a);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
+}
+
+template <int SRC_DT, QuantMode MODE>
+static int dispatch_mode(const QuantScatterArgs& a, int scheme, hipStream_t st) {
+  switch (scheme) {
+    case PIKV_Q_I8_SYM: return launch_mode<PIKV_Q_I8_SYM, SRC_DT, MODE>(a, st);
+    case PIKV_Q_I8_ASYM: return launch_mode<PIKV_Q_I8_ASYM, SRC_DT, MODE>(a, st);
+    case PIKV_Q_I4_ASYM: return launch_mode<PIKV_Q_I4_ASYM, SRC_DT, MODE>(a, st);
+    default: return launch_mode<PIKV_Q_I4_SYM, SRC_DT, MODE>(a, st);
+  }
 }
 
 static int check_quant_shape(int D, int group, int scheme) {
@@ -379,13 +392,7 @@ extern "C" int pikv_quant_scatter_routed(const float* k_src, const float* v_src,
   a.src_div = per_token; a.v_rows = n_tokens;
   a.n_tensors = 2;
   a.n_caches = n_caches;
-  hipStream_t st = (hipStream_t)stream;
-  switch (scheme) {
-    case PIKV_Q_I8_SYM: return launch_routed<PIKV_Q_I8_SYM>(a, st);
-    case PIKV_Q_I8_ASYM: return launch_routed<PIKV_Q_I8_ASYM>(a, st);
-    case PIKV_Q_I4_ASYM: return launch_routed<PIKV_Q_I4_ASYM>(a, st);
-    default: return launch_routed<PIKV_Q_I4_SYM>(a, st);
-  }
+  return dispatch_mode<PIKV_F32, ROUTED>(a, scheme, (hipStream_t)stream);
 }
 
 extern "C" int pikv_quant_append(const void* k_src, const void* v_src, int src_dtype, int64_t rows_per_cache, int D,
@@ -411,7 +418,9 @@ extern "C" int pikv_quant_append(const void* k_src, const void* v_src, int src_d
   a.n_src = rows_per_cache * n_caches; a.rows_per_cache = rows_per_cache; a.fanout = 1; a.D = D; a.group = group;
   a.n_tensors = v_src ? 2 : 1;
   a.n_caches = n_caches;
-  return dispatch_quant(a, scheme, src_dtype, (hipStream_t)stream);
+  hipStream_t st = (hipStream_t)stream;
+  return src_dtype == PIKV_BF16 ? dispatch_mode<PIKV_BF16, APPEND>(a, scheme, st)
+                                : dispatch_mode<PIKV_F32, APPEND>(a, scheme, st);
 }
 
 extern "C" int pikv_quant_gather(const void* k_src, const void* v_src, int src_dtype, int D,
