@@ -1007,7 +1007,13 @@ __global__ __launch_bounds__(64) void slot_scan_kernel(int32_t* __restrict__ ws,
 // SELF_PREFIX: ws holds the raw per-chunk histograms and every block adds up the chunks before
 // its own by itself (integer sums: the order does not matter); the last block also writes the
 // totals.  For short assignment streams this saves the scan launch, which is all latency there.
-template <bool SELF_PREFIX>
+// SELF_COUNT: no histograms at all, every block counts the assignments before its own chunk itself (and the last one
+// writes the totals): one launch instead of two for streams of up to kSlotSelfCountChunks chunks, where the last block
+// reads 30 KB for it (with the accumulation's own statistics in read_path.hip: a prefill step of 3 x 577 tokens
+// 70 -> 65 us).
+enum SlotPrefix { SCANNED, SELF_PREFIX, SELF_COUNT };
+constexpr int64_t kSlotSelfCountChunks = 16;
+template <SlotPrefix PREFIX>
 __global__ __launch_bounds__(256) void slot_rank_kernel(const int32_t* __restrict__ idx, int64_t A,
                                                         int E, int64_t capacity,
                                                         const int32_t* __restrict__ ws,
@@ -1017,7 +1023,35 @@ __global__ __launch_bounds__(256) void slot_rank_kernel(const int32_t* __restric
   __shared__ int wcnt[4][64];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  if constexpr (SELF_PREFIX) {
+  // lanes with the same expert: one ballot per bit of the expert id, and every lane keeps
+  // the side of each ballot it is on (six ballots instead of one round per distinct expert)
+  auto same_expert = [&](int e, bool valid) {
+    uint64_t same = __ballot(valid);
+#pragma unroll
+    for (int bit = 0; bit < 6; ++bit) {
+      const uint64_t ones = __ballot(valid && ((e >> bit) & 1));
+      same &= ((e >> bit) & 1) ? ones : ~ones;
+    }
+    return same;
+  };
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  if constexpr (PREFIX == SELF_COUNT) {
+    if (threadIdx.x < 64) running[threadIdx.x] = 0;
+    __syncthreads();
+    const int n = (int)blockIdx.x * kSlotChunk;   // all below A: only the last chunk can be short
+    for (int p0 = threadIdx.x; p0 < n; p0 += 256 * 8) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = (p0 + u * 256 < n) ? idx[p0 + u * 256] : -1;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const bool valid = (unsigned)v[u] < (unsigned)E;
+        const uint64_t same = same_expert(v[u], valid);
+        if (valid && (same & lt_mask) == 0) atomicAdd(&running[v[u]], __popcll(same));
+      }
+    }
+    __syncthreads();
+  } else if constexpr (PREFIX == SELF_PREFIX) {
     if (threadIdx.x < 64) running[threadIdx.x] = 0;
     __syncthreads();
     const int n = (int)blockIdx.x * E;  // words of the earlier chunks, [chunk][expert]
@@ -1037,7 +1071,6 @@ __global__ __launch_bounds__(256) void slot_rank_kernel(const int32_t* __restric
       running[threadIdx.x] = ((int)threadIdx.x < E) ? ws[(int64_t)blockIdx.x * E + threadIdx.x] : 0;
   }
   const int64_t base = (int64_t)blockIdx.x * kSlotChunk;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   for (int step = 0; step < kSlotChunk / 256; ++step) {
     wcnt[wave][lane] = 0;
     __syncthreads();
@@ -1048,14 +1081,7 @@ __global__ __launch_bounds__(256) void slot_rank_kernel(const int32_t* __restric
       if ((unsigned)e >= (unsigned)E) e = -1;  // out-of-range ids get slot -1
     }
     const bool valid = e >= 0;
-    // lanes with the same expert: one ballot per bit of the expert id, and every lane keeps
-    // the side of each ballot it is on (six ballots instead of one round per distinct expert)
-    uint64_t same = __ballot(valid);
-#pragma unroll
-    for (int bit = 0; bit < 6; ++bit) {
-      const uint64_t ones = __ballot(valid && ((e >> bit) & 1));
-      same &= ((e >> bit) & 1) ? ones : ~ones;
-    }
+    const uint64_t same = same_expert(e, valid);
     const int rank = __popcll(same & lt_mask);
     if (valid && rank == 0) wcnt[wave][e] = __popcll(same);
     __syncthreads();
@@ -1072,6 +1098,8 @@ __global__ __launch_bounds__(256) void slot_rank_kernel(const int32_t* __restric
                               wcnt[3][threadIdx.x];
     __syncthreads();
   }
+  if (PREFIX == SELF_COUNT && count && blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < E)
+    count[threadIdx.x] = running[threadIdx.x];
 }
 
 static int64_t slot_chunks(int64_t A) { return (A + kSlotChunk - 1) / kSlotChunk; }
@@ -1095,13 +1123,19 @@ static int launch_slots(const int32_t* idx, int64_t A, int E, int64_t capacity, 
   if (ws_bytes < slot_workspace_bytes(A, E)) return PIKV_ERR_WORKSPACE;
   const int64_t nb = slot_chunks(A);
   if (nb > 0x7fffffffLL) return PIKV_ERR_SHAPE;
+  if (nb <= kSlotSelfCountChunks) {
+    hipLaunchKernelGGL((slot_rank_kernel<SELF_COUNT>), dim3((unsigned)nb), dim3(256), 0, st, idx, A, E, capacity,
+                       (const int32_t*)nullptr, slot, count);
+    PIKV_CHECK_LAUNCH();
+    return PIKV_OK;
+  }
   hipLaunchKernelGGL(slot_hist_kernel, dim3((unsigned)nb), dim3(256), 0, st, idx, A, E, (int32_t*)ws);
   if (nb * E <= kSlotSelfPrefixWords) {
-    hipLaunchKernelGGL((slot_rank_kernel<true>), dim3((unsigned)nb), dim3(256), 0, st, idx, A, E, capacity,
+    hipLaunchKernelGGL((slot_rank_kernel<SELF_PREFIX>), dim3((unsigned)nb), dim3(256), 0, st, idx, A, E, capacity,
                        (const int32_t*)ws, slot, count);
   } else {
     hipLaunchKernelGGL(slot_scan_kernel, dim3((unsigned)E), dim3(64), 0, st, (int32_t*)ws, nb, E, count);
-    hipLaunchKernelGGL((slot_rank_kernel<false>), dim3((unsigned)nb), dim3(256), 0, st, idx, A, E, capacity,
+    hipLaunchKernelGGL((slot_rank_kernel<SCANNED>), dim3((unsigned)nb), dim3(256), 0, st, idx, A, E, capacity,
                        (const int32_t*)ws, slot, count);
   }
   PIKV_CHECK_LAUNCH();

@@ -146,3 +146,66 @@ def test_prefill_attend(dev, scheme, heads, hq, dh, group, S, lens, causal):
             p = np.exp(s - s.max(axis=1, keepdims=True))
             want = (p / p.sum(axis=1, keepdims=True)) @ vv[:, h // (hq // heads)]
             assert np.abs(got[b, :, h] - want).max() <= 4 * 2.0 ** -24 * np.sqrt(dh + n + S) * size
+
+
+@pytest.mark.parametrize("A", [1, 255, 512, 513, 8191, 8192, 8193, 16000])
+@pytest.mark.parametrize("E,capacity", [(1, 5000), (8, 700), (64, 90)])
+def test_capacity_slots_chunks(dev, A, E, capacity):
+    """Slots and totals on both sides of the lengths where blocks count the assignments before them by themselves,
+    ids out of range among them."""
+    from pikv_amd import ops
+    r = rng(A + E)
+    idx = r.integers(0, E, A).astype(np.int32)
+    idx[3::97] = E
+    idx[5::89] = -1
+    slot, count = (np_of(t) for t in ops.capacity_slots(to_dev(idx, dev), E, capacity))
+    seen = np.zeros(E, dtype=np.int64)
+    for a, e in enumerate(idx):
+        want = -1
+        if 0 <= e < E:
+            want = seen[e] if seen[e] < capacity else -1
+            seen[e] += 1
+        assert slot[a] == want
+    assert np.array_equal(count, seen)
+
+
+@pytest.mark.parametrize("cap,lens,hq", [(64, [64, 0], 1), (2048, [2048, 65], 64), (2049, [2049, 1], 64),
+                                         (2048, [1983, 64], 65)])
+@pytest.mark.parametrize("write_probs", [False, True])
+def test_h2o_accumulate_own_statistics(dev, cap, lens, hq, write_probs):
+    """On both sides of 32 tiles and 64 heads, where the accumulation merges the tile statistics by itself: importance,
+    accumulators, probabilities and head statistics against float64.  Probabilities are float32 exponentials of score
+    differences below 30: 2^-24 * 30 of each, with a factor of four."""
+    from pikv_amd import ops
+    import torch
+    r = rng(cap + hq)
+    pool = ops.CachePool([cap] * 2, 1, 64, 64, O.Q_I8_SYM, dev)
+    pool.fill.copy_(torch.tensor(lens, dtype=torch.int32))
+    s = (4 * r.standard_normal((2, hq, cap))).astype(np.float32)
+    n_tiles = (cap + 63) // 64
+    tmax = np.full((2, n_tiles, hq), -np.inf, dtype=np.float32)
+    tsum = np.zeros((2, n_tiles, hq), dtype=np.float32)
+    for c, n in enumerate(lens):
+        for t in range((n + 63) // 64):
+            x = s[c, :, 64 * t:min(64 * t + 64, n)].astype(np.float64)
+            tmax[c, t] = x.max(axis=1)
+            tsum[c, t] = np.exp(x - x.max(axis=1, keepdims=True)).sum(axis=1)
+    sd = to_dev(s, dev)
+    imp = np_of(pool.h2o_accumulate(sd, to_dev(tmax, dev), to_dev(tsum, dev), now=2.0, write_probs=write_probs,
+                                    return_importance=True))
+    stats, acc, ts, probs = np_of(pool.head_stats), np_of(pool.acc), np_of(pool.ts), np_of(sd)
+    tol = 4 * 30 * 2.0 ** -24
+    for c, n in enumerate(lens):
+        if n == 0:
+            assert not acc[c * cap:(c + 1) * cap].any() and np.isneginf(stats[c, :, 0]).all()
+            continue
+        x = s[c, :, :n].astype(np.float64)
+        p = np.exp(x - x.max(axis=1, keepdims=True))
+        np.testing.assert_allclose(stats[c, :, 0], x.max(axis=1), rtol=0)
+        np.testing.assert_allclose(stats[c, :, 1], p.sum(axis=1), rtol=tol)
+        p /= p.sum(axis=1, keepdims=True)
+        np.testing.assert_allclose(imp[c, :n], p.sum(axis=0), rtol=tol)
+        np.testing.assert_allclose(acc[c * cap:c * cap + n], p.sum(axis=0), rtol=tol)
+        assert (ts[c * cap:c * cap + n] == 2.0).all() and not acc[c * cap + n:(c + 1) * cap].any()
+        if write_probs:
+            np.testing.assert_allclose(probs[c, :, :n], p, rtol=tol)
