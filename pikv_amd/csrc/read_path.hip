@@ -1241,9 +1241,15 @@ static void launch_head_stats(const float* tile_max, const float* tile_sum, cons
 
 // VEC consecutive tokens per thread (16-byte accesses when VEC = 4) and four q
 // heads per round, their loads issued before any store of the round.
-template <int VEC, bool WRITE_PROBS>
+// OWN_STATS: every block merges the tile statistics of its cache's heads by itself (and the first block of a cache
+// leaves them in head_stats) instead of a head_stats_kernel launch before it: up to kOwnStatHeads heads and
+// kOwnStatTiles tiles, 16 KB of statistics, where that launch's 4.4 us are latency (with the one-launch capacity
+// slots: a prefill step of 3 x 577 tokens 70 -> 65 us).
+constexpr int kOwnStatHeads = 64, kOwnStatTiles = 32;
+template <int VEC, bool WRITE_PROBS, bool OWN_STATS = false>
 __global__ __launch_bounds__(256) void h2o_accumulate_kernel(
-    float* __restrict__ scores, const float* __restrict__ head_stats, int n_q_heads,
+    float* __restrict__ scores, const float* __restrict__ tile_max, const float* __restrict__ tile_sum, int64_t n_tiles,
+    float* __restrict__ head_stats, int n_q_heads,
     const int64_t* __restrict__ row_base, const int32_t* __restrict__ fill, int64_t max_len,
     int64_t score_stride, float decay, float now, float* __restrict__ row_acc, float* __restrict__ row_ts,
     float* __restrict__ importance_out) {
@@ -1251,9 +1257,42 @@ __global__ __launch_bounds__(256) void h2o_accumulate_kernel(
   const int c = blockIdx.y;
   const int64_t n0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
   const int64_t len = fill[c] < max_len ? (int64_t)fill[c] : max_len;
+  const float* hs = head_stats + (int64_t)c * n_q_heads * 2;
+  if constexpr (OWN_STATS) {
+    __shared__ float sm[4][kOwnStatHeads], sz[4][kOwnStatHeads], merged[2 * kOwnStatHeads];
+    const int hq = threadIdx.x & 63, tl = threadIdx.x >> 6;   // one head per lane, every fourth tile per wavefront
+    const int lim = (int)((len + kTile - 1) / kTile);          // at most n_tiles
+    float m = -__builtin_inff(), z = 0.f;
+    if (hq < n_q_heads) {
+      float tm[kOwnStatTiles / 4], ts[kOwnStatTiles / 4];
+#pragma unroll
+      for (int u = 0; u < kOwnStatTiles / 4; ++u) {
+        const int t = tl + 4 * u;
+        const int64_t i = ((int64_t)c * n_tiles + (t < lim ? t : 0)) * n_q_heads + hq;
+        tm[u] = t < lim ? tile_max[i] : -__builtin_inff();
+        ts[u] = t < lim ? tile_sum[i] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < kOwnStatTiles / 4; ++u) stat_merge(m, z, tm[u], ts[u]);
+    }
+    sm[tl][hq] = m;
+    sz[tl][hq] = z;
+    __syncthreads();
+    if (tl == 0 && hq < n_q_heads) {
+#pragma unroll
+      for (int k = 1; k < 4; ++k) stat_merge(m, z, sm[k][hq], sz[k][hq]);
+      merged[2 * hq] = m;
+      merged[2 * hq + 1] = z;
+      if (blockIdx.x == 0) {
+        head_stats[((int64_t)c * n_q_heads + hq) * 2] = m;
+        head_stats[((int64_t)c * n_q_heads + hq) * 2 + 1] = z;
+      }
+    }
+    __syncthreads();
+    hs = merged;
+  }
   if (n0 >= len) return;
   const int cnt = (len - n0 < VEC) ? (int)(len - n0) : VEC;
-  const float* hs = head_stats + (int64_t)c * n_q_heads * 2;
   float* sc = scores + (int64_t)c * n_q_heads * score_stride + n0;
   float imp[VEC];
 #pragma unroll
@@ -1543,9 +1582,10 @@ extern "C" int pikv_h2o_accumulate(float* scores, const float* tile_max, const f
   if (max_len == 0) return PIKV_OK;
   const int64_t n_tiles = (max_len + kTile - 1) / kTile;
   hipStream_t st = (hipStream_t)stream;
-  launch_head_stats(tile_max, tile_sum, cache_fill, n_q_heads, n_tiles, n_caches, head_stats, st);
-  // nothing to normalise or accumulate: the caller only wanted the statistics
-  if (!write_probs && !row_acc && !row_ts && !importance_out) {
+  const bool stats_only = !write_probs && !row_acc && !row_ts && !importance_out;
+  const bool own_stats = !stats_only && n_q_heads <= kOwnStatHeads && n_tiles <= kOwnStatTiles;
+  if (!own_stats) launch_head_stats(tile_max, tile_sum, cache_fill, n_q_heads, n_tiles, n_caches, head_stats, st);
+  if (stats_only) {   // nothing to normalise or accumulate
     PIKV_CHECK_LAUNCH();
     return PIKV_OK;
   }
@@ -1559,11 +1599,15 @@ extern "C" int pikv_h2o_accumulate(float* scores, const float* tile_max, const f
   const int64_t nb = (max_len + per_block - 1) / per_block;
   if (nb > 0x7fffffffLL) return PIKV_ERR_SHAPE;
   const dim3 grid((unsigned)nb, (unsigned)n_caches);
-#define PIKV_H2O_LAUNCH(V, W)                                                                       \
-  hipLaunchKernelGGL((h2o_accumulate_kernel<V, W>), grid, dim3(256), 0, st, scores, head_stats,     \
-                     n_q_heads, cache_row_base, cache_fill, max_len, score_stride, decay, now, row_acc, \
+#define PIKV_H2O_LAUNCH(...)                                                                        \
+  hipLaunchKernelGGL((h2o_accumulate_kernel<__VA_ARGS__>), grid, dim3(256), 0, st, scores, tile_max, tile_sum, n_tiles, \
+                     head_stats, n_q_heads, cache_row_base, cache_fill, max_len, score_stride, decay, now, row_acc, \
                      row_ts, importance_out)
-  if (vec4) {
+  if (own_stats && vec4) {
+    if (write_probs) PIKV_H2O_LAUNCH(4, true, true); else PIKV_H2O_LAUNCH(4, false, true);
+  } else if (own_stats) {
+    if (write_probs) PIKV_H2O_LAUNCH(1, true, true); else PIKV_H2O_LAUNCH(1, false, true);
+  } else if (vec4) {
     if (write_probs) PIKV_H2O_LAUNCH(4, true); else PIKV_H2O_LAUNCH(4, false);
   } else {
     if (write_probs) PIKV_H2O_LAUNCH(1, true); else PIKV_H2O_LAUNCH(1, false);
