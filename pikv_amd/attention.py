@@ -262,9 +262,9 @@ class PiKVAttention(nn.Module):
             return False
         if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
             return False
-        if not (q.dtype == k.dtype == v.dtype == torch.float32):
+        if not all(type(t) is torch.Tensor and t.dtype == torch.float32 for t in (q, k, v)) or not dense.ordinary_call():
             return False
-        if type(self.attn_dropout) is not nn.Dropout or (self.attn_dropout.training and self.attn_dropout.p > 0):
+        if not dense.plain(self.attn_dropout, nn.Dropout) or (self.attn_dropout.training and self.attn_dropout.p > 0):
             return False
         return 0 < q.shape[1] * (self.num_heads // self.num_kv_heads) <= 65535 * 32
 

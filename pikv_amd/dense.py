@@ -25,26 +25,26 @@ def plain(m, cls) -> bool:
     return type(m) is cls and _no_hooks(m)
 
 
-def _ordinary_call() -> bool:
+def ordinary_call() -> bool:
     return not (_module._has_any_global_hook() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
                 or torch.compiler.is_compiling() or forward_ad._current_level >= 0
                 or torch._C._functorch.peek_interpreter_stack() is not None)
 
 
-def _ordinary_tensor(t, device, dtype=torch.float32) -> bool:
+def ordinary_tensor(t, device, dtype=torch.float32) -> bool:
     return (type(t) in (torch.Tensor, nn.Parameter) and t.device == device and t.dtype == dtype and t.is_contiguous()
             and torch._C._has_storage(t) and t.data_ptr() % 16 == 0)      # a batched tensor has none
 
 
 def forward_only(x) -> bool:
     """A float32 GPU input of a pass that records nothing."""
-    return not torch.is_grad_enabled() and x.is_cuda and _ordinary_tensor(x, x.device) and _ordinary_call()
+    return not torch.is_grad_enabled() and x.is_cuda and ordinary_tensor(x, x.device) and ordinary_call()
 
 
 def linear_ok(m, n_in: int, n_out: int, device) -> bool:
     """A plain nn.Linear of this shape with a bias, as linear_group reads it."""
     return (plain(m, nn.Linear) and m.bias is not None and m.weight.shape == (n_out, n_in)
-            and _ordinary_tensor(m.weight, device) and _ordinary_tensor(m.bias, device))
+            and ordinary_tensor(m.weight, device) and ordinary_tensor(m.bias, device))
 
 
 def mlp_ok(seq, acts, sizes, device) -> bool:

@@ -226,7 +226,7 @@ class PiKVMoE(nn.Module):
     def _lora_ok(self, m, rank, device):
         H = config['hidden_size']
         return (dense.plain(m, LoRALayer) and type(m.scaling) in (int, float) and m.lora_A.shape == (H, rank) and m.lora_B.shape == (rank, H)
-                and dense._ordinary_tensor(m.lora_A, device) and dense._ordinary_tensor(m.lora_B, device)
+                and dense.ordinary_tensor(m.lora_A, device) and dense.ordinary_tensor(m.lora_B, device)
                 and dense.plain(m.dropout, nn.Dropout) and not (m.dropout.training and m.dropout.p > 0))
 
     def _native_experts(self, x, routing_weights) -> bool:
@@ -237,7 +237,7 @@ class PiKVMoE(nn.Module):
         if not (not self.training and dense.forward_only(x) and x.numel() > 0 and H % 128 == 0 and H == config['hidden_size']
                 and E == config['num_experts'] <= dense.MAX_LAYERS and len(self.kv_caches) == E):
             return False
-        if not (dense._ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)
+        if not (dense.ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)
                 and x.shape[0] * x.shape[1] <= 65535 * 32):
             return False
         rank = self.key_lora.lora_A.shape[1]

@@ -151,3 +151,32 @@ def test_moe_native_forward_equals_module_path(dev, H, policy):
     finally:
         config.clear()
         config.update(saved)
+
+
+def test_native_prompt_attention_leaves_other_calls_alone(dev):
+    """Hooks, dropout, masks, gradients, other types and forward-mode tangents keep the torch path; the two paths agree
+    on what both take (float32 sums of some 200 products: 1e-5 of outputs of order one)."""
+    import torch
+    from torch.autograd import forward_ad
+    from pikv_amd.attention import PiKVAttention
+    torch.manual_seed(0)
+    layer = PiKVAttention(128, 4, head_dim=64, cache_size=64, num_kv_heads=2).to(dev).eval()
+    q, k, v = (torch.randn(2, 9, h, 64, device=dev) for h in (4, 2, 2))
+    with torch.no_grad():
+        assert layer._native_prefill(q, k, v, None)
+        assert not layer._native_prefill(q, k, v, torch.ones(2, 9, device=dev))
+        assert not layer._native_prefill(q.bfloat16(), k.bfloat16(), v.bfloat16(), None)
+        with forward_ad.dual_level():
+            assert not layer._native_prefill(forward_ad.make_dual(q, q), k, v, None)
+        handle = layer.attn_dropout.register_forward_hook(lambda *a: None)
+        x = torch.randn(2, 9, 128, device=dev)
+        assert not layer._native_prefill(q, k, v, None)
+        want = [layer(x)[0] for _ in range(2)]           # the second call attends to the first one's rows
+        handle.remove()
+        layer.reset_cache()
+        for w in want:
+            assert torch.allclose(layer(x)[0], w, rtol=0, atol=1e-5)
+        layer.train()
+        assert not layer._native_prefill(q, k, v, None)
+    layer.eval()
+    assert not layer._native_prefill(q.requires_grad_(), k, v, None)
