@@ -45,6 +45,13 @@ struct PrefillArgs {
   float scale_qk;
 };
 
+// Orders the LDS accesses of a wavefront's lanes before it against those after it.
+__device__ __forceinline__ void wave_lds_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The tile's K rows, 16 bytes a lane along the rows, into the wavefront's LDS rows of QP floats.
 template <int DH, int QP>
 __device__ __forceinline__ void stage_own_k(const float* k, int D, int last, int lane, float* rows) {
@@ -172,10 +179,10 @@ __global__ __launch_bounds__(64 * kPfWaves, 2) void prefill_attend_kernel(Prefil
     // the tile's rows; rows past the end are read from the last one and masked
     const int last = n_keys - key0 < kPfKeys ? (int)(n_keys - key0) - 1 : kPfKeys - 1;
     const int64_t own0 = (((int64_t)b * a.S + key0) * a.n_kv + kvh) * DH;   // of the chunk's own rows
-    __builtin_amdgcn_wave_barrier();     // the reads of the tile before come first
+    wave_lds_exchange();                 // the reads of the tile before come first
     if (past) stage_cached_k<SCHEME, DH, QP>(a, base + key0, kvh, last, lane, krows);
     else stage_own_k<DH, QP>(a.k + own0, D, last, lane, krows);
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_exchange();
     // V of keys 16 g + 4 half + (0..3) and 16 g + 8 + 4 half + (0..3): the first half of them is in flight
     // during the scores, the second during the softmax
     auto load_v = [&](int g, float (&vf)[8][NC]) {
