@@ -2,7 +2,8 @@
 
 linear_group / adaptive_router / expert_combine (csrc/moe.hip) serve forward passes without autograd,
 over modules that are what their class says: a subclass, a hook, an instance-level forward, autocast,
-a functorch transform or forward-mode differentiation all go through the module's own call.
+a functorch transform, forward-mode differentiation, a tracer or any other mode that watches torch's calls
+all go through the module's own call.
 """
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
+from torch.utils._device import DeviceContext
 
 MAX_LORA_RANK = 8
 MAX_LAYERS = 20          # of one linear_group or expert_combine launch
@@ -25,8 +27,17 @@ def plain(m, cls) -> bool:
     return type(m) is cls and _no_hooks(m)
 
 
+def _watched() -> bool:
+    """A function or dispatch mode (make_fx, a user's) sees torch's calls; to it the output of a kernel launched beside them is a
+    constant.  A default device is a function mode too, but one that only places new tensors."""
+    if torch._C._len_torch_dispatch_stack() or torch._ops._len_torch_dispatch_stack_pre_dispatch():
+        return True
+    n = torch._C._len_torch_function_stack()
+    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
+
+
 def ordinary_call() -> bool:
-    return not (_module._has_any_global_hook() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+    return not (_watched() or _module._has_any_global_hook() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
                 or torch.compiler.is_compiling() or forward_ad._current_level >= 0
                 or torch._C._functorch.peek_interpreter_stack() is not None)
 
