@@ -7,11 +7,35 @@ all go through the module's own call.
 """
 from __future__ import annotations
 
+from functools import reduce
+
 import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
-from torch.nn.modules import module as _module
-from torch.utils._device import DeviceContext
+
+try:
+    from torch.utils._device import DeviceContext as _DeviceContext
+except ImportError:
+    _DeviceContext = None
+
+
+def _internal(path: str):
+    """torch.<path>, or None in a version of torch that does not have it."""
+    return reduce(lambda o, name: getattr(o, name, None), path.split("."), torch)
+
+
+# What tells whether something watches a call is internal to torch.  Where a name is missing the answer is yes:
+# every layer takes its module's own call.
+_dispatch_modes = _internal("_C._len_torch_dispatch_stack")
+_pre_dispatch_modes = _internal("_ops._len_torch_dispatch_stack_pre_dispatch")
+_function_modes = _internal("_C._len_torch_function_stack")
+_function_mode_at = _internal("_C._get_function_stack_at")
+_has_global_hook = _internal("nn.modules.module._has_any_global_hook")
+_transforms = _internal("_C._functorch.peek_interpreter_stack")
+_has_storage = _internal("_C._has_storage")
+_KNOWN = (hasattr(forward_ad, "_current_level")
+          and None not in (_dispatch_modes, _pre_dispatch_modes, _function_modes, _function_mode_at, _DeviceContext,
+                           _has_global_hook, _transforms, _has_storage))
 
 MAX_LORA_RANK = 8
 MAX_LAYERS = 20          # of one linear_group or expert_combine launch
@@ -30,26 +54,27 @@ def plain(m, cls) -> bool:
 def _watched() -> bool:
     """A function or dispatch mode (make_fx, a user's) sees torch's calls; to it the output of a kernel launched beside them is a
     constant.  A default device is a function mode too, but one that only places new tensors."""
-    if torch._C._len_torch_dispatch_stack() or torch._ops._len_torch_dispatch_stack_pre_dispatch():
+    if _dispatch_modes() or _pre_dispatch_modes():
         return True
-    n = torch._C._len_torch_function_stack()
-    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
+    n = _function_modes()
+    return n > 0 and any(type(_function_mode_at(i)) is not _DeviceContext for i in range(n))
 
 
 def ordinary_call() -> bool:
-    return not (_watched() or _module._has_any_global_hook() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
-                or torch.compiler.is_compiling() or forward_ad._current_level >= 0
-                or torch._C._functorch.peek_interpreter_stack() is not None)
+    # (is_compiling comes first: what follows it would break a compiled graph)
+    return _KNOWN and not (torch.compiler.is_compiling() or _watched() or _has_global_hook()
+                           or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+                           or forward_ad._current_level >= 0 or _transforms() is not None)
 
 
 def ordinary_tensor(t, device, dtype=torch.float32) -> bool:
     return (type(t) in (torch.Tensor, nn.Parameter) and t.device == device and t.dtype == dtype and t.is_contiguous()
-            and torch._C._has_storage(t) and t.data_ptr() % 16 == 0)      # a batched tensor has none
+            and _has_storage(t) and t.data_ptr() % 16 == 0)      # a batched tensor has none
 
 
 def forward_only(x) -> bool:
     """A float32 GPU input of a pass that records nothing."""
-    return not torch.is_grad_enabled() and x.is_cuda and ordinary_tensor(x, x.device) and ordinary_call()
+    return not torch.is_grad_enabled() and x.is_cuda and ordinary_call() and ordinary_tensor(x, x.device)
 
 
 def linear_ok(m, n_in: int, n_out: int, device) -> bool:

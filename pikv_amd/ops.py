@@ -40,10 +40,16 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# the raw handle of torch.cuda.current_stream(), without building the stream object (every caller holds a GPU
+# tensor, so the runtime is up); by the public way in a version of torch that names the two calls otherwise
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> int:
-    # the raw handle of torch.cuda.current_stream(), without building the stream object (every caller holds a GPU
-    # tensor, so the runtime is up)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _dt(t: torch.Tensor, name: str) -> int:

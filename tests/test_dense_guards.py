@@ -1,12 +1,15 @@
 """When the native forms of float32 layers stand back: CPU checks of the conditions on the call."""
 import contextlib
+import importlib
+from types import SimpleNamespace
 
 import pytest
 import torch
+import torch.utils._device
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from pikv_amd import dense
+from pikv_amd import dense, ops
 
 
 class _FunctionMode(TorchFunctionMode):
@@ -43,3 +46,33 @@ def test_make_fx_is_noticed(tracing, pre_dispatch):
 
     make_fx(f, tracing_mode=tracing, pre_dispatch=pre_dispatch)(torch.ones(3))
     assert seen and not any(seen)
+
+
+def test_compiled_call_is_noticed_without_a_graph_break():
+    def f(x):
+        return x + 1 if dense.ordinary_call() else x + 2
+
+    assert torch.compile(f, backend="eager", fullgraph=True)(torch.zeros(())) == 2
+
+
+@pytest.mark.parametrize("name", [
+    "_C._len_torch_dispatch_stack", "_ops._len_torch_dispatch_stack_pre_dispatch", "_C._len_torch_function_stack",
+    "_C._get_function_stack_at", "utils._device.DeviceContext", "nn.modules.module._has_any_global_hook",
+    "_C._functorch.peek_interpreter_stack", "_C._has_storage", "autograd.forward_ad._current_level"])
+def test_without_a_torch_internal_the_modules_run(monkeypatch, name):
+    """A version of torch that lacks one of the internals: no error, and nothing counts as an ordinary call."""
+    owner, attr = torch, name.split(".")
+    for a in attr[:-1]:
+        owner = getattr(owner, a)
+    with monkeypatch.context() as m:
+        m.delattr(owner, attr[-1])
+        importlib.reload(dense)
+        ordinary = dense.ordinary_call()
+    importlib.reload(dense)
+    assert ordinary is False and dense.ordinary_call()
+
+
+def test_stream_without_the_raw_call(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=77))
+    monkeypatch.setattr(ops, "_raw_stream", None, raising=False)
+    assert ops._stream() == 77
