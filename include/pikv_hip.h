@@ -276,12 +276,14 @@ int pikv_quant_gather(const void* k_src, const void* v_src, int src_dtype,
 
 /* The same for rows that go to the caches in order: source row c*rows_per_cache + i
  * becomes row first_row[c] + i of cache c (dropped at cache_cap[c]).  first_row is the
- * cache_fill before the rows came, e.g. the new_len of pikv_cache_make_room.
+ * cache_fill before the rows came, e.g. the new_len of pikv_cache_make_room.  cache_fill
+ * [n_caches] (NULL: left alone) = min(first_row + rows_per_cache, cache_cap), written with
+ * the rows; it must not be first_row itself (PIKV_ERR_UNSUPPORTED).
  * Replaces: PiKVAttention._update_cache's write (core/single/pikv_attention.py:92-100). */
 int pikv_quant_append(const void* k_src, const void* v_src, int src_dtype,
                       int64_t rows_per_cache, int D, int group, int scheme,
                       const int64_t* cache_row_base, const int32_t* first_row,
-                      const int32_t* cache_cap, int n_caches,
+                      int32_t* cache_fill, const int32_t* cache_cap, int n_caches,
                       void* k_codes, void* v_codes,
                       void* k_scale, void* v_scale,
                       void* k_zero, void* v_zero,
@@ -534,7 +536,8 @@ int pikv_compact_rows(void* const* plane_ptrs_host,
  *     PIKV_EVICT_LRU  drop the fill + n_new - cap rows of smallest row_ts
  *     PIKV_EVICT_ALL  drop every row
  *   Planes as in pikv_compact_rows; new_len [n_caches] = rows kept (cache_fill for a cache
- *   that did not evict); cache_fill = new_len, or min(new_len + n_new, cap) with append != 0.
+ *   that did not evict); cache_fill = new_len, or min(new_len + n_new, cap) with append != 0 -
+ *   before the rows are there: a caller whose write may still fail lets pikv_quant_append advance it.
  *   keep_flag, keep_index [rows_total] and budgets int32 [3*n_caches] are scratch;
  *   max_len >= max_c cache_fill[c]; workspace as in pikv_evict_select. */
 int pikv_cache_make_room(int policy, const int32_t* count, int64_t count_all, int64_t per_call_limit,

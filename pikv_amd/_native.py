@@ -43,7 +43,7 @@ SIGNATURES = {
     "pikv_cache_advance": (_i, [_p, _p, _p, _i, _l, _p]),
     "pikv_quant_gather": (_i, [_p, _p, _i, _i, _i, _i, _p, _p, _p, _l, _p, _p, _p, _p, _i,
                                _p, _p, _p, _p, _p, _p, _p, _p, _f, _p]),
-    "pikv_quant_append": (_i, [_p, _p, _i, _l, _i, _i, _i, _p, _p, _p, _i,
+    "pikv_quant_append": (_i, [_p, _p, _i, _l, _i, _i, _i, _p, _p, _p, _p, _i,
                                _p, _p, _p, _p, _p, _p, _p, _p, _f, _p]),
     "pikv_quantize_rows": (_i, [_p, _i, _l, _i, _i, _i, _l, _p, _p, _p, _p]),
     "pikv_quant8_minshift": (_i, [_p, _i, _l, _i, _p, _p, _p, _p, _p]),

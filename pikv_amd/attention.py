@@ -132,11 +132,11 @@ class PiKVAttention(nn.Module):
         # ones, or (on_overflow="reset") none
         policy = ops.EVICT_ALL if self.on_overflow == "reset" else ops.EVICT_H2O
         pool.make_room(policy, count_all=S, heavy_ratio=self.heavy_ratio, recent_ratio=self.recent_ratio,
-                       leave_room=True, append=True)
+                       leave_room=True)
         self.clock += 1
         if k.dtype not in (torch.float32, torch.bfloat16):
             k = k.float()
-        pool.append_rows(k.contiguous(), v.to(k.dtype).contiguous(), now=float(self.clock))
+        pool.append_rows(k.contiguous(), v.to(k.dtype).contiguous(), now=float(self.clock), advance=True)
 
     def _split_past(self, past_key_values, layer_idx: Optional[int]):
         """(k, v) tensors of one layer out of what callers carry: a (k, v) pair, a tuple of

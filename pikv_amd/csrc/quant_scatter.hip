@@ -41,7 +41,8 @@ struct QuantScatterArgs {
   int64_t n_src;
   int64_t dst_row0;     // used when cache_id == nullptr
   int64_t rows_per_cache;  // append mode: source row s goes to cache s / rows_per_cache
-                           // as its new row s % rows_per_cache
+                           // as its new row s % rows_per_cache ...
+  int32_t* new_fill;       //   and its first row leaves the fill behind the new rows here, unless null
   int fanout;
   int D;
   int group;
@@ -150,6 +151,8 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(QuantScatterArgs a) 
         const int c = (int)(s / a.rows_per_cache);
         const int64_t r = (int64_t)a.fill[c] + (s - (int64_t)c * a.rows_per_cache);
         if (r < a.cap[c]) dst[j] = a.row_base[c] + r;
+        if (a.new_fill != nullptr && part == 0 && s == (int64_t)c * a.rows_per_cache)
+          a.new_fill[c] = r + a.rows_per_cache < a.cap[c] ? (int32_t)(r + a.rows_per_cache) : a.cap[c];
       } else if (a.seg_index != nullptr) {
         dst[j] = gather_dst;
       } else if (a.cache_id == nullptr) {
@@ -397,11 +400,12 @@ extern "C" int pikv_quant_scatter_routed(const float* k_src, const float* v_src,
 
 extern "C" int pikv_quant_append(const void* k_src, const void* v_src, int src_dtype, int64_t rows_per_cache, int D,
                                  int group, int scheme, const int64_t* cache_row_base, const int32_t* first_row,
-                                 const int32_t* cache_cap, int n_caches, void* k_codes, void* v_codes, void* k_scale,
+                                 int32_t* cache_fill, const int32_t* cache_cap, int n_caches, void* k_codes, void* v_codes, void* k_scale,
                                  void* v_scale, void* k_zero, void* v_zero, float* row_acc, float* row_ts, float now,
                                  void* stream) {
   if (!k_src || !k_codes || !k_scale || !cache_row_base || !first_row || !cache_cap) return PIKV_ERR_NULL;
   if (src_dtype != PIKV_F32 && src_dtype != PIKV_BF16) return PIKV_ERR_UNSUPPORTED;
+  if (cache_fill == first_row) return PIKV_ERR_UNSUPPORTED;   // every row of a cache reads its first_row
   if (rows_per_cache < 1 || n_caches < 1) return PIKV_ERR_SHAPE;
   int rc = check_quant_shape(D, group, scheme);
   if (rc != PIKV_OK) return rc;
@@ -413,7 +417,7 @@ extern "C" int pikv_quant_append(const void* k_src, const void* v_src, int src_d
   a.codes[0] = k_codes; a.codes[1] = v_codes;
   a.scale[0] = k_scale; a.scale[1] = v_scale;
   a.zero[0] = k_zero; a.zero[1] = v_zero;
-  a.row_base = cache_row_base; a.fill = first_row; a.cap = cache_cap;
+  a.row_base = cache_row_base; a.fill = first_row; a.cap = cache_cap; a.new_fill = cache_fill;
   a.row_acc = row_acc; a.row_ts = row_ts; a.now = now;
   a.n_src = rows_per_cache * n_caches; a.rows_per_cache = rows_per_cache; a.fanout = 1; a.D = D; a.group = group;
   a.n_tensors = v_src ? 2 : 1;

@@ -938,8 +938,8 @@ class CachePool:
                   leave_room: bool = False, append: bool = False):
         """Caches that min(count[c] or count_all, limit, cap[c]) new rows would overflow evict by
         `policy` (EVICT_H2O, EVICT_LRU, EVICT_ALL) and are compacted; the others keep their rows.
-        new_len = the rows kept; fill = new_len, or the fill after the new rows with append=True
-        (for an append_rows call that follows)."""
+        new_len = the rows kept; fill = new_len, or the fill after the new rows with append=True (for an
+        append_rows call that is sure to follow: until then the caches claim rows they do not hold)."""
         if count is not None:
             count = _need(count, "count", dtype=torch.int32, ndim=1)
             if count.numel() != self.n_caches:
@@ -957,9 +957,10 @@ class CachePool:
                _ptr(self.fill), _ptr(self.cap), self.n_caches, self.max_cap, ptrs, rbs, len(ps), _ptr(self.keep_flag),
                _ptr(self.keep_index), _ptr(self.new_len), _ptr(self._budgets), _ptr(ws), ws_bytes, _stream())
 
-    def append_rows(self, k_src, v_src, now: float = 0.0):
+    def append_rows(self, k_src, v_src, now: float = 0.0, advance: bool = False):
         """Quantise k_src / v_src [n_caches * rows, D] (cache-major) behind the new_len rows of every
-        cache, as make_room(append=True) has left them; rows past the capacity are dropped."""
+        cache, as make_room has left them; rows past the capacity are dropped.  advance=True also moves
+        fill behind them, in the same launch (after make_room(append=True) it is there already)."""
         k_src = _need(k_src, "k_src")
         dt = _dt(k_src, "k_src")
         rows = k_src.numel() // (self.D * self.n_caches)
@@ -972,8 +973,8 @@ class CachePool:
         if rows == 0:
             return
         N.call("pikv_quant_append", _ptr(k_src), _ptr(v_src) if self.with_v else None, dt, rows, self.D, self.group,
-               self.scheme, _ptr(self.row_base), _ptr(self.new_len), _ptr(self.cap), self.n_caches,
-               _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero),
+               self.scheme, _ptr(self.row_base), _ptr(self.new_len), _ptr(self.fill) if advance else None, _ptr(self.cap),
+               self.n_caches, _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero),
                _ptr(self.v_zero), _ptr(self.acc), _ptr(self.ts), float(now), _stream())
 
     def evict(self, policy: int, **kw):

@@ -112,6 +112,47 @@ def test_make_room_and_append(dev, policy, caps, D, heavy, recent):
         assert (ts2[base + m:base + m + w] == 9.0).all() and (acc2[base + m:base + m + w] == 0.0).all()
 
 
+@pytest.mark.parametrize("caps,rows", [([9, 40, 3, 64], 1), ([9, 40, 3, 64], 5), ([300] * 3, 299), ([0, 7], 7)])
+@pytest.mark.parametrize("D,scheme", [(64, O.Q_I8_SYM), (96, O.Q_I4_ASYM), (2048, O.Q_I8_ASYM)])
+def test_append_rows_advances_with_the_write(dev, caps, rows, D, scheme):
+    """append_rows(advance=True) behind a plain make_room leaves what make_room(append=True) + append_rows does; a
+    write that is refused leaves the fill at the rows that are there."""
+    import torch
+    from pikv_amd import ops
+    r = rng(D + rows)
+    pools = [ops.CachePool(caps, 1, D, 32, scheme, dev) for _ in range(2)]
+    fills = np.array([max(0, c - 3) for c in caps], np.int32)
+    k, v = (to_dev(r.standard_normal((len(caps) * rows, D)).astype(np.float32), dev) for _ in range(2))
+    for pool, append in zip(pools, (True, False)):
+        pool.fill.copy_(to_dev(fills, dev))
+        pool.make_room(ops.EVICT_LRU, count_all=rows, append=append)
+    held = pools[1].fill.clone()
+    assert torch.equal(held, pools[1].new_len)
+    with pytest.raises(ValueError):
+        pools[1].append_rows(k, v[:-1], now=2.0, advance=True)
+    assert torch.equal(pools[1].fill, held)
+    pools[0].append_rows(k, v, now=2.0)
+    pools[1].append_rows(k, v, now=2.0, advance=True)
+    for a, b in zip([pools[0].fill, *pools[0].planes()], [pools[1].fill, *pools[1].planes()]):
+        assert torch.equal(a, b)
+
+
+def test_attention_cache_after_a_refused_write(dev):
+    """A layer whose new rows are refused claims none of them."""
+    import torch
+    from pikv_amd.attention import PiKVAttention
+    layer = PiKVAttention(128, 2, head_dim=64, cache_size=16).to(dev).eval()
+    x = torch.randn(2, 5, 128, device=dev)
+    with torch.no_grad():
+        layer(x)
+        k = torch.randn(2, 4, 2, 64, device=dev)
+        with pytest.raises(ValueError):
+            layer._update_cache(k, k[:, :3])
+        assert layer.cache_ptr.tolist() == [5, 5]
+        layer._update_cache(k, k)
+    assert layer.cache_ptr.tolist() == [9, 9]
+
+
 @pytest.mark.parametrize("scheme,heads,hq,dh,group", [
     (O.Q_I8_SYM, 2, 4, 128, 128), (O.Q_I8_ASYM, 4, 4, 64, 32), (O.Q_I4_ASYM, 2, 6, 64, 32), (O.Q_I4_SYM, 1, 7, 128, 64)])
 @pytest.mark.parametrize("S,lens", [(1, [5]), (2, [0, 33]), (31, [1, 64]), (33, None), (70, [32, 300]), (5, [1500])])
