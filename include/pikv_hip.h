@@ -455,7 +455,8 @@ int64_t pikv_decode_attend_workspace_bytes(int n_caches, int n_q_heads, int head
  *   (core/single/pikv_attention.py:104-191, :240-244) where no mask, dropout or gradient is
  *   asked for.
  *   q [n_seqs][S][n_q_heads][head_dim], k / v [n_seqs][S][n_kv_heads][head_dim], out as q, all
- *   float and contiguous; head_dim 64 or 128; sequence b attends to cache b's
+ *   float and contiguous, q, k and v 16-byte aligned (PIKV_ERR_UNSUPPORTED otherwise); head_dim
+ *   64 or 128; sequence b attends to cache b's
  *   min(cache_fill[b], max_cached) rows (k_codes == NULL: no cached rows) and to the own rows
  *   0 .. i of query i (all S with causal == 0).
  *   workspace: pikv_prefill_attend_workspace_bytes(...) bytes (0 for most shapes), 256-byte

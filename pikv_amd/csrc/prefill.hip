@@ -359,6 +359,7 @@ extern "C" int pikv_prefill_attend(const float* q, const float* k, const float* 
   if (n_seqs < 1 || S < 1 || n_kv_heads < 1 || n_q_heads < 1 || n_q_heads % n_kv_heads != 0 || max_cached < 0)
     return PIKV_ERR_SHAPE;
   if (head_dim != 64 && head_dim != 128) return PIKV_ERR_UNSUPPORTED;
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 != 0) return PIKV_ERR_UNSUPPORTED;   // read as float4
   if (scheme < 0 || scheme > 3) return PIKV_ERR_UNSUPPORTED;
   const bool asym = (scheme == PIKV_Q_I8_ASYM || scheme == PIKV_Q_I4_ASYM);
   const int epl = (scheme == PIKV_Q_I8_SYM || scheme == PIKV_Q_I8_ASYM) ? 16 : 32;

@@ -526,6 +526,8 @@ def prefill_attend(q, k, v, pool: Optional["CachePool"] = None, causal: bool = T
         raise ValueError("the query heads must be a multiple of the kv heads")
     if dh not in (64, 128):
         raise ValueError(f"head_dim must be 64 or 128, got {dh}")
+    # the kernel reads 16 bytes at a time: rows that begin elsewhere (a view into a larger buffer) are copied
+    q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
     if pool is not None and (pool.n_caches != B or pool.n_heads != hkv or pool.head_dim != dh or not pool.with_v):
         raise ValueError("the pool's caches do not match k and v")
     out = torch.empty_like(q)

@@ -92,6 +92,16 @@ def test_pure_host_entry_points():
                                   1, 1, ws - 1, None) == -4
 
 
+@pytest.mark.parametrize("odd", [0, 1, 2])
+def test_prefill_attend_refuses_rows_that_begin_between_16_bytes(odd):
+    """The kernel reads q, k and v as 16-byte vectors."""
+    from pikv_amd import _native as N
+    qkv = [4096, 8192, 12288]
+    qkv[odd] += 4
+    assert N.lib().pikv_prefill_attend(*qkv, 1, 5, 2, 4, 64, 1, 0.125, None, None, None, None, None, None, 0, 0,
+                                       None, None, 0, 16384, None, 0, None) == -3
+
+
 def test_integration_stub_matches_header():
     """The ctypes stub shown to maintainers binds the declared number of arguments."""
     doc = open(os.path.join(ROOT, "INTEGRATION.md")).read()

@@ -189,6 +189,23 @@ def test_prefill_attend(dev, scheme, heads, hq, dh, group, S, lens, causal):
             assert np.abs(got[b, :, h] - want).max() <= 4 * 2.0 ** -24 * np.sqrt(dh + n + S) * size
 
 
+@pytest.mark.parametrize("dh,scheme", [(64, O.Q_I4_SYM), (128, O.Q_I8_SYM)])
+def test_prefill_attend_takes_views(dev, dh, scheme):
+    """Rows that begin one, two and three floats into a buffer give what the same rows give in a buffer of their own."""
+    import torch
+    from pikv_amd import ops
+    r = rng(dh)
+    q, k, v = (to_dev(r.standard_normal((2, 37, h, dh)).astype(np.float32), dev) for h in (4, 2, 2))
+    pool, _ = _fill_pool(dev, r, [40] * 2, [40, 7], 2, dh, 32, scheme)
+    want = ops.prefill_attend(q, k, v, pool)
+    views = []
+    for i, t in enumerate((q, k, v)):
+        buf = torch.empty(t.numel() + 4, device=dev)
+        views.append(buf[i + 1:i + 1 + t.numel()].view(t.shape).copy_(t))
+        assert views[-1].data_ptr() % 16
+    assert torch.equal(ops.prefill_attend(*views, pool), want)
+
+
 @pytest.mark.parametrize("A", [1, 255, 512, 513, 8191, 8192, 8193, 16000])
 @pytest.mark.parametrize("E,capacity", [(1, 5000), (8, 700), (64, 90)])
 def test_capacity_slots_chunks(dev, A, E, capacity):
