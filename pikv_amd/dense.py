@@ -41,6 +41,27 @@ MAX_LORA_RANK = 8
 MAX_LAYERS = 20          # of one linear_group or expert_combine launch
 
 
+# The kernels of csrc/moe.hip spend few launches on little work: a tile is 32 x 32 whatever the shape, weights and
+# inputs come from L2 without an LDS tile, and some of them are one block.  Where a call is more than that the library's
+# kernels win, and these rules end the native form.  Times in us, a pass among others, native / torch.
+
+def router_pays(T: int, H: int, E: int) -> bool:
+    """AdaptiveRouter of T tokens.  Inside both the pass and its kernels are faster: 128 x 256, 4 experts 106 / 377; 1024 x 1024,
+    64 experts 268 / 416 (kernels 266 / 284); 8192 x 128, 16 experts 130 / 422; 128 x 2048, 8 experts 204 / 435 (kernels 201 / 208).
+    Outside: 2048 x 1024, 64 experts 394 / 380; 8192 x 512, 8 experts 310 / 375 with 311 / 288 of kernels; 1024 x 2048 464 / 416;
+    16 x 4096 493 / 413 (the selector's weights go through one block); 65536 x 128, 64 experts 5228 / 439 (the balance loss
+    is one block)."""
+    if H <= 1024:
+        return T * H <= 1 << 20 and T * E <= 1 << 17
+    return H <= 2048 and T <= 128 and E <= 8
+
+
+def key_projection_pays(T: int, H: int) -> bool:
+    """One [H, H] layer with LoRA: 1024 x 512 22 / 71, 2048 x 512 34 / 69, 256 x 1024 23 / 74, 128 x 2048 38 / 71; outside
+    8192 x 512 111 / 79, 2048 x 1024 90 / 79, 512 x 2048 91 / 71, 128 x 4096 105 / 89."""
+    return H <= 512 and T * H <= 1 << 20 or H <= 2048 and T * H <= 1 << 18
+
+
 def _no_hooks(m: nn.Module) -> bool:
     return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
                 or "forward" in m.__dict__)

@@ -230,15 +230,14 @@ class PiKVMoE(nn.Module):
                 and dense.plain(m.dropout, nn.Dropout) and not (m.dropout.training and m.dropout.p > 0))
 
     def _native_experts(self, x, routing_weights) -> bool:
-        """Whether the key projection, the value terms and everything behind the experts' products run natively
+        """Whether the key projection (while it pays), the value terms and everything behind the experts' products run natively
         (_experts_forward): a float32 forward in evaluation mode, without autograd, over unmodified layers of widths
         the kernels have (13 launches an expert otherwise)."""
         E, H = len(self.experts), x.shape[-1]
         if not (not self.training and dense.forward_only(x) and x.numel() > 0 and H % 128 == 0 and H == config['hidden_size']
                 and E == config['num_experts'] <= dense.MAX_LAYERS and len(self.kv_caches) == E):
             return False
-        if not (dense.ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)
-                and x.shape[0] * x.shape[1] <= 65535 * 32):
+        if not (dense.ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)):
             return False
         rank = self.key_lora.lora_A.shape[1]
         if not (1 <= rank <= dense.MAX_LORA_RANK and self._lora_ok(self.key_lora, rank, x.device)
@@ -250,16 +249,20 @@ class PiKVMoE(nn.Module):
 
     def _experts_forward(self, x, cached, routing_weights):
         """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]): the experts' products by the
-        library, bit for bit those of LoRAExpert.forward, the rest in four launches."""
+        library, bit for bit those of LoRAExpert.forward, the rest in four launches (the key projection of many
+        or wide rows by the library too)."""
         H = x.shape[-1]
         x2 = x.reshape(-1, H)
         T, E = x2.shape[0], len(self.experts)
         lora = [c.value_lora for c in self.kv_caches]
         add = ops.value_lora(cached, [m.lora_A for m in lora], [m.lora_B for m in lora], [m.scaling for m in lora])
-        keys = torch.empty(T, H, dtype=torch.float32, device=x.device)
-        ops.linear_group(x2, [dict(weight=self.key_proj.weight, bias=self.key_proj.bias, lora_a=self.key_lora.lora_A,
-                                   lora_b=self.key_lora.lora_B, scaling=self.key_lora.scaling, out=keys)],
-                         rank=self.key_lora.lora_A.shape[1])
+        if dense.key_projection_pays(T, H):
+            keys = torch.empty(T, H, dtype=torch.float32, device=x.device)
+            ops.linear_group(x2, [dict(weight=self.key_proj.weight, bias=self.key_proj.bias, lora_a=self.key_lora.lora_A,
+                                       lora_b=self.key_lora.lora_B, scaling=self.key_lora.scaling, out=keys)],
+                             rank=self.key_lora.lora_A.shape[1])
+        else:
+            keys = self.key_proj(x2) + self.key_lora(x2)
         products, terms = [], []
         for e in self.experts:
             products.append(F.linear(x2, e.dense.weight, e.dense.bias))

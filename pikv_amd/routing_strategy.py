@@ -2,7 +2,8 @@
 LoadBalancingRouter, ImportanceAwareRouter and their blend, AdaptiveRouter - same
 constructors, parameter names (a reference state_dict loads) and return tuples.
 
-AdaptiveRouter in evaluation mode and without autograd runs natively as a whole (_forward_native).  Otherwise the small
+AdaptiveRouter of a few thousand tokens at most, in evaluation mode and without autograd, runs natively as a whole
+(_forward_native).  Otherwise the small
 MLPs (gate, importance predictor, router selector) and the losses built on their outputs stay in
 torch.  What runs natively in every case: every softmax + top-k + renormalise
 (`pikv_router_tail`, one wavefront per token), with this build's total order - value
@@ -126,11 +127,12 @@ class AdaptiveRouter(nn.Module):
 
     def _native(self, x, expert_mask) -> bool:
         """Whether the three hidden layers run in one launch and everything behind them in three: a float32 forward
-        in evaluation mode, without autograd, over unmodified layers (35 launches otherwise, 128 tokens as well as 2048)."""
+        in evaluation mode, without autograd, over unmodified layers, of a size where that is faster than the 35
+        launches otherwise (dense.router_pays)."""
         H, E = self.hidden_size, self.num_experts
         lb, imp = self.load_balancing_router, self.importance_router
         if not (not self.training and dense.forward_only(x) and x.dim() == 3 and x.numel() > 0 and x.shape[-1] == H and H % 128 == 0
-                and 1 <= E <= 64 and 1 <= min(self.top_k, E) <= 8 and x.shape[0] * x.shape[1] <= 65535 * 32):
+                and 1 <= E <= 64 and 1 <= min(self.top_k, E) <= 8 and dense.router_pays(x.shape[0] * x.shape[1], H, E)):
             return False
         if expert_mask is not None and not (dense.ordinary_tensor(expert_mask, x.device) and expert_mask.shape == (E,)):
             return False

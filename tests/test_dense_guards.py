@@ -76,3 +76,20 @@ def test_stream_without_the_raw_call(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=77))
     monkeypatch.setattr(ops, "_raw_stream", None, raising=False)
     assert ops._stream() == 77
+
+
+@pytest.mark.parametrize("T,H,E,pays", [
+    (1, 128, 4, True), (8192, 128, 16, True), (2048, 256, 64, True), (2048, 512, 64, True), (1024, 1024, 64, True),
+    (128, 1536, 8, True), (128, 2048, 8, True),
+    (8192, 128, 64, False), (65536, 128, 8, False), (8192, 512, 8, False), (2048, 1024, 64, False), (8192, 1024, 8, False),
+    (256, 2048, 64, False), (1024, 2048, 4, False), (1, 4096, 4, False), (65536, 4096, 64, False)])
+def test_router_rule_against_measured_sizes(T, H, E, pays):
+    """Sizes where the native router was measured faster (pass and kernels) and where it was not."""
+    assert dense.router_pays(T, H, E) is pays
+
+
+@pytest.mark.parametrize("T,H,pays", [
+    (1, 128, True), (8192, 128, True), (2048, 256, True), (1024, 512, True), (256, 1024, True), (128, 2048, True),
+    (8192, 512, False), (2048, 1024, False), (512, 2048, False), (1, 4096, False), (8192, 4096, False)])
+def test_key_projection_rule_against_measured_sizes(T, H, pays):
+    assert dense.key_projection_pays(T, H) is pays

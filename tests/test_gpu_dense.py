@@ -119,6 +119,24 @@ def test_adaptive_router_native(dev, B, S, H, E, k, mask):
     assert torch.allclose(got[2][same], ref[2][same], atol=64 * 2.0 ** -24 * np.sqrt(H))
 
 
+@pytest.mark.parametrize("T,H,E,native", [(2048, 512, 64, True), (2049, 512, 64, False), (128, 2048, 8, True),
+                                          (129, 2048, 8, False), (1, 2176, 2, False)])
+def test_adaptive_router_size_rule(dev, T, H, E, native):
+    """Both sides of the sizes where the native pass ends: one selection, values to the rounding of the sums."""
+    import torch
+    from pikv_amd.routing_strategy import AdaptiveRouter
+    torch.manual_seed(T + H)
+    m = AdaptiveRouter(H, E, top_k=2).to(dev).eval()
+    x = torch.randn(1, T, H, device=dev)
+    ref = m(x)
+    with torch.no_grad():
+        assert m._native(x, None) is native
+        got = m(x)
+    assert (got[1] == ref[1]).float().mean() > 0.99
+    for i in (0, 3, 4):
+        assert torch.allclose(got[i], ref[i], rtol=0, atol=64 * 2.0 ** -24 * np.sqrt(H))
+
+
 @pytest.mark.parametrize("H,policy", [(128, "lru"), (256, "h2o")])
 def test_moe_native_forward_equals_module_path(dev, H, policy):
     """PiKVMoE without autograd through the native experts and through the modules (a hook on one expert)."""
