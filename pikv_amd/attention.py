@@ -241,13 +241,13 @@ class PiKVAttention(nn.Module):
                                   scale_qk=1.0 / math.sqrt(self.head_dim))
 
     def _project(self, x: torch.Tensor):
-        """q, k, v of x [B, S, hidden]: in one launch for up to 64 tokens without autograd - 8 tokens, 1024 -> 1024: 25 us
-        for the three, 58 as library calls, 64 tokens of 2048: 37 and 59 - and by the library otherwise (128 tokens:
-        55 and 59)."""
+        """q, k, v of x [B, S, hidden]: in one launch for up to 64 tokens without autograd and weights of a size where
+        that is faster (dense.projections_pay), by the library otherwise."""
         layers = (self.q_proj, self.k_proj, self.v_proj)
         T, H = x.shape[0] * x.shape[1], x.shape[2]
         dq, dkv = self.num_heads * self.head_dim, self.num_kv_heads * self.head_dim
-        if not (0 < T <= 64 and H % 128 == 0 and dq % 32 == 0 and dkv % 32 == 0 and dense.forward_only(x)
+        if not (T > 0 and dense.projections_pay(T, H, dq + 2 * dkv) and H % 128 == 0 and dq % 32 == 0 and dkv % 32 == 0
+                and dense.forward_only(x)
                 and all(dense.linear_ok(m, H, n, x.device) for m, n in zip(layers, (dq, dkv, dkv)))):
             return tuple(m(x) for m in layers)
         out = [torch.empty(T, n, dtype=torch.float32, device=x.device) for n in (dq, dkv, dkv)]

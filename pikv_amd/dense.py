@@ -56,6 +56,13 @@ def router_pays(T: int, H: int, E: int) -> bool:
     return H <= 2048 and T <= 128 and E <= 8
 
 
+def projections_pay(T: int, H: int, N: int) -> bool:
+    """q, k and v of T tokens, N columns in all: 8 x 1024 x 3072 23 / 61, 64 x 2048 x 6144 37 / 60, 8 x 2560 x 7680 25 / 60,
+    32 x 3584 x 5376 35 / 62; outside 64 x 3072 x 9216 75 / 61, 8 x 4096 x 12288 51 / 61 with 47 / 41 in a replayed graph,
+    64 x 4096 x 12288 101 / 69, 8 x 8192 x 12288 140 / 100; 128 tokens of 2048 x 6144 55 / 59."""
+    return T <= 64 and H <= 3584 and H * N <= (20_000_000 if T <= 32 else 13_000_000)
+
+
 def key_projection_pays(T: int, H: int) -> bool:
     """One [H, H] layer with LoRA: 1024 x 512 22 / 71, 2048 x 512 34 / 69, 256 x 1024 23 / 74, 128 x 2048 38 / 71; outside
     8192 x 512 111 / 79, 2048 x 1024 90 / 79, 512 x 2048 91 / 71, 128 x 4096 105 / 89."""

@@ -93,3 +93,11 @@ def test_router_rule_against_measured_sizes(T, H, E, pays):
     (8192, 512, False), (2048, 1024, False), (512, 2048, False), (1, 4096, False), (8192, 4096, False)])
 def test_key_projection_rule_against_measured_sizes(T, H, pays):
     assert dense.key_projection_pays(T, H) is pays
+
+
+@pytest.mark.parametrize("T,H,N,pays", [
+    (1, 256, 384, True), (64, 1024, 3072, True), (64, 2048, 6144, True), (32, 2560, 7680, True), (32, 3584, 5376, True),
+    (16, 3072, 6144, True), (65, 256, 384, False), (64, 3072, 9216, False), (64, 4096, 6144, False), (32, 4096, 12288, False),
+    (8, 8192, 12288, False), (1, 8192, 1024, False)])
+def test_projection_rule_against_measured_sizes(T, H, N, pays):
+    assert dense.projections_pay(T, H, N) is pays

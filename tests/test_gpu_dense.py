@@ -171,6 +171,25 @@ def test_moe_native_forward_equals_module_path(dev, H, policy):
         config.update(saved)
 
 
+@pytest.mark.parametrize("T,hidden,heads,kv,native", [(64, 1024, 32, 32, True), (65, 1024, 32, 32, False),
+                                                      (32, 3584, 56, 14, True), (33, 3584, 56, 14, False), (1, 3712, 2, 2, False)])
+def test_projection_size_rule(dev, monkeypatch, T, hidden, heads, kv, native):
+    """Both sides of the sizes where the projections end to be one launch: the modules' values to float32 sums."""
+    import torch
+    from pikv_amd import ops
+    from pikv_amd.attention import PiKVAttention
+    torch.manual_seed(T + hidden)
+    layer = PiKVAttention(hidden, heads, head_dim=64, num_kv_heads=kv, cache_size=8).to(dev).eval()
+    calls, group = [], ops.linear_group
+    monkeypatch.setattr(ops, "linear_group", lambda *a, **kw: calls.append(1) or group(*a, **kw))
+    x = torch.randn(1, T, hidden, device=dev)
+    with torch.no_grad():
+        for got, m in zip(layer._project(x), (layer.q_proj, layer.k_proj, layer.v_proj)):
+            want = m(x).view(got.shape)
+            assert torch.allclose(got, want, rtol=0, atol=16 * 2.0 ** -24 * np.sqrt(hidden) * float(want.abs().max()))
+    assert bool(calls) is native
+
+
 def test_native_prompt_attention_leaves_other_calls_alone(dev):
     """Hooks, dropout, masks, gradients, other types and forward-mode tangents keep the torch path; the two paths agree
     on what both take (float32 sums of some 200 products: 1e-5 of outputs of order one)."""
