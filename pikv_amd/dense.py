@@ -95,9 +95,10 @@ def ordinary_call() -> bool:
                            or forward_ad._current_level >= 0 or _transforms() is not None)
 
 
-def ordinary_tensor(t, device, dtype=torch.float32) -> bool:
+def ordinary_tensor(t, device, dtype=torch.float32, align: int = 16) -> bool:
+    """A dense tensor a kernel may read by its address, `align` bytes at a time."""
     return (type(t) in (torch.Tensor, nn.Parameter) and t.device == device and t.dtype == dtype and t.is_contiguous()
-            and _has_storage(t) and t.data_ptr() % 16 == 0)      # a batched tensor has none
+            and _has_storage(t) and t.data_ptr() % align == 0)      # a batched tensor has no storage
 
 
 def forward_only(x) -> bool:

@@ -237,7 +237,8 @@ class PiKVMoE(nn.Module):
         if not (not self.training and dense.forward_only(x) and x.numel() > 0 and H % 128 == 0 and H == config['hidden_size']
                 and E == config['num_experts'] <= dense.MAX_LAYERS and len(self.kv_caches) == E):
             return False
-        if not (dense.ordinary_tensor(routing_weights, x.device) and routing_weights.shape == (*x.shape[:2], E)):
+        # (the router's weights follow its probabilities in one buffer: read as single floats, they begin anywhere)
+        if not (dense.ordinary_tensor(routing_weights, x.device, align=4) and routing_weights.shape == (*x.shape[:2], E)):
             return False
         rank = self.key_lora.lora_A.shape[1]
         if not (1 <= rank <= dense.MAX_LORA_RANK and self._lora_ok(self.key_lora, rank, x.device)

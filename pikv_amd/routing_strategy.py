@@ -134,7 +134,7 @@ class AdaptiveRouter(nn.Module):
         if not (not self.training and dense.forward_only(x) and x.dim() == 3 and x.numel() > 0 and x.shape[-1] == H and H % 128 == 0
                 and 1 <= E <= 64 and 1 <= min(self.top_k, E) <= 8 and dense.router_pays(x.shape[0] * x.shape[1], H, E)):
             return False
-        if expert_mask is not None and not (dense.ordinary_tensor(expert_mask, x.device) and expert_mask.shape == (E,)):
+        if expert_mask is not None and not (dense.ordinary_tensor(expert_mask, x.device, align=4) and expert_mask.shape == (E,)):
             return False
         if not (dense.plain(lb, LoadBalancingRouter) and dense.plain(imp, ImportanceAwareRouter)
                 and all(type(v) in (int, float) for v in (lb.temperature, imp.temperature, lb.balance_weight))

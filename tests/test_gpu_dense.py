@@ -40,16 +40,18 @@ def test_linear_group(dev, T, K, widths, rank):
 
 @pytest.mark.parametrize("E,T,H", [(1, 1, 4), (3, 37, 132), (20, 5, 64)])
 def test_expert_combine(dev, E, T, H):
-    """Bit for bit what the torch operations give, a NaN and infinities among the products."""
+    """Bit for bit what the torch operations give, each rounded on its own (a scaling that is no power of two: a fused
+    multiply-add would show), a NaN and infinities among the products."""
     import torch
     from pikv_amd import ops
     torch.manual_seed(E)
+    scaling = [0.3 + 0.1 * e for e in range(E)]
     d, l, c, w = (torch.randn(*s, device=dev) for s in ((E, T, H), (E, T, H), (E, H), (T, E)))
     d[0, 0, 0], d[E - 1, T - 1, 1], l[0, 0, 2] = float("nan"), float("inf"), float("-inf")
-    outs, mix = ops.expert_combine(list(d), list(l), [0.25] * E, c, w)
+    outs, mix = ops.expert_combine(list(d), list(l), scaling, c, w)
     want = torch.zeros(T, H, device=dev)
     for e in range(E):
-        o = torch.relu(d[e] + l[e] * 0.25) + c[e]
+        o = torch.relu(d[e] + l[e] * scaling[e]) + c[e]
         assert torch.equal(o.nan_to_num(7.0), outs[e].nan_to_num(7.0))
         want = want + o * w[:, e:e + 1]
     assert torch.equal(want.nan_to_num(7.0), mix.nan_to_num(7.0))
@@ -137,20 +139,23 @@ def test_adaptive_router_size_rule(dev, T, H, E, native):
         assert torch.allclose(got[i], ref[i], rtol=0, atol=64 * 2.0 ** -24 * np.sqrt(H))
 
 
-@pytest.mark.parametrize("H,policy", [(128, "lru"), (256, "h2o")])
-def test_moe_native_forward_equals_module_path(dev, H, policy):
-    """PiKVMoE without autograd through the native experts and through the modules (a hook on one expert)."""
+@pytest.mark.parametrize("H,policy,seqs,seq", [(128, "lru", 2, 37), (256, "h2o", 2, 37), (640, "lru", 6, 70)])
+def test_moe_native_forward_equals_module_path(dev, H, policy, seqs, seq):
+    """PiKVMoE without autograd through the native experts and through the modules (a hook on one expert); 640 x 420 rows
+    take the key projection from the library.  Logits to float32 sums; the cached rows are quantised from values that differ
+    by a rounding, so a code may move by one: within a scale of each other, and nearly all equal."""
     import torch
-    from pikv_amd import moe
+    from pikv_amd import dense, moe
     from pikv_amd.config import config
     from pikv_amd.scheduling import SchedulingPolicy
     saved = dict(config)
     try:
-        config.update(hidden_size=H, num_experts=3, kv_cache_size=60, kv_heads=2, kv_quant="int8", kv_group=None,
+        config.update(hidden_size=H, num_experts=3, kv_cache_size=60, kv_heads=2, kv_quant="int8", kv_group=128 if H == 640 else None,
                       vocab_size=512, cache_decrement=5, top_k=2, capacity_factor=1.5)
+        assert dense.key_projection_pays(seqs * seq, H) is (H != 640)
         pol = SchedulingPolicy.H2O if policy == "h2o" else SchedulingPolicy.LRU
-        models = []
-        for _ in range(2):
+        models, native = [], [0, 0]
+        for i in range(2):
             torch.manual_seed(1)
             m = moe.PiKVMoE(use_cache_scheduling=True, cache_scheduling_policy=pol).to(dev).eval()
             with torch.no_grad():
@@ -158,14 +163,30 @@ def test_moe_native_forward_equals_module_path(dev, H, policy):
                     e.lora.lora_B.normal_(0.0, 0.05)
                 for c in m.kv_caches:
                     c.value_lora.lora_B.normal_(0.0, 0.05)
+                m.key_lora.lora_B.normal_(0.0, 0.05)
+
+            def counted(*a, i=i, inner=m._experts_forward):
+                native[i] += 1
+                return inner(*a)
+            m._experts_forward = counted
             models.append(m)
         models[1].experts[0].register_forward_hook(lambda *a: None)
-        ids = torch.randint(512, (2, 37), device=dev)
+        ids = torch.randint(512, (seqs, seq), device=dev)
         with torch.no_grad():
             for _ in range(3):
                 a, b = (m(ids) for m in models)
                 assert torch.allclose(a, b, rtol=0, atol=1e-5 * float(b.abs().max()))
-        assert torch.equal(models[0].pool.fill, models[1].pool.fill)
+        assert native == [3, 0]
+        pa, pb = (m.pool for m in models)
+        assert torch.equal(pa.fill, pb.fill) and int(pa.fill.min()) > 0
+        live = torch.cat([base + torch.arange(int(n), device=dev) for base, n in zip(pa.base_host, pa.fill.tolist())])
+        for which in ("k", "v"):
+            ra, rb = (p.gather_dequant(which)[live] for p in (pa, pb))
+            scale = getattr(pb, which + "_scale")[live].repeat_interleave(pb.group, dim=1)
+            assert ((ra - rb).abs() <= 1.001 * scale).all()
+            assert ((ra - rb).abs() > 0.5 * scale).float().mean() < 0.01
+        assert torch.equal(pa.ts[live], pb.ts[live])
+        assert torch.allclose(pa.acc[live], pb.acc[live], rtol=1e-3, atol=1e-5)
     finally:
         config.clear()
         config.update(saved)
