@@ -663,13 +663,14 @@ __global__ void set_fill_kernel(int32_t* __restrict__ fill, const int32_t* __res
 // ---- making room: budgets, selection, compaction and fill of every cache that would overflow ------------------
 //
 // A cache takes n_new = min(count[c] (count_all), limit, cap[c]) rows.  One that has the space keeps all its rows:
-// its block writes the fill and ends - what almost every decode step finds, so the call costs one launch.
+// its block writes the fill and ends - what almost every decode step finds, so the call costs one launch (caches of up
+// to kRoomMaxLen rows).
 // Caches of up to kRoomMaxLen rows are selected by one block each, flags and survivor list in LDS, and - unless the
 // survivors are many bytes - compacted by the same block: the launches between the steps (3 to 5 us each, and as
 // much on the host) cost more than the other compute units would give back.  Longer caches take the multi-block
-// selection.
+// selection, all of its launches whether or not a cache evicts; only the moves are left out where none does.
 // One decode step of 8 caches x 3000 rows that all have the space: 24 launches (budgets as elementwise torch
-// operations, selection, two compactions, fill), 105 us of GPU time, before; now one of 2.5 us.
+// operations, selection, two compactions, fill), 105 us of GPU time, before; now one of 4 to 5 us.
 constexpr int kRoomMaxLen = 8192;
 
 struct RoomArgs {
@@ -748,7 +749,7 @@ __device__ __forceinline__ void room_move(char* plane, int64_t base_row, int64_t
       dst[k] = -1;
       val[k] = V{};
       if (u < total) {
-        const int j = (int)((uint32_t)u / (uint32_t)per_row);   // (total < 2^31: kRoomMaxLen rows of at most 2^17 pieces)
+        const int j = (int)((uint32_t)u / (uint32_t)per_row);   // (total < 2^21: a megabyte of survivors, single bytes at worst)
         const int col = (int)(u - (int64_t)j * per_row);
         const int src = list[j];
         if (src != j) {
@@ -977,7 +978,10 @@ extern "C" int pikv_cache_make_room(int policy, const int32_t* count, int64_t co
     int64_t row = 0;
     for (int p = 0; p < n_planes; ++p) row += pl.row_bytes[p];
     double kept = (double)max_len;
-    if (policy == PIKV_EVICT_H2O) kept *= heavy_ratio + recent_ratio < 1.0 ? heavy_ratio + recent_ratio : 1.0;
+    if (policy == PIKV_EVICT_H2O) {   // as room_budget: either set has a row at least, whatever its ratio
+      const double part = (heavy_ratio > 0.0 ? heavy_ratio : 0.0) + (recent_ratio > 0.0 ? recent_ratio : 0.0);
+      if (part < 1.0) kept = kept * part + 2.0 < kept ? kept * part + 2.0 : kept;
+    }
     const double most = row > 1200 ? 640.0 * 1024.0 : 1024.0 * 1024.0;
     const bool here = policy == PIKV_EVICT_ALL || kept * (double)row <= most;
     CompactPlanes none{};

@@ -62,6 +62,7 @@ def test_decode_attend_few_ranges(dev, scheme, qdtype, length):
 @pytest.mark.parametrize("caps,D,heavy,recent", [
     ([128, 118, 1, 90], 64, 0.1, 0.1),          # selected and compacted by one block per cache
     ([1024, 1500, 1025], 2048, 0.5, 0.3),       # selected by one block, more than a megabyte of survivors
+    ([1024, 1500, 1025], 2048, -0.5, 0.8),      # a ratio below zero: one row of that set
     ([200, 190, 170], 2048, 0.9, 0.05),         # wide rows: between two thirds of a megabyte and one
     ([150, 140, 100], 2048, 0.9, 0.05),         # ... and below
     ([8192, 8000], 32, 0.06, 0.01),             # the longest caches of the one-block form
