@@ -257,7 +257,8 @@ class PiKVAttention(nn.Module):
     def _native_prefill(self, q, k, v, attention_mask) -> bool:
         """Whether a chunk goes through ops.prefill_attend: float32 without a mask, dropout or gradient, and a head
         width that kernel has.  Everything else keeps the torch path below, whose score matrix, masks and copies
-        of the cached rows cost more than the products: 2 x 500 tokens x 16 heads over 500 cached rows."""
+        of the cached rows cost more than the products at every size measured, 2 to 4096 tokens over 0 to 20000 cached
+        rows: 4 x 2 tokens of 32 heads over none 125 us a layer call against 277, 16 x 64 over 20000 rows 6.2 ms against 17.8."""
         if attention_mask is not None or self.head_dim not in (64, 128) or not q.is_cuda:
             return False
         if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):

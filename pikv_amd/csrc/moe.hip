@@ -9,8 +9,10 @@
 // float64 2.1e-7 where the library's is 4.1e-7.  The experts' own products stay with the library: their outputs are
 // quantised into the caches and come back as means in the next call, where another order of their sums - 2e-7, a code
 // in 10^4 - grew to 1e-4 of a cached row's scale.
-// Measured: linear_group, three layers of 2048 x 2048 over 8 rows 26 us (59 as three library calls), over 128 rows 55
-// and 59; adaptive router with 128 tokens, 4 experts 7.6 + 5.1 + 7.1 + 2.9 us for 35 launches.
+// Measured: linear_group, three layers of 2048 x 2048 over 8 rows 23 us a call and 19 in a replayed graph (61 and 26 as
+// three library calls), over 128 rows 55 a call (59); adaptive router with 128 tokens of 256, 4 experts 7.7 + 5.2 + 7.0 +
+// 3.0 us of kernels for 35 launches.  The kernels are made for that scale: no LDS tile in linear_group, one block a sequence
+// for the blend, one block for the balance loss.  dense.py holds the sizes where the library takes over, with both sides.
 #include "common.hpp"
 
 namespace pikv {

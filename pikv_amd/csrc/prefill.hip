@@ -14,10 +14,15 @@
 // of the chip idle.  A wavefront stages its K tile in LDS along the rows - read straight into the operand layout, a
 // lane to a row, a load touched 64 lines and every line came from L2 up to eight times - and reads V along the rows.
 //
-// Measured, 2 x 500 tokens, 16 heads of 128 over 8 kv heads, kernel time: 46.7 us for the first chunk and 110 us for
-// the second (over 500 cached rows of 8 bits), 59.4 and 129 us with K read into the operand layout and the longest
-// blocks side by side; the whole layer call 1104 us with the score matrix in torch, 544 us now, of which 410 us are
-// its four projections.  Against float64 the error is that of the torch path or below (4.7e-7 and 6.2e-7).
+// Measured, 2 x 500 tokens, 16 heads of 128 over 8 kv heads, kernel time: 45 us for the first chunk and 107 us for
+// the second (over 500 cached rows of 8 bits), 59 and 129 us with K read into the operand layout and the longest
+// blocks side by side; the two layer calls 1104 us with the score matrix in torch, 541 us now, of which 410 us are
+// their projections.  Heads of 128 use all 256 registers and spill: 10 values with 8-bit rows, 26 with 4-bit asymmetric,
+// 11 with 4-bit symmetric ones (44, 108 and 48 bytes of scratch a lane); heads of 64 use 200 and spill none.
+// Against float64 the error is that of the torch path or below (4.7e-7 and 6.2e-7).
+//
+// A NaN or infinity in a V row that a query does not see reaches that query only from the query's own last tile (a
+// zero probability times it); a product over the whole score matrix spreads it to every row.
 #include "common.hpp"
 
 namespace pikv {
@@ -67,7 +72,7 @@ __device__ __forceinline__ void stage_own_k(const float* k, int D, int last, int
 #pragma unroll
     for (int i = 0; i < N; ++i)
       *reinterpret_cast<float4*>(rows + ((g * N + i) * (64 / LPR) + lane / LPR) * QP + lane % LPR * 4) = x[i];
-    __builtin_amdgcn_sched_barrier(0);   // with all rounds in flight at once registers spill
+    __builtin_amdgcn_sched_barrier(0);   // with all rounds in flight at once more registers spill
   }
 }
 

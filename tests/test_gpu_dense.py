@@ -238,3 +238,23 @@ def test_native_prompt_attention_leaves_other_calls_alone(dev):
         assert not layer._native_prefill(q, k, v, None)
     layer.eval()
     assert not layer._native_prefill(q.requires_grad_(), k, v, None)
+
+
+@pytest.mark.parametrize("S,masked,dtype", [(5, False, "float32"), (5, True, "float32"), (1, False, "float32"),
+                                            (5, False, "bfloat16")])
+def test_context_of_another_batch_size_is_refused(dev, S, masked, dtype):
+    """On every path of a layer, the native ones among them, and nothing of the context is lost; an empty one is replaced."""
+    import torch
+    from pikv_amd.attention import PiKVAttention
+    dt = getattr(torch, dtype)
+    layer = PiKVAttention(128, 2, head_dim=64, cache_size=32).to(dev, dt).eval()
+    x = torch.randn(3, S, 128, device=dev, dtype=dt)
+    mask = torch.ones(3, S, device=dev) if masked else None
+    with torch.no_grad():
+        layer(x[:2].expand(2, S, 128).contiguous())
+        with pytest.raises(ValueError):
+            layer(x, attention_mask=mask)
+        assert layer.cache_ptr.tolist() == [S, S]
+        layer.reset_cache()
+        layer(x, attention_mask=mask)
+    assert layer.cache_ptr.tolist() == [S] * 3
