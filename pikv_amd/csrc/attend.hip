@@ -1454,7 +1454,7 @@ extern "C" int pikv_attend_values(const float* scores, const float* head_stats, 
 static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
 struct DecodeWs {
-  int64_t n_tiles, stride, scores, tmax, tsum, stats, partial, total;
+  int64_t n_tiles, stride, scores, tmax, tsum, stats, partial, ranges, total;
 };
 static DecodeWs decode_ws(int n_caches, int n_q_heads, int head_dim, int64_t max_len) {
   DecodeWs w;
@@ -1462,16 +1462,16 @@ static DecodeWs decode_ws(int n_caches, int n_q_heads, int head_dim, int64_t max
   w.stride = w.n_tiles * PIKV_SCORE_TILE;
   w.scores = 0;  // float scores [cache][head][stride], or the exchange rows [cache][tile][head][64] (same size)
   // (the two tile tables have room for one tile more than max_len holds: the one-pass form keeps a spare
-  // record per cache there, and its ranges' statistics - 8 bytes per head and range of at least 64 tokens -
-  // lie in the second table)
+  // record per cache there; its ranges' statistics - 8 bytes per head and range of at least 64 tokens - come last)
   w.tmax = align256((int64_t)n_caches * n_q_heads * w.stride * 4);
   w.tsum = w.tmax + align256((int64_t)n_caches * (w.n_tiles + 1) * n_q_heads * 4);
-  w.stats = w.tsum + align256((int64_t)n_caches * (w.n_tiles + 1) * n_q_heads * 8);
+  w.stats = w.tsum + align256((int64_t)n_caches * (w.n_tiles + 1) * n_q_heads * 4);
   w.partial = w.stats + align256((int64_t)n_caches * n_q_heads * 2 * 4);
   const int64_t fused_tpb = fused_min_tokens_per_block(n_caches, max_len);
   const int64_t fused = (max_len + fused_tpb - 1) / fused_tpb * n_caches * (int64_t)n_q_heads * head_dim * (int64_t)sizeof(float);
   const int64_t two_kernel = pikv_attend_workspace_bytes(n_caches, n_q_heads, head_dim, max_len);
-  w.total = w.partial + align256(fused > two_kernel ? fused : two_kernel);
+  w.ranges = w.partial + align256(fused > two_kernel ? fused : two_kernel);
+  w.total = w.ranges + align256((max_len + fused_tpb - 1) / fused_tpb * n_caches * (int64_t)n_q_heads * 8);
   return w;
 }
 
@@ -1502,7 +1502,7 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
   float* tsum = reinterpret_cast<float*>(ws + w.tsum);
   float* stats = reinterpret_cast<float*>(ws + w.stats);
   void* partial = ws + w.partial;
-  const int64_t partial_bytes = w.total - w.partial;
+  const int64_t partial_bytes = w.ranges - w.partial;
   hipStream_t st = (hipStream_t)stream;
   if (max_len == 0)  // nothing cached anywhere: the output is zero (the reduction writes it)
     return pikv_attend_values(reinterpret_cast<const float*>(out), nullptr, 0, v_codes, v_scale, v_zero, scheme, group,
@@ -1513,14 +1513,14 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
   // one pass over K and V (no score matrix): heads of 128, bf16 queries; 4-bit codes with up to 4 query heads per
   // kv head, 8-bit codes (scale per kv head or coarser) with up to 8.
   // Its halves (n_q_heads * 128 bytes per tile and one spare tile per cache) lie where the float scores would
-  // (256 bytes per head and tile), the tiles' reference maxima in the tile-maximum table, the ranges' statistics
-  // in the tile-sum table.
+  // (256 bytes per head and tile), the tiles' reference maxima in the tile-maximum table.
   if (decode_fused_serves(scheme, group, n_kv_heads, n_q_heads, head_dim, q_dtype, row_acc != nullptr) && (!any_asym || (k_zero && v_zero)) &&
       n_caches <= 65535) {
     const int tpb = fused_tokens_per_block(n_caches, n_kv_heads, n_q_heads, scheme, q_dtype, max_len);
     return decode_fused_launch(k_codes, k_scale, k_zero, v_codes, v_scale, v_zero, scheme, group, n_kv_heads, n_q_heads, q,
                                q_dtype, scale_qk, cache_row_base, cache_fill, n_caches, max_len, tpb, decay, now, row_acc, row_ts,
-                               out, ws + w.scores, tmax, tsum, reinterpret_cast<float*>(partial), stats, st);
+                               out, ws + w.scores, tmax, reinterpret_cast<float*>(ws + w.ranges), reinterpret_cast<float*>(partial), stats,
+                               st);
   }
   // the 4-bit matrix-core kernels meeting in the exchange format
   const int rep = n_q_heads % n_kv_heads == 0 ? n_q_heads / n_kv_heads : 0;
