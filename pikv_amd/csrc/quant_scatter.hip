@@ -40,18 +40,19 @@ struct QuantScatterArgs {
   const float* seg_score;  // optional: initial accumulator of a gathered row, by source row
   int64_t n_src;
   int64_t dst_row0;     // used when cache_id == nullptr
-  int64_t rows_per_cache;  // append mode: source row s goes to cache s / rows_per_cache
-                           // as its new row s % rows_per_cache ...
-  int32_t* new_fill;       //   and its first row leaves the fill behind the new rows here, unless null
   int fanout;
   int D;
   int group;
   int n_tensors;        // 1 (K only) or 2 (K and V)
   int n_caches;
-  int src_div;          // routed mode: assignment s belongs to token s / src_div, its K row ...
-  int64_t v_rows;       //   and its V row is that token's of the slab of v_rows rows of its cache
   int lpr_shift;        // log2(lanes per row) or -1 when it is not a power of two
   int lpg_shift;        // log2(lanes per group)
+  // what only the other modes read stands last: the plain mode's arguments keep their cache lines
+  int64_t rows_per_cache;  // append mode: source row s goes to cache s / rows_per_cache
+                           // as its new row s % rows_per_cache ...
+  int32_t* new_fill;       //   and its first row leaves the fill behind the new rows here, unless null
+  int64_t v_rows;       // routed mode: assignment s belongs to token s / src_div, its K row and its V row are
+  int src_div;          //   that token's, the V row of the slab of v_rows rows of its cache
 };
 
 template <int DT, int EPL>
