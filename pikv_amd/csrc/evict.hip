@@ -982,8 +982,8 @@ extern "C" int pikv_cache_make_room(int policy, const int32_t* count, int64_t co
   if (policy == PIKV_EVICT_ALL || max_len <= kRoomMaxLen) {
     // The block that selects a cache also moves its survivors while those are at most a megabyte - two thirds of it
     // for rows of more than 1200 bytes, where the launches that spread over the columns of a row get ahead earlier.
-    // 1 to 16 caches, LRU, us for one block / for the launches: 1900 rows of 536 bytes 59-61 / 77-88, 900 of 1096 54-55 /
-    // 54-63, 300 of 2120 41-44 / 37-44, 480 of 2120 54-56 / 40-48, 120 of 8456 51-54 / 34-39.
+    // 1 to 16 caches, LRU, us for one block / for the launches: 1900 rows of 536 bytes 57-58 / 75-89, 900 of 1096 51-53 /
+    // 54-62, 300 of 2120 40-43 / 37-44, 480 of 2120 53-54 / 40-48, 120 of 8456 49-51 / 33-39.
     int64_t row = 0;
     for (int p = 0; p < n_planes; ++p) row += pl.row_bytes[p];
     double kept = (double)max_len;

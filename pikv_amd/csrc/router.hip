@@ -1008,11 +1008,12 @@ __global__ __launch_bounds__(64) void slot_scan_kernel(int32_t* __restrict__ ws,
 // its own by itself (integer sums: the order does not matter); the last block also writes the
 // totals.  For short assignment streams this saves the scan launch, which is all latency there.
 // SELF_COUNT: no histograms at all, every block counts the assignments before its own chunk itself (and the last one
-// writes the totals): one launch instead of two for streams of up to kSlotSelfCountChunks chunks, where the last block
-// reads 30 KB for it (with the accumulation's own statistics in read_path.hip: a prefill step of 3 x 577 tokens
-// 70 -> 65 us).
+// writes the totals): one launch instead of two.  The last block's count is a chain of 0.6 us per chunk - in a replayed
+// graph 4.8 us for 2048 assignments, 6.6 for 4096, 10.3 for 8192 against 5.4 for the two launches, which cost 5 us more on
+// the host - so it is taken for up to kSlotSelfCountChunks chunks: prefill steps of 8176 assignments 70-73 us with it, 65-68
+// without; of 3462 within 1 us where the card is busy and 3 us faster where the host is.
 enum SlotPrefix { SCANNED, SELF_PREFIX, SELF_COUNT };
-constexpr int64_t kSlotSelfCountChunks = 16;
+constexpr int64_t kSlotSelfCountChunks = 8;
 template <SlotPrefix PREFIX>
 __global__ __launch_bounds__(256) void slot_rank_kernel(const int32_t* __restrict__ idx, int64_t A,
                                                         int E, int64_t capacity,

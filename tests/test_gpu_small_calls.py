@@ -209,7 +209,7 @@ def test_prefill_attend_takes_views(dev, dh, scheme):
     assert torch.equal(ops.prefill_attend(*views, pool), want)
 
 
-@pytest.mark.parametrize("A", [1, 255, 512, 513, 8191, 8192, 8193, 16000])
+@pytest.mark.parametrize("A", [1, 255, 512, 513, 4095, 4096, 4097, 8191, 8192, 8193, 16000])
 @pytest.mark.parametrize("E,capacity", [(1, 5000), (8, 700), (64, 90)])
 def test_capacity_slots_chunks(dev, A, E, capacity):
     """Slots and totals on both sides of the lengths where blocks count the assignments before them by themselves,
