@@ -33,6 +33,7 @@ _function_mode_at = _internal("_C._get_function_stack_at")
 _has_global_hook = _internal("nn.modules.module._has_any_global_hook")
 _transforms = _internal("_C._functorch.peek_interpreter_stack")
 _has_storage = _internal("_C._has_storage")
+_is_compiling, _is_tracing, _is_autocast = torch.compiler.is_compiling, torch.jit.is_tracing, torch.is_autocast_enabled
 _KNOWN = (hasattr(forward_ad, "_current_level")
           and None not in (_dispatch_modes, _pre_dispatch_modes, _function_modes, _function_mode_at, _DeviceContext,
                            _has_global_hook, _transforms, _has_storage))
@@ -90,8 +91,7 @@ def _watched() -> bool:
 
 def ordinary_call() -> bool:
     # (is_compiling comes first: what follows it would break a compiled graph)
-    return _KNOWN and not (torch.compiler.is_compiling() or _watched() or _has_global_hook()
-                           or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+    return _KNOWN and not (_is_compiling() or _watched() or _has_global_hook() or _is_autocast("cuda") or _is_tracing()
                            or forward_ad._current_level >= 0 or _transforms() is not None)
 
 
