@@ -13,4 +13,4 @@ extern "C" const char* pikv_status_string(int status) {
   return "unknown status";
 }
 
-extern "C" int pikv_abi_version(void) { return 1003; }  // 1.3: + pikv_quant8_minshift, pikv_decode_attend, pikv_stream_probe
+extern "C" int pikv_abi_version(void) { return 1004; }  // 1.4: + pikv_quant_append (and the entry points of prefill.hip and moe.hip), pikv_cache_make_room, pikv_quant_scatter_routed
