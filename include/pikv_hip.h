@@ -566,6 +566,13 @@ int pikv_linear_group(const float* x, int64_t T, int K, int n_layers, const floa
                       float* const* out, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t pikv_linear_group_workspace_bytes(int64_t T, int n_layers, int rank);
 
+/* The same without activation or LoRA for many tokens (matrix-core tiles through LDS), one launch:
+ *   out[g][t][n] = x[t] . w[g][n] + bias[g][n]
+ *   K a multiple of 64, any n_out; x and w 16-byte aligned, out too where its n_out is a multiple of 4.  Other sizes:
+ *   PIKV_ERR_UNSUPPORTED. */
+int pikv_linear_tiled(const float* x, int64_t T, int K, int n_layers, const float* const* w, const float* const* bias,
+                      const int32_t* n_out, float* const* out, void* stream);
+
 /* out [n_caches][D] = mean of every cache's dequantised rows (zero for an empty cache).
  * max_len >= max_c cache_fill[c]; workspace: pikv_cache_mean_workspace_bytes(...) bytes. */
 int pikv_cache_mean(const void* codes, const void* scale, const void* zero, int scheme, int group,

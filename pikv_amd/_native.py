@@ -70,6 +70,7 @@ SIGNATURES = {
     "pikv_linear_group": (_i, [_p, _l, _i, _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(C.c_int32), C.POINTER(C.c_int32),
                                _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), C.POINTER(_p), _p, _l, _p]),
     "pikv_linear_group_workspace_bytes": (_l, [_l, _i, _i]),
+    "pikv_linear_tiled": (_i, [_p, _l, _i, _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(C.c_int32), C.POINTER(_p), _p]),
     "pikv_cache_mean": (_i, [_p, _p, _p, _i, _i, _i, _p, _p, _i, _l, _p, _p, _l, _p]),
     "pikv_cache_mean_workspace_bytes": (_l, [_i, _i, _l]),
     "pikv_value_lora": (_i, [_p, _i, _i, _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), _p, _p]),

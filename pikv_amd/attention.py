@@ -241,17 +241,21 @@ class PiKVAttention(nn.Module):
                                   scale_qk=1.0 / math.sqrt(self.head_dim))
 
     def _project(self, x: torch.Tensor):
-        """q, k, v of x [B, S, hidden]: in one launch for up to 64 tokens without autograd and weights of a size where
-        that is faster (dense.projections_pay), by the library otherwise."""
+        """q, k, v of x [B, S, hidden]: in one launch without autograd and at sizes where that is faster (dense.projections_pay
+        for few tokens, dense.tiled_pays for more), by the library otherwise."""
         layers = (self.q_proj, self.k_proj, self.v_proj)
         T, H = x.shape[0] * x.shape[1], x.shape[2]
         dq, dkv = self.num_heads * self.head_dim, self.num_kv_heads * self.head_dim
-        if not (T > 0 and dense.projections_pay(T, H, dq + 2 * dkv) and H % 128 == 0 and dq % 32 == 0 and dkv % 32 == 0
-                and dense.forward_only(x)
-                and all(dense.linear_ok(m, H, n, x.device) for m, n in zip(layers, (dq, dkv, dkv)))):
+        widths = (dq, dkv, dkv)
+        few = T > 0 and dense.projections_pay(T, H, dq + 2 * dkv) and H % 128 == 0 and dq % 32 == 0 and dkv % 32 == 0
+        if not ((few or (T > 0 and H % 64 == 0 and dq % 4 == 0 and dkv % 4 == 0 and dense.tiled_pays(T, H, widths)))
+                and dense.forward_only(x) and all(dense.linear_ok(m, H, n, x.device) for m, n in zip(layers, widths))):
             return tuple(m(x) for m in layers)
-        out = [torch.empty(T, n, dtype=torch.float32, device=x.device) for n in (dq, dkv, dkv)]
-        ops.linear_group(x.view(T, H), [dict(weight=m.weight, bias=m.bias, out=o) for m, o in zip(layers, out)])
+        out = [torch.empty(T, n, dtype=torch.float32, device=x.device) for n in widths]
+        if few:
+            ops.linear_group(x.view(T, H), [dict(weight=m.weight, bias=m.bias, out=o) for m, o in zip(layers, out)])
+        else:
+            ops.linear_tiled(x.view(T, H), [(m.weight, m.bias, o) for m, o in zip(layers, out)])
         return out
 
     def _native_prefill(self, q, k, v, attention_mask) -> bool:

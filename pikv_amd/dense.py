@@ -39,7 +39,7 @@ _KNOWN = (hasattr(forward_ad, "_current_level")
                            _has_global_hook, _transforms, _has_storage))
 
 MAX_LORA_RANK = 8
-MAX_LAYERS = 20          # of one linear_group or expert_combine launch
+MAX_LAYERS = 20          # of one linear_group, linear_tiled or expert_combine launch
 
 
 # The kernels of csrc/moe.hip spend few launches on little work: a tile is 32 x 32 whatever the shape, weights and
@@ -62,6 +62,21 @@ def projections_pay(T: int, H: int, N: int) -> bool:
     32 x 3584 x 5376 35 / 62; outside 64 x 3072 x 9216 75 / 61, 8 x 4096 x 12288 51 / 61 with 47 / 41 in a replayed graph,
     64 x 4096 x 12288 101 / 69, 8 x 8192 x 12288 140 / 100; 128 tokens of 2048 x 6144 55 / 59."""
     return T <= 64 and H <= 3584 and H * N <= (20_000_000 if T <= 32 else 13_000_000)
+
+
+def tiled_pays(T: int, H: int, widths) -> bool:
+    """The same for 256 tokens and more, in LDS tiles (csrc/linear.hip).  Up to 3.5e9 multiply-adds the library's three calls are
+    bound by the host (250 x 512 x 2048 9 / 56, 1000 x 512 x 2048 21 / 56, 500 x 1536 x 4096 52 / 66); beyond, one round of 128 x 128
+    tiles that fills the chip (1000 x 2048 x 4096 125 / 143).  Outside 1000 x 3072 x 3072 150 / 146, 4000 x 3072 x 3072 537 / 528.  Fewer
+    than 256 tokens would be faster too (130 x 1024 x 3072 32 / 57), but there the library sums in another order for most widths, and
+    2e-7 of a query is 1e-5 of a probability where scores reach 100; from 256 on nearly all sums are bit for bit the library's."""
+    if T < 256:
+        return False
+    N = sum(widths)
+    if T * H * N <= 3_500_000_000:
+        return True
+    tiles = -(-T // 128) * sum(-(-n // 128) for n in widths)
+    return tiles <= 256 and T * N >= 0.85 * 256 * 128 * 128
 
 
 def key_projection_pays(T: int, H: int) -> bool:

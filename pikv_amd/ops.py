@@ -440,6 +440,24 @@ def linear_group(x, layers, rank: int = 0):
            _ptr_array([l["out"] for l in layers]), _ptr(ws), nb, _stream())
 
 
+def linear_tiled(x, layers):
+    """Linear layers over one input x [T, K] float32 in one launch of LDS tiles, for many tokens.  `layers`: (weight [N, K],
+    bias [N], out [T, N]) of each, at most 20; K a multiple of 64."""
+    x = _need(x, "x", dtype=torch.float32, ndim=2)
+    T, K = x.shape
+    for l in layers:
+        w, b, o = (_need(t, n, dtype=torch.float32) for t, n in zip(l, ("weight", "bias", "out")))
+        N_ = w.shape[0]
+        if w.shape != (N_, K) or b.shape != (N_,) or o.shape != (T, N_):
+            raise ValueError("a layer's weight, bias or out does not match x")
+    if T == 0:
+        return
+    n = len(layers)
+    w, b, o = zip(*layers)
+    N.call("pikv_linear_tiled", _ptr(x), T, K, n, _ptr_array(w), _ptr_array(b), (C.c_int32 * n)(*[t.shape[0] for t in w]),
+           _ptr_array(o), _stream())
+
+
 def value_lora(mean, lora_a, lora_b, scaling):
     """mean[e] + ((mean[e] lora_a[e]) lora_b[e]) * scaling[e] for mean [E, H] float32 and lists of E."""
     mean = _need(mean, "mean", dtype=torch.float32, ndim=2)

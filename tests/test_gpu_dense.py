@@ -38,6 +38,27 @@ def test_linear_group(dev, T, K, widths, rank):
         _near(l["out"], y, K * max(rank, 1), 4.5)
 
 
+@pytest.mark.parametrize("T,K,widths", [(1, 64, [1]), (31, 64, [65, 3, 64]), (33, 192, [64] * 20), (129, 128, [50257]),   # 32 x 64 tiles, 64 x 64
+                                        (256, 64, [4000]), (300, 320, [1000, 1500, 50]),                  # 64 x 64
+                                        (511, 128, [2048, 1025, 1000]),                                   # 64 x 128
+                                        (1000, 64, [2048, 1024, 1024]), (641, 448, [5000, 130])])         # 128 x 128
+def test_linear_tiled(dev, T, K, widths):
+    from pikv_amd import ops
+    import torch
+    r = rng(T + K)
+    x = r.standard_normal((T, K)).astype(np.float32)
+    layers, want = [], []
+    for n in widths:
+        w, b = (r.standard_normal(s).astype(np.float32) for s in ((n, K), (n,)))
+        want.append(x.astype(np.float64) @ w.T.astype(np.float64) + b)
+        # a guard row behind the outputs: a tile's last rows and columns must not be written
+        layers.append((to_dev(w, dev), to_dev(b, dev), torch.full((T + 1, n), 7.0, device=dev)))
+    ops.linear_tiled(to_dev(x, dev), [(w, b, o[:T]) for w, b, o in layers])
+    for (_, _, o), y in zip(layers, want):
+        _near(o[:T], y, K, 4.5)
+        assert bool((o[T] == 7.0).all())
+
+
 @pytest.mark.parametrize("E,T,H", [(1, 1, 4), (3, 37, 132), (20, 5, 64)])
 def test_expert_combine(dev, E, T, H):
     """Bit for bit what the torch operations give, each rounded on its own (a scaling that is no power of two: a fused
