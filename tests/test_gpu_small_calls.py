@@ -209,6 +209,30 @@ def test_prefill_attend_takes_views(dev, dh, scheme):
     assert torch.equal(ops.prefill_attend(*views, pool), want)
 
 
+@pytest.mark.parametrize("dh", [64, 128])
+def test_prefill_attend_nan_rows_and_unaligned_output(dev, dh):
+    """A NaN or infinite query makes its own output NaN and no other; an output that begins between 16 bytes holds the same
+    values, and nothing beside it is written."""
+    import torch
+    from pikv_amd import _native as N, ops
+    r = rng(dh + 1)
+    q, k, v = (to_dev(r.standard_normal((2, 45, h, dh)).astype(np.float32), dev) for h in (4, 2, 2))
+    pool, _ = _fill_pool(dev, r, [70] * 2, [70, 9], 2, dh, 32, O.Q_I4_ASYM)
+    want = ops.prefill_attend(q, k, v, pool)
+    bad = q.clone()
+    bad[0, 7, 1, 3], bad[1, 44, 2, 0] = float("nan"), float("inf")
+    got = ops.prefill_attend(bad, k, v, pool)
+    hit = torch.zeros(2, 45, 4, 1, dtype=torch.bool, device=dev)
+    hit[0, 7, 1], hit[1, 44, 2] = True, True
+    assert bool(got.isnan().eq(hit).all()) and torch.equal(torch.where(hit, want, got), want)
+    buf = torch.full((q.numel() + 2,), 7.0, device=dev)
+    p = lambda t: t.data_ptr()
+    N.call("pikv_prefill_attend", p(q), p(k), p(v), 2, 45, 2, 4, dh, 1, dh ** -0.5, *map(p, (*pool._planes("k"), *pool._planes("v"))),
+           pool.scheme, pool.group, p(pool.row_base), p(pool.fill), pool.max_cap, p(buf) + 4, None, 0,
+           torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(buf[1:-1].view_as(want), want) and float(buf[0]) == float(buf[-1]) == 7.0
+
+
 @pytest.mark.parametrize("A", [1, 255, 512, 513, 4095, 4096, 4097, 8191, 8192, 8193, 16000])
 @pytest.mark.parametrize("E,capacity", [(1, 5000), (8, 700), (64, 90)])
 def test_capacity_slots_chunks(dev, A, E, capacity):
