@@ -510,6 +510,13 @@ int pikv_h2o_budget(const int32_t* cache_fill, int n_caches,
                     double heavy_ratio, double recent_ratio,
                     int32_t* n_heavy, int32_t* n_recent, void* stream);
 
+/* pikv_h2o_budget and pikv_evict_select(PIKV_EVICT_H2O, ...) in one call and, for the caches that several blocks select, a launch
+ * less; n_heavy and n_recent [n_caches] are written. */
+int pikv_evict_select_h2o(double heavy_ratio, double recent_ratio, const float* row_acc, const float* row_ts,
+                          const int64_t* cache_row_base, const int32_t* cache_fill, int32_t* n_heavy, int32_t* n_recent,
+                          int n_caches, int64_t max_len, uint8_t* keep_flag, int32_t* keep_index, int32_t* new_len,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Move surviving rows to the front of every cache, in place and in ascending
  * order, for up to PIKV_MAX_PLANES planes (codes, scales, zeros, acc, ts ...),
  * then set cache_fill[c] = new_len[c].

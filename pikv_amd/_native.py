@@ -62,6 +62,7 @@ SIGNATURES = {
                                  _p, _p, _l, _p, _p, _l, _p]),
     "pikv_prefill_attend_workspace_bytes": (_l, [_i, _i, _i, _i, _i, _l]),
     "pikv_evict_select": (_i, [_i, _p, _p, _p, _p, _p, _p, _i, _l, _p, _p, _p, _p, _l, _p]),
+    "pikv_evict_select_h2o": (_i, [_d, _d, _p, _p, _p, _p, _p, _p, _i, _l, _p, _p, _p, _p, _l, _p]),
     "pikv_evict_workspace_bytes": (_l, [_i, _l]),
     "pikv_h2o_budget": (_i, [_p, _i, _d, _d, _p, _p, _p]),
     "pikv_cache_make_room": (_i, [_i, _p, _l, _l, _d, _d, _i, _i, _p, _p, _p, _p, _p, _i, _l,

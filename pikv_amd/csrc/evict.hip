@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kSelThreads) void evict_select_kernel(
 // order-preserving key is split into three digits (11 + 11 + 10 bits); pass p builds
 // the histogram of digit p over the keys that match the digits already chosen
 // (integer atomics into a per-cache table, so the result does not depend on
-// scheduling), and every later kernel re-derives the chosen digits from the tables.
+// scheduling), and every block of the next kernel picks the digit from the table by itself.
 // Kernels, in stream order: zero tables | hist 0 | hist 1 | hist 2 | mark | list.
 // A thread owns 16 CONSECUTIVE rows, so ranks in index order are a thread-local count
 // plus one block scan plus the per-chunk counts of the earlier chunks.
@@ -283,7 +283,7 @@ struct MbArgs {
   uint8_t* keep_flag;
   int32_t* keep_index;
   int32_t* new_len;
-  int* hist;       // [cache][pass 0..2][slot 0..1][kMbBins]
+  int* hist;       // [cache][pass 0..2][slot 0..1][kMbBins]; pass 2 has 1024 bins, and mb_prefix's picks behind them
   int* blk_hist2;  // [cache][chunk][slot][1024]: last-digit histogram of every chunk
   int* blk_kept;   // [cache][chunk]
   int n_chunks;
@@ -373,22 +373,60 @@ __device__ __forceinline__ int mb_pick(const int* __restrict__ hist, int nb, int
   return sh[4];
 }
 
-// Digits chosen by the first `passes` passes for one slot: key prefix and what remains.
-__device__ __forceinline__ uint32_t mb_prefix(const MbArgs& a, int c, int slot, int passes, int& remaining,
+// Digits chosen by the first `passes` passes for one slot: key prefix and what remains.  All but the last of them were chosen by
+// the blocks of the pass before: that of the first chunk has left them in picks (every block picking from all tables
+// again cost the last two kernels 5 us each).
+__device__ __forceinline__ uint32_t mb_prefix(const MbArgs& a, int c, int slot, int passes, int chunk, int& remaining,
                                               int* sh, int* last_digit) {
+  if (passes == 0) return 0;
+  // (key prefix up to the digit, rows left to take, behind the 1024 bins of the last digit's table)
+  int2* const picks = reinterpret_cast<int2*>(a.hist + (((int64_t)c * 3 + 2) * 2 + slot) * kMbBins + 1024);
   uint32_t prefix = 0;
-  for (int p = 0; p < passes; ++p) {
-    const int* h = a.hist + (((int64_t)c * 3 + p) * 2 + slot) * kMbBins;
-    const int d = mb_pick(h, p == 2 ? 1024 : kMbBins, remaining, sh);
-    prefix |= (uint32_t)d << (p == 0 ? 21 : p == 1 ? 10 : 0);
-    if (last_digit) *last_digit = d;
+  if (passes > 1) {
+    const int2 p = picks[passes - 2];
+    prefix = (uint32_t)p.x;
+    remaining = p.y;
   }
+  const int* h = a.hist + (((int64_t)c * 3 + passes - 1) * 2 + slot) * kMbBins;
+  const int d = mb_pick(h, passes == 3 ? 1024 : kMbBins, remaining, sh);
+  prefix |= (uint32_t)d << (passes == 1 ? 21 : passes == 2 ? 10 : 0);
+  if (last_digit) *last_digit = d;
+  if (passes < 3 && chunk == 0 && threadIdx.x == 0) picks[passes - 1] = make_int2((int)prefix, remaining);
   return prefix;
 }
 
-__global__ void mb_zero_kernel(int* __restrict__ p, int64_t n) {
+__device__ __forceinline__ void h2o_budget(int fill, double heavy_ratio, double recent_ratio, int32_t& n_heavy, int32_t& n_recent) {
+  const double len = (double)fill;
+  int h = (int)(len * heavy_ratio);
+  int r = (int)(len * recent_ratio);
+  n_heavy = h < 1 ? 1 : h;
+  n_recent = r < 1 ? 1 : r;
+}
+
+// Clears the tables; with budgets to make (n_heavy not null) the first blocks make those of the caches.
+__global__ void mb_zero_kernel(int* __restrict__ p, int64_t n, const int32_t* __restrict__ fill, int n_caches, double heavy_ratio,
+                               double recent_ratio, int32_t* __restrict__ n_heavy, int32_t* __restrict__ n_recent) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
+  if (n_heavy != nullptr && i < n_caches) h2o_budget(fill[i], heavy_ratio, recent_ratio, n_heavy[i], n_recent[i]);
+  if (4 * i < n) *reinterpret_cast<int4*>(p + 4 * i) = make_int4(0, 0, 0, 0);   // n: a multiple of the bins
+}
+
+// The thread's 16 keys, rows i0 .. i0 + 15 of v; those from len on are not looked at.  Four 16-byte loads where they lie so: sixteen of
+// 4 bytes, every lane on a line of its own, had kept the address unit busy for 7 of a kernel's 12 us.
+__device__ __forceinline__ void mb_keys(const float* __restrict__ v, int64_t i0, int64_t len, bool smallest, uint32_t (&key)[kMbItems]) {
+  if (i0 + kMbItems <= len && (reinterpret_cast<uintptr_t>(v + i0) & 15) == 0) {
+#pragma unroll
+    for (int j = 0; j < kMbItems / 4; ++j) {
+      const float4 x = *reinterpret_cast<const float4*>(v + i0 + 4 * j);
+      key[4 * j] = order_key(x.x, smallest);
+      key[4 * j + 1] = order_key(x.y, smallest);
+      key[4 * j + 2] = order_key(x.z, smallest);
+      key[4 * j + 3] = order_key(x.w, smallest);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kMbItems; ++j) key[j] = i0 + j < len ? order_key(v[i0 + j], smallest) : 0u;
+  }
 }
 
 template <int PASS>
@@ -407,20 +445,18 @@ __global__ __launch_bounds__(kMbThreads) void mb_hist_kernel(MbArgs a) {
     // lies inside the cache, for selections that need a threshold)
     if (!s.partial || (int64_t)chunk * kMbChunk >= len) continue;  // uniform
     int remaining = s.m;
-    const uint32_t prefix = mb_prefix(a, c, slot, PASS, remaining, sh, nullptr);
+    const uint32_t prefix = mb_prefix(a, c, slot, PASS, chunk, remaining, sh, nullptr);
     const uint32_t pmask = mb_mask(PASS);
     for (int b = threadIdx.x; b < NB; b += kMbThreads) lh[b] = 0;
     __syncthreads();
     // neighbouring rows often share a digit (timestamps grow along the cache, scores of a
     // region are of one magnitude): a run of equal digits costs one LDS atomic, not one per row
     int run_digit = -1, run = 0;
+    uint32_t key[kMbItems];
+    mb_keys(s.v, i0, len, s.smallest, key);
 #pragma unroll
     for (int j = 0; j < kMbItems; ++j) {
-      int d = -1;
-      if (i0 + j < len) {
-        const uint32_t key = order_key(s.v[i0 + j], s.smallest);
-        if ((key & pmask) == prefix) d = mb_digit(key, PASS);
-      }
+      const int d = i0 + j < len && (key[j] & pmask) == prefix ? mb_digit(key[j], PASS) : -1;
       if (d != run_digit) {
         if (run_digit >= 0) atomicAdd(&lh[run_digit], run);
         run_digit = d;
@@ -458,20 +494,20 @@ __global__ __launch_bounds__(kMbThreads) void mb_mark_kernel(MbArgs a) {
       continue;
     }
     int remaining = s.m, d2 = 0;
-    const uint32_t kstar = mb_prefix(a, c, slot, 3, remaining, sh, &d2);
+    const uint32_t kstar = mb_prefix(a, c, slot, 3, chunk, remaining, sh, &d2);
     // rows equal to the threshold key in earlier chunks
     int part = 0;
     for (int b = threadIdx.x; b < chunk; b += kMbThreads)
       part += a.blk_hist2[(((int64_t)c * a.n_chunks + b) * 2 + slot) * 1024 + d2];
     int eq_before;
     mb_block_scan(part, sh, eq_before);
-    uint32_t gt = 0, eq = 0;
+    uint32_t gt = 0, eq = 0, key[kMbItems];
+    mb_keys(s.v, i0, len, s.smallest, key);
 #pragma unroll
     for (int j = 0; j < kMbItems; ++j) {
       if (i0 + j < len) {
-        const uint32_t key = order_key(s.v[i0 + j], s.smallest);
-        gt |= (key > kstar ? 1u : 0u) << j;
-        eq |= (key == kstar ? 1u : 0u) << j;
+        gt |= (key[j] > kstar ? 1u : 0u) << j;
+        eq |= (key[j] == kstar ? 1u : 0u) << j;
       }
     }
     int tot;
@@ -550,12 +586,7 @@ __global__ void h2o_budget_kernel(const int32_t* __restrict__ fill, int n, doubl
                                   double recent_ratio, int32_t* __restrict__ n_heavy,
                                   int32_t* __restrict__ n_recent) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  const double len = (double)fill[c];
-  int h = (int)(len * heavy_ratio);
-  int r = (int)(len * recent_ratio);
-  n_heavy[c] = h < 1 ? 1 : h;
-  n_recent[c] = r < 1 ? 1 : r;
+  if (c < n) h2o_budget(fill[c], heavy_ratio, recent_ratio, n_heavy[c], n_recent[c]);
 }
 
 // ---- compaction -------------------------------------------------------------------
@@ -567,7 +598,7 @@ struct CompactPlanes {
 };
 
 constexpr int kSlabBytes = 256;
-constexpr int kRowsUnroll = 16;
+constexpr int kHeadUnroll = 16, kTailUnroll = 8;   // rows of a thread in flight
 
 // Survivor j of a cache moves from row keep[j] to row j (keep ascending, keep[j] >= j).
 // The m survivors split at j* = first j with keep[j] >= m:
@@ -578,36 +609,40 @@ constexpr int kRowsUnroll = 16;
 //     destinations [j*, m) are read by the head only - once the head is done they can move
 //     in any order, by as many blocks as there are.
 // After an eviction that keeps a small fraction nearly every survivor is in the tail.
+// Either kernel tells a row's part from its source; a search for j* would be a dozen dependent loads in every block.  All
+// source numbers of a pass are loaded before the first row: with each row behind its own number the moves of 64 x 32768 rows to a
+// half took 961 us, now 634 (4.3 TB/s of bytes read and written), to a 14th 124, now 94 (pieces of 64 to 256 bytes).
 template <typename V, bool TAIL>
 __device__ __forceinline__ void compact_slab(char* plane, int64_t row_bytes, int64_t base_row,
                                              int64_t col0, int slab_bytes,
-                                             const int32_t* __restrict__ keep, int j_begin, int j_end,
-                                             int chunk, int n_chunks) {
+                                             const int32_t* __restrict__ keep, int m, int chunk, int n_chunks) {
+  constexpr int U = TAIL ? kTailUnroll : kHeadUnroll;
   const int lanes_per_row = slab_bytes / (int)sizeof(V);
   const int rows_per_pass = 256 / lanes_per_row;
   const int lane_in_row = threadIdx.x % lanes_per_row;
   const int row_in_pass = threadIdx.x / lanes_per_row;
   const bool active = row_in_pass < rows_per_pass;  // 256 % lanes_per_row may be non-zero
-  const int step_rows = rows_per_pass * kRowsUnroll;
+  const int step_rows = rows_per_pass * U;
   const int64_t col = col0 + (int64_t)lane_in_row * sizeof(V);
-  for (int j0 = j_begin + chunk * step_rows; j0 < j_end; j0 += n_chunks * step_rows) {
-    V val[kRowsUnroll];
-    int src[kRowsUnroll];
+  for (int j0 = chunk * step_rows; j0 < m; j0 += n_chunks * step_rows) {
+    if (!TAIL && keep[j0] >= m) break;               // uniform: the rest are the tail's
+    V val[U];
+    int src[U];
 #pragma unroll
-    for (int u = 0; u < kRowsUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int j = j0 + u * rows_per_pass + row_in_pass;
-      src[u] = -1;
+      src[u] = active && j < m ? keep[j] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = j0 + u * rows_per_pass + row_in_pass;
+      if (TAIL ? src[u] < m : src[u] >= m || src[u] == j) src[u] = -1;
       val[u] = V{};
-      if (active && j < j_end) {
-        const int s = keep[j];
-        if (s != j) src[u] = s;
-      }
-      if (src[u] >= 0)
-        val[u] = *reinterpret_cast<const V*>(plane + (base_row + src[u]) * row_bytes + col);
+      if (src[u] >= 0) val[u] = *reinterpret_cast<const V*>(plane + (base_row + src[u]) * row_bytes + col);
     }
     if (!TAIL) __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kRowsUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int j = j0 + u * rows_per_pass + row_in_pass;
       if (src[u] >= 0) *reinterpret_cast<V*>(plane + (base_row + j) * row_bytes + col) = val[u];
     }
@@ -615,16 +650,19 @@ __device__ __forceinline__ void compact_slab(char* plane, int64_t row_bytes, int
   }
 }
 
-// grid (slabs of all planes, caches, chunks).  TAIL = false: chunks == 1.  SOME: caches with active[c] == 0 are left alone.
+// grid (slabs of all planes, caches, chunks).  TAIL = false: chunks == 1, and cache_fill (or null) becomes new_len.
+// SOME: caches with active[c] == 0 are left alone.
 template <bool TAIL, bool SOME>
 __global__ __launch_bounds__(256) void compact_rows_kernel(CompactPlanes pl,
                                                            const int64_t* __restrict__ row_base,
                                                            const int32_t* __restrict__ keep_index,
                                                            const int32_t* __restrict__ new_len,
-                                                           const int32_t* __restrict__ active) {
+                                                           const int32_t* __restrict__ active, int32_t* __restrict__ cache_fill) {
   const int c = blockIdx.y;
   if (SOME && active[c] == 0) return;                // every row of this cache stays where it is
   const int slab = blockIdx.x;
+  const int m = new_len[c];
+  if (!TAIL && cache_fill != nullptr && slab == 0 && threadIdx.x == 0) cache_fill[c] = m;
   int p = 0;
   while (p + 1 < pl.n_planes && slab >= pl.slab_begin[p + 1]) ++p;
   const int64_t rb = pl.row_bytes[p];
@@ -632,29 +670,19 @@ __global__ __launch_bounds__(256) void compact_rows_kernel(CompactPlanes pl,
   const int64_t left = rb - col0;
   const int slab_bytes = left < kSlabBytes ? (int)left : kSlabBytes;
   const int64_t base = row_base[c];
-  const int m = new_len[c];
   const int32_t* keep = keep_index + base;
-  // j* = first survivor whose source lies beyond the final region (binary search, uniform)
-  int lo = 0, hi = m;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (keep[mid] >= m) hi = mid; else lo = mid + 1;
-  }
-  const int j_begin = TAIL ? lo : 0;
-  const int j_end = TAIL ? m : lo;
-  if (j_begin >= j_end) return;  // uniform
   char* plane = reinterpret_cast<char*>(pl.ptr[p]);
   const int chunk = TAIL ? (int)blockIdx.z : 0;
   const int n_chunks = TAIL ? (int)gridDim.z : 1;
   // widest element that every row start is aligned to
   if (rb % 16 == 0)
-    compact_slab<uint4, TAIL>(plane, rb, base, col0, slab_bytes, keep, j_begin, j_end, chunk, n_chunks);
+    compact_slab<uint4, TAIL>(plane, rb, base, col0, slab_bytes, keep, m, chunk, n_chunks);
   else if (rb % 4 == 0)
-    compact_slab<uint32_t, TAIL>(plane, rb, base, col0, slab_bytes, keep, j_begin, j_end, chunk, n_chunks);
+    compact_slab<uint32_t, TAIL>(plane, rb, base, col0, slab_bytes, keep, m, chunk, n_chunks);
   else if (rb % 2 == 0)
-    compact_slab<uint16_t, TAIL>(plane, rb, base, col0, slab_bytes, keep, j_begin, j_end, chunk, n_chunks);
+    compact_slab<uint16_t, TAIL>(plane, rb, base, col0, slab_bytes, keep, m, chunk, n_chunks);
   else
-    compact_slab<uint8_t, TAIL>(plane, rb, base, col0, slab_bytes, keep, j_begin, j_end, chunk, n_chunks);
+    compact_slab<uint8_t, TAIL>(plane, rb, base, col0, slab_bytes, keep, m, chunk, n_chunks);
 }
 
 __global__ void set_fill_kernel(int32_t* __restrict__ fill, const int32_t* __restrict__ new_len, int n) {
@@ -845,12 +873,16 @@ extern "C" int64_t pikv_evict_workspace_bytes(int n_caches, int64_t max_len) {
   return (int64_t)n_caches * (3 * 2 * kMbBins + nch * 2 * 1024 + nch) * (int64_t)sizeof(int);
 }
 
-extern "C" int pikv_evict_select(int policy, const float* row_acc, const float* row_ts,
-                                 const int64_t* cache_row_base, const int32_t* cache_fill,
-                                 const int32_t* n_heavy, const int32_t* n_recent, int n_caches,
-                                 int64_t max_len, uint8_t* keep_flag, int32_t* keep_index,
-                                 int32_t* new_len, void* workspace, int64_t workspace_bytes,
-                                 void* stream) {
+// Budgets the kernels make first (H2O), from the caches' fill.
+struct SelectRatios {
+  double heavy, recent;
+  int32_t *n_heavy, *n_recent;
+};
+
+static int evict_select(int policy, const float* row_acc, const float* row_ts, const int64_t* cache_row_base,
+                        const int32_t* cache_fill, const int32_t* n_heavy, const int32_t* n_recent, const SelectRatios* ratios,
+                        int n_caches, int64_t max_len, uint8_t* keep_flag, int32_t* keep_index, int32_t* new_len,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
   if (!row_ts || !cache_row_base || !cache_fill || !n_heavy || !keep_flag || !keep_index || !new_len)
     return PIKV_ERR_NULL;
   if (policy != PIKV_EVICT_H2O && policy != PIKV_EVICT_LRU) return PIKV_ERR_UNSUPPORTED;
@@ -870,7 +902,9 @@ extern "C" int pikv_evict_select(int policy, const float* row_acc, const float* 
     a.blk_hist2 = a.hist + (int64_t)n_caches * 3 * 2 * kMbBins;
     a.blk_kept = a.blk_hist2 + (int64_t)n_caches * nch * 2 * 1024;
     const int64_t nz = (int64_t)n_caches * 3 * 2 * kMbBins;
-    hipLaunchKernelGGL(mb_zero_kernel, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, st, a.hist, nz);
+    const SelectRatios r = ratios ? *ratios : SelectRatios{};
+    hipLaunchKernelGGL(mb_zero_kernel, dim3((unsigned)((nz / 4 + 255) / 256)), dim3(256), 0, st, a.hist, nz, cache_fill, n_caches,
+                       r.heavy, r.recent, r.n_heavy, r.n_recent);
     const dim3 grid((unsigned)nch, (unsigned)n_caches);
     const dim3 grid2((unsigned)nch, (unsigned)n_caches, 2);
     hipLaunchKernelGGL(mb_hist_kernel<0>, grid2, dim3(kMbThreads), 0, st, a);
@@ -881,11 +915,33 @@ extern "C" int pikv_evict_select(int policy, const float* row_acc, const float* 
     PIKV_CHECK_LAUNCH();
     return PIKV_OK;
   }
+  if (ratios)
+    hipLaunchKernelGGL(h2o_budget_kernel, dim3((n_caches + 63) / 64), dim3(64), 0, st, cache_fill, n_caches, ratios->heavy,
+                       ratios->recent, ratios->n_heavy, ratios->n_recent);
   hipLaunchKernelGGL(evict_select_kernel, dim3((unsigned)n_caches), dim3(kSelThreads), 0, st, policy,
                      row_acc, row_ts, cache_row_base, cache_fill, n_heavy, n_recent, keep_flag,
                      keep_index, new_len);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
+}
+
+extern "C" int pikv_evict_select(int policy, const float* row_acc, const float* row_ts,
+                                 const int64_t* cache_row_base, const int32_t* cache_fill,
+                                 const int32_t* n_heavy, const int32_t* n_recent, int n_caches,
+                                 int64_t max_len, uint8_t* keep_flag, int32_t* keep_index,
+                                 int32_t* new_len, void* workspace, int64_t workspace_bytes,
+                                 void* stream) {
+  return evict_select(policy, row_acc, row_ts, cache_row_base, cache_fill, n_heavy, n_recent, nullptr, n_caches, max_len,
+                      keep_flag, keep_index, new_len, workspace, workspace_bytes, stream);
+}
+
+extern "C" int pikv_evict_select_h2o(double heavy_ratio, double recent_ratio, const float* row_acc, const float* row_ts,
+                                     const int64_t* cache_row_base, const int32_t* cache_fill, int32_t* n_heavy,
+                                     int32_t* n_recent, int n_caches, int64_t max_len, uint8_t* keep_flag, int32_t* keep_index,
+                                     int32_t* new_len, void* workspace, int64_t workspace_bytes, void* stream) {
+  const SelectRatios r{heavy_ratio, recent_ratio, n_heavy, n_recent};
+  return evict_select(PIKV_EVICT_H2O, row_acc, row_ts, cache_row_base, cache_fill, n_heavy, n_recent, &r, n_caches, max_len,
+                      keep_flag, keep_index, new_len, workspace, workspace_bytes, stream);
 }
 
 extern "C" int pikv_h2o_budget(const int32_t* cache_fill, int n_caches, double heavy_ratio,
@@ -917,26 +973,30 @@ static int make_planes(void* const* plane_ptrs_host, const int64_t* plane_row_by
   return PIKV_OK;
 }
 
-// active [n_caches] or nullptr: caches with active[c] == 0 are left alone
 template <bool SOME>
 static void launch_compact_form(const CompactPlanes& pl, const int64_t* cache_row_base, const int32_t* keep_index,
-                                const int32_t* new_len, const int32_t* active, int n_caches, hipStream_t st) {
+                                const int32_t* new_len, const int32_t* active, int32_t* cache_fill, int n_caches, hipStream_t st) {
   const int slabs = pl.slab_begin[pl.n_planes];
   if (slabs > 0) {
     // ordered head first, then the free-moving tail spread over enough blocks to fill the chip
     hipLaunchKernelGGL((compact_rows_kernel<false, SOME>), dim3((unsigned)slabs, (unsigned)n_caches), dim3(256), 0,
-                       st, pl, cache_row_base, keep_index, new_len, active);
-    int64_t chunks = 4096 / ((int64_t)slabs * n_caches);
+                       st, pl, cache_row_base, keep_index, new_len, active, cache_fill);
+    // (us of both launches with 8 rows a thread and 4096 / 8192 / 16384 blocks: 64 caches x 32768 rows of 1288 bytes to a 14th
+    // 99 / 94 / 93, to a half 645 / 634 / 625; 20 x 12000 rows of 600 bytes 15 / 17 / 19)
+    int64_t chunks = 8192 / ((int64_t)slabs * n_caches);
     chunks = chunks < 1 ? 1 : (chunks > 64 ? 64 : chunks);
     hipLaunchKernelGGL((compact_rows_kernel<true, SOME>), dim3((unsigned)slabs, (unsigned)n_caches, (unsigned)chunks),
-                       dim3(256), 0, st, pl, cache_row_base, keep_index, new_len, active);
+                       dim3(256), 0, st, pl, cache_row_base, keep_index, new_len, active, nullptr);
+  } else if (cache_fill) {
+    hipLaunchKernelGGL(set_fill_kernel, dim3((n_caches + 63) / 64), dim3(64), 0, st, cache_fill, new_len, n_caches);
   }
 }
 
+// active [n_caches] or nullptr: caches with active[c] == 0 are left alone; cache_fill or nullptr: becomes new_len
 static void launch_compact(const CompactPlanes& pl, const int64_t* cache_row_base, const int32_t* keep_index,
-                           const int32_t* new_len, const int32_t* active, int n_caches, hipStream_t st) {
-  if (active != nullptr) launch_compact_form<true>(pl, cache_row_base, keep_index, new_len, active, n_caches, st);
-  else launch_compact_form<false>(pl, cache_row_base, keep_index, new_len, active, n_caches, st);
+                           const int32_t* new_len, const int32_t* active, int32_t* cache_fill, int n_caches, hipStream_t st) {
+  if (active != nullptr) launch_compact_form<true>(pl, cache_row_base, keep_index, new_len, active, cache_fill, n_caches, st);
+  else launch_compact_form<false>(pl, cache_row_base, keep_index, new_len, active, cache_fill, n_caches, st);
 }
 
 extern "C" int pikv_compact_rows(void* const* plane_ptrs_host, const int64_t* plane_row_bytes_host,
@@ -951,10 +1011,7 @@ extern "C" int pikv_compact_rows(void* const* plane_ptrs_host, const int64_t* pl
   CompactPlanes pl;
   const int rc = make_planes(plane_ptrs_host, plane_row_bytes_host, n_planes, pl);
   if (rc != PIKV_OK) return rc;
-  launch_compact(pl, cache_row_base, keep_index, new_len, nullptr, n_caches, st);
-  if (cache_fill)
-    hipLaunchKernelGGL(set_fill_kernel, dim3((n_caches + 63) / 64), dim3(64), 0, st, cache_fill,
-                       new_len, n_caches);
+  launch_compact(pl, cache_row_base, keep_index, new_len, nullptr, cache_fill, n_caches, st);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
 }
@@ -995,7 +1052,7 @@ extern "C" int pikv_cache_make_room(int policy, const int32_t* count, int64_t co
     const bool here = policy == PIKV_EVICT_ALL || kept * (double)row <= most;
     CompactPlanes none{};
     hipLaunchKernelGGL(room_small_kernel, dim3((unsigned)n_caches), dim3(kSelThreads), 0, st, a, here ? pl : none);
-    if (!here) launch_compact(pl, cache_row_base, keep_index, new_len, a.active, n_caches, st);
+    if (!here) launch_compact(pl, cache_row_base, keep_index, new_len, a.active, nullptr, n_caches, st);
     PIKV_CHECK_LAUNCH();
     return PIKV_OK;
   }
@@ -1004,7 +1061,7 @@ extern "C" int pikv_cache_make_room(int policy, const int32_t* count, int64_t co
   rc = pikv_evict_select(policy, row_acc, row_ts, cache_row_base, cache_fill, a.n_heavy, a.n_recent, n_caches, max_len,
                          keep_flag, keep_index, new_len, workspace, workspace_bytes, stream);
   if (rc != PIKV_OK) return rc;
-  launch_compact(pl, cache_row_base, keep_index, new_len, a.active, n_caches, st);
+  launch_compact(pl, cache_row_base, keep_index, new_len, a.active, nullptr, n_caches, st);
   hipLaunchKernelGGL(room_fill_kernel, cgrid, dim3(64), 0, st, a);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;

@@ -913,14 +913,12 @@ class CachePool:
         ratios (per cache, from its current fill) or explicit int32 tensors;
         LRU: n_evict int32 [n_caches].  multi_block=False withholds the workspace, so
         that one block selects each cache whatever its length (same result)."""
-        if policy == EVICT_H2O:
-            if n_heavy is None:
-                N.call("pikv_h2o_budget", _ptr(self.fill), self.n_caches, float(heavy_ratio),
-                       float(recent_ratio), _ptr(self.n_heavy), _ptr(self.n_recent), _stream())
-                nh, nr = self.n_heavy, self.n_recent
-            else:
-                nh = _need(n_heavy, "n_heavy", dtype=torch.int32, ndim=1)
-                nr = _need(n_recent, "n_recent", dtype=torch.int32, ndim=1)
+        ratios = policy == EVICT_H2O and n_heavy is None
+        if ratios:
+            nh, nr = self.n_heavy, self.n_recent
+        elif policy == EVICT_H2O:
+            nh = _need(n_heavy, "n_heavy", dtype=torch.int32, ndim=1)
+            nr = _need(n_recent, "n_recent", dtype=torch.int32, ndim=1)
         elif policy == EVICT_LRU:
             nh = _need(n_evict, "n_evict", dtype=torch.int32, ndim=1)
             nr = None
@@ -933,9 +931,12 @@ class CachePool:
             if getattr(self, "_evict_ws", None) is None:
                 self._evict_ws = _evict_workspace(self.n_caches, self.max_cap, self.device)
             ws, ws_bytes = self._evict_ws
-        N.call("pikv_evict_select", policy, _ptr(self.acc), _ptr(self.ts), _ptr(self.row_base),
-               _ptr(self.fill), _ptr(nh), _ptr(nr), self.n_caches, self.max_cap, _ptr(self.keep_flag),
-               _ptr(self.keep_index), _ptr(self.new_len), _ptr(ws), ws_bytes, _stream())
+        args = (_ptr(self.acc), _ptr(self.ts), _ptr(self.row_base), _ptr(self.fill), _ptr(nh), _ptr(nr), self.n_caches,
+                self.max_cap, _ptr(self.keep_flag), _ptr(self.keep_index), _ptr(self.new_len), _ptr(ws), ws_bytes, _stream())
+        if ratios:
+            N.call("pikv_evict_select_h2o", float(heavy_ratio), float(recent_ratio), *args)
+        else:
+            N.call("pikv_evict_select", policy, *args)
 
     def planes(self):
         ps = [self.k_codes, self.k_scale, self.k_zero, self.v_codes, self.v_scale, self.v_zero,

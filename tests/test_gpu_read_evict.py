@@ -375,6 +375,35 @@ def test_h2o_select_long_cache(dev, ties, multi_block):
     _check_compacted(pool, ref, O.Q_I8_SYM, keeps)
 
 
+@pytest.mark.parametrize("policy,heavy", [(0, 0.07), (0, 0.6), (1, None)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_long_caches_at_odd_rows(dev, ties, policy, heavy):
+    """Caches whose rows begin at no multiple of four (keys read one by one) beside ones that do, budgets from the ratios in the
+    call that selects, survivors inside and beyond the final region over several passes of the moves, and the fill after them."""
+    r = rng(57 + ties)
+    caps = [20001, 9002, 4, 20003, 12000]
+    lens = [20001, 9001, 4, 8192, 11999]
+    pool, ref = _fill_pool(dev, r, caps, lens, 2, 32, 32, O.Q_I4_ASYM, dtype="f32")
+    _set_state(pool, ref, r, ties)
+    ne = np.array([10000, 1, 4, 8000, 6000], dtype=np.int32)
+    if policy == 0:
+        pool.evict_select(0, heavy_ratio=heavy, recent_ratio=0.01)
+    else:
+        pool.evict_select(1, n_evict=to_dev(ne, dev))
+    keeps = []
+    for c, L in enumerate(lens):
+        rows = ref.valid_rows(c)
+        if policy == 0:
+            nh, nr = O.h2o_budget(L, heavy, 0.01)
+            assert (int(np_of(pool.n_heavy)[c]), int(np_of(pool.n_recent)[c])) == (nh, nr)
+            keeps.append(O.h2o_keep(ref.acc[rows], ref.ts[rows], nh, nr))
+        else:
+            keeps.append(O.lru_keep(ref.ts[rows], int(ne[c])))
+        assert np.array_equal(np_of(pool.keep_flag)[rows].astype(bool), keeps[-1]), c
+    pool.compact()
+    _check_compacted(pool, ref, O.Q_I4_ASYM, keeps)
+
+
 @pytest.mark.parametrize("ties", [False, True])
 def test_select_chunked_edges(dev, ties):
     """Several blocks per cache: empty cache, lengths around the 4096-row chunk edge,
