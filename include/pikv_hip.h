@@ -599,6 +599,10 @@ int pikv_value_lora(const float* mean, int n_experts, int H, int rank, const flo
 int pikv_expert_combine(const float* const* dense, const float* const* lora, const float* scaling,
                         const float* add, const float* weights, int64_t T, int E, int H, float* outs,
                         float* mix, void* stream);
+/* The same with lora[e] = lora_t[e] lora_b[e], lora_t [T][rank], lora_b [rank][H] (16-byte aligned). */
+int pikv_expert_combine_factors(const float* const* dense, const float* const* lora_t, const float* const* lora_b, int rank,
+                                const float* scaling, const float* add, const float* weights, int64_t T, int E, int H,
+                                float* outs, float* mix, void* stream);
 
 /* AdaptiveRouter (core/single/routing_strategy.py:100-150) behind its hidden layers, T = n_seqs * S:
  *   blend [n_seqs][2] = softmax(relu(x_mean sel_w1^T + sel_b1) sel_w2^T + sel_b2)

@@ -76,6 +76,8 @@ SIGNATURES = {
     "pikv_cache_mean_workspace_bytes": (_l, [_i, _i, _l]),
     "pikv_value_lora": (_i, [_p, _i, _i, _i, C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), _p, _p]),
     "pikv_expert_combine": (_i, [C.POINTER(_p), C.POINTER(_p), C.POINTER(_f), _p, _p, _l, _i, _i, _p, _p, _p]),
+    "pikv_expert_combine_factors": (_i, [C.POINTER(_p), C.POINTER(_p), C.POINTER(_p), _i, C.POINTER(_f), _p, _p, _l, _i, _i,
+                                         _p, _p, _p]),
     "pikv_adaptive_router": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _f, _p, _p, _p,
                                   _p, _f, _p, _p, _p, _p, _p, _p, _p, _p]),
     "pikv_quant_scatter_routed": (_i, [_p, _p, _l, _i, _i, _i, _i, _p, _p, _p, _p, _p, _i,

@@ -6,9 +6,10 @@
 // single compute unit (one 256 x 128 tile, 33 us).  Here a tile is 32 x 32 and the contraction is split over the
 // wavefronts of its block, so that one launch of all layers covers the chip and no chain is longer than a quarter of
 // the contraction.  Everything is float32 (v_mfma_f32_32x32x2_f32): products, sums and results; error against
-// float64 2.1e-7 where the library's is 4.1e-7.  The experts' own products stay with the library: their outputs are
-// quantised into the caches and come back as means in the next call, where another order of their sums - 2e-7, a code
-// in 10^4 - grew to 1e-4 of a cached row's scale.
+// float64 2.1e-7 where the library's is 4.1e-7.  The experts' own products keep the library's order of sums - one launch
+// of linear_tiled at the sizes where that order is the same, library calls elsewhere: their outputs are quantised into the
+// caches and come back as means in the next call, where another order - 2e-7, a code in 10^4 - grew to 1e-4 of a cached row's
+// scale.  The second factor of their LoRA is taken in expert_combine.  Evaluation pass of 128 tokens x 256, 4 experts: 644 -> 513 us.
 // Measured: linear_group, three layers of 2048 x 2048 over 8 rows 23 us a call and 19 in a replayed graph (61 and 26 as
 // three library calls), over 128 rows 55 a call (59); adaptive router with 128 tokens of 256, 4 experts 7.7 + 5.2 + 7.0 +
 // 3.0 us of kernels for 35 launches.  The kernels are made for that scale: no LDS tile in linear_group, one block a sequence
@@ -237,17 +238,21 @@ __global__ __launch_bounds__(256) void value_lora_kernel(ValueLoraArgs a) {
 // ---- experts behind their products ----------------------------------------------------------------
 struct ExpertArgs {
   const float* dense[kMaxGroups];   // [T][H]
-  const float* lora[kMaxGroups];    // [T][H]
+  const float* lora[kMaxGroups];    // [T][H]; with factors [T][rank]
+  const float* lora_b[kMaxGroups];  // with factors [rank][H]
   float scaling[kMaxGroups];
   const float* add;                 // [E][H]
   const float* w;                   // [T][E]
   float* outs;                      // [E][T][H]
   float* mix;                       // [T][H]
   int64_t T;
-  int E, H4;
+  int E, H4, rank;
 };
 
 // outs[e] = relu(dense[e] + lora[e] * scaling[e]) + add[e]; mix[t] = sum over e, in order, of outs[e][t] * w[t][e].
+// FACTORS: lora[e] is the product of two factors of a small rank, added up here by fused multiply-adds in ascending order - to the
+// last bit what the library's product of that rank gives, without its launch (8 us each for 128 tokens of 256).
+template <bool FACTORS>
 __global__ __launch_bounds__(256) void expert_combine_kernel(ExpertArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= a.T * a.H4) return;
@@ -256,7 +261,16 @@ __global__ __launch_bounds__(256) void expert_combine_kernel(ExpertArgs a) {
   float s[4] = {0.f, 0.f, 0.f, 0.f};
   for (int e = 0; e < a.E; ++e) {
     const float4 d = reinterpret_cast<const float4*>(a.dense[e])[i];
-    const float4 l = reinterpret_cast<const float4*>(a.lora[e])[i];
+    float4 l = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (FACTORS) {
+      for (int j = 0; j < a.rank; ++j) {
+        const float u = a.lora[e][t * a.rank + j];
+        const float4 b = reinterpret_cast<const float4*>(a.lora_b[e])[j * a.H4 + h];
+        l = make_float4(fmaf(u, b.x, l.x), fmaf(u, b.y, l.y), fmaf(u, b.z, l.z), fmaf(u, b.w, l.w));
+      }
+    } else {
+      l = reinterpret_cast<const float4*>(a.lora[e])[i];
+    }
     const float4 c = reinterpret_cast<const float4*>(a.add)[(int64_t)e * a.H4 + h];
     const float dv[4] = {d.x, d.y, d.z, d.w}, lv[4] = {l.x, l.y, l.z, l.w}, cv[4] = {c.x, c.y, c.z, c.w};
     const float we = a.w[t * a.E + e];
@@ -534,22 +548,38 @@ extern "C" int pikv_value_lora(const float* mean, int n_experts, int H, int rank
   return PIKV_OK;
 }
 
-extern "C" int pikv_expert_combine(const float* const* dense, const float* const* lora, const float* scaling,
-                                   const float* add, const float* weights, int64_t T, int E, int H, float* outs,
-                                   float* mix, void* stream) {
+static int expert_combine(const float* const* dense, const float* const* lora, const float* const* lora_b, int rank,
+                          const float* scaling, const float* add, const float* weights, int64_t T, int E, int H, float* outs,
+                          float* mix, void* stream) {
   if (!dense || !lora || !scaling || !add || !weights || !outs || !mix) return PIKV_ERR_NULL;
   if (T < 1 || E < 1 || H < 4 || H % 4 != 0 || (T * (H / 4) + 255) / 256 > 0x7fffffffLL) return PIKV_ERR_SHAPE;
   if (E > kMaxGroups) return PIKV_ERR_UNSUPPORTED;
   ExpertArgs a{};
   for (int e = 0; e < E; ++e) {
-    if (!dense[e] || !lora[e]) return PIKV_ERR_NULL;
+    if (!dense[e] || !lora[e] || (lora_b && !lora_b[e])) return PIKV_ERR_NULL;
     a.dense[e] = dense[e]; a.lora[e] = lora[e]; a.scaling[e] = scaling[e];
+    if (lora_b) a.lora_b[e] = lora_b[e];
   }
-  a.add = add; a.w = weights; a.outs = outs; a.mix = mix; a.T = T; a.E = E; a.H4 = H / 4;
-  hipLaunchKernelGGL(expert_combine_kernel, dim3((unsigned)((T * (H / 4) + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream, a);
+  a.add = add; a.w = weights; a.outs = outs; a.mix = mix; a.T = T; a.E = E; a.H4 = H / 4; a.rank = rank;
+  const dim3 grid((unsigned)((T * (H / 4) + 255) / 256));
+  if (lora_b) hipLaunchKernelGGL(expert_combine_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, a);
+  else hipLaunchKernelGGL(expert_combine_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, a);
   PIKV_CHECK_LAUNCH();
   return PIKV_OK;
+}
+
+extern "C" int pikv_expert_combine(const float* const* dense, const float* const* lora, const float* scaling,
+                                   const float* add, const float* weights, int64_t T, int E, int H, float* outs,
+                                   float* mix, void* stream) {
+  return expert_combine(dense, lora, nullptr, 0, scaling, add, weights, T, E, H, outs, mix, stream);
+}
+
+extern "C" int pikv_expert_combine_factors(const float* const* dense, const float* const* lora_t, const float* const* lora_b,
+                                           int rank, const float* scaling, const float* add, const float* weights, int64_t T,
+                                           int E, int H, float* outs, float* mix, void* stream) {
+  if (!lora_b) return PIKV_ERR_NULL;
+  if (rank < 1) return PIKV_ERR_SHAPE;
+  return expert_combine(dense, lora_t, lora_b, rank, scaling, add, weights, T, E, H, outs, mix, stream);
 }
 
 extern "C" int pikv_adaptive_router(const float* x_mean, int n_seqs, int S, int H, int H2, int E, int top_k,

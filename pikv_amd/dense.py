@@ -79,6 +79,15 @@ def tiled_pays(T: int, H: int, widths) -> bool:
     return tiles <= 256 and T * N >= 0.85 * 256 * 128 * 128
 
 
+def experts_tiled(T: int, H: int, E: int) -> bool:
+    """The products of E experts [H, H] in one launch of LDS tiles: 128 x 256, 4 experts 14 us for four library calls of 34 on one
+    compute unit each; 2048 x 512, 4 experts 45 / 80.  Only where the library sums in the same order to the last bit: what the
+    experts put out is cached in codes, and the means of the caches come back in the next call.  That is from 33 tokens on but
+    for 257 to 1024 tokens of less than 384 columns (128 columns: 257 on), and for few tokens of more than 512."""
+    return (33 <= T and (T <= 256 or H >= 384 or (H >= 256 and T > 1024)) and (H <= 512 or T >= 512)
+            and T * H * H * E <= 3_500_000_000)
+
+
 def key_projection_pays(T: int, H: int) -> bool:
     """One [H, H] layer with LoRA: 1024 x 512 22 / 71, 2048 x 512 34 / 69, 256 x 1024 23 / 74, 128 x 2048 38 / 71; outside
     8192 x 512 111 / 79, 2048 x 1024 90 / 79, 512 x 2048 91 / 71, 128 x 4096 105 / 89."""

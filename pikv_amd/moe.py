@@ -249,9 +249,9 @@ class PiKVMoE(nn.Module):
                    for e, c in zip(self.experts, self.kv_caches))
 
     def _experts_forward(self, x, cached, routing_weights):
-        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]): the experts' products by the
-        library, bit for bit those of LoRAExpert.forward, the rest in four launches (the key projection of many
-        or wide rows by the library too)."""
+        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]): the experts' products bit for bit
+        those of LoRAExpert.forward - in one launch where that sums in the library's order (dense.experts_tiled), by the
+        library otherwise - and the rest in four launches (the key projection of many or wide rows by the library too)."""
         H = x.shape[-1]
         x2 = x.reshape(-1, H)
         T, E = x2.shape[0], len(self.experts)
@@ -264,12 +264,15 @@ class PiKVMoE(nn.Module):
                              rank=self.key_lora.lora_A.shape[1])
         else:
             keys = self.key_proj(x2) + self.key_lora(x2)
-        products, terms = [], []
-        for e in self.experts:
-            products.append(F.linear(x2, e.dense.weight, e.dense.bias))
-            terms.append(torch.mm(torch.mm(x2, e.lora.lora_A), e.lora.lora_B))
-        outs, mix = ops.expert_combine(products, terms, [e.lora.scaling for e in self.experts], add,
-                                       routing_weights.view(T, E))
+        scaling = [e.lora.scaling for e in self.experts]
+        weights = routing_weights.view(T, E)
+        if dense.experts_tiled(T, H, E):
+            products = torch.empty(E, T, H, dtype=torch.float32, device=x.device).unbind()
+            ops.linear_tiled(x2, [(e.dense.weight, e.dense.bias, o) for e, o in zip(self.experts, products)])
+        else:
+            products = [F.linear(x2, e.dense.weight, e.dense.bias) for e in self.experts]
+        inner = [torch.mm(x2, e.lora.lora_A) for e in self.experts]
+        outs, mix = ops.expert_combine(products, inner, scaling, add, weights, lora_b=[e.lora.lora_B for e in self.experts])
         return outs, keys, mix
 
     def update_cache(self, expert_idx, key, value, importance):

@@ -475,16 +475,20 @@ def value_lora(mean, lora_a, lora_b, scaling):
     return out
 
 
-def expert_combine(dense, lora, scaling, add, weights):
+def expert_combine(dense, lora, scaling, add, weights, lora_b=None):
     """(outs [E, T, H], mix [T, H]): outs[e] = relu(dense[e] + lora[e] * scaling[e]) + add[e], mix the sum over e, in
     order, of outs[e][t] * weights[t][e].  dense, lora: lists of E (at most 20) tensors [T, H]; add [E, H]; weights
-    [T, E]; float32."""
+    [T, E]; float32.  With lora_b (E tensors [rank, H]) lora[e] is [T, rank], and its product with lora_b[e] is taken."""
     E, (T, H) = len(dense), dense[0].shape
     if not 1 <= E == len(lora) == len(scaling) or H % 4:
         raise ValueError("one lora and scaling per expert, and a width that is a multiple of 4")
-    for t in (*dense, *lora):
-        if _need(t, "an expert's product", dtype=torch.float32).shape != (T, H) or t.data_ptr() % 16:
-            raise ValueError(f"the experts' products must be [{T}, {H}] and 16-byte aligned")
+    rank = H if lora_b is None else lora_b[0].shape[0]
+    for ts, shape, align in ((dense, (T, H), 16), (lora, (T, rank), 16 if lora_b is None else 4), (lora_b or (), (rank, H), 16)):
+        for t in ts:
+            if _need(t, "an expert's product", dtype=torch.float32).shape != shape or t.data_ptr() % align:
+                raise ValueError(f"the experts' products must be {list(shape)} and {align}-byte aligned")
+    if lora_b is not None and len(lora_b) != E:
+        raise ValueError("one lora_b per expert")
     add = _need(add, "add", dtype=torch.float32, ndim=2)
     weights = _need(weights, "weights", dtype=torch.float32, ndim=2)
     if add.shape != (E, H) or weights.shape != (T, E) or add.data_ptr() % 16:
@@ -492,8 +496,11 @@ def expert_combine(dense, lora, scaling, add, weights):
     outs = torch.empty(E, T, H, dtype=torch.float32, device=add.device)
     mix = torch.empty(T, H, dtype=torch.float32, device=add.device)
     if mix.numel():
-        N.call("pikv_expert_combine", _ptr_array(dense), _ptr_array(lora), (C.c_float * E)(*[float(v) for v in scaling]),
-               _ptr(add), _ptr(weights), T, E, H, _ptr(outs), _ptr(mix), _stream())
+        rest = ((C.c_float * E)(*[float(v) for v in scaling]), _ptr(add), _ptr(weights), T, E, H, _ptr(outs), _ptr(mix), _stream())
+        if lora_b is None:
+            N.call("pikv_expert_combine", _ptr_array(dense), _ptr_array(lora), *rest)
+        else:
+            N.call("pikv_expert_combine_factors", _ptr_array(dense), _ptr_array(lora), _ptr_array(lora_b), rank, *rest)
     return outs, mix
 
 

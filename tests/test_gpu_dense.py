@@ -78,6 +78,35 @@ def test_expert_combine(dev, E, T, H):
     assert torch.equal(want.nan_to_num(7.0), mix.nan_to_num(7.0))
 
 
+@pytest.mark.parametrize("E,T,H,rank", [(1, 1, 4, 1), (3, 37, 132, 4), (20, 5, 64, 8)])
+def test_expert_combine_factors(dev, E, T, H, rank):
+    """Bit for bit the form that is given the products, as torch.mm makes them."""
+    import torch
+    from pikv_amd import ops
+    torch.manual_seed(E)
+    scaling = [0.3 + 0.1 * e for e in range(E)]
+    d, t, b, c, w = (torch.randn(*s, device=dev) for s in ((E, T, H), (E, T, rank), (E, rank, H), (E, H), (T, E)))
+    d[0, 0, 0], t[E - 1, T - 1, 0] = float("nan"), float("inf")
+    want = ops.expert_combine(list(d), [torch.mm(x, y) for x, y in zip(t, b)], scaling, c, w)
+    got = ops.expert_combine(list(d), list(t), scaling, c, w, lora_b=list(b))
+    for g, x in zip(got, want):
+        assert torch.equal(g.nan_to_num(7.0), x.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("T,H", [(33, 128), (17, 256), (256, 256), (257, 256), (1025, 256), (40, 512), (1000, 512), (700, 1024)])
+def test_tiled_experts_sum_in_the_librarys_order(dev, T, H):
+    import torch
+    from pikv_amd import dense, ops
+    torch.manual_seed(T)
+    x, w, b = torch.randn(T, H, device=dev), torch.randn(H, H, device=dev) * 0.05, torch.randn(H, device=dev)
+    if dense.experts_tiled(T, H, 4):
+        o = torch.empty(T, H, device=dev)
+        ops.linear_tiled(x, [(w, b, o)])
+        assert torch.equal(o, torch.nn.functional.linear(x, w, b))
+    else:
+        assert (T, H) in ((17, 256), (257, 256))
+
+
 @pytest.mark.parametrize("scheme,D,group", [(O.Q_I8_SYM, 272, 16), (O.Q_I8_ASYM, 256, 256), (O.Q_I4_ASYM, 1088, 32),
                                             (O.Q_I4_SYM, 64, 64)])
 @pytest.mark.parametrize("lens", [[0, 1, 63], [65, 64, 130], [5000, 4097, 2]])
