@@ -1,4 +1,5 @@
-"""ctypes binding of libpikv_hip.so (the C ABI declared in include/pikv_hip.h).
+"""Binding of libpikv_hip.so (the C ABI declared in include/pikv_hip.h): ctypes signatures, and call() through the typed entry
+points of csrc/call.cpp.
 
 The library is the only compute path of this package: if it is missing, or a
 call returns a non-zero status, an exception is raised.  There is no CPU or
@@ -123,8 +124,35 @@ def check(code: int, what: str) -> None:
         raise PiKVNativeError(f"{what} failed: {status_string(code)} (status {code})")
 
 
+try:
+    from . import _call
+except ImportError:                      # not built: whoever needs it is told
+    _call = None
+_entries = None
+
+
+def entries():
+    """The module of typed entry points (csrc/call.cpp), bound to the library that lib() loads.  Every call of this package
+    goes through it; lib() remains for a ctypes caller."""
+    global _entries
+    if _entries is None:
+        lib()
+        with _lock:
+            if _entries is None:
+                if _call is None:
+                    raise PiKVNativeError("pikv_amd/_call is not built: build it with `python -m pikv_amd.build`")
+                _call.load(LIB_PATH)
+                _entries = _call
+    return _entries
+
+
 def call(name: str, *args) -> None:
-    """Call an int-status entry point and raise on a non-zero status."""
-    code = getattr(_lib or lib(), name)(*args)
+    """Call an int-status entry point and raise on a non-zero status.  Pointers: tensors, addresses, None; lists for host arrays."""
+    code = getattr(_entries or entries(), name)(*args)
     if code:
         check(code, name)
+
+
+def size(name: str, *args) -> int:
+    """Call an entry point that returns a number of bytes."""
+    return getattr(_entries or entries(), name)(*args)

@@ -1,0 +1,273 @@
+// Python entry to libpikv_hip.so: one function per entry point of include/pikv_hip.h, typed by its declaration.
+//
+// A call of one launch spends about 2.5 us in the launch; through ctypes the conversion of its 12 to 25 arguments, a Python call
+// per tensor for its address among them, took 5 us more, which is what bounded the small calls (a decode step of 1 x 700
+// tokens: three calls, 31 addresses).  Arguments here: tensors (anything with data_ptr()), addresses as int, None, numbers;
+// a list for a parameter that is a host array, of tensors or numbers; an object with a buffer for any pointer.
+// Beside them the two checks that run for every tensor of a call (56 and 47 times in an evaluation pass of the
+// mixture-of-experts model).  The symbols come from the library that load() is given; the GIL is released around each call.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <dlfcn.h>
+
+#include <cstdint>
+#include <cstring>
+#include <tuple>
+#include <type_traits>
+#include <utility>
+
+#include "../../include/pikv_hip.h"
+
+namespace {
+
+PyObject *g_data_ptr, *g_is_cuda, *g_is_contiguous, *g_dtype, *g_device, *g_dim;
+PyObject *g_tensor, *g_parameter;        // torch.Tensor, torch.nn.Parameter
+PyObject *g_refuse, *g_has_storage;      // ops._refuse, torch._C._has_storage
+
+// Host arrays of one call.
+struct Arena {
+  alignas(16) unsigned char bytes[4096];
+  size_t used = 0;
+  void* take(size_t n) {
+    const size_t at = (used + 15) / 16 * 16;
+    if (n > sizeof(bytes) - at) {
+      PyErr_SetString(PyExc_ValueError, "argument lists are too long");
+      return nullptr;
+    }
+    used = at + n;
+    return bytes + at;
+  }
+};
+
+bool address(PyObject* o, void*& p) {
+  if (o == Py_None) {
+    p = nullptr;
+    return true;
+  }
+  if (PyLong_Check(o)) {
+    p = PyLong_AsVoidPtr(o);
+    return !PyErr_Occurred();
+  }
+  if (PyObject_CheckBuffer(o)) {
+    Py_buffer b;
+    if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) return false;
+    p = b.buf;                           // the caller's reference keeps the object over the call
+    PyBuffer_Release(&b);
+    return true;
+  }
+  PyObject* a = PyObject_CallMethodNoArgs(o, g_data_ptr);
+  if (!a) return false;
+  p = PyLong_AsVoidPtr(a);
+  Py_DECREF(a);
+  return !PyErr_Occurred();
+}
+
+template <typename T>
+bool number(PyObject* o, T& v) {
+  if constexpr (std::is_floating_point_v<T>) {
+    const double d = PyFloat_AsDouble(o);
+    if (d == -1.0 && PyErr_Occurred()) return false;
+    v = (T)d;
+  } else {
+    PyObject* i = PyNumber_Index(o);
+    if (!i) return false;
+    const long long n = PyLong_AsLongLong(i);
+    Py_DECREF(i);
+    if (n == -1 && PyErr_Occurred()) return false;
+    v = (T)n;
+    if ((long long)v != n) {
+      PyErr_SetString(PyExc_OverflowError, "an integer argument does not fit its parameter");
+      return false;
+    }
+  }
+  return true;
+}
+
+template <typename T>
+bool convert(PyObject* o, T& v, Arena& arena) {
+  if constexpr (std::is_pointer_v<T>) {
+    using E = std::remove_cv_t<std::remove_pointer_t<T>>;
+    if constexpr (!std::is_void_v<E>) {
+      if (PyList_Check(o) || PyTuple_Check(o)) {
+        const Py_ssize_t n = PySequence_Fast_GET_SIZE(o);
+        E* a = static_cast<E*>(arena.take((size_t)n * sizeof(E)));
+        if (!a) return false;
+        for (Py_ssize_t i = 0; i < n; ++i) {
+          PyObject* e = PySequence_Fast_GET_ITEM(o, i);
+          if constexpr (std::is_pointer_v<E>) {
+            void* p = nullptr;
+            if (!address(e, p)) return false;
+            a[i] = static_cast<E>(p);
+          } else if (!number(e, a[i])) {
+            return false;
+          }
+        }
+        v = a;
+        return true;
+      }
+    }
+    void* p = nullptr;
+    if (!address(o, p)) return false;
+    v = static_cast<T>(p);
+    return true;
+  } else {
+    return number(o, v);
+  }
+}
+
+template <typename R, typename... A, size_t... I>
+PyObject* invoke(R (*f)(A...), const char* name, PyObject* const* args, Py_ssize_t n, std::index_sequence<I...>) {
+  if (!f) return PyErr_Format(PyExc_RuntimeError, "%s: no library loaded", name);
+  if (n != (Py_ssize_t)sizeof...(A)) return PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %zd", name, (int)sizeof...(A), n);
+  Arena arena;
+  std::tuple<std::decay_t<A>...> v{};
+  if (!(convert(args[I], std::get<I>(v), arena) && ...)) return nullptr;
+  R r;
+  Py_BEGIN_ALLOW_THREADS
+  r = f(std::get<I>(v)...);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLongLong((long long)r);
+}
+template <typename R, typename... A>
+PyObject* invoke(R (*f)(A...), const char* name, PyObject* const* args, Py_ssize_t n) {
+  return invoke(f, name, args, n, std::index_sequence_for<A...>());
+}
+
+struct Entry {
+  const char* name;
+  void** slot;
+};
+
+#define PIKV_ENTRIES(X)                                                                                                       \
+  X(pikv_abi_version) X(pikv_router_fused) X(pikv_router_tail) X(pikv_capacity_slots) X(pikv_capacity_slots_static)           \
+  X(pikv_capacity_slots_static_max) X(pikv_router_workspace_bytes) X(pikv_router_fused_workspace_bytes) X(pikv_quant_scatter) \
+  X(pikv_cache_advance) X(pikv_quant_gather) X(pikv_quant_append) X(pikv_quantize_rows) X(pikv_quant8_minshift)               \
+  X(pikv_gather_dequant) X(pikv_gather_dequant_scores) X(pikv_h2o_accumulate) X(pikv_attend_values)                           \
+  X(pikv_attend_workspace_bytes) X(pikv_decode_attend) X(pikv_decode_attend_workspace_bytes) X(pikv_prefill_attend)           \
+  X(pikv_prefill_attend_workspace_bytes) X(pikv_evict_select) X(pikv_evict_select_h2o) X(pikv_evict_workspace_bytes)          \
+  X(pikv_h2o_budget) X(pikv_cache_make_room) X(pikv_compact_rows) X(pikv_linear_group) X(pikv_linear_group_workspace_bytes)   \
+  X(pikv_linear_tiled) X(pikv_cache_mean) X(pikv_cache_mean_workspace_bytes) X(pikv_value_lora) X(pikv_expert_combine)        \
+  X(pikv_expert_combine_factors) X(pikv_adaptive_router) X(pikv_quant_scatter_routed) X(pikv_fakequant_colblocks)             \
+  X(pikv_fakequant_workspace_bytes) X(pikv_fakequant_preset)
+
+#define PIKV_DEFINE(name)                                                                     \
+  decltype(&::name) f_##name = nullptr;                                                       \
+  PyObject* c_##name(PyObject*, PyObject* const* args, Py_ssize_t n) { return invoke(f_##name, #name, args, n); }
+PIKV_ENTRIES(PIKV_DEFINE)
+
+#define PIKV_SLOT(name) {#name, reinterpret_cast<void**>(&f_##name)},
+const Entry g_entries[] = {PIKV_ENTRIES(PIKV_SLOT)};
+
+PyObject* load(PyObject*, PyObject* path) {
+  const char* p = PyUnicode_AsUTF8(path);
+  if (!p) return nullptr;
+  void* lib = dlopen(p, RTLD_NOW | RTLD_LOCAL);
+  if (!lib) return PyErr_Format(PyExc_OSError, "%s", dlerror());
+  for (const Entry& e : g_entries) {
+    void* s = dlsym(lib, e.name);
+    if (!s) return PyErr_Format(PyExc_OSError, "%s: no symbol %s", p, e.name);
+    *e.slot = s;
+  }
+  Py_RETURN_NONE;
+}
+
+// -1: an exception is set
+int is_true(PyObject* o) {
+  if (!o) return -1;
+  const int r = PyObject_IsTrue(o);
+  Py_DECREF(o);
+  return r;
+}
+int is_same(PyObject* o, PyObject* want) {
+  if (!o) return -1;
+  Py_DECREF(o);
+  return o == want;
+}
+
+PyObject* setup(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 4) return PyErr_Format(PyExc_TypeError, "setup takes 4 arguments");
+  PyObject** const to[] = {&g_tensor, &g_parameter, &g_refuse, &g_has_storage};
+  for (int i = 0; i < 4; ++i) {
+    Py_INCREF(args[i]);
+    Py_XSETREF(*to[i], args[i]);
+  }
+  Py_RETURN_NONE;
+}
+
+// need(t, name, *, dtype=None, ndim=None, optional=False): t, if it is a contiguous GPU tensor of that dtype and number of
+// dimensions (or None and optional); what it is not, g_refuse(t, name, dtype, ndim) says in an exception.
+PyObject* need(PyObject*, PyObject* const* args, Py_ssize_t n, PyObject* kw) {
+  if (n != 2 || !g_tensor) return PyErr_Format(PyExc_TypeError, "need(t, name, *, dtype, ndim, optional)");
+  PyObject *t = args[0], *dtype = Py_None, *ndim = Py_None;
+  bool optional = false;
+  for (Py_ssize_t i = 0; kw && i < PyTuple_GET_SIZE(kw); ++i) {
+    const char* k = PyUnicode_AsUTF8(PyTuple_GET_ITEM(kw, i));
+    if (!k) return nullptr;
+    PyObject* v = args[n + i];
+    if (std::strcmp(k, "dtype") == 0) dtype = v;
+    else if (std::strcmp(k, "ndim") == 0) ndim = v;
+    else if (std::strcmp(k, "optional") == 0) { const int o = PyObject_IsTrue(v); if (o < 0) return nullptr; optional = o; }
+    else return PyErr_Format(PyExc_TypeError, "need: no argument %s", k);
+  }
+  int ok;
+  if (t == Py_None) ok = optional;
+  else ok = PyType_IsSubtype(Py_TYPE(t), reinterpret_cast<PyTypeObject*>(g_tensor));
+  if (ok > 0 && t != Py_None) {
+    ok = is_true(PyObject_GetAttr(t, g_is_cuda));
+    if (ok > 0) ok = is_true(PyObject_CallMethodNoArgs(t, g_is_contiguous));
+    if (ok > 0 && dtype != Py_None) ok = is_same(PyObject_GetAttr(t, g_dtype), dtype);
+    if (ok > 0 && ndim != Py_None) {
+      PyObject* d = PyObject_CallMethodNoArgs(t, g_dim);
+      ok = d ? PyObject_RichCompareBool(d, ndim, Py_EQ) : -1;
+      Py_XDECREF(d);
+    }
+  }
+  if (ok < 0) return nullptr;
+  if (ok) return Py_NewRef(t);
+  PyObject* said = PyObject_CallFunctionObjArgs(g_refuse, t, args[1], dtype, ndim, nullptr);
+  if (!said) return nullptr;
+  Py_DECREF(said);
+  return PyErr_Format(PyExc_ValueError, "%U is not what the operator needs", args[1]);
+}
+
+// ordinary(t, device, dtype, align): whether t is a dense tensor (no subclass but Parameter) of that device and dtype that a kernel
+// may read by its address, `align` bytes at a time.
+PyObject* ordinary(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (n != 4 || !g_tensor) return PyErr_Format(PyExc_TypeError, "ordinary(t, device, dtype, align)");
+  PyObject* t = args[0];
+  PyObject* const type = reinterpret_cast<PyObject*>(Py_TYPE(t));
+  if (type != g_tensor && type != g_parameter) Py_RETURN_FALSE;
+  PyObject* d = PyObject_GetAttr(t, g_device);
+  int ok = d ? PyObject_RichCompareBool(d, args[1], Py_EQ) : -1;
+  Py_XDECREF(d);
+  if (ok > 0) ok = is_same(PyObject_GetAttr(t, g_dtype), args[2]);
+  if (ok > 0) ok = is_true(PyObject_CallMethodNoArgs(t, g_is_contiguous));
+  if (ok > 0) ok = is_true(PyObject_CallOneArg(g_has_storage, t));     // a batched tensor has none
+  if (ok > 0) {
+    void* p = nullptr;
+    const long long align = PyLong_AsLongLong(args[3]);
+    ok = align < 1 || !address(t, p) ? -1 : reinterpret_cast<uintptr_t>(p) % (uintptr_t)align == 0;
+    if (ok < 0 && !PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "align");
+  }
+  if (ok < 0) return nullptr;
+  return PyBool_FromLong(ok);
+}
+
+#define PIKV_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(c_##name)), METH_FASTCALL, nullptr},
+PyMethodDef g_methods[] = {PIKV_ENTRIES(PIKV_METHOD){"load", load, METH_O, nullptr},
+                          {"setup", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(setup)), METH_FASTCALL, nullptr},
+                          {"need", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(need)), METH_FASTCALL | METH_KEYWORDS, nullptr},
+                          {"ordinary", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(ordinary)), METH_FASTCALL, nullptr},
+                          {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_call", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__call() {
+  PyObject** const names[] = {&g_data_ptr, &g_is_cuda, &g_is_contiguous, &g_dtype, &g_device, &g_dim};
+  const char* const text[] = {"data_ptr", "is_cuda", "is_contiguous", "dtype", "device", "dim"};
+  for (int i = 0; i < 6; ++i)
+    if (!(*names[i] = PyUnicode_InternFromString(text[i]))) return nullptr;
+  return PyModule_Create(&g_module);
+}

@@ -13,6 +13,8 @@ import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
 
+from . import _native
+
 try:
     from torch.utils._device import DeviceContext as _DeviceContext
 except ImportError:
@@ -120,9 +122,8 @@ def ordinary_call() -> bool:
 
 
 def ordinary_tensor(t, device, dtype=torch.float32, align: int = 16) -> bool:
-    """A dense tensor a kernel may read by its address, `align` bytes at a time."""
-    return (type(t) in (torch.Tensor, nn.Parameter) and t.device == device and t.dtype == dtype and t.is_contiguous()
-            and _has_storage(t) and t.data_ptr() % align == 0)      # a batched tensor has no storage
+    """A dense tensor a kernel may read by its address, `align` bytes at a time (csrc/call.cpp)."""
+    return _native._call.ordinary(t, device, dtype, align)
 
 
 def forward_only(x) -> bool:
@@ -132,8 +133,11 @@ def forward_only(x) -> bool:
 
 def linear_ok(m, n_in: int, n_out: int, device) -> bool:
     """A plain nn.Linear of this shape with a bias, as linear_group reads it."""
-    return (plain(m, nn.Linear) and m.bias is not None and m.weight.shape == (n_out, n_in)
-            and ordinary_tensor(m.weight, device) and ordinary_tensor(m.bias, device))
+    if not plain(m, nn.Linear):
+        return False
+    w, b = m._parameters.get("weight"), m._parameters.get("bias")    # (m.weight looks through three tables for it)
+    return (w is not None and b is not None and w.shape == (n_out, n_in) and ordinary_tensor(w, device)
+            and ordinary_tensor(b, device))
 
 
 def mlp_ok(seq, acts, sizes, device) -> bool:

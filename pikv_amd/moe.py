@@ -224,10 +224,13 @@ class PiKVMoE(nn.Module):
         return torch.stack(means) / pool.fill.clamp_min(1).unsqueeze(1).float()
 
     def _lora_ok(self, m, rank, device):
+        if not dense.plain(m, LoRALayer):
+            return False
         H = config['hidden_size']
-        return (dense.plain(m, LoRALayer) and type(m.scaling) in (int, float) and m.lora_A.shape == (H, rank) and m.lora_B.shape == (rank, H)
-                and dense.ordinary_tensor(m.lora_A, device) and dense.ordinary_tensor(m.lora_B, device)
-                and dense.plain(m.dropout, nn.Dropout) and not (m.dropout.training and m.dropout.p > 0))
+        a, b, drop = m._parameters.get("lora_A"), m._parameters.get("lora_B"), m._modules.get("dropout")
+        return (a is not None and b is not None and type(m.scaling) in (int, float) and a.shape == (H, rank) and b.shape == (rank, H)
+                and dense.ordinary_tensor(a, device) and dense.ordinary_tensor(b, device)
+                and dense.plain(drop, nn.Dropout) and not (drop.training and drop.p > 0))
 
     def _native_experts(self, x, routing_weights) -> bool:
         """Whether the key projection (while it pays), the value terms and everything behind the experts' products run natively
@@ -264,15 +267,16 @@ class PiKVMoE(nn.Module):
                              rank=self.key_lora.lora_A.shape[1])
         else:
             keys = self.key_proj(x2) + self.key_lora(x2)
-        scaling = [e.lora.scaling for e in self.experts]
+        layers = [(e.dense, e.lora) for e in self.experts]
         weights = routing_weights.view(T, E)
         if dense.experts_tiled(T, H, E):
             products = torch.empty(E, T, H, dtype=torch.float32, device=x.device).unbind()
-            ops.linear_tiled(x2, [(e.dense.weight, e.dense.bias, o) for e, o in zip(self.experts, products)])
+            ops.linear_tiled(x2, [(m.weight, m.bias, o) for (m, _), o in zip(layers, products)])
         else:
-            products = [F.linear(x2, e.dense.weight, e.dense.bias) for e in self.experts]
-        inner = [torch.mm(x2, e.lora.lora_A) for e in self.experts]
-        outs, mix = ops.expert_combine(products, inner, scaling, add, weights, lora_b=[e.lora.lora_B for e in self.experts])
+            products = [F.linear(x2, m.weight, m.bias) for m, _ in layers]
+        inner = [torch.mm(x2, m.lora_A) for _, m in layers]
+        outs, mix = ops.expert_combine(products, inner, [m.scaling for _, m in layers], add, weights,
+                                       lora_b=[m.lora_B for _, m in layers])
         return outs, keys, mix
 
     def update_cache(self, expert_idx, key, value, importance):

@@ -15,7 +15,6 @@ compact (core/single/cache_scheduling.py:391-436), H2O bookkeeping (:69-99).
 """
 from __future__ import annotations
 
-import ctypes as C
 import math
 from typing import Optional, Sequence
 
@@ -35,10 +34,6 @@ __all__ = [
 # --------------------------------------------------------------------------
 # helpers
 # --------------------------------------------------------------------------
-
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
-
 
 # the raw handle of torch.cuda.current_stream(), without building the stream object (every caller holds a GPU
 # tensor, so the runtime is up); by the public way in a version of torch that names the two calls otherwise
@@ -60,10 +55,9 @@ def _dt(t: torch.Tensor, name: str) -> int:
     raise ValueError(f"{name}: dtype must be float32 or bfloat16, got {t.dtype}")
 
 
-def _need(t, name, *, dtype=None, ndim=None, optional=False):
+def _refuse(t, name, dtype, ndim):
+    """Says what `t` is not (for _need)."""
     if t is None:
-        if optional:
-            return None
         raise ValueError(f"{name} is required")
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch.Tensor")
@@ -73,9 +67,18 @@ def _need(t, name, *, dtype=None, ndim=None, optional=False):
         raise ValueError(f"{name} must be contiguous")
     if dtype is not None and t.dtype != dtype:
         raise ValueError(f"{name}: dtype must be {dtype}, got {t.dtype}")
-    if ndim is not None and t.dim() != ndim:
-        raise ValueError(f"{name}: expected {ndim} dimensions, got {tuple(t.shape)}")
-    return t
+    raise ValueError(f"{name}: expected {ndim} dimensions, got {tuple(t.shape)}")
+
+
+def _need(*a, **k):
+    """_need(t, name, *, dtype=None, ndim=None, optional=False): t, if it is a contiguous GPU tensor of that dtype and
+    number of dimensions (or None where that may be); in csrc/call.cpp."""
+    raise N.PiKVNativeError("pikv_amd/_call is not built: build it with `python -m pikv_amd.build`")
+
+
+if N._call is not None:
+    N._call.setup(torch.Tensor, torch.nn.Parameter, _refuse, torch._C._has_storage if hasattr(torch._C, "_has_storage") else bool)
+    _need = N._call.need
 
 
 def _vecf(t, name, n, device):
@@ -153,7 +156,7 @@ def _router_common(T, E, k, capacity, device, want_probs=True, want_logits=False
             raise ValueError("capacity must be >= 0")
         slot = torch.empty(T, k, dtype=torch.int32, device=device)
         count = torch.empty(E, dtype=torch.int32, device=device)
-        ws_bytes = int(N.lib().pikv_router_workspace_bytes(T, E, k))
+        ws_bytes = N.size("pikv_router_workspace_bytes", T, E, k)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=device)
     return probs, logits, idx, w, slot, count, ws, ws_bytes
 
@@ -190,17 +193,17 @@ def router_fused(x, weight, bias=None, *, top_k=2, capacity=None, expert_scale=N
     expert_mask = _vecf(expert_mask, "expert_mask", E, dev)
     probs, logits, idx, w, slot, count, ws, ws_bytes = _router_common(
         T, E, top_k, capacity, dev, True, return_logits)
-    ws_bytes = int(N.lib().pikv_router_fused_workspace_bytes(T, H, E, top_k))
+    ws_bytes = N.size("pikv_router_fused_workspace_bytes", T, H, E, top_k)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
     if T == 0:  # nothing to route (empty tensors have no device address)
         if count is not None:
             count.zero_()
         return RouterOut(probs, idx, w, slot, count, logits, capacity)
-    N.call("pikv_router_fused", _ptr(x), _ptr(weight), dt, _ptr(bias), _ptr(expert_scale),
-           _ptr(expert_mask), float(temperature), float(renorm_eps), _arith(module_arithmetic),
+    N.call("pikv_router_fused", x, weight, dt, bias, expert_scale,
+           expert_mask, float(temperature), float(renorm_eps), _arith(module_arithmetic),
            T, H, E, top_k,
-           int(capacity or 0), _ptr(probs), _ptr(logits), _ptr(idx), _ptr(w), _ptr(slot),
-           _ptr(count), _ptr(ws), ws_bytes, _stream())
+           int(capacity or 0), probs, logits, idx, w, slot,
+           count, ws, ws_bytes, _stream())
     return RouterOut(probs, idx, w, slot, count, logits, capacity)
 
 
@@ -228,10 +231,10 @@ def router_tail(logits, *, top_k=2, capacity=None, logits_b=None, select=None,
         if count is not None:
             count.zero_()
         return RouterOut(probs, idx, w, slot, count, None, capacity)
-    N.call("pikv_router_tail", _ptr(logits), _ptr(logits_b), _ptr(select), _ptr(expert_scale),
-           _ptr(expert_mask), float(temperature), float(renorm_eps), int(bool(use_softmax)),
-           _arith(module_arithmetic), T, E, top_k, int(capacity or 0), _ptr(probs), _ptr(idx), _ptr(w), _ptr(slot),
-           _ptr(count), _ptr(ws), ws_bytes, _stream())
+    N.call("pikv_router_tail", logits, logits_b, select, expert_scale,
+           expert_mask, float(temperature), float(renorm_eps), int(bool(use_softmax)),
+           _arith(module_arithmetic), T, E, top_k, int(capacity or 0), probs, idx, w, slot,
+           count, ws, ws_bytes, _stream())
     return RouterOut(probs, idx, w, slot, count, None, capacity)
 
 
@@ -246,12 +249,12 @@ def capacity_slots(expert_idx, num_experts: int, capacity: int):
     dev = expert_idx.device
     slot = torch.empty_like(expert_idx)
     count = torch.empty(num_experts, dtype=torch.int32, device=dev)
-    ws_bytes = int(N.lib().pikv_router_workspace_bytes(A, num_experts, 1))
+    ws_bytes = N.size("pikv_router_workspace_bytes", A, num_experts, 1)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
     if A == 0:
         return slot, count.zero_()
-    N.call("pikv_capacity_slots", _ptr(expert_idx), A, num_experts, int(capacity), _ptr(slot),
-           _ptr(count), _ptr(ws), ws_bytes, _stream())
+    N.call("pikv_capacity_slots", expert_idx, A, num_experts, int(capacity), slot,
+           count, ws, ws_bytes, _stream())
     return slot, count
 
 
@@ -272,8 +275,8 @@ def quantize_rows(x, group: int, scheme: int):
     zero = torch.empty_like(scale) if _scheme_asym(scheme) else None
     if n == 0:
         return codes, scale, zero
-    N.call("pikv_quantize_rows", _ptr(x), dt, n, D, group, scheme, 0, _ptr(codes), _ptr(scale),
-           _ptr(zero), _stream())
+    N.call("pikv_quantize_rows", x, dt, n, D, group, scheme, 0, codes, scale,
+           zero, _stream())
     return codes, scale, zero
 
 
@@ -292,7 +295,7 @@ def quant8_minshift(x, want_dq: bool = True):
     scale = torch.empty(n, 1, dtype=torch.float32, device=dev)
     mn = torch.empty(n, 1, dtype=torch.float32, device=dev)
     if n:
-        N.call("pikv_quant8_minshift", _ptr(x), dt, n, D, _ptr(codes), _ptr(dq), _ptr(scale), _ptr(mn), _stream())
+        N.call("pikv_quant8_minshift", x, dt, n, D, codes, dq, scale, mn, _stream())
     return dq, codes, scale, mn
 
 
@@ -321,8 +324,8 @@ def dequantize_rows(codes, scale, zero, group: int, scheme: int, out_dtype=torch
     out = torch.empty(cnt, D, dtype=out_dtype, device=codes.device)
     if cnt == 0:
         return out
-    N.call("pikv_gather_dequant", _ptr(codes), _ptr(scale), _ptr(zero), D, group, scheme,
-           _ptr(rows), row0, cnt, _ptr(out), F32 if out_dtype == torch.float32 else BF16,
+    N.call("pikv_gather_dequant", codes, scale, zero, D, group, scheme,
+           rows, row0, cnt, out, F32 if out_dtype == torch.float32 else BF16,
            _stream())
     return out
 
@@ -339,10 +342,10 @@ def fakequant_colblocks(x, group: int, bits: int = 8, symmetric: bool = False):
     out = torch.empty_like(x)
     stats = torch.zeros(nblk, 4, dtype=torch.float32, device=dev)
     mse = torch.zeros(nblk, dtype=torch.float32, device=dev)
-    ws_bytes = int(N.lib().pikv_fakequant_workspace_bytes(Nr, H, group))
+    ws_bytes = N.size("pikv_fakequant_workspace_bytes", Nr, H, group)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    N.call("pikv_fakequant_colblocks", _ptr(x), Nr, H, group, bits, int(bool(symmetric)),
-           _ptr(out), _ptr(stats), _ptr(mse), _ptr(ws), ws_bytes, _stream())
+    N.call("pikv_fakequant_colblocks", x, Nr, H, group, bits, int(bool(symmetric)),
+           out, stats, mse, ws, ws_bytes, _stream())
     return out, stats, mse
 
 
@@ -361,10 +364,10 @@ def fakequant_preset(x, preset, group: int, bits: int = 8, symmetric: bool = Fal
     dev = x.device
     out = torch.empty_like(x)
     mse = torch.zeros(nblk, dtype=torch.float32, device=dev)
-    ws_bytes = int(N.lib().pikv_fakequant_workspace_bytes(Nr, H, group))
+    ws_bytes = N.size("pikv_fakequant_workspace_bytes", Nr, H, group)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    N.call("pikv_fakequant_preset", _ptr(x), Nr, H, group, bits, int(bool(symmetric)),
-           _ptr(preset), _ptr(out), _ptr(mse), _ptr(ws), ws_bytes, _stream())
+    N.call("pikv_fakequant_preset", x, Nr, H, group, bits, int(bool(symmetric)),
+           preset, out, mse, ws, ws_bytes, _stream())
     return out, mse
 
 
@@ -373,7 +376,7 @@ def fakequant_preset(x, preset, group: int, bits: int = 8, symmetric: bool = Fal
 # --------------------------------------------------------------------------
 
 def _evict_workspace(n_caches: int, max_len: int, device):
-    nbytes = int(N.lib().pikv_evict_workspace_bytes(n_caches, max_len))
+    nbytes = N.size("pikv_evict_workspace_bytes", n_caches, max_len)
     return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device), nbytes
 
 
@@ -400,14 +403,10 @@ def select_top_rows(score, seg_base, seg_len, n_keep, max_len: Optional[int] = N
         max_len = score.numel()
     ws, ws_bytes = _evict_workspace(n, int(max_len), dev)
     # H2O selection with an empty "recent" budget; the score doubles as the (unused) timestamp
-    N.call("pikv_evict_select", EVICT_H2O, _ptr(score), _ptr(score), _ptr(seg_base), _ptr(seg_len),
-           _ptr(n_keep), _ptr(zero), n, int(max_len), _ptr(flag), _ptr(index), _ptr(kept), _ptr(ws),
+    N.call("pikv_evict_select", EVICT_H2O, score, score, seg_base, seg_len,
+           n_keep, zero, n, int(max_len), flag, index, kept, ws,
            ws_bytes, _stream())
     return flag, index, kept
-
-
-def _ptr_array(ts):
-    return (C.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
 
 
 def linear_group(x, layers, rank: int = 0):
@@ -430,14 +429,14 @@ def linear_group(x, layers, rank: int = 0):
     if T == 0:
         return
     n = len(layers)
-    nb = int(N.lib().pikv_linear_group_workspace_bytes(T, n, rank))
+    nb = N.size("pikv_linear_group_workspace_bytes", T, n, rank)
     ws = torch.empty(nb, dtype=torch.uint8, device=x.device) if nb else None
-    N.call("pikv_linear_group", _ptr(x), T, K, n, _ptr_array([l["weight"] for l in layers]),
-           _ptr_array([l["bias"] for l in layers]), (C.c_int32 * n)(*[l["weight"].shape[0] for l in layers]),
-           (C.c_int32 * n)(*[int(bool(l.get("relu"))) for l in layers]), rank,
-           _ptr_array([l.get("lora_a") for l in layers]), _ptr_array([l.get("lora_b") for l in layers]),
-           (C.c_float * n)(*[float(l.get("scaling", 0.0)) for l in layers]),
-           _ptr_array([l["out"] for l in layers]), _ptr(ws), nb, _stream())
+    N.call("pikv_linear_group", x, T, K, n, [l["weight"] for l in layers],
+           [l["bias"] for l in layers], [l["weight"].shape[0] for l in layers],
+           [int(bool(l.get("relu"))) for l in layers], rank,
+           [l.get("lora_a") for l in layers], [l.get("lora_b") for l in layers],
+           [float(l.get("scaling", 0.0)) for l in layers],
+           [l["out"] for l in layers], ws, nb, _stream())
 
 
 def linear_tiled(x, layers):
@@ -454,8 +453,8 @@ def linear_tiled(x, layers):
         return
     n = len(layers)
     w, b, o = zip(*layers)
-    N.call("pikv_linear_tiled", _ptr(x), T, K, n, _ptr_array(w), _ptr_array(b), (C.c_int32 * n)(*[t.shape[0] for t in w]),
-           _ptr_array(o), _stream())
+    N.call("pikv_linear_tiled", x, T, K, n, w, b, [t.shape[0] for t in w],
+           o, _stream())
 
 
 def value_lora(mean, lora_a, lora_b, scaling):
@@ -470,8 +469,8 @@ def value_lora(mean, lora_a, lora_b, scaling):
                 or _need(b, "lora_b", dtype=torch.float32).shape != (rank, H)):
             raise ValueError("lora_a must be [H, rank], lora_b [rank, H]")
     out = torch.empty_like(mean)
-    N.call("pikv_value_lora", _ptr(mean), E, H, rank, _ptr_array(lora_a), _ptr_array(lora_b),
-           (C.c_float * E)(*[float(v) for v in scaling]), _ptr(out), _stream())
+    N.call("pikv_value_lora", mean, E, H, rank, lora_a, lora_b,
+           [float(v) for v in scaling], out, _stream())
     return out
 
 
@@ -496,11 +495,11 @@ def expert_combine(dense, lora, scaling, add, weights, lora_b=None):
     outs = torch.empty(E, T, H, dtype=torch.float32, device=add.device)
     mix = torch.empty(T, H, dtype=torch.float32, device=add.device)
     if mix.numel():
-        rest = ((C.c_float * E)(*[float(v) for v in scaling]), _ptr(add), _ptr(weights), T, E, H, _ptr(outs), _ptr(mix), _stream())
+        rest = ([float(v) for v in scaling], add, weights, T, E, H, outs, mix, _stream())
         if lora_b is None:
-            N.call("pikv_expert_combine", _ptr_array(dense), _ptr_array(lora), *rest)
+            N.call("pikv_expert_combine", dense, lora, *rest)
         else:
-            N.call("pikv_expert_combine_factors", _ptr_array(dense), _ptr_array(lora), _ptr_array(lora_b), rank, *rest)
+            N.call("pikv_expert_combine_factors", dense, lora, lora_b, rank, *rest)
     return outs, mix
 
 
@@ -527,10 +526,10 @@ def adaptive_router(x_mean, selector, lb, imp, predictor, seq_len: int, top_k: i
     topk_w = torch.empty(T, top_k, dtype=torch.float32, device=dev)
     importance = torch.empty(T, dtype=torch.float32, device=dev)
     loss = torch.empty((), dtype=torch.float32, device=dev)
-    N.call("pikv_adaptive_router", _ptr(x_mean), B, seq_len, H, H2, E, top_k, *[_ptr(t) for t in selector],
-           *[_ptr(t) for t in lb], float(temp_lb), *[_ptr(t) for t in imp], float(temp_imp),
-           *[_ptr(t) for t in predictor], _ptr(mask), float(balance_weight), _ptr(blend), _ptr(probs[0]), _ptr(probs[1]),
-           _ptr(idx), _ptr(topk_w), _ptr(importance), _ptr(loss), _stream())
+    N.call("pikv_adaptive_router", x_mean, B, seq_len, H, H2, E, top_k, *selector,
+           *lb, float(temp_lb), *imp, float(temp_imp),
+           *predictor, mask, float(balance_weight), blend, probs[0], probs[1],
+           idx, topk_w, importance, loss, _stream())
     return probs[1], idx, topk_w, loss, importance
 
 
@@ -559,14 +558,14 @@ def prefill_attend(q, k, v, pool: Optional["CachePool"] = None, causal: bool = T
     if out.numel() == 0:
         return out
     max_cached = pool.max_cap if pool is not None and pool.rows > 0 else 0
-    planes = [None] * 6 if max_cached == 0 else [_ptr(p) for p in (*pool._planes("k"), *pool._planes("v"))]
-    nb = int(N.lib().pikv_prefill_attend_workspace_bytes(B, S, hkv, hq, dh, max_cached))
+    planes = [None] * 6 if max_cached == 0 else [*pool._planes("k"), *pool._planes("v")]
+    nb = N.size("pikv_prefill_attend_workspace_bytes", B, S, hkv, hq, dh, max_cached)
     ws = torch.empty(nb, dtype=torch.uint8, device=q.device) if nb else None
-    N.call("pikv_prefill_attend", _ptr(q), _ptr(k), _ptr(v), B, S, hkv, hq, dh, int(bool(causal)),
+    N.call("pikv_prefill_attend", q, k, v, B, S, hkv, hq, dh, int(bool(causal)),
            float(1.0 / math.sqrt(dh) if scale_qk is None else scale_qk), *planes,
            pool.scheme if max_cached else Q_I8_SYM, pool.group if max_cached else 0,
-           _ptr(pool.row_base) if max_cached else None, _ptr(pool.fill) if max_cached else None, max_cached,
-           _ptr(out), _ptr(ws), nb, _stream())
+           pool.row_base if max_cached else None, pool.fill if max_cached else None, max_cached,
+           out, ws, nb, _stream())
     return out
 
 
@@ -619,6 +618,7 @@ class CachePool:
         self.n_heavy = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
         self.n_recent = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
         self._budgets = torch.empty(3 * self.n_caches, dtype=torch.int32, device=dev)
+        self._row_bytes = [math.prod(p.shape[1:]) * p.element_size() for p in self.planes()]
 
     # ---- checkpoint ----
     _STATE_PLANES = ("k_codes", "k_scale", "k_zero", "v_codes", "v_scale", "v_zero", "acc", "ts")
@@ -701,11 +701,11 @@ class CachePool:
             raise ValueError(f"cache_id/slot must have n_src*fanout = {n_src * fanout} elements")
         if n_src == 0:
             return
-        N.call("pikv_quant_scatter", _ptr(k2), _ptr(v2), dt, n_src, fanout, self.D, self.group,
-               self.scheme, _ptr(cache_id), _ptr(slot), _ptr(self.row_base), _ptr(self.fill),
-               _ptr(self.cap), self.n_caches, _ptr(self.k_codes), _ptr(self.v_codes),
-               _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero), _ptr(self.v_zero),
-               _ptr(self.acc), _ptr(self.ts), float(now), _stream())
+        N.call("pikv_quant_scatter", k2, v2, dt, n_src, fanout, self.D, self.group,
+               self.scheme, cache_id, slot, self.row_base, self.fill,
+               self.cap, self.n_caches, self.k_codes, self.v_codes,
+               self.k_scale, self.v_scale, self.k_zero, self.v_zero,
+               self.acc, self.ts, float(now), _stream())
 
     def quant_scatter_routed(self, k_src, v_src, cache_id, slot, per_token: int, now: float = 0.0):
         """quant_scatter for rows that differ per cache: assignment j of token t (cache_id / slot
@@ -724,10 +724,10 @@ class CachePool:
             raise ValueError("cache_id and slot must have n * per_token elements")
         if n == 0:
             return
-        N.call("pikv_quant_scatter_routed", _ptr(k_src), _ptr(v_src), n, per_token, self.D, self.group, self.scheme,
-               _ptr(cache_id), _ptr(slot), _ptr(self.row_base), _ptr(self.fill), _ptr(self.cap), self.n_caches,
-               _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero),
-               _ptr(self.v_zero), _ptr(self.acc), _ptr(self.ts), float(now), _stream())
+        N.call("pikv_quant_scatter_routed", k_src, v_src, n, per_token, self.D, self.group, self.scheme,
+               cache_id, slot, self.row_base, self.fill, self.cap, self.n_caches,
+               self.k_codes, self.v_codes, self.k_scale, self.v_scale, self.k_zero,
+               self.v_zero, self.acc, self.ts, float(now), _stream())
 
     def quant_gather(self, k_src, v_src, src_row_base, src_index, n_take, max_take: int,
                      src_score=None, now: float = 0.0):
@@ -757,11 +757,11 @@ class CachePool:
                 raise ValueError("src_score must have one entry per source row")
         if max_take <= 0 or k2.shape[0] == 0:
             return
-        N.call("pikv_quant_gather", _ptr(k2), _ptr(v2), dt, self.D, self.group, self.scheme,
-               _ptr(src_row_base), _ptr(src_index), _ptr(n_take), int(max_take), _ptr(src_score),
-               _ptr(self.row_base), _ptr(self.fill), _ptr(self.cap), self.n_caches,
-               _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale),
-               _ptr(self.k_zero), _ptr(self.v_zero), _ptr(self.acc), _ptr(self.ts), float(now),
+        N.call("pikv_quant_gather", k2, v2, dt, self.D, self.group, self.scheme,
+               src_row_base, src_index, n_take, int(max_take), src_score,
+               self.row_base, self.fill, self.cap, self.n_caches,
+               self.k_codes, self.v_codes, self.k_scale, self.v_scale,
+               self.k_zero, self.v_zero, self.acc, self.ts, float(now),
                _stream())
 
     def advance(self, count, per_call_limit: int = -1):
@@ -769,7 +769,7 @@ class CachePool:
         count = _need(count, "count", dtype=torch.int32, ndim=1)
         if count.numel() != self.n_caches:
             raise ValueError("count must have one entry per cache")
-        N.call("pikv_cache_advance", _ptr(self.fill), _ptr(count), _ptr(self.cap), self.n_caches,
+        N.call("pikv_cache_advance", self.fill, count, self.cap, self.n_caches,
                int(per_call_limit), _stream())
 
     # ---- read path ----
@@ -791,10 +791,10 @@ class CachePool:
         out = torch.empty(self.n_caches, self.D, dtype=torch.float32, device=self.device)
         if self.rows == 0:
             return out.zero_()
-        nb = int(N.lib().pikv_cache_mean_workspace_bytes(self.n_caches, self.D, self.max_cap))
+        nb = N.size("pikv_cache_mean_workspace_bytes", self.n_caches, self.D, self.max_cap)
         ws = torch.empty(nb, dtype=torch.uint8, device=self.device)
-        N.call("pikv_cache_mean", _ptr(codes), _ptr(scale), _ptr(zero), self.scheme, self.group, self.D,
-               _ptr(self.row_base), _ptr(self.fill), self.n_caches, self.max_cap, _ptr(out), _ptr(ws), nb, _stream())
+        N.call("pikv_cache_mean", codes, scale, zero, self.scheme, self.group, self.D,
+               self.row_base, self.fill, self.n_caches, self.max_cap, out, ws, nb, _stream())
         return out
 
     def scores(self, q, n_q_heads: int, scale_qk: Optional[float] = None,
@@ -817,10 +817,10 @@ class CachePool:
         tsum = torch.empty_like(tmax)
         if scale_qk is None:
             scale_qk = 1.0 / (self.head_dim ** 0.5)
-        N.call("pikv_gather_dequant_scores", _ptr(self.k_codes), _ptr(self.k_scale),
-               _ptr(self.k_zero), self.scheme, self.group, self.n_heads, n_q_heads, self.head_dim,
-               _ptr(q), qdt, float(scale_qk), _ptr(self.row_base), _ptr(self.fill), self.n_caches,
-               max_len, stride, _ptr(scores), _ptr(tmax), _ptr(tsum), _stream())
+        N.call("pikv_gather_dequant_scores", self.k_codes, self.k_scale,
+               self.k_zero, self.scheme, self.group, self.n_heads, n_q_heads, self.head_dim,
+               q, qdt, float(scale_qk), self.row_base, self.fill, self.n_caches,
+               max_len, stride, scores, tmax, tsum, _stream())
         return scores, tmax, tsum
 
     def h2o_accumulate(self, scores, tile_max, tile_sum, now: float, decay: float = 1.0,
@@ -841,10 +841,10 @@ class CachePool:
         dev = self.device
         imp = torch.zeros(nc, stride, dtype=torch.float32, device=dev) if return_importance else None
         head_stats = torch.empty(nc, hq, 2, dtype=torch.float32, device=dev)
-        N.call("pikv_h2o_accumulate", _ptr(scores), _ptr(tile_max), _ptr(tile_sum), hq,
-               _ptr(self.row_base), _ptr(self.fill), nc, stride, stride, float(decay), float(now),
-               int(bool(write_probs)), None if stats_only else _ptr(self.acc),
-               None if stats_only else _ptr(self.ts), _ptr(imp), _ptr(head_stats), _stream())
+        N.call("pikv_h2o_accumulate", scores, tile_max, tile_sum, hq,
+               self.row_base, self.fill, nc, stride, stride, float(decay), float(now),
+               int(bool(write_probs)), None if stats_only else self.acc,
+               None if stats_only else self.ts, imp, head_stats, _stream())
         self.head_stats = head_stats   # (max, sum) per (cache, head): what attend_values normalises with
         return imp
 
@@ -870,13 +870,13 @@ class CachePool:
         out = torch.zeros(nc, hq, self.head_dim, dtype=torch.float32, device=dev)
         if stride == 0:
             return out
-        ws_bytes = int(N.lib().pikv_attend_workspace_bytes(nc, hq, self.head_dim, stride))
+        ws_bytes = N.size("pikv_attend_workspace_bytes", nc, hq, self.head_dim, stride)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-        N.call("pikv_attend_values", _ptr(scores), _ptr(head_stats), stride, _ptr(self.v_codes),
-               _ptr(self.v_scale), _ptr(self.v_zero), self.scheme, self.group, self.n_heads, hq,
-               self.head_dim, _ptr(self.row_base), _ptr(self.fill), nc, stride, float(decay), float(now),
-               _ptr(self.acc) if accumulate else None, _ptr(self.ts) if accumulate else None,
-               _ptr(out), _ptr(ws), ws_bytes, _stream())
+        N.call("pikv_attend_values", scores, head_stats, stride, self.v_codes,
+               self.v_scale, self.v_zero, self.scheme, self.group, self.n_heads, hq,
+               self.head_dim, self.row_base, self.fill, nc, stride, float(decay), float(now),
+               self.acc if accumulate else None, self.ts if accumulate else None,
+               out, ws, ws_bytes, _stream())
         return out
 
     def decode_attend(self, q, n_q_heads: int, now: float = 0.0, scale_qk: Optional[float] = None,
@@ -901,16 +901,16 @@ class CachePool:
         out = torch.empty(self.n_caches, n_q_heads, self.head_dim, dtype=torch.float32, device=dev)
         key = (n_q_heads, max_len)
         if getattr(self, "_decode_ws_key", None) != key:
-            nb = int(N.lib().pikv_decode_attend_workspace_bytes(self.n_caches, n_q_heads, self.head_dim, max_len))
+            nb = N.size("pikv_decode_attend_workspace_bytes", self.n_caches, n_q_heads, self.head_dim, max_len)
             self._decode_ws = torch.empty(max(nb, 256), dtype=torch.uint8, device=dev)
             self._decode_ws_key = key
         ws = self._decode_ws
-        N.call("pikv_decode_attend", _ptr(self.k_codes), _ptr(self.k_scale), _ptr(self.k_zero),
-               _ptr(self.v_codes), _ptr(self.v_scale), _ptr(self.v_zero), self.scheme, self.group,
-               self.n_heads, n_q_heads, self.head_dim, _ptr(q), dt, float(scale_qk), _ptr(self.row_base),
-               _ptr(self.fill), self.n_caches, max_len, float(decay), float(now),
-               _ptr(self.acc) if accumulate else None, _ptr(self.ts) if accumulate else None,
-               _ptr(out), _ptr(ws), ws.numel(), _stream())
+        N.call("pikv_decode_attend", self.k_codes, self.k_scale, self.k_zero,
+               self.v_codes, self.v_scale, self.v_zero, self.scheme, self.group,
+               self.n_heads, n_q_heads, self.head_dim, q, dt, float(scale_qk), self.row_base,
+               self.fill, self.n_caches, max_len, float(decay), float(now),
+               self.acc if accumulate else None, self.ts if accumulate else None,
+               out, ws, ws.numel(), _stream())
         return out
 
     # ---- eviction ----
@@ -938,8 +938,8 @@ class CachePool:
             if getattr(self, "_evict_ws", None) is None:
                 self._evict_ws = _evict_workspace(self.n_caches, self.max_cap, self.device)
             ws, ws_bytes = self._evict_ws
-        args = (_ptr(self.acc), _ptr(self.ts), _ptr(self.row_base), _ptr(self.fill), _ptr(nh), _ptr(nr), self.n_caches,
-                self.max_cap, _ptr(self.keep_flag), _ptr(self.keep_index), _ptr(self.new_len), _ptr(ws), ws_bytes, _stream())
+        args = (self.acc, self.ts, self.row_base, self.fill, nh, nr, self.n_caches,
+                self.max_cap, self.keep_flag, self.keep_index, self.new_len, ws, ws_bytes, _stream())
         if ratios:
             N.call("pikv_evict_select_h2o", float(heavy_ratio), float(recent_ratio), *args)
         else:
@@ -956,10 +956,9 @@ class CachePool:
         ps = self.planes() + [_need(p, "extra plane") for p in extra_planes]
         if len(ps) > N.MAX_PLANES:
             raise ValueError(f"at most {N.MAX_PLANES} planes")
-        ptrs = (C.c_void_p * len(ps))(*[p.data_ptr() for p in ps])
-        rbs = (C.c_int64 * len(ps))(*[math.prod(p.shape[1:]) * p.element_size() for p in ps])
-        N.call("pikv_compact_rows", ptrs, rbs, len(ps), _ptr(self.row_base), _ptr(self.keep_index),
-               _ptr(self.new_len), _ptr(self.fill), self.n_caches, _stream())
+        rbs = self._row_bytes + [math.prod(p.shape[1:]) * p.element_size() for p in extra_planes]
+        N.call("pikv_compact_rows", ps, rbs, len(ps), self.row_base, self.keep_index,
+               self.new_len, self.fill, self.n_caches, _stream())
 
     def make_room(self, policy: int, *, count: Optional[torch.Tensor] = None, count_all: int = 0,
                   limit: int = -1, heavy_ratio: float = 0.1, recent_ratio: float = 0.1,
@@ -975,15 +974,14 @@ class CachePool:
         if policy not in (EVICT_H2O, EVICT_LRU, EVICT_ALL):
             raise ValueError(f"unknown eviction policy {policy}")
         ps = self.planes()
-        ptrs = (C.c_void_p * len(ps))(*[p.data_ptr() for p in ps])
-        rbs = (C.c_int64 * len(ps))(*[math.prod(p.shape[1:]) * p.element_size() for p in ps])
+        rbs = self._row_bytes
         if getattr(self, "_evict_ws", None) is None:
             self._evict_ws = _evict_workspace(self.n_caches, self.max_cap, self.device)
         ws, ws_bytes = self._evict_ws
-        N.call("pikv_cache_make_room", policy, _ptr(count), int(count_all), int(limit), float(heavy_ratio),
-               float(recent_ratio), int(leave_room), int(append), _ptr(self.acc), _ptr(self.ts), _ptr(self.row_base),
-               _ptr(self.fill), _ptr(self.cap), self.n_caches, self.max_cap, ptrs, rbs, len(ps), _ptr(self.keep_flag),
-               _ptr(self.keep_index), _ptr(self.new_len), _ptr(self._budgets), _ptr(ws), ws_bytes, _stream())
+        N.call("pikv_cache_make_room", policy, count, int(count_all), int(limit), float(heavy_ratio),
+               float(recent_ratio), int(leave_room), int(append), self.acc, self.ts, self.row_base,
+               self.fill, self.cap, self.n_caches, self.max_cap, ps, rbs, len(ps), self.keep_flag,
+               self.keep_index, self.new_len, self._budgets, ws, ws_bytes, _stream())
 
     def append_rows(self, k_src, v_src, now: float = 0.0, advance: bool = False):
         """Quantise k_src / v_src [n_caches * rows, D] (cache-major) behind the new_len rows of every
@@ -1000,10 +998,10 @@ class CachePool:
                 raise ValueError("v_src must match k_src")
         if rows == 0:
             return
-        N.call("pikv_quant_append", _ptr(k_src), _ptr(v_src) if self.with_v else None, dt, rows, self.D, self.group,
-               self.scheme, _ptr(self.row_base), _ptr(self.new_len), _ptr(self.fill) if advance else None, _ptr(self.cap),
-               self.n_caches, _ptr(self.k_codes), _ptr(self.v_codes), _ptr(self.k_scale), _ptr(self.v_scale), _ptr(self.k_zero),
-               _ptr(self.v_zero), _ptr(self.acc), _ptr(self.ts), float(now), _stream())
+        N.call("pikv_quant_append", k_src, v_src if self.with_v else None, dt, rows, self.D, self.group,
+               self.scheme, self.row_base, self.new_len, self.fill if advance else None, self.cap,
+               self.n_caches, self.k_codes, self.v_codes, self.k_scale, self.v_scale, self.k_zero,
+               self.v_zero, self.acc, self.ts, float(now), _stream())
 
     def evict(self, policy: int, **kw):
         self.evict_select(policy, **kw)

@@ -1,0 +1,68 @@
+"""CPU checks of the typed Python entry (csrc/call.cpp): conversions, what it refuses, and the tensor checks beside it."""
+import numpy as np
+import pytest
+import torch
+
+from pikv_amd import _native as N, dense, ops
+
+
+def test_every_entry_point_is_there():
+    assert set(N.SIGNATURES) - {"pikv_status_string"} <= set(dir(N.entries()))
+
+
+def test_sizes_agree_with_ctypes():
+    for name, args in (("pikv_router_workspace_bytes", (32768, 8, 2)), ("pikv_evict_workspace_bytes", (3, 70000)),
+                       ("pikv_decode_attend_workspace_bytes", (4, 32, 128, 5000)), ("pikv_capacity_slots_static_max", ())):
+        assert N.size(name, *args) == getattr(N.lib(), name)(*args)
+
+
+@pytest.mark.parametrize("array", [[8, 16], (8, 16), np.array([8, 16], dtype=np.int32)])
+def test_host_arrays_reach_the_library(array):
+    """A bad layer width inside a host array is found by the library itself, whatever the array came as."""
+    def call(widths):
+        return N.entries().pikv_linear_group(64, 4, 128, 2, [64, 64], [64, 64], widths, [0, 1], 0, None, None, None, [64, 64],
+                                             None, 0, None)
+    assert call(array) == -3 and call([32, 0]) == -2     # widths that are no multiple of 32; no width at all
+
+
+def test_refusals():
+    f = N.entries()
+    with pytest.raises(TypeError):
+        f.pikv_evict_workspace_bytes(1)
+    with pytest.raises(OverflowError):
+        f.pikv_evict_workspace_bytes(1 << 40, 5)
+    with pytest.raises(TypeError):
+        f.pikv_evict_workspace_bytes(1.5, 5)
+    with pytest.raises(AttributeError):
+        f.pikv_h2o_budget(object(), 1, 0.1, 0.1, None, None, None)
+    with pytest.raises(ValueError):
+        f.pikv_linear_tiled(64, 4, 64, 1, [64] * 5000, [64], [4], [64], None)
+    with pytest.raises(N.PiKVNativeError):
+        N.call("pikv_h2o_budget", None, 1, 0.1, 0.1, None, None, None)
+
+
+def test_need():
+    t = torch.zeros(3, 4)
+    assert ops._need(None, "x", optional=True) is None
+    for args, kw, text in (((None, "x"), {}, "x is required"), ((5, "x"), {}, "must be a torch.Tensor"),
+                           ((t, "x"), {"ndim": 2}, "must live on the GPU")):
+        with pytest.raises(ValueError, match=text):
+            ops._need(*args, **kw)
+    for kw, text in (({"dtype": torch.int32}, "dtype"), ({"ndim": 3}, "dimensions")):
+        with pytest.raises(ValueError, match=text):
+            ops._refuse(type("T", (torch.Tensor,), {"is_cuda": True})(t), "x", kw.get("dtype"), kw.get("ndim"))
+    with pytest.raises(TypeError):
+        ops._need(t, "x", shape=3)
+
+
+def test_ordinary_tensor():
+    cpu = torch.device("cpu")
+    t = torch.zeros(8, 4)
+    assert dense.ordinary_tensor(t, cpu) and dense.ordinary_tensor(torch.nn.Parameter(t), cpu)
+    assert not dense.ordinary_tensor(t.t(), cpu) and not dense.ordinary_tensor(t.double(), cpu)
+    assert not dense.ordinary_tensor(t, torch.device("meta")) and not dense.ordinary_tensor(None, cpu)
+    assert not dense.ordinary_tensor(t.view(-1)[1:], cpu) and dense.ordinary_tensor(t.view(-1)[1:], cpu, align=4)
+    assert not dense.ordinary_tensor(t.as_subclass(type("S", (torch.Tensor,), {})), cpu)
+    seen = []
+    torch.func.vmap(lambda x: seen.append(dense.ordinary_tensor(x, cpu)) or x)(torch.zeros(2, 3))
+    assert seen == [False]
