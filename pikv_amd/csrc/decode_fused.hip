@@ -882,6 +882,25 @@ __device__ __forceinline__ uint2 bytes_to_bf16(uint32_t w) {
                     __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf2)));
 }
 
+// A block that holds few tiles is mostly its start: the loads of the fill, the first row, the queries and the first tile's
+// metadata, each waited for before the next was issued, took 9.5 of 35 thousand cycles of four tiles.  Here the first three go
+// out together (also from the blocks that then find no tokens), and the queries are unpacked when the first tile is on its
+// way: one call over 24 x <= 4000 tokens (4 x 28 heads) 31.3 -> 30.7 us, 2 x 7271 (8 x 40) 21.5 -> 20.7.  (The 4-bit kernels, which
+// start with two tiles on their way, measured slower that way: 16.1 -> 16.7 us for 1 x 700, 24.8 -> 25.5 for 3 x 8183.)
+// Tokens of cache c.
+__device__ __forceinline__ int64_t cache_len(const int32_t* fill, int c, int64_t max_len) {
+  const int n = fill[c];
+  return n < max_len ? (int64_t)n : max_len;
+}
+// Raw bits of 16 elements of either half of a head of 128.
+template <typename E, int N>
+__device__ __forceinline__ void load_query_halves(const E* q, uint4 (&raw)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    raw[k] = ld16(reinterpret_cast<const char*>(q + k / (N / 2) * 64) + 16 * (k % (N / 2)));
+  asm volatile("" ::: "memory");
+}
+
 // QF32: float32 queries as two bf16 limbs, q = hi + lo to 2^-18 |q| (hi = the float rounded to bf16, lo = the
 // rest rounded to bf16); both limbs are multiplied with the same converted codes into the same accumulators.
 template <int SCHEME, bool BOOK, bool QF32 = false>
@@ -903,7 +922,14 @@ __global__ __launch_bounds__(512) void decode_fused_i8_kernel(Fused8Args a) {
   const int g0 = (blockIdx.y % a.blocks_per_range) * nwb;
   const int g = g0 + wv;                            // this wavefront's kv head
   const int rep = a.n_q_heads / HK;
-  const int64_t len = a.fill[c] < a.max_len ? (int64_t)a.fill[c] : a.max_len;
+  const int64_t len = cache_len(a.fill, c, a.max_len), base = a.row_base[c];
+  const int nl = lane & 15, rg = lane >> 4;
+  uint4 qraw[QF32 ? 8 : 4];   // dimensions 16 rg .. + 15 of either half of the head
+  {
+    const int64_t qo = ((int64_t)c * a.n_q_heads + g * rep + (nl < rep ? nl : 0)) * 128 + rg * 16;
+    if constexpr (QF32) load_query_halves(reinterpret_cast<const float*>(a.q) + qo, qraw);
+    else load_query_halves(reinterpret_cast<const uint16_t*>(a.q) + qo, qraw);
+  }
   const int64_t t0 = (int64_t)xr * a.tokens_per_block;
   if (t0 >= len) return;   // the merge skips ranges that hold no token
   const int span = (int)((t0 + a.tokens_per_block < len ? t0 + a.tokens_per_block : len) - t0);
@@ -912,13 +938,12 @@ __global__ __launch_bounds__(512) void decode_fused_i8_kernel(Fused8Args a) {
   // roles.  Score product: lane = (column nl: a token, k-slice rg: 16 dimensions of each half of the head);
   // result lane (nl, rg) holds heads 4 rg .. 4 rg + 3 of its token.  Softmax and weights: heads
   // hq0 .. hq0 + 3, tokens tp, tp + 1.  Output product: lane = (A row / dimension i, k-slice kg: 8 tokens).
-  const int nl = lane & 15, rg = lane >> 4;
   const int i = nl, kg = rg;
   const int hq0 = 4 * (rg & 1);
   const int tp = 4 * nl + 2 * (rg >> 1);
   const int row_codes = HK * 128;                       // bytes per cached row in the code planes
   const int gpr = row_codes / a.group;                  // metadata entries per cached row
-  const int64_t urow = a.row_base[c] + t0;
+  const int64_t urow = base + t0;
   const char* const kc = reinterpret_cast<const char*>(a.k_codes) + urow * row_codes + g * 128;
   const char* const vc = reinterpret_cast<const char*>(a.v_codes) + urow * row_codes + g * 128;
 
@@ -934,54 +959,8 @@ __global__ __launch_bounds__(512) void decode_fused_i8_kernel(Fused8Args a) {
   const float* const vsb = reinterpret_cast<const float*>(a.v_scale) + urow * gpr + m_ent;
   const float* const vzb = reinterpret_cast<const float*>(a.v_zero) + urow * gpr + m_ent;
 
-  // ---- queries: A rows = the kv head's query heads, k-step (half, o) = dimensions 64 half + 16 rg + 8 o .. + 7 ----
-  uint4 aq[4], aql[QF32 ? 4 : 1];
-  float qs0, qs1;   // sum of the head's query over the dimensions of half 0 / half 1 (lane's row nl)
-  {
-    const bool a_on = nl < rep;
-    const int64_t qoff = ((int64_t)c * a.n_q_heads + g * rep + (a_on ? nl : 0)) * 128 + rg * 16;
-    float part[2] = {0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int64_t eo = qoff + (k >> 1) * 64 + (k & 1) * 8;
-      if constexpr (QF32) {
-        const float* qf = reinterpret_cast<const float*>(a.q) + eo;
-        uint32_t hb[8], lb[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float f = a_on ? qf[e] : 0.f;
-          hb[e] = bf16_limb_bits(f, 0);
-          lb[e] = bf16_limb_bits(f, 1);
-          part[k >> 1] += __uint_as_float(hb[e] << 16);
-          part[k >> 1] += __uint_as_float(lb[e] << 16);
-        }
-        aq[k] = make_uint4(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16), hb[4] | (hb[5] << 16), hb[6] | (hb[7] << 16));
-        aql[k] = make_uint4(lb[0] | (lb[1] << 16), lb[2] | (lb[3] << 16), lb[4] | (lb[5] << 16), lb[6] | (lb[7] << 16));
-      } else {
-        uint4 d = make_uint4(0, 0, 0, 0);
-        if (a_on) d = ld16(reinterpret_cast<const uint16_t*>(a.q) + eo);
-        aq[k] = d;
-        const uint32_t w[4] = {d.x, d.y, d.z, d.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          part[k >> 1] += __uint_as_float(w[e] << 16);
-          part[k >> 1] += __uint_as_float(w[e] & 0xffff0000u);
-        }
-      }
-    }
-    part[0] += __shfl_xor(part[0], 16, PIKV_WAVE);
-    part[0] += __shfl_xor(part[0], 32, PIKV_WAVE);
-    part[1] += __shfl_xor(part[1], 16, PIKV_WAVE);
-    part[1] += __shfl_xor(part[1], 32, PIKV_WAVE);
-    qs0 = part[0];
-    qs1 = part[1];
-  }
-  // ... of the four heads in this lane's result rows 4 rg .. 4 rg + 3 (rows past the heads: zero)
+  uint4 aq[4], aql[QF32 ? 4 : 1];   // the queries, filled below
   float4 q0v, q1v;
-  q0v.x = __shfl(qs0, 4 * rg + 0, PIKV_WAVE); q0v.y = __shfl(qs0, 4 * rg + 1, PIKV_WAVE);
-  q0v.z = __shfl(qs0, 4 * rg + 2, PIKV_WAVE); q0v.w = __shfl(qs0, 4 * rg + 3, PIKV_WAVE);
-  q1v.x = __shfl(qs1, 4 * rg + 0, PIKV_WAVE); q1v.y = __shfl(qs1, 4 * rg + 1, PIKV_WAVE);
-  q1v.z = __shfl(qs1, 4 * rg + 2, PIKV_WAVE); q1v.w = __shfl(qs1, 4 * rg + 3, PIKV_WAVE);
 
   pikv_f32x4 C[8];
 #pragma unroll
@@ -1045,13 +1024,65 @@ __global__ __launch_bounds__(512) void decode_fused_i8_kernel(Fused8Args a) {
   };
 
   issue_meta(0);
-  stage_meta(0);
+  const float fks = mks, fkz = mkz, fvs = mvs, fvz = mvz;
   pin_order();
   issue_meta(kFTile);
   issue_v(0);
   pin_order();
   issue_k(0);
   pin_order();
+  // ---- queries: A rows = the kv head's query heads, k-step (half, o) = dimensions 64 half + 16 rg + 8 o .. + 7 ----
+  float qs0, qs1;   // sum of the head's query over the dimensions of half 0 / half 1 (lane's row nl)
+  {
+    const bool a_on = nl < rep;
+    float part[2] = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (QF32) {
+        const uint4 f0 = qraw[2 * k], f1 = qraw[2 * k + 1];
+        const uint32_t fw[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+        uint32_t hb[8], lb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float f = a_on ? __uint_as_float(fw[e]) : 0.f;
+          hb[e] = bf16_limb_bits(f, 0);
+          lb[e] = bf16_limb_bits(f, 1);
+          part[k >> 1] += __uint_as_float(hb[e] << 16);
+          part[k >> 1] += __uint_as_float(lb[e] << 16);
+        }
+        aq[k] = make_uint4(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16), hb[4] | (hb[5] << 16), hb[6] | (hb[7] << 16));
+        aql[k] = make_uint4(lb[0] | (lb[1] << 16), lb[2] | (lb[3] << 16), lb[4] | (lb[5] << 16), lb[6] | (lb[7] << 16));
+      } else {
+        uint4 d = make_uint4(0, 0, 0, 0);
+        if (a_on) d = qraw[k];
+        aq[k] = d;
+        const uint32_t w[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          part[k >> 1] += __uint_as_float(w[e] << 16);
+          part[k >> 1] += __uint_as_float(w[e] & 0xffff0000u);
+        }
+      }
+    }
+    part[0] += __shfl_xor(part[0], 16, PIKV_WAVE);
+    part[0] += __shfl_xor(part[0], 32, PIKV_WAVE);
+    part[1] += __shfl_xor(part[1], 16, PIKV_WAVE);
+    part[1] += __shfl_xor(part[1], 32, PIKV_WAVE);
+    qs0 = part[0];
+    qs1 = part[1];
+  }
+  // ... of the four heads in this lane's result rows 4 rg .. 4 rg + 3 (rows past the heads: zero)
+  q0v.x = __shfl(qs0, 4 * rg + 0, PIKV_WAVE); q0v.y = __shfl(qs0, 4 * rg + 1, PIKV_WAVE);
+  q0v.z = __shfl(qs0, 4 * rg + 2, PIKV_WAVE); q0v.w = __shfl(qs0, 4 * rg + 3, PIKV_WAVE);
+  q1v.x = __shfl(qs1, 4 * rg + 0, PIKV_WAVE); q1v.y = __shfl(qs1, 4 * rg + 1, PIKV_WAVE);
+  q1v.z = __shfl(qs1, 4 * rg + 2, PIKV_WAVE); q1v.w = __shfl(qs1, 4 * rg + 3, PIKV_WAVE);
+
+  {
+    const float nks = mks, nkz = mkz, nvs = mvs, nvz = mvz;
+    mks = fks; mkz = fkz; mvs = fvs; mvz = fvz;
+    stage_meta(0);
+    mks = nks; mkz = nkz; mvs = nvs; mvz = nvz;
+  }
 
   for (int n0 = 0; n0 < span; n0 += kFTile) {
     const int par = (n0 / kFTile) & 1;
