@@ -1275,6 +1275,7 @@ static void launch_attend_mfma(int n_slabs, int heads_per_slab, dim3 grid, hipSt
     const int room = (nsets == 2 ? 4 : 8) / n_slabs;
     ti = room >= 8 ? 8 : room >= 4 ? 4 : room >= 2 ? 2 : 1;
     while (ti > 1 && a.tokens_per_block % (kAttTile * ti) != 0) ti >>= 1;
+    if (ti == 2 && n_slabs * ti < (nsets == 2 ? 4 : 6)) ti = 1;   // no such kernel
     // 4 slabs already fill the wavefronts; pairs of rows gain 5 % on the exchange rows and lose 4 % on float scores
     if (n_slabs == 4 && !EXCH) ti = 1;
   }
@@ -1304,7 +1305,9 @@ static void launch_attend_mfma(int n_slabs, int heads_per_slab, dim3 grid, hipSt
   }
 }
 
-// out[c,h,d] = sum over the splits that hold tokens of cache c, in split order
+// out[c,h,d] = sum over the splits that hold tokens of cache c, in split order.  The sum is a chain, the loads are not:
+// 16 of them are asked for together (2 caches x 21346 tokens x 36 heads of 128, 84 splits of 295 KB: 25 -> 10 us).
+constexpr int kReduceUnroll = 16;
 __global__ __launch_bounds__(256) void attend_reduce_kernel(const float* __restrict__ partial,
                                                            const int32_t* __restrict__ fill, int n_caches,
                                                            int n_q_heads, int head_dim, int n_splits,
@@ -1315,8 +1318,17 @@ __global__ __launch_bounds__(256) void attend_reduce_kernel(const float* __restr
   const int c = (int)(idx / per_cache);
   const int64_t used = ((int64_t)fill[c] + tokens_per_block - 1) / tokens_per_block;
   const int lim = used < n_splits ? (int)used : n_splits;
+  const float* p = partial + idx;
+  const int64_t step = per_cache * n_caches;
   float s = 0.f;
-  for (int sp = 0; sp < lim; ++sp) s += partial[(int64_t)sp * per_cache * n_caches + idx];
+  for (int sp = 0; sp < lim; sp += kReduceUnroll) {
+    float v[kReduceUnroll];
+#pragma unroll
+    for (int u = 0; u < kReduceUnroll; ++u) v[u] = sp + u < lim ? p[(int64_t)u * step] : 0.f;
+#pragma unroll
+    for (int u = 0; u < kReduceUnroll; ++u) s = sp + u < lim ? s + v[u] : s;
+    p += kReduceUnroll * step;
+  }
   out[idx] = s;
 }
 
@@ -1344,23 +1356,33 @@ static int attend_tokens_per_block(int n_caches, int64_t max_len) {
   }
   return best;
 }
-static int64_t attend_splits(int n_caches, int64_t max_len) {
-  const int tpb = attend_tokens_per_block(n_caches, max_len);
-  return (max_len + tpb - 1) / tpb;
+// ... inside pikv_decode_attend, whose workspace holds a partial per 64 tokens: while the pieces leave compute
+// units without a block they are halved, down to one tile.  Whole call, pieces of 256 / 128 / 64 tokens, us:
+// 8 caches x 3001 tokens x 16 heads of 64 (96 / 192 / 376 blocks) 44.4 / 40.2 / 40.3; 4 x 1500 x 16 of 256, 8-bit
+// (24 / 48 / 96) 62.9 / 42.3 / 32.9; 28 x 628 x 36 on 4 (84 / 140 / 280) 48.0 / 35.8 / 32.1; with a block for every
+// unit the prologues cost more than they bring: 17 x 5488 x 12 of 64 (374 / 731) 56.8 / 55.7 / 59.0, 64 x 3000 x 8
+// (768 / 1536) 90.4 / 93.8 / 98.3.
+// passes: blocks of one piece (the vector form's groups of query heads, and its windows).
+static int decode_tokens_per_block(int n_caches, int64_t max_len, int64_t passes) {
+  constexpr int64_t kUnits = 256;
+  int tpb = attend_tokens_per_block(n_caches, max_len);
+  while (tpb > kAttTile && passes * n_caches * ((max_len + tpb - 1) / tpb) < kUnits) tpb >>= 1;
+  return tpb;
 }
+static int64_t attend_splits(int tpb, int64_t max_len) { return (max_len + tpb - 1) / tpb; }
 
 extern "C" int64_t pikv_attend_workspace_bytes(int n_caches, int n_q_heads, int head_dim, int64_t max_len) {
   if (n_caches < 1 || n_q_heads < 1 || head_dim < 1 || max_len < 0) return 0;
-  return attend_splits(n_caches, max_len) * n_caches * (int64_t)n_q_heads * head_dim * (int64_t)sizeof(float);
+  return attend_splits(attend_tokens_per_block(n_caches, max_len), max_len) * n_caches * (int64_t)n_q_heads * head_dim * (int64_t)sizeof(float);
 }
 
-extern "C" int pikv_attend_values(const float* scores, const float* head_stats, int64_t score_stride,
-                                  const void* v_codes, const void* v_scale, const void* v_zero,
-                                  int scheme, int group, int n_kv_heads, int n_q_heads, int head_dim,
-                                  const int64_t* cache_row_base, const int32_t* cache_fill,
-                                  int n_caches, int64_t max_len, float decay, float now,
-                                  float* row_acc, float* row_ts, float* out, void* workspace,
-                                  int64_t workspace_bytes, void* stream) {
+static int attend_values(const float* scores, const float* head_stats, int64_t score_stride,
+                         const void* v_codes, const void* v_scale, const void* v_zero,
+                         int scheme, int group, int n_kv_heads, int n_q_heads, int head_dim,
+                         const int64_t* cache_row_base, const int32_t* cache_fill,
+                         int n_caches, int64_t max_len, float decay, float now,
+                         float* row_acc, float* row_ts, float* out, void* workspace,
+                         int64_t workspace_bytes, bool fine, void* stream) {
   if (!scores || !v_codes || !v_scale || !cache_row_base || !cache_fill || !out) return PIKV_ERR_NULL;
   if (scheme < 0 || scheme > 3) return PIKV_ERR_UNSUPPORTED;
   const bool eight = (scheme == PIKV_Q_I8_SYM || scheme == PIKV_Q_I8_ASYM);
@@ -1378,49 +1400,51 @@ extern "C" int pikv_attend_values(const float* scores, const float* head_stats, 
   if (head_dim / epl > 256) return PIKV_ERR_UNSUPPORTED;   // one kv head must fit a block of the vector form
   hipStream_t st = (hipStream_t)stream;
   const int64_t total = (int64_t)n_caches * n_q_heads * head_dim;
-  const int64_t splits = attend_splits(n_caches, max_len);
+  const int rep = n_q_heads / n_kv_heads;
+  // the matrix-core kernels see 128-dimension slabs of the row: one kv head, or 2 / 4 narrow ones
+  const int hps = mfma_heads_per_slab(head_dim, n_kv_heads);
+  const int slabs = hps > 0 ? n_kv_heads / hps : 0;
+  const bool slabs_ok = (slabs >= 1 && slabs <= 8) || (hps == 1 && slabs > 8 && slabs % 8 == 0 && slabs / 8 <= 32768);   // 32768 x 65535 splits
+  const bool mfma4 = !eight && group == 32 && slabs_ok && (rep * hps <= 8 || slabs <= 4);
+  const bool mfma8 = eight && slabs >= 1 && slabs <= 8 && group % head_dim == 0 && rep * hps >= 2 &&
+                     (rep * hps <= 8 || (hps == 1 && (n_q_heads <= 64 || slabs <= 4)));
+  // the vector form: heads of a kv group per pass (the float accumulators of one lane must fit), and for rows of more
+  // than 256 lanes windows of kv heads, preferably of a lane count that divides the block
+  const int rp = eight ? (rep >= 8 ? 8 : rep >= 4 ? 4 : rep >= 2 ? 2 : 1) : (rep >= 2 ? 2 : 1);
+  int window = 0;
+  if (lanes_per_row > 256) {
+    const int lph = head_dim / epl;
+    for (int w = n_kv_heads; w >= 1; --w)
+      if (n_kv_heads % w == 0 && w * lph <= 256 && (window == 0 || (256 % (w * lph) == 0 && 256 % (window * lph) != 0)))
+        window = w;
+  }
+  const int64_t passes = mfma4 || mfma8 ? 1 : (int64_t)((rep + rp - 1) / rp) * (window ? n_kv_heads / window : 1);
+  const int tpb = fine ? decode_tokens_per_block(n_caches, max_len, passes) : attend_tokens_per_block(n_caches, max_len);
+  const int64_t splits = attend_splits(tpb, max_len);
   if (splits > 65535) return PIKV_ERR_SHAPE;
   if (max_len > 0) {
     if (!workspace) return PIKV_ERR_NULL;
-    if (workspace_bytes < pikv_attend_workspace_bytes(n_caches, n_q_heads, head_dim, max_len))
-      return PIKV_ERR_WORKSPACE;
+    if (workspace_bytes < splits * total * (int64_t)sizeof(float)) return PIKV_ERR_WORKSPACE;
   }
   AttendArgs a{scores, head_stats, v_codes, v_scale, v_zero, cache_row_base, cache_fill,
                (float*)workspace, score_stride, group, n_kv_heads, n_q_heads, head_dim, n_caches,
-               row_acc, row_ts, decay, now, max_len, nullptr, nullptr, 0, 0, attend_tokens_per_block(n_caches, max_len)};
-  const int rep = n_q_heads / n_kv_heads;
+               row_acc, row_ts, decay, now, max_len, nullptr, nullptr, 0, 0, tpb};
   if (max_len > 0) {
-    // the matrix-core kernels see 128-dimension slabs of the row: one kv head, or 2 / 4 narrow ones
-    const int hps = mfma_heads_per_slab(head_dim, n_kv_heads);
-    const int slabs = hps > 0 ? n_kv_heads / hps : 0;
-    const bool slabs_ok = (slabs >= 1 && slabs <= 8) || (hps == 1 && slabs > 8 && slabs % 8 == 0 && splits * (slabs / 8) <= 0x7fffffffLL);
-    if (!eight && group == 32 && slabs_ok && (rep * hps <= 8 || slabs <= 4)) {
+    if (mfma4) {
       const dim3 grid((unsigned)splits, (unsigned)n_caches);
       if (scheme == PIKV_Q_I4_ASYM) launch_attend_mfma<PIKV_Q_I4_ASYM>(slabs, rep * hps, grid, st, a);
       else launch_attend_mfma<PIKV_Q_I4_SYM>(slabs, rep * hps, grid, st, a);
-    } else if (eight && slabs >= 1 && slabs <= 8 && group % head_dim == 0 && rep * hps >= 2 &&
-               (rep * hps <= 8 || (hps == 1 && (n_q_heads <= 64 || slabs <= 4)))) {
+    } else if (mfma8) {
       const dim3 grid((unsigned)splits, (unsigned)n_caches);
       if (scheme == PIKV_Q_I8_SYM) launch_attend_mfma8<PIKV_Q_I8_SYM>(slabs, hps, grid, st, a);
       else launch_attend_mfma8<PIKV_Q_I8_ASYM>(slabs, hps, grid, st, a);
     } else {
+      if (passes > 65535) return PIKV_ERR_SHAPE;
       if (row_acc || row_ts)
         hipLaunchKernelGGL(attend_importance_kernel, dim3((unsigned)((max_len + 255) / 256), (unsigned)n_caches),
                            dim3(256), 0, st, a);
-      // heads of a kv group per pass: the float accumulators of one lane must fit
-      const int rp = eight ? (rep >= 8 ? 8 : rep >= 4 ? 4 : rep >= 2 ? 2 : 1) : (rep >= 2 ? 2 : 1);
-      // rows of more than 256 lanes: windows of kv heads, preferably of a lane count that divides the block
-      int n_win = 1;
-      if (lanes_per_row > 256) {
-        const int lph = head_dim / epl;
-        int wk = 0;
-        for (int w = n_kv_heads; w >= 1; --w)
-          if (n_kv_heads % w == 0 && w * lph <= 256 && (wk == 0 || (256 % (w * lph) == 0 && 256 % (wk * lph) != 0))) wk = w;
-        a.kv_window = wk;
-        n_win = n_kv_heads / wk;
-      }
-      if ((int64_t)((rep + rp - 1) / rp) * n_win > 65535) return PIKV_ERR_SHAPE;
-      const dim3 grid((unsigned)splits, (unsigned)n_caches, (unsigned)((rep + rp - 1) / rp * n_win));
+      a.kv_window = window;
+      const dim3 grid((unsigned)splits, (unsigned)n_caches, (unsigned)passes);
 #define PIKV_ATTEND_CASE(S)                                                                        \
   case S:                                                                                          \
     if (rp == 8) hipLaunchKernelGGL((attend_valu_kernel<S, 8>), grid, dim3(256), 0, st, a);        \
@@ -1450,6 +1474,18 @@ extern "C" int pikv_attend_values(const float* scores, const float* head_stats, 
   return PIKV_OK;
 }
 
+extern "C" int pikv_attend_values(const float* scores, const float* head_stats, int64_t score_stride,
+                                  const void* v_codes, const void* v_scale, const void* v_zero,
+                                  int scheme, int group, int n_kv_heads, int n_q_heads, int head_dim,
+                                  const int64_t* cache_row_base, const int32_t* cache_fill,
+                                  int n_caches, int64_t max_len, float decay, float now,
+                                  float* row_acc, float* row_ts, float* out, void* workspace,
+                                  int64_t workspace_bytes, void* stream) {
+  return attend_values(scores, head_stats, score_stride, v_codes, v_scale, v_zero, scheme, group, n_kv_heads, n_q_heads,
+                       head_dim, cache_row_base, cache_fill, n_caches, max_len, decay, now, row_acc, row_ts, out, workspace,
+                       workspace_bytes, false, stream);
+}
+
 // ---- one call for the decode read: scores, softmax, attention output, H2O bookkeeping ----
 static int64_t align256(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
@@ -1469,7 +1505,7 @@ static DecodeWs decode_ws(int n_caches, int n_q_heads, int head_dim, int64_t max
   w.partial = w.stats + align256((int64_t)n_caches * n_q_heads * 2 * 4);
   const int64_t fused_tpb = fused_min_tokens_per_block(n_caches, max_len);
   const int64_t fused = (max_len + fused_tpb - 1) / fused_tpb * n_caches * (int64_t)n_q_heads * head_dim * (int64_t)sizeof(float);
-  const int64_t two_kernel = pikv_attend_workspace_bytes(n_caches, n_q_heads, head_dim, max_len);
+  const int64_t two_kernel = attend_splits(decode_tokens_per_block(n_caches, max_len, 1), max_len) * n_caches * (int64_t)n_q_heads * head_dim * (int64_t)sizeof(float);
   w.ranges = w.partial + align256(fused > two_kernel ? fused : two_kernel);
   w.total = w.ranges + align256((max_len + fused_tpb - 1) / fused_tpb * n_caches * (int64_t)n_q_heads * 8);
   return w;
@@ -1527,7 +1563,8 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
   const int hps = mfma_heads_per_slab(head_dim, n_kv_heads);   // 128-dimension slabs: one kv head, or 2 / 4 narrow ones
   const int slabs = hps > 0 ? n_kv_heads / hps : 0;
   const bool hk_ok = (slabs >= 1 && slabs <= 8) || (hps == 1 && slabs > 8 && slabs % 8 == 0);
-  const int64_t splits = attend_splits(n_caches, max_len);
+  const int tpb = decode_tokens_per_block(n_caches, max_len, 1);
+  const int64_t splits = attend_splits(tpb, max_len);
   if ((scheme == PIKV_Q_I4_ASYM || scheme == PIKV_Q_I4_SYM) && group == 32 && rep >= 1 &&
       (rep * hps <= 8 || slabs <= 4) && hk_ok && (q_dtype == PIKV_BF16 || q_dtype == PIKV_F32) && n_caches <= 65535 && splits <= 65535 && (!asym || (k_zero && v_zero))) {
     float* esc = reinterpret_cast<float*>(ws + w.scores);
@@ -1537,7 +1574,7 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
     if (rc == PIKV_OK) {
       AttendArgs a{nullptr, stats, v_codes, v_scale, v_zero, cache_row_base, cache_fill,
                    (float*)partial, 0, group, n_kv_heads, n_q_heads, head_dim, n_caches,
-                   row_acc, row_ts, decay, now, max_len, esc, tmax, w.n_tiles, 0, attend_tokens_per_block(n_caches, max_len)};
+                   row_acc, row_ts, decay, now, max_len, esc, tmax, w.n_tiles, 0, tpb};
       const dim3 grid((unsigned)splits, (unsigned)n_caches);
       if (asym) launch_attend_mfma<PIKV_Q_I4_ASYM, true>(slabs, rep * hps, grid, st, a);
       else launch_attend_mfma<PIKV_Q_I4_SYM, true>(slabs, rep * hps, grid, st, a);
@@ -1559,7 +1596,7 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
   rc = pikv_h2o_accumulate(scores, tmax, tsum, n_q_heads, cache_row_base, cache_fill, n_caches, max_len, w.stride,
                            1.0f, now, 0, nullptr, nullptr, nullptr, stats, stream);
   if (rc != PIKV_OK) return rc;
-  return pikv_attend_values(scores, stats, w.stride, v_codes, v_scale, v_zero, scheme, group, n_kv_heads, n_q_heads,
-                            head_dim, cache_row_base, cache_fill, n_caches, max_len, decay, now, row_acc, row_ts, out,
-                            partial, partial_bytes, stream);
+  return attend_values(scores, stats, w.stride, v_codes, v_scale, v_zero, scheme, group, n_kv_heads, n_q_heads, head_dim,
+                       cache_row_base, cache_fill, n_caches, max_len, decay, now, row_acc, row_ts, out, partial, partial_bytes,
+                       true, stream);
 }

@@ -363,6 +363,38 @@ def test_attend_block_lengths(dev, n_caches, length, scheme, heads, hq):
         np.testing.assert_allclose(acc3[rows], imp, rtol=1e-3, atol=1e-6)
 
 
+@pytest.mark.parametrize("scheme,group,heads,hq,dh,qdtype", [
+    (O.Q_I4_ASYM, 32, 16, 16, 64, "f32"),    # exchange format
+    (O.Q_I4_ASYM, 32, 1, 8, 128, "bf16"),    # ... rows too narrow for pairs of them in these pieces
+    (O.Q_I4_SYM, 32, 3, 9, 128, "bf16"),     # ... pairs of rows
+    (O.Q_I8_ASYM, 128, 3, 30, 128, "bf16"),  # float scores, 8-bit matrix-core form
+    (O.Q_I8_SYM, 256, 2, 4, 256, "bf16"),    # vector form
+    (O.Q_I4_SYM, 64, 1, 7, 64, "f32"),       # ... two lanes to a row
+])
+@pytest.mark.parametrize("n_caches,longest", [(20, 1700), (33, 1700), (90, 129), (3, 65)])
+def test_decode_attend_pieces(dev, n_caches, longest, scheme, group, heads, hq, dh, qdtype):
+    """Pieces of 128, 256, 128 and 64 cached tokens per block of the decode read, lengths around their edges, against
+    the three public steps (pieces of 256 or more).  Both add up at most 1700 products of 24 bits whose
+    probabilities sum to one, in another order, from scores that are equal or differ by a rounding of the
+    largest, below 64: 2 x 1700 x 2^-24 and 64 x 2^-23 of the largest value row element."""
+    r = rng(n_caches + heads)
+    edge = [0, 1, 63, 64, 65, 127, 128, 129, 255, 256, 257, longest - 1]
+    lens = [longest] + [min(edge[c % len(edge)], longest) for c in range(n_caches - 1)]
+    pool, ref = _fill_pool(dev, r, [longest] * n_caches, lens, heads, dh, group, scheme)
+    q = to_dev(O.bf16_round(r.standard_normal((n_caches, hq, dh)).astype(np.float32)), dev, qdtype)
+    pool.acc.zero_()
+    out = np_of(pool.decode_attend(q, hq, now=3.0))
+    acc = np_of(pool.acc).copy()
+    scores, tmax, tsum = pool.scores(q, hq)
+    pool.acc.zero_()
+    pool.h2o_accumulate(scores, tmax, tsum, now=3.0, stats_only=True)
+    want = np_of(pool.attend_values(scores, pool.head_stats, accumulate=True, now=3.0))
+    rows = np.concatenate([ref.valid_rows(c)[:L] for c, L in enumerate(lens)])
+    v_max = np.abs(O.dequantize_groups(ref.v_codes[rows], ref.v_scale[rows], ref.v_zero[rows], group)).max()
+    assert np.abs(out - want).max() <= (2 * 1700 * 2.0 ** -24 + 64 * 2.0 ** -23) * v_max
+    np.testing.assert_allclose(acc, np_of(pool.acc), rtol=hq * 2.0 ** -22 + 64 * 2.0 ** -23, atol=1e-12)
+
+
 def _decode_reference(ref, q, lens_now, acc_before, heads, group, scale_qk, decay):
     """softmax(q k^T) v and the H2O sums of every cache in float64 on the restatement's dequantised rows."""
     outs, accs = [], acc_before.copy()
