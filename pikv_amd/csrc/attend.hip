@@ -56,7 +56,7 @@ struct AttendArgs {
   const float* escores;
   const float* tile_max;
   int64_t n_tiles;
-  int head_off;  // attend_mfma_i4_kernel: first query head of every kv group handled by this launch
+  int head_off;  // matrix-core kernels: first query head of every kv group of this launch's first blocks (grid z: the next sets)
   int tokens_per_block;  // cached tokens per block (a multiple of 64): block x covers tokens [x * tokens_per_block, ...)
   int kv_window;         // attend_valu_kernel: kv heads per block when a whole row has more than 256 lanes (0: all)
   int row_slabs;         // attend_mfma_i4_kernel<SPLIT>: 128-dimension slabs of a whole cached row (the block takes 8 of them)
@@ -74,7 +74,8 @@ template <int SCHEME, int RP>
 __global__ __launch_bounds__(256) void attend_valu_kernel(AttendArgs a) {
   using Q = QScheme<SCHEME>;
   constexpr int EPL = Q::epl;
-  __shared__ float red[256 * EPL];
+  constexpr int RS = 257;                         // padded: consecutive dimensions of a lane lie in different banks
+  __shared__ float red[RS * EPL];                 // [dimension of a lane][thread]
   const int c = blockIdx.y;
   const int64_t len = a.fill[c] < a.max_len ? (int64_t)a.fill[c] : a.max_len;
   const int64_t t0 = (int64_t)blockIdx.x * a.tokens_per_block;
@@ -93,7 +94,6 @@ __global__ __launch_bounds__(256) void attend_valu_kernel(AttendArgs a) {
   const int gpart = (blockIdx.z % n_win) * lanes_per_row + part;   // piece of the whole row
   const int tok_in_step = threadIdx.x / lanes_per_row;
   const int kvh = gpart / lanes_per_head;
-  const int d0 = (part % lanes_per_head) * EPL;
   const bool normalise = a.head_stats != nullptr;
 
   float acc[RP][EPL];
@@ -148,49 +148,70 @@ __global__ __launch_bounds__(256) void attend_valu_kernel(AttendArgs a) {
       }
     }
   }
-  // add the token slots of the block (threads that share `part`), one head at a time
+  // Add the token slots of the block (threads that share `part`), one head at a time.  Rows of up to 32 lanes have many
+  // slots and few outputs: there all threads take part, `seg` of them to an output where there are fewer outputs than
+  // threads (two lanes of 71 heads x 64, 4-bit, 128 slots: by two threads 975 us, by all 122 us at 24 caches x 2401
+  // tokens; the wide rows' two to five slots go through LDS in 16-byte pieces, 13.0 against 15.2 us at 3532 tokens x 8
+  // heads of 256).
+  const int n_out = lanes_per_row * EPL;            // outputs of the window per query head of a group
+  const int seg = n_out < 256 ? 256 / n_out : 1;
+  const int sg = threadIdx.x / n_out;               // 0 where n_out >= 256
+  const int hd_bits = 31 - __builtin_clz(a.head_dim);
+  const int kv0 = (blockIdx.z % n_win) * wk;
 #pragma unroll
   for (int r = 0; r < RP; ++r) {
+    if (r0 + r >= rep) break;  // uniform
     __syncthreads();
+    float* const out = a.partial + (((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads + kv0 * rep + r0 + r) * a.head_dim;
+    auto out_at = [&](int o) -> float* {            // output o of the window: heads side by side, a power of two each
+      return out + (o >> hd_bits) * rep * a.head_dim + (o & (a.head_dim - 1));
+    };
+    if (lanes_per_row > 32) {
 #pragma unroll
-    for (int j = 0; j < EPL; ++j) red[threadIdx.x * EPL + j] = acc[r][j] - zacc[r];
+      for (int j = 0; j < EPL; ++j) red[threadIdx.x * EPL + j] = acc[r][j] - zacc[r];
+      __syncthreads();
+      if (tok_in_step == 0) {
+        float sum[EPL];
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) sum[j] = 0.f;
+        for (int t = 0; t < tok_per_step; ++t)
+#pragma unroll
+          for (int j = 0; j < EPL; ++j) sum[j] += red[(t * lanes_per_row + part) * EPL + j];
+        float* const o = out_at(part * EPL);
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) o[j] = sum[j];
+      }
+      continue;
+    }
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) red[j * RS + threadIdx.x] = acc[r][j] - zacc[r];
     __syncthreads();
-    if (tok_in_step == 0 && r0 + r < rep) {
-      float sum[EPL];
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) sum[j] = 0.f;
-      for (int s = 0; s < tok_per_step; ++s)
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) sum[j] += red[(s * lanes_per_row + part) * EPL + j];
-      const int hq = kvh * rep + r0 + r;
-      float* o = a.partial + (((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads + hq) * a.head_dim + d0;
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) o[j] = sum[j];
+    if (seg == 1) {
+      for (int o = threadIdx.x; o < n_out; o += 256) {
+        const float* p = red + (o % EPL) * RS + o / EPL;
+        float sum = 0.f;
+        for (int t = 0; t < tok_per_step; ++t) sum += p[t * lanes_per_row];
+        *out_at(o) = sum;
+      }
+    } else {
+      const int o = threadIdx.x - sg * n_out;
+      const float* p = red + (o % EPL) * RS + o / EPL;
+      float sum = 0.f;
+      if (sg < seg)
+        for (int t = sg; t < tok_per_step; t += seg) sum += p[t * lanes_per_row];
+      __syncthreads();
+      red[threadIdx.x] = sum;
+      __syncthreads();
+      if (sg == 0) {
+        for (int k = 1; k < seg; ++k) sum += red[k * n_out + o];
+        *out_at(o) = sum;
+      }
     }
   }
 }
 
-// Importance of every cached token (sum of its probabilities over the query heads, in
-// head order) for callers of the vector-unit form.
-__global__ __launch_bounds__(256) void attend_importance_kernel(AttendArgs a) {
-  const int c = blockIdx.y;
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (n >= a.fill[c] || n >= a.max_len) return;
-  const bool normalise = a.head_stats != nullptr;
-  float imp = 0.f;
-  for (int h0 = 0; h0 < a.n_q_heads; h0 += 8) {   // eight heads in flight per thread
-    float sv[8], mx[8], hz[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int64_t hi = (int64_t)c * a.n_q_heads + (h0 + u < a.n_q_heads ? h0 + u : 0);
-      sv[u] = a.scores[hi * a.score_stride + n];
-      mx[u] = normalise ? a.head_stats[hi * 2] : 0.f;
-      hz[u] = normalise ? a.head_stats[hi * 2 + 1] : 1.f;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (h0 + u < a.n_q_heads) imp = imp + prob_of(sv[u], mx[u], 1.0f / hz[u], normalise);
-  }
+// H2O bookkeeping of token n of cache c
+__device__ __forceinline__ void add_importance(const AttendArgs& a, int c, int64_t n, float imp) {
   const int64_t row = a.row_base[c] + n;
   if (a.row_acc) {
     float acc = a.row_acc[row];
@@ -198,6 +219,39 @@ __global__ __launch_bounds__(256) void attend_importance_kernel(AttendArgs a) {
     a.row_acc[row] = acc + imp;
   }
   if (a.row_ts) a.row_ts[row] = a.now;
+}
+
+// Importance of every cached token (sum of its probabilities over the query heads) for callers of the vector-unit form
+// and for sets of query heads side by side.  One block per 64 tokens; four lanes per token add every fourth head, then the four
+// partial sums (a lane per token, head after head: 8 caches x 32520 tokens x
+// 71 heads 18.2 -> 16.5 us, 3 x 4430 x 32 6.8 -> 4.4).
+__global__ __launch_bounds__(256) void attend_importance_kernel(AttendArgs a) {
+  __shared__ float part[4][kAttTile];
+  const int c = blockIdx.y;
+  const int64_t n0 = (int64_t)blockIdx.x * kAttTile;
+  const int64_t len = a.fill[c] < a.max_len ? (int64_t)a.fill[c] : a.max_len;
+  if (n0 >= len) return;  // uniform
+  const int t = threadIdx.x & 63, hl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool in = n0 + t < len;
+  const int64_t n = in ? n0 + t : n0;
+  const bool normalise = a.head_stats != nullptr;
+  float imp = 0.f;
+  for (int h0 = hl; h0 < a.n_q_heads; h0 += 4 * 8) {   // eight heads in flight per thread
+    float sv[8], mx[8], hz[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t hi = (int64_t)c * a.n_q_heads + (h0 + 4 * u < a.n_q_heads ? h0 + 4 * u : hl);
+      sv[u] = a.scores[hi * a.score_stride + n];
+      mx[u] = normalise ? a.head_stats[hi * 2] : 0.f;
+      hz[u] = normalise ? a.head_stats[hi * 2 + 1] : 1.f;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (h0 + 4 * u < a.n_q_heads) imp = imp + prob_of(sv[u], mx[u], 1.0f / hz[u], normalise);
+  }
+  part[hl][t] = imp;
+  __syncthreads();
+  if (hl == 0 && in) add_importance(a, c, n, (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
 }
 
 // H2O bookkeeping from the exchange format of pikv_decode_attend, for the attention kernels that
@@ -211,7 +265,7 @@ __global__ __launch_bounds__(256) void exch_importance_kernel(AttendArgs a) {
   const int64_t len = a.fill[c] < a.max_len ? (int64_t)a.fill[c] : a.max_len;
   const int64_t n0 = tile * kAttTile;
   if (n0 >= len) return;  // uniform
-  const int t = threadIdx.x & 63, hl = threadIdx.x >> 6;
+  const int t = threadIdx.x & 63, hl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t trow = ((int64_t)c * a.n_tiles + tile) * a.n_q_heads;
   float imp = 0.f;
   for (int h0 = hl; h0 < a.n_q_heads; h0 += 4 * 8) {   // eight heads in flight per thread
@@ -232,16 +286,7 @@ __global__ __launch_bounds__(256) void exch_importance_kernel(AttendArgs a) {
   }
   part[hl][t] = imp;
   __syncthreads();
-  if (hl == 0 && n0 + t < len) {
-    imp = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
-    const int64_t row = a.row_base[c] + n0 + t;
-    if (a.row_acc) {
-      float acc = a.row_acc[row];
-      if (a.decay != 1.0f) acc = acc * a.decay;
-      a.row_acc[row] = acc + imp;
-    }
-    if (a.row_ts) a.row_ts[row] = a.now;
-  }
+  if (hl == 0 && n0 + t < len) add_importance(a, c, n0 + t, (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]));
 }
 
 // ---- matrix-core form -----------------------------------------------------------------
@@ -316,6 +361,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   if (threadIdx.x < 8) reinterpret_cast<uint32_t*>(azero)[threadIdx.x] = 0u;  // visible after the loop's first barrier
 
   const int c = blockIdx.y;
+  const int head_off = a.head_off + blockIdx.z * 4 * NSETS;   // first query head of every slab of this block
   const int64_t len = a.fill[c] < a.max_len ? (int64_t)a.fill[c] : a.max_len;
   static_assert(!SPLIT || !NARROW, "split rows: groups of HK slabs, heads of 128 dimensions");
   const int n_groups = SPLIT ? a.row_slabs / HK : 1;
@@ -331,11 +377,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       a.partial[(((int64_t)xb * a.n_caches + c) * a.n_q_heads + (SPLIT ? (blockIdx.x % n_groups) * nh : 0)) * hd + idx] = 0.f;
     return;
   }
-  // A launch covers up to 4 query heads of every kv group: heads head_off .. head_off+nr-1.
-  // More than 4 heads per kv head are served by a second launch over the same codes.
+  // A block covers up to 4 query heads of every kv group and set: heads head_off .. head_off + rep + rep_b - 1.
+  // More heads per slab are other blocks (grid z) over the same codes.
   const int rep_all = a.n_q_heads / row_slabs;   // query heads per slab
-  const int rep = rep_all - a.head_off < 4 ? rep_all - a.head_off : 4;  // heads of a group in this launch (first set)
-  const int rep_b = NSETS == 1 ? 0 : rep_all - a.head_off - 4 < 0 ? 0 : rep_all - a.head_off - 4 < 4 ? rep_all - a.head_off - 4 : 4;  // second set
+  const int rep = rep_all - head_off < 4 ? rep_all - head_off : 4;  // heads of a group in this launch (first set)
+  const int rep_b = NSETS == 1 ? 0 : rep_all - head_off - 4 < 0 ? 0 : rep_all - head_off - 4 < 4 ? rep_all - head_off - 4 : 4;  // second set
   // matrix-core roles: A row / B,C column i, token group kg
   const int i = lane & 15;
   const int kg = lane >> 4;
@@ -366,7 +412,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const int s_set = NSETS == 1 && TI == 1 ? 0 : sh / (4 * HR);
   const int s_g = NSETS == 1 && TI == 1 ? sh >> 2 : (sh >> 2) % HR;
   const bool s_on = s_set < NSETS && s_g < HR && (sh & 3) < (s_set ? rep_b : rep);
-  const int s_hq = s_on ? (kv_off + s_g) * rep_all + a.head_off + 4 * s_set + (sh & 3) : 0;
+  const int s_hq = s_on ? (kv_off + s_g) * rep_all + head_off + 4 * s_set + (sh & 3) : 0;
   const float* srow = a.scores + ((int64_t)c * a.n_q_heads + s_hq) * a.score_stride;
   float smx = 0.f, srz = 1.f;
   if (normalise) {
@@ -739,12 +785,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     for (int idx = threadIdx.x; idx < HR * 4 * NSETS * 128; idx += 256) {
       const int row = idx >> 7, g = row / (4 * NSETS), hl = row % (4 * NSETS), d = idx & 127;
       if (hl >= heads) continue;
-      const int64_t ohead = ((int64_t)xb * a.n_caches + c) * a.n_q_heads + g * rep_all + a.head_off + hl;
+      const int64_t ohead = ((int64_t)xb * a.n_caches + c) * a.n_q_heads + g * rep_all + head_off + hl;
       if constexpr (!NARROW) {
         a.partial[ohead * 128 + d] = ol[idx];
       } else {
         // a narrow head keeps the dimensions of its own kv head of the slab
-        const int hh = (a.head_off + hl) / rep1;
+        const int hh = (head_off + hl) / rep1;
         if (d / a.head_dim == hh) a.partial[ohead * a.head_dim + d - hh * a.head_dim] = ol[idx];
       }
     }
@@ -759,7 +805,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     for (int rr = 0; rr < 2; ++rr) {
       const int ro = 2 * kg + rr;  // head (inside the set) held by this lane
       if (ro >= (set ? rep_b : rep)) continue;
-      const int hro = a.head_off + 4 * set + ro;   // head inside the kv group
+      const int hro = head_off + 4 * set + ro;   // head inside the kv group
       const int64_t ohead = ((int64_t)xb * a.n_caches + c) * a.n_q_heads + (kv_off + g) * rep_all + hro;
       if constexpr (!NARROW) {
         float* o = a.partial + ohead * 128;
@@ -841,6 +887,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
                                           4 * (2 * 16 * kAtt8ARow));
 
   const int c = blockIdx.y;
+  const int head_off = a.head_off + blockIdx.z * 8;   // first query head of every kv head (slab) of this block
   const int64_t len = a.fill[c] < a.max_len ? (int64_t)a.fill[c] : a.max_len;
   const int64_t t0 = (int64_t)blockIdx.x * a.tokens_per_block;
   const int64_t t1 = (t0 + a.tokens_per_block < len) ? t0 + a.tokens_per_block : len;
@@ -849,10 +896,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       a.partial[((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads * a.head_dim + idx] = 0.f;
     return;
   }
-  // a launch serves heads a.head_off .. a.head_off + rep - 1 of every kv head (more than 8 per kv head: two
+  // a launch serves heads head_off .. head_off + rep - 1 of every kv head (more than 8 per kv head: two
   // launches; narrow heads are launched with head_off = 0 only); the staged rows count these heads alone
   const int rep_all = a.n_q_heads / HKR;
-  const int rep = rep_all - a.head_off < 8 ? rep_all - a.head_off : 8;  // 1..8
+  const int rep = rep_all - head_off < 8 ? rep_all - head_off : 8;  // 1..8
   const int nql = HKR * rep;         // staged heads: row (kv head) * rep + head of the launch
   const int rep1 = rep / HPS;        // query heads per stored kv head
   const int groups_per_row = (HKR * 128) / a.group;
@@ -877,7 +924,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const int sh = threadIdx.x / (4 * TI);
   const int st8 = (threadIdx.x % (4 * TI)) * 8;
   const bool s_on = sh < nql;
-  const int s_hq = s_on ? (sh / rep) * rep_all + a.head_off + sh % rep : 0;   // the query head itself
+  const int s_hq = s_on ? (sh / rep) * rep_all + head_off + sh % rep : 0;   // the query head itself
   const float* srow = a.scores + ((int64_t)c * a.n_q_heads + s_hq) * a.score_stride;
   float smx = 0.f, srz = 1.f;
   if (normalise) {
@@ -1150,7 +1197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     for (int idx = threadIdx.x; idx < HKR * 8 * 128; idx += 256) {
       const int row = idx >> 7, g = row >> 3, ro = row & 7;
       if (ro < rep)
-        a.partial[(((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads + g * rep_all + a.head_off + ro) * 128 + (idx & 127)] = ol[idx];
+        a.partial[(((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads + g * rep_all + head_off + ro) * 128 + (idx & 127)] = ol[idx];
     }
     return;
   }
@@ -1163,7 +1210,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       const int ro = 2 * kg + rr;  // head (inside the kv group) held by this lane
       if (ro >= rep) continue;
       const int hh = HPS > 1 ? ro / rep1 : 0;   // stored kv head of the slab that owns this head: blocks db with db * HPS / 8 == hh
-      float* o = a.partial + (((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads + g * rep_all + a.head_off + ro) * (128 / HPS) -
+      float* o = a.partial + (((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads + g * rep_all + head_off + ro) * (128 / HPS) -
                  hh * (128 / HPS);
 #pragma unroll
       for (int db = 0; db < 8; ++db)
@@ -1188,12 +1235,31 @@ static void launch_attend_mfma8_slabs(int n_slabs, dim3 grid, hipStream_t st, co
 }
 template <int SCHEME>
 static void launch_attend_mfma8_heads(int n_slabs, int hps, dim3 grid, hipStream_t st, const AttendArgs& a);
-// All query heads of every kv head: up to eight per launch; a later launch (same codes, next heads) adds its
-// share of the importance to the accumulators that the first one has decayed.
+// The H2O bookkeeping as a launch of its own, for blocks that see only some of a token's query heads.
+template <bool EXCH>
+static void launch_importance(hipStream_t st, AttendArgs& a) {
+  const dim3 grid((unsigned)((a.max_len + kAttTile - 1) / kAttTile), (unsigned)a.n_caches);
+  if (a.row_acc || a.row_ts) {
+    if (EXCH) hipLaunchKernelGGL(exch_importance_kernel, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(attend_importance_kernel, grid, dim3(256), 0, st, a);
+  }
+  a.row_acc = nullptr;
+  a.row_ts = nullptr;
+}
+// Sets of query heads beyond a block's: as blocks side by side (grid z) with the bookkeeping before them while one
+// set leaves the chip half empty (whole read, 48 query heads on one kv head of 128, 4-bit: 9 caches x 259 tokens 65 -> 22 us,
+// 50 x 3417 143 -> 102), and one launch after the other beyond, where the bookkeeping is cheaper inside them (each
+// adds its share to the accumulators that the first one has decayed) than another pass over the scores.
+static bool sets_side_by_side(dim3 grid) { return (int64_t)grid.x * grid.y < 512; }
 template <int SCHEME>
 static void launch_attend_mfma8(int n_slabs, int hps, dim3 grid, hipStream_t st, AttendArgs a) {
   const int rep = a.n_q_heads / n_slabs;
-  for (int off = 0; off < rep; off += 8) {
+  const bool side = rep > 8 && sets_side_by_side(grid);
+  if (side) {
+    launch_importance<false>(st, a);
+    grid.z = (unsigned)((rep + 7) / 8);
+  }
+  for (int off = 0; off < rep; off += 8 * (int)grid.z) {
     a.head_off = off;
     if (off > 0) a.decay = 1.0f;
     launch_attend_mfma8_heads<SCHEME>(n_slabs, hps, grid, st, a);
@@ -1249,23 +1315,14 @@ static void launch_attend_mfma(int n_slabs, int heads_per_slab, dim3 grid, hipSt
   const int gs = wide && n_slabs >= 8 && n_slabs % 4 == 0 ? 4 : wide && n_slabs == 6 ? 3 : n_slabs > 8 ? 8 : 0;
   if (gs) {
     // the groups of a token range are neighbouring blocks; the H2O bookkeeping runs first, as a kernel of its own
-    if (a.row_acc || a.row_ts) {
-      const dim3 ig((unsigned)((a.max_len + kAttTile - 1) / kAttTile), (unsigned)a.n_caches);
-      if (EXCH) hipLaunchKernelGGL(exch_importance_kernel, ig, dim3(256), 0, st, a);
-      else hipLaunchKernelGGL(attend_importance_kernel, dim3((unsigned)((a.max_len + 255) / 256), (unsigned)a.n_caches), dim3(256), 0, st, a);
-    }
-    a.row_acc = nullptr;
-    a.row_ts = nullptr;
+    launch_importance<EXCH>(st, a);
     a.row_slabs = n_slabs;
+    const int nsets = gs == 8 ? 1 : 2;   // (as many sets as a slab has heads: up to 4, up to 8)
     const dim3 sgrid(grid.x * (unsigned)(n_slabs / gs), grid.y);
-    const int nsets = gs == 8 ? 1 : 2;
     const size_t lds = attend_mfma_lds_bytes(gs, a.n_q_heads, nsets);
-    for (int off = 0; off < heads_per_slab; off += 4 * nsets) {
-      a.head_off = off;
-      if (gs == 8) hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 8, EXCH, false, 1, true>), sgrid, dim3(256), lds, st, a);
-      else if (gs == 4) hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 4, EXCH, false, 2, true>), sgrid, dim3(256), lds, st, a);
-      else hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 3, EXCH, false, 2, true>), sgrid, dim3(256), lds, st, a);
-    }
+    if (gs == 8) hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 8, EXCH, false, 1, true>), sgrid, dim3(256), lds, st, a);
+    else if (gs == 4) hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 4, EXCH, false, 2, true>), sgrid, dim3(256), lds, st, a);
+    else hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 3, EXCH, false, 2, true>), sgrid, dim3(256), lds, st, a);
     return;
   }
   const int nsets = (n_slabs <= 4 && heads_per_slab > 4) ? 2 : 1;
@@ -1279,7 +1336,11 @@ static void launch_attend_mfma(int n_slabs, int heads_per_slab, dim3 grid, hipSt
     // 4 slabs already fill the wavefronts; pairs of rows gain 5 % on the exchange rows and lose 4 % on float scores
     if (n_slabs == 4 && !EXCH) ti = 1;
   }
-  for (int off = 0; off < heads_per_slab; off += 4 * nsets) {
+  if (heads_per_slab > 4 * nsets && sets_side_by_side(grid)) {
+    launch_importance<EXCH>(st, a);
+    grid.z = (unsigned)((heads_per_slab + 4 * nsets - 1) / (4 * nsets));
+  }
+  for (int off = 0; off < heads_per_slab; off += 4 * nsets * (int)grid.z) {
     a.head_off = off;
     if (off > 0) a.decay = 1.0f;
     if (ti > 1) {
@@ -1362,12 +1423,17 @@ static int attend_tokens_per_block(int n_caches, int64_t max_len) {
 // (24 / 48 / 96) 62.9 / 42.3 / 32.9; 28 x 628 x 36 on 4 (84 / 140 / 280) 48.0 / 35.8 / 32.1; with a block for every
 // unit the prologues cost more than they bring: 17 x 5488 x 12 of 64 (374 / 731) 56.8 / 55.7 / 59.0, 64 x 3000 x 8
 // (768 / 1536) 90.4 / 93.8 / 98.3.
-// passes: blocks of one piece (the vector form's groups of query heads, and its windows).
+// passes: blocks of one piece (groups of query heads, and the vector form's windows).
 static int decode_tokens_per_block(int n_caches, int64_t max_len, int64_t passes) {
   constexpr int64_t kUnits = 256;
   int tpb = attend_tokens_per_block(n_caches, max_len);
   while (tpb > kAttTile && passes * n_caches * ((max_len + tpb - 1) / tpb) < kUnits) tpb >>= 1;
   return tpb;
+}
+// ... blocks of a piece in the matrix-core form: sets of query heads of a slab
+static int64_t mfma_passes(bool eight, int slabs, int heads_per_slab) {
+  const int set = eight || (slabs <= 4 && heads_per_slab > 4) ? 8 : 4;
+  return (heads_per_slab + set - 1) / set;
 }
 static int64_t attend_splits(int tpb, int64_t max_len) { return (max_len + tpb - 1) / tpb; }
 
@@ -1418,7 +1484,7 @@ static int attend_values(const float* scores, const float* head_stats, int64_t s
       if (n_kv_heads % w == 0 && w * lph <= 256 && (window == 0 || (256 % (w * lph) == 0 && 256 % (window * lph) != 0)))
         window = w;
   }
-  const int64_t passes = mfma4 || mfma8 ? 1 : (int64_t)((rep + rp - 1) / rp) * (window ? n_kv_heads / window : 1);
+  const int64_t passes = mfma4 || mfma8 ? mfma_passes(eight, slabs, rep * hps) : (int64_t)((rep + rp - 1) / rp) * (window ? n_kv_heads / window : 1);
   const int tpb = fine ? decode_tokens_per_block(n_caches, max_len, passes) : attend_tokens_per_block(n_caches, max_len);
   const int64_t splits = attend_splits(tpb, max_len);
   if (splits > 65535) return PIKV_ERR_SHAPE;
@@ -1440,9 +1506,7 @@ static int attend_values(const float* scores, const float* head_stats, int64_t s
       else launch_attend_mfma8<PIKV_Q_I8_ASYM>(slabs, hps, grid, st, a);
     } else {
       if (passes > 65535) return PIKV_ERR_SHAPE;
-      if (row_acc || row_ts)
-        hipLaunchKernelGGL(attend_importance_kernel, dim3((unsigned)((max_len + 255) / 256), (unsigned)n_caches),
-                           dim3(256), 0, st, a);
+      launch_importance<false>(st, a);
       a.kv_window = window;
       const dim3 grid((unsigned)splits, (unsigned)n_caches, (unsigned)passes);
 #define PIKV_ATTEND_CASE(S)                                                                        \
@@ -1563,7 +1627,7 @@ extern "C" int pikv_decode_attend(const void* k_codes, const void* k_scale, cons
   const int hps = mfma_heads_per_slab(head_dim, n_kv_heads);   // 128-dimension slabs: one kv head, or 2 / 4 narrow ones
   const int slabs = hps > 0 ? n_kv_heads / hps : 0;
   const bool hk_ok = (slabs >= 1 && slabs <= 8) || (hps == 1 && slabs > 8 && slabs % 8 == 0);
-  const int tpb = decode_tokens_per_block(n_caches, max_len, 1);
+  const int tpb = decode_tokens_per_block(n_caches, max_len, slabs > 0 ? mfma_passes(false, slabs, rep * hps) : 1);
   const int64_t splits = attend_splits(tpb, max_len);
   if ((scheme == PIKV_Q_I4_ASYM || scheme == PIKV_Q_I4_SYM) && group == 32 && rep >= 1 &&
       (rep * hps <= 8 || slabs <= 4) && hk_ok && (q_dtype == PIKV_BF16 || q_dtype == PIKV_F32) && n_caches <= 65535 && splits <= 65535 && (!asym || (k_zero && v_zero))) {

@@ -133,7 +133,10 @@ struct ScoreArgs {
   int tiles_per_block;   // scores_mfma_i8_kernel: consecutive tiles of a block, 1 to kI8TilesPerBlock
 };
 
-template <int SCHEME, int REP, int Q_DT>
+// UN: token steps per batch of loads.  Rows of few lanes take the steps of a tile in fewer, larger strides: with the
+// four of the wide rows a row of 4 lanes had its 64 tokens read and multiplied four times over (58 caches x 3091 tokens
+// x 25 heads of 64, 8-bit: 160 -> 51 us, with five heads to a block instead of one; 24 x 2401 x 71 on one, 4-bit: 424 -> 188).
+template <int SCHEME, int REP, int Q_DT, int UN>
 __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   using Q = QScheme<SCHEME>;
   constexpr int EPL = Q::epl;
@@ -147,6 +150,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   // queries they share are fetched from memory once, not once per piece.  (Any dispatch order gives
   // the same results; a ragged last run keeps the plain order.)
   const int c = blockIdx.y;
+  const int head_off = a.head_off + blockIdx.z * REP;   // first query head of every kv group of this block
   const unsigned run = 8u * (unsigned)a.head_split;
   const unsigned run0 = blockIdx.x / run * run;
   int64_t tile;
@@ -170,7 +174,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   const int D = a.n_kv_heads * a.head_dim;
   const int lanes_per_row = D / EPL;                         // lanes of a whole cached row
   const int lanes_per_head = a.head_dim / EPL;               // power of two
-  const int lanes_blk = kv_blk * lanes_per_head;             // <= 256, divides 256
+  const int lanes_blk = kv_blk * lanes_per_head;             // <= 256
   const int groups_per_row = D / a.group;
   const int tok_per_step = 256 / lanes_blk;
   const int part_blk = threadIdx.x % lanes_blk;
@@ -180,7 +184,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   const int kvh = kv0 + kvl;
   const int d0 = (part % lanes_per_head) * EPL;
 
-  constexpr int UN = 4;  // token steps per batch of loads
+  const bool slot = tok_in_step < tok_per_step;              // threads beyond the last whole row stage nothing
   const int batch = tok_per_step * UN;  // tokens of the tile covered by one batch
 
   // Two register sets: the loads of the next batch are in flight while the current one is
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   float qsum[REP];
 #pragma unroll
   for (int r = 0; r < REP; ++r) {
-    const int hq = kvh * a.rep + a.head_off + r;
+    const int hq = kvh * a.rep + head_off + r;
     load_as_float<Q_DT, EPL>(a.q, ((int64_t)c * a.n_q_heads + hq) * a.head_dim + d0, qv[r]);
     float sacc = 0.f;
 #pragma unroll
@@ -241,7 +245,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
         for (int j = 0; j < EPL; ++j) d = fmaf(qv[r][j], cf[j], d);
         d = (d - zu * qsum[r]) * t.sc[u];
         d = group_sum_dpp(d, lanes_per_head);
-        if ((part % lanes_per_head) == 0 && tl < kTile)
+        if ((part % lanes_per_head) == 0 && tl < kTile && slot)
           stage[(kvl * REP + r) * kTile + tl] = ok ? d * a.scale_qk : -__builtin_inff();
       }
     }
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   const int wave = threadIdx.x >> 6;
   const int hq_blk = kv_blk * REP;
   for (int hl = wave; hl < hq_blk; hl += 4) {
-    const int hq = (kv0 + hl / REP) * a.rep + a.head_off + hl % REP;
+    const int hq = (kv0 + hl / REP) * a.rep + head_off + hl % REP;
     const float s = stage[hl * kTile + lane];
     const bool ok = n0 + lane < len;
     if (ok) a.scores[((int64_t)c * a.n_q_heads + hq) * a.score_stride + n0 + lane] = s;
@@ -580,15 +584,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NKV * NSET 
   uint16_t* zmeta = smeta + kTile * meta_stride;
 
   const int c = blockIdx.y;
+  const int head_off = SPLIT ? 0 : blockIdx.z * 4 * NSET;   // first query head of every slab of this block
   const int len = a.fill[c] < a.max_len ? a.fill[c] : a.max_len;
   const int n_groups = SPLIT ? a.row_slabs / a.n_kv_heads : 1;
   const int64_t tile0 = (int64_t)(SPLIT ? blockIdx.x / n_groups : blockIdx.x) * kGqaTilesPerBlock;
   const int64_t tok0 = tile0 * kTile;
   if (tok0 >= len) return;  // uniform for the block
-  // query heads per slab; a launch serves heads a.head_off .. a.head_off + rep - 1 of every slab, rep <= 4 NSET
-  // (more than 8 heads per slab: two launches; split rows are launched with head_off = 0 only)
+  // query heads per slab; a block serves heads head_off .. head_off + rep - 1 of every slab, rep <= 4 NSET
+  // (more than 8 heads per slab: grid z; split rows have no more)
   const int rep_all = a.n_q_heads / (SPLIT ? a.row_slabs : a.n_kv_heads);
-  const int rep = rep_all - a.head_off < 4 * NSET ? rep_all - a.head_off : 4 * NSET;
+  const int rep = rep_all - head_off < 4 * NSET ? rep_all - head_off : 4 * NSET;
   // Heads narrower than 128: a.n_kv_heads counts 128-dimension slabs of the cached row, each the
   // stored bytes of hps = 128 / head_dim neighbouring kv heads, and the rep query heads of a slab
   // are the heads of those kv heads, rep1 each, in order.  Query head r of a slab belongs to kv
@@ -600,7 +605,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NKV * NSET 
   const int gshift = head_dim == 64 ? 1 : 0;          // log2 of a narrow head's groups of 32
   const int rep1 = head_dim == 64 ? rep_all >> 1 : rep_all >> 2;
   auto owns = [&](int r, int gq) {                    // group gq of the slab belongs to the kv head of the launch's query head r
-    const int ra = r + a.head_off;                    // ... which is head ra of the slab
+    const int ra = r + head_off;                    // ... which is head ra of the slab
     return !NARROW || (gq >> gshift) == (ra >= rep1) + (ra >= 2 * rep1) + (ra >= 3 * rep1);
   };
   auto group_in_head = [&](int gq) { return NARROW ? gq & ((1 << gshift) - 1) : gq; };
@@ -611,8 +616,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NKV * NSET 
   const int nl = lane & 15;
   const int rg = lane >> 4;
   // (the queries of this block's slabs: heads kv_off * rep ...)
-  const uint16_t* qbase = reinterpret_cast<const uint16_t*>(a.q) + ((int64_t)c * a.n_q_heads + kv_off * rep_all + a.head_off) * head_dim;
-  const float* qfbase = reinterpret_cast<const float*>(a.q) + ((int64_t)c * a.n_q_heads + kv_off * rep_all + a.head_off) * head_dim;
+  const uint16_t* qbase = reinterpret_cast<const uint16_t*>(a.q) + ((int64_t)c * a.n_q_heads + kv_off * rep_all + head_off) * head_dim;
+  const float* qfbase = reinterpret_cast<const float*>(a.q) + ((int64_t)c * a.n_q_heads + kv_off * rep_all + head_off) * head_dim;
   // bf16 bits of limb `set` of a float32 query element
   auto limb_bits = [](float v, int set) -> uint32_t { return bf16_limb_bits(v, set); };
   const int64_t base_row = a.row_base[c];
@@ -781,8 +786,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NKV * NSET 
     }
     __syncthreads();
 
-    if constexpr (EXCH) tile_stats_exchange<true, SL>(a, stage, c, tile, n0, len, wave, rg, nl, rep, kv_off * rep_all + a.head_off, rep_all);
-    else tile_stats_store<true, SL>(a, stage, c, tile, n0, len, wave, rg, nl, rep, kv_off * rep_all + a.head_off, rep_all);
+    if constexpr (EXCH) tile_stats_exchange<true, SL>(a, stage, c, tile, n0, len, wave, rg, nl, rep, kv_off * rep_all + head_off, rep_all);
+    else tile_stats_store<true, SL>(a, stage, c, tile, n0, len, wave, rg, nl, rep, kv_off * rep_all + head_off, rep_all);
     __syncthreads();  // stage and the metadata rows are reused by the next tile
     return true;
   };
@@ -830,13 +835,14 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
   float* stage = i8_lds + kI8QsFloats;  // [q head][token in tile]
 
   const int c = blockIdx.y;
+  const int head_off = blockIdx.z * 16;   // first query head of every kv head of this block
   const int len = a.fill[c] < a.max_len ? a.fill[c] : a.max_len;
   const int64_t tile0 = (int64_t)blockIdx.x * a.tiles_per_block;
   if (tile0 * kTile >= len) return;  // uniform for the block
-  // a launch serves heads a.head_off .. a.head_off + rep - 1 of every kv head (more than 16 per kv head: several
+  // a block serves heads head_off .. head_off + rep - 1 of every kv head (more than 16 per kv head: grid z
   // launches, heads of 128 only); the staged rows are those heads, rep per kv head
   const int rep_all = a.n_q_heads / a.n_kv_heads;
-  const int rep = rep_all - a.head_off < 16 ? rep_all - a.head_off : 16;
+  const int rep = rep_all - head_off < 16 ? rep_all - head_off : 16;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int nl = lane & 15;   // token of a slice (B, C column) / query head (A row)
@@ -884,7 +890,7 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
       uint2 qd = make_uint2(0, 0);
       const int ds = 64 * (ks >> 2) + 16 * rg + 4 * (ks & 3);   // dimension inside the slab
       if (on && (HPS == 1 || ds / (128 / HPS) == hh_a)) {
-        const int64_t qo = (int64_t)(g * rep_all + a.head_off + (nl >> RSH)) * (128 / HPS) + (ds - hh_a * (128 / HPS));
+        const int64_t qo = (int64_t)(g * rep_all + head_off + (nl >> RSH)) * (128 / HPS) + (ds - hh_a * (128 / HPS));
         if constexpr (QF32) {
           float f4[4];
           load_as_float<PIKV_F32, 4>(qfbase, qo, f4);
@@ -1018,7 +1024,7 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
         const int64_t tile = tile0 + round * tpr + k;
         if (tile * kTile < len) {  // uniform
           if (rep == rep_all) tile_stats_store<false>(a, stage + k * a.n_q_heads * kTile, c, tile, tile * kTile, len, wave, rg, nl);
-          else tile_stats_store<true, 0>(a, stage + k * a.n_q_heads * kTile, c, tile, tile * kTile, len, wave, rg, nl, rep, a.head_off, rep_all);
+          else tile_stats_store<true, 0>(a, stage + k * a.n_q_heads * kTile, c, tile, tile * kTile, len, wave, rg, nl, rep, head_off, rep_all);
         }
       }
       __syncthreads();  // the staging areas are reused by the next round
@@ -1037,7 +1043,7 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
     }
     __syncthreads();
     if (rep == rep_all) tile_stats_store<false>(a, stage, c, tile, n0, len, wave, rg, nl);
-    else tile_stats_store<true, 0>(a, stage, c, tile, n0, len, wave, rg, nl, rep, a.head_off, rep_all);
+    else tile_stats_store<true, 0>(a, stage, c, tile, n0, len, wave, rg, nl, rep, head_off, rep_all);
     __syncthreads();  // stage is reused by the next tile
   }
 }
@@ -1061,9 +1067,10 @@ static void launch_i8_mfma_q(const ScoreArgs& a0, int n_caches, int64_t n_tiles,
   // 32 blocks of 4 tiles 39.8 us, 128 blocks of one 13.3 us
   const int fewest = a.n_kv_heads <= 2 ? kI8TilesPerBlock / a.n_kv_heads : 1;
   a.tiles_per_block = kI8TilesPerBlock;
-  while (a.tiles_per_block > fewest && (n_tiles + a.tiles_per_block - 1) / a.tiles_per_block * n_caches < 512)
+  const int sets = (a.n_q_heads / a.n_kv_heads + 15) / 16;   // blocks of 16 query heads per kv head (slab)
+  while (a.tiles_per_block > fewest && (n_tiles + a.tiles_per_block - 1) / a.tiles_per_block * n_caches * sets < 512)
     a.tiles_per_block >>= 1;
-  const dim3 grid((unsigned)((n_tiles + a.tiles_per_block - 1) / a.tiles_per_block), (unsigned)n_caches);
+  const dim3 grid((unsigned)((n_tiles + a.tiles_per_block - 1) / a.tiles_per_block), (unsigned)n_caches, (unsigned)sets);
   if (a.n_kv_heads <= 4)
     hipLaunchKernelGGL((scores_mfma_i8_kernel<SCHEME, 1, HPS, QF32>), grid, dim3(256), lds, st, a);
   else if (a.n_kv_heads <= 8)
@@ -1084,11 +1091,11 @@ static int launch_gqa_slabs(const ScoreArgs& a0, int n_caches, int64_t n_tiles, 
   const int rep = a.n_q_heads / a.n_kv_heads;
   const int nset = rep <= 4 ? 1 : 2;
   const size_t lds = gqa_lds_bytes(a.n_kv_heads, nset, qf32 ? 2 * nset : nset);   // float32 queries: a copy of the A operands per limb
-  // more than 8 query heads per slab (rows of up to 4 slabs): launches of eight heads each over the same codes
+  // more than 8 query heads per slab (rows of up to 4 slabs): eight heads per block, grid z
   if (rep > 8 && a.n_kv_heads > 4) return PIKV_ERR_UNSUPPORTED;
   if (lds > 64 * 1024 || a.n_kv_heads > (qf32 ? 8 : kGqaMaxKvHeads)) return PIKV_ERR_UNSUPPORTED;
-  for (a.head_off = 0; a.head_off < rep; a.head_off += 4 * nset) {
-  const dim3 grid((unsigned)((n_tiles + kGqaTilesPerBlock - 1) / kGqaTilesPerBlock), (unsigned)n_caches);
+  const dim3 grid((unsigned)((n_tiles + kGqaTilesPerBlock - 1) / kGqaTilesPerBlock), (unsigned)n_caches,
+                  (unsigned)((rep + 4 * nset - 1) / (4 * nset)));
   // (rows of 1 or 2 slabs have a kernel of their own: fewer registers, 8 instead of 6 blocks per compute unit,
   // and with 5 KB tiles the bytes in flight are what bounds them - 1 kv head x 4 q heads 61.3 -> 52.1 us,
   // 2 x 8: 83.6 -> 76.8 us at 64 caches x 32768 tokens)
@@ -1123,7 +1130,6 @@ static int launch_gqa_slabs(const ScoreArgs& a0, int n_caches, int64_t n_tiles, 
       hipLaunchKernelGGL((scores_mfma_i4_gqa_kernel<SCHEME, 4, 2, EXCH, NARROW>), grid, dim3(256), lds, st, a);
     else
       hipLaunchKernelGGL((scores_mfma_i4_gqa_kernel<SCHEME, 8, 2, EXCH, NARROW>), grid, dim3(256), lds, st, a);
-  }
   }
   return PIKV_OK;
 }
@@ -1368,25 +1374,36 @@ template <int SCHEME, int REP>
 static void launch_scores_q(dim3 grid, hipStream_t st, int q_dtype, const ScoreArgs& a) {
   // staged scores of the block's query heads: the fewer, the more blocks share a compute unit
   const size_t lds = (size_t)(a.n_kv_heads / a.head_split) * REP * kTile * sizeof(float);
-  if (q_dtype == PIKV_BF16)
-    hipLaunchKernelGGL((scores_kernel<SCHEME, REP, PIKV_BF16>), grid, dim3(256), lds, st, a);
-  else
-    hipLaunchKernelGGL((scores_kernel<SCHEME, REP, PIKV_F32>), grid, dim3(256), lds, st, a);
+  // steps per batch: as many as waste no more of the tile's last batch than fewer would
+  const int tps = 256 / (a.n_kv_heads / a.head_split * (a.head_dim / QScheme<SCHEME>::epl));
+  auto covered = [tps](int un) { return (kTile + tps * un - 1) / (tps * un) * tps * un; };
+  const int un = covered(4) <= covered(2) && covered(4) <= covered(1) ? 4 : covered(2) <= covered(1) ? 2 : 1;
+#define PIKV_SCORES_UN(U)                                                                                       \
+  if (un == U) {                                                                                                \
+    if (q_dtype == PIKV_BF16)                                                                                   \
+      hipLaunchKernelGGL((scores_kernel<SCHEME, REP, PIKV_BF16, U>), grid, dim3(256), lds, st, a);              \
+    else                                                                                                        \
+      hipLaunchKernelGGL((scores_kernel<SCHEME, REP, PIKV_F32, U>), grid, dim3(256), lds, st, a);               \
+  }
+  PIKV_SCORES_UN(4)
+  PIKV_SCORES_UN(2)
+  PIKV_SCORES_UN(1)
+#undef PIKV_SCORES_UN
 }
 
 template <int SCHEME>
 static int launch_scores(int rep, dim3 grid, hipStream_t st, int q_dtype, ScoreArgs a) {
   // The kernel is compiled for 8, 4, 2 and 1 query heads per kv head; any other ratio is served
-  // as the sum of those (7 = 4 + 2 + 1), one launch each over the same codes.
+  // as the sum of those (15 = 8 + 4 + 2 + 1), one launch each over the same codes, the eights side by side.
   a.rep = rep;
-  for (int off = 0; off < rep;) {
-    const int left = rep - off;
-    a.head_off = off;
-    if (left >= 8) { launch_scores_q<SCHEME, 8>(grid, st, q_dtype, a); off += 8; }
-    else if (left >= 4) { launch_scores_q<SCHEME, 4>(grid, st, q_dtype, a); off += 4; }
-    else if (left >= 2) { launch_scores_q<SCHEME, 2>(grid, st, q_dtype, a); off += 2; }
-    else { launch_scores_q<SCHEME, 1>(grid, st, q_dtype, a); off += 1; }
+  a.head_off = 0;
+  if (rep >= 8) {
+    launch_scores_q<SCHEME, 8>(dim3(grid.x, grid.y, (unsigned)(rep / 8)), st, q_dtype, a);
+    a.head_off = rep / 8 * 8;
   }
+  if (rep & 4) { launch_scores_q<SCHEME, 4>(grid, st, q_dtype, a); a.head_off += 4; }
+  if (rep & 2) { launch_scores_q<SCHEME, 2>(grid, st, q_dtype, a); a.head_off += 2; }
+  if (rep & 1) launch_scores_q<SCHEME, 1>(grid, st, q_dtype, a);
   return PIKV_OK;
 }
 
@@ -1531,28 +1548,23 @@ extern "C" int pikv_gather_dequant_scores(const void* k_codes, const void* k_sca
   // (heads of 64 or 32 dimensions as 128-dimension slabs of two or four neighbouring kv heads)
   // (float32 queries as two bf16 limbs, two operand rows per head: up to 8 heads per slab)
   const bool qf32 = q_dtype == PIKV_F32;
-  // (more than 16 bf16 query heads per kv head of 128 on rows of up to 4 kv heads: launches of 16 heads each)
+  // (more than 16 bf16 query heads per kv head of 128 on rows of up to 4 kv heads: 16 heads per block, grid z)
   const bool many = hps == 1 && !qf32 && n_kv_heads <= 4 && rep > 16;
   if (eight && hps > 0 && group % head_dim == 0 && rep >= 2 && (rep * hps <= (qf32 ? 8 : 16) || many) && n_kv_heads / hps <= 16 &&
       i8_mfma_lds_bytes(n_kv_heads / hps, n_q_heads) <= kI8MfmaMaxLds) {
     ScoreArgs as = a;
     as.n_kv_heads = n_kv_heads / hps;
     const bool sym = scheme == PIKV_Q_I8_SYM;
-    if (many) {
-      for (as.head_off = 0; as.head_off < rep; as.head_off += 16)
-        sym ? launch_i8_mfma<PIKV_Q_I8_SYM>(as, n_caches, n_tiles, st, false) : launch_i8_mfma<PIKV_Q_I8_ASYM>(as, n_caches, n_tiles, st, false);
-    } else if (hps == 1) sym ? launch_i8_mfma<PIKV_Q_I8_SYM>(as, n_caches, n_tiles, st, qf32) : launch_i8_mfma<PIKV_Q_I8_ASYM>(as, n_caches, n_tiles, st, qf32);
+    if (hps == 1) sym ? launch_i8_mfma<PIKV_Q_I8_SYM>(as, n_caches, n_tiles, st, qf32) : launch_i8_mfma<PIKV_Q_I8_ASYM>(as, n_caches, n_tiles, st, qf32);
     else if (hps == 2) sym ? launch_i8_mfma<PIKV_Q_I8_SYM, 2>(as, n_caches, n_tiles, st, qf32) : launch_i8_mfma<PIKV_Q_I8_ASYM, 2>(as, n_caches, n_tiles, st, qf32);
     else sym ? launch_i8_mfma<PIKV_Q_I8_SYM, 4>(as, n_caches, n_tiles, st, qf32) : launch_i8_mfma<PIKV_Q_I8_ASYM, 4>(as, n_caches, n_tiles, st, qf32);
     PIKV_CHECK_LAUNCH();
     return PIKV_OK;
   }
-  // The blocks of a tile own a power-of-two number of kv heads each (a block's lanes per token must
-  // divide 256): 12 kv heads are three blocks of four.  Rows wider than 512 bytes are split further:
-  // short-lived blocks of 64 tokens x 512 bytes keep more loads in flight per compute unit than
-  // fewer, longer ones.
-  a.head_split = n_kv_heads / (n_kv_heads & -n_kv_heads);
-  while (lanes_per_row / a.head_split > 32 && n_kv_heads % (a.head_split * 2) == 0) a.head_split *= 2;
+  // The blocks of a tile own the same number of kv heads each, up to 512 bytes of a row: short-lived
+  // blocks of 64 tokens x 512 bytes keep more loads in flight per compute unit than fewer, longer ones.
+  // (25 kv heads are five blocks of five, the 256 threads twelve rows and 16 idle.)
+  while (a.head_split < n_kv_heads && (n_kv_heads % a.head_split != 0 || lanes_per_row / a.head_split > 32)) ++a.head_split;
   if (lanes_per_row / a.head_split > 256) return PIKV_ERR_UNSUPPORTED;
   if (n_tiles * a.head_split > 0x7fffffffLL) return PIKV_ERR_SHAPE;
   const dim3 vgrid((unsigned)(n_tiles * a.head_split), (unsigned)n_caches);

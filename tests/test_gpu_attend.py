@@ -370,11 +370,14 @@ def test_attend_block_lengths(dev, n_caches, length, scheme, heads, hq):
     (O.Q_I8_ASYM, 128, 3, 30, 128, "bf16"),  # float scores, 8-bit matrix-core form
     (O.Q_I8_SYM, 256, 2, 4, 256, "bf16"),    # vector form
     (O.Q_I4_SYM, 64, 1, 7, 64, "f32"),       # ... two lanes to a row
+    (O.Q_I8_ASYM, 64, 5, 5, 64, "bf16"),     # ... twenty, 256 threads hold twelve rows
+    (O.Q_I4_SYM, 32, 2, 40, 128, "bf16"),    # sets of query heads side by side, exchange format
+    (O.Q_I8_SYM, 128, 1, 20, 128, "bf16"),   # ... float scores
 ])
-@pytest.mark.parametrize("n_caches,longest", [(20, 1700), (33, 1700), (90, 129), (3, 65)])
+@pytest.mark.parametrize("n_caches,longest", [(20, 1700), (33, 1700), (90, 129), (3, 65), (130, 1025)])
 def test_decode_attend_pieces(dev, n_caches, longest, scheme, group, heads, hq, dh, qdtype):
-    """Pieces of 128, 256, 128 and 64 cached tokens per block of the decode read, lengths around their edges, against
-    the three public steps (pieces of 256 or more).  Both add up at most 1700 products of 24 bits whose
+    """Pieces of 128, 256, 128, 64 and 256 (sets one after the other) cached tokens per block of the decode read, lengths
+    around their edges, against the three public steps (pieces of 256 or more).  Both add up at most 1700 products of 24 bits whose
     probabilities sum to one, in another order, from scores that are equal or differ by a rounding of the
     largest, below 64: 2 x 1700 x 2^-24 and 64 x 2^-23 of the largest value row element."""
     r = rng(n_caches + heads)
@@ -393,6 +396,34 @@ def test_decode_attend_pieces(dev, n_caches, longest, scheme, group, heads, hq, 
     v_max = np.abs(O.dequantize_groups(ref.v_codes[rows], ref.v_scale[rows], ref.v_zero[rows], group)).max()
     assert np.abs(out - want).max() <= (2 * 1700 * 2.0 ** -24 + 64 * 2.0 ** -23) * v_max
     np.testing.assert_allclose(acc, np_of(pool.acc), rtol=hq * 2.0 ** -22 + 64 * 2.0 ** -23, atol=1e-12)
+
+
+@pytest.mark.parametrize("scheme,group,heads,hq,dh", [
+    (O.Q_I8_SYM, 64, 25, 25, 64),    # five blocks of 20 lanes: twelve rows per step, 16 threads without one
+    (O.Q_I4_SYM, 64, 1, 71, 64),     # 2 lanes: a tile in one step, eight sets of eight heads side by side
+    (O.Q_I8_ASYM, 64, 1, 13, 64),    # 4 lanes
+    (O.Q_I4_ASYM, 64, 7, 21, 64),    # 14 lanes, 18 rows per step
+    (O.Q_I8_SYM, 32, 3, 6, 32),      # 6 lanes, 42 rows
+    (O.Q_I4_ASYM, 32, 9, 9, 32),     # 9 lanes, 28 rows
+    (O.Q_I8_ASYM, 64, 8, 8, 64),     # 32 lanes, 8 rows
+])
+@pytest.mark.parametrize("qdtype", ["f32", "bf16"])
+def test_scores_lane_counts(dev, scheme, group, heads, hq, dh, qdtype):
+    """Vector-form scores over rows of any lane count.  A score sums dh products q * code and takes off the zero point
+    times the sum of q, each with a rounding of 2^-24: with codes and zero points up to four times the
+    largest dequantised element in units of the scale, within (dh + 8) * 2^-24 * 4 * max |k| * sum |q| / sqrt(dh)."""
+    r = rng(heads * 3 + dh)
+    lens = [257, 64, 63, 1, 0, 129]
+    pool, ref = _fill_pool(dev, r, [300] * len(lens), lens, heads, dh, group, scheme)
+    q = O.bf16_round(r.standard_normal((len(lens), hq, dh)).astype(np.float32))
+    sc = np_of(pool.scores(to_dev(q, dev, qdtype), hq)[0])
+    for c, L in enumerate(lens):
+        if L:
+            rows = ref.valid_rows(c)[:L]
+            k_hat = O.dequantize_groups(ref.k_codes[rows], ref.k_scale[rows], ref.k_zero[rows], group)
+            want = O.attention_scores(q[c], k_hat, heads, 1.0 / np.sqrt(dh))
+            tol = (dh + 8) * 2.0 ** -24 * 4 * np.abs(k_hat).max() * np.abs(q[c]).sum(-1).max() / np.sqrt(dh)
+            assert np.abs(sc[c, :, :L] - want).max() <= tol, c
 
 
 def _decode_reference(ref, q, lens_now, acc_before, heads, group, scale_qk, decay):
