@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   // queries they share are fetched from memory once, not once per piece.  (Any dispatch order gives
   // the same results; a ragged last run keeps the plain order.)
   const int c = blockIdx.y;
-  const int head_off = a.head_off + blockIdx.z * REP;   // first query head of every kv group of this block
+  const int head_off = REP == 8 ? blockIdx.z * REP : a.head_off;   // first query head of every kv group of this block
   const unsigned run = 8u * (unsigned)a.head_split;
   const unsigned run0 = blockIdx.x / run * run;
   int64_t tile;
@@ -179,8 +179,9 @@ __global__ __launch_bounds__(256) void scores_kernel(ScoreArgs a) {
   const int tok_per_step = 256 / lanes_blk;
   const int part_blk = threadIdx.x % lanes_blk;
   const int part = kv0 * lanes_per_head + part_blk;          // fixed (kv head, slice) of this lane
-  // (the threads beyond the last whole row: a token past the tile, read from its last row and not staged)
-  const int tok_in_step = (int)threadIdx.x < tok_per_step * lanes_blk ? threadIdx.x / lanes_blk : kTile;
+  // (the threads beyond the last whole row, which UN = 4 does not have: a token past the tile, read from its last row
+  // and not staged)
+  const int tok_in_step = UN == 4 || (int)threadIdx.x < tok_per_step * lanes_blk ? threadIdx.x / lanes_blk : kTile;
   const int kvl = part_blk / lanes_per_head;                 // kv head inside the block
   const int kvh = kv0 + kvl;
   const int d0 = (part % lanes_per_head) * EPL;
@@ -1408,9 +1409,9 @@ static void launch_scores_q(dim3 grid, hipStream_t st, int q_dtype, const ScoreA
   // staged scores of the block's query heads: the fewer, the more blocks share a compute unit
   const size_t lds = (size_t)(a.n_kv_heads / a.head_split) * REP * kTile * sizeof(float);
   // steps per batch: as many as waste no more of the tile's last batch than fewer would
-  const int tps = 256 / (a.n_kv_heads / a.head_split * (a.head_dim / QScheme<SCHEME>::epl));
+  const int lanes = a.n_kv_heads / a.head_split * (a.head_dim / QScheme<SCHEME>::epl), tps = 256 / lanes;
   auto covered = [tps](int un) { return (kTile + tps * un - 1) / (tps * un) * tps * un; };
-  const int un = covered(4) <= covered(2) && covered(4) <= covered(1) ? 4 : covered(2) <= covered(1) ? 2 : 1;
+  const int un = 256 % lanes == 0 && covered(4) <= covered(2) && covered(4) <= covered(1) ? 4 : covered(2) <= covered(1) ? 2 : 1;
 #define PIKV_SCORES_UN(U)                                                                                       \
   if (un == U) {                                                                                                \
     if (q_dtype == PIKV_BF16)                                                                                   \
