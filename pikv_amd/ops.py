@@ -953,10 +953,11 @@ class CachePool:
     def compact(self, extra_planes: Sequence[torch.Tensor] = ()):
         """Move survivors (keep_index/new_len) to the front of every plane and
         set fill = new_len."""
-        ps = self.planes() + [_need(p, "extra plane") for p in extra_planes]
+        extra = [_need(p, "extra plane") for p in extra_planes]      # (an iterator gives them once)
+        ps = self.planes() + extra
         if len(ps) > N.MAX_PLANES:
             raise ValueError(f"at most {N.MAX_PLANES} planes")
-        rbs = self._row_bytes + [math.prod(p.shape[1:]) * p.element_size() for p in extra_planes]
+        rbs = self._row_bytes + [math.prod(p.shape[1:]) * p.element_size() for p in extra]
         N.call("pikv_compact_rows", ps, rbs, len(ps), self.row_base, self.keep_index,
                self.new_len, self.fill, self.n_caches, _stream())
 

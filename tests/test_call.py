@@ -66,3 +66,20 @@ def test_ordinary_tensor():
     seen = []
     torch.func.vmap(lambda x: seen.append(dense.ordinary_tensor(x, cpu)) or x)(torch.zeros(2, 3))
     assert seen == [False]
+
+
+@pytest.mark.parametrize("kind", [list, tuple, iter])
+def test_every_plane_of_a_compaction_has_its_row_bytes(monkeypatch, kind):
+    """The library reads as many widths as there are planes, whatever the extra ones come in."""
+    pool = object.__new__(ops.CachePool)
+    pool.k_codes, pool.k_scale, pool.acc, pool.ts = torch.zeros(4, 64, dtype=torch.int8), torch.zeros(4, 2), torch.zeros(4), torch.zeros(4)
+    pool.k_zero = pool.v_codes = pool.v_scale = pool.v_zero = None
+    pool.row_base = pool.keep_index = pool.new_len = pool.fill = None
+    pool.n_caches, pool._row_bytes = 1, [64, 8, 4, 4]
+    seen = []
+    monkeypatch.setattr(ops, "_need", lambda t, name: t)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(N, "call", lambda name, *args: seen.append(args))
+    pool.compact(extra_planes=kind([torch.zeros(4, 3), torch.zeros(4, dtype=torch.int64)]))
+    planes, widths, n = seen[0][:3]
+    assert len(planes) == len(widths) == n == 6 and widths == [64, 8, 4, 4, 12, 8]
