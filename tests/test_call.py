@@ -1,4 +1,6 @@
 """CPU checks of the typed Python entry (csrc/call.cpp): conversions, what it refuses, and the tensor checks beside it."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -39,6 +41,54 @@ def test_refusals():
         f.pikv_linear_tiled(64, 4, 64, 1, [64] * 5000, [64], [4], [64], None)
     with pytest.raises(N.PiKVNativeError):
         N.call("pikv_h2o_budget", None, 1, 0.1, 0.1, None, None, None)
+
+
+class _Tensor:
+    def __init__(self, is_cuda):
+        self.is_cuda, self.asked = is_cuda, 0
+
+    def data_ptr(self):
+        self.asked += 1
+        return 64
+
+
+@pytest.mark.parametrize("name", sorted(set(N.SIGNATURES) - {"pikv_status_string"}))
+def test_pointer_parameters_take_what_they_are(name):
+    """A pointer that a kernel reads never comes from host memory, a host array never from the GPU.  (No call here gets as far
+    as the library.)"""
+    _, types = N.SIGNATURES[name]
+    plain = [0.0 if t in (C.c_float, C.c_double) else 0 if t is not C.c_void_p and not hasattr(t, "contents") else None
+             for t in types]
+    for i, t in enumerate(types):
+        if t is C.c_void_p:
+            wrong = [[64], (64,), np.zeros(4, np.float32), np.int64(64), (C.c_float * 4)(), b"abcd", bytearray(8),
+                     torch.zeros(4), _Tensor(False)]
+        elif hasattr(t, "contents"):
+            numbers = t._type_ is not C.c_void_p
+            wrong = [64, _Tensor(True), torch.zeros(4), np.zeros(4, np.float16), np.zeros((2, 2), np.int32), np.int64(64),
+                     (C.c_double * 2)(), b"abcd", np.zeros(8, np.int64)[::2]]
+            wrong += [C.c_void_p(64), [None], [_Tensor(True)], np.zeros(4, np.int32 if t._type_ is C.c_float else np.float32)] if numbers else [
+                [torch.zeros(4)], [np.zeros(4)], [[64]], np.zeros(4, np.int32)]
+        else:
+            continue
+        for w in wrong:
+            with pytest.raises((TypeError, ValueError)):       # (numpy: a strided array gives no plain buffer, a ValueError)
+                getattr(N.entries(), name)(*plain[:i], w, *plain[i + 1:])
+
+
+def test_pointer_values():
+    f = N.entries()
+    # (n_caches = 0 is refused behind the null pointers: -1 null, -2 a bad size)
+    for p, status in ((None, -1), (C.c_void_p(None), -1), (C.POINTER(C.c_int32)(), -1), (64, -2), (C.c_void_p(64), -2),
+                      (C.cast(64, C.POINTER(C.c_int32)), -2), (_Tensor(True), -2)):
+        assert f.pikv_h2o_budget(p, 0, 0.1, 0.1, 64, 64, None) == status, p
+        if not isinstance(p, _Tensor):
+            assert N.lib().pikv_h2o_budget(p, 0, 0.1, 0.1, 64, 64, None) == status
+    # host arrays of ctypes, as the ctypes signatures take them: the width 0 is found behind them
+    for widths in ((C.c_int32 * 2)(32, 0), C.cast((C.c_int32 * 2)(32, 0), C.POINTER(C.c_int32)), np.array([32, 0], np.int32)):
+        w = (C.c_void_p * 2)(64, 64)
+        assert f.pikv_linear_group(64, 4, 128, 2, w, w, widths, [0, 1], 0, None, None, None, w, None, 0, None) == -2
+    assert f.pikv_linear_group(64, 4, 128, 1, [64], [64], C.byref(C.c_int32(0)), [0], 0, None, None, None, [64], None, 0, None) == -2
 
 
 def test_need():
