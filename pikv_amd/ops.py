@@ -461,6 +461,7 @@ def value_lora(mean, lora_a, lora_b, scaling):
     """mean[e] + ((mean[e] lora_a[e]) lora_b[e]) * scaling[e] for mean [E, H] float32 and lists of E."""
     mean = _need(mean, "mean", dtype=torch.float32, ndim=2)
     E, H = mean.shape
+    lora_a, lora_b = list(lora_a), list(lora_b)          # (a stacked tensor or a ParameterList, too)
     rank = lora_a[0].shape[1]
     if not len(lora_a) == len(lora_b) == len(scaling) == E:
         raise ValueError("one lora_a, lora_b and scaling per row of mean")
@@ -478,6 +479,7 @@ def expert_combine(dense, lora, scaling, add, weights, lora_b=None):
     """(outs [E, T, H], mix [T, H]): outs[e] = relu(dense[e] + lora[e] * scaling[e]) + add[e], mix the sum over e, in
     order, of outs[e][t] * weights[t][e].  dense, lora: lists of E (at most 20) tensors [T, H]; add [E, H]; weights
     [T, E]; float32.  With lora_b (E tensors [rank, H]) lora[e] is [T, rank], and its product with lora_b[e] is taken."""
+    dense, lora, lora_b = list(dense), list(lora), None if lora_b is None else list(lora_b)     # (stacked tensors, too)
     E, (T, H) = len(dense), dense[0].shape
     if not 1 <= E == len(lora) == len(scaling) or H % 4:
         raise ValueError("one lora and scaling per expert, and a width that is a multiple of 4")

@@ -133,3 +133,21 @@ def test_every_plane_of_a_compaction_has_its_row_bytes(monkeypatch, kind):
     pool.compact(extra_planes=kind([torch.zeros(4, 3), torch.zeros(4, dtype=torch.int64)]))
     planes, widths, n = seen[0][:3]
     assert len(planes) == len(widths) == n == 6 and widths == [64, 8, 4, 4, 12, 8]
+
+
+@pytest.mark.parametrize("kind", [list, tuple, torch.stack, torch.nn.ParameterList])
+def test_experts_factors_come_in_any_sequence(monkeypatch, kind):
+    """What holds the experts' tensors becomes a host array of their addresses, not itself an address."""
+    seen = []
+    monkeypatch.setattr(ops, "_need", lambda t, name, **kw: t)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(N, "call", lambda name, *args: seen.append((name, args)))
+    a, b, d = ([torch.ones(s) for _ in range(3)] for s in ((8, 2), (2, 8), (5, 8)))
+    t = [torch.ones(5, 2) for _ in range(3)]
+    ops.value_lora(torch.ones(3, 8), kind(a), kind(b), [1.0] * 3)
+    ops.expert_combine(kind(d), kind(d), [1.0] * 3, torch.ones(3, 8), torch.ones(5, 3))
+    ops.expert_combine(kind(d), kind(t), [1.0] * 3, torch.ones(3, 8), torch.ones(5, 3), lora_b=kind(b))
+    assert [name for name, _ in seen] == ["pikv_value_lora", "pikv_expert_combine", "pikv_expert_combine_factors"]
+    for (_, args), arrays in zip(seen, ((4, 5), (0, 1), (0, 1, 2))):
+        for i in arrays:
+            assert type(args[i]) in (list, tuple) and [type(x) in (torch.Tensor, torch.nn.Parameter) for x in args[i]] == [True] * 3
