@@ -126,9 +126,17 @@ def check(code: int, what: str) -> None:
 
 try:
     from . import _call
-except ImportError:                      # not built: whoever needs it is told
-    _call = None
+except ImportError as e:                 # not built, or it does not load: whoever needs it is told
+    _call, _call_error = None, e
 _entries = None
+
+
+def entry_module():
+    """The extension module of csrc/call.cpp."""
+    if _call is None:
+        raise PiKVNativeError(f"pikv_amd/_call is not built or does not load ({_call_error}): build it with "
+                              "`python -m pikv_amd.build`") from _call_error
+    return _call
 
 
 def entries():
@@ -139,10 +147,9 @@ def entries():
         lib()
         with _lock:
             if _entries is None:
-                if _call is None:
-                    raise PiKVNativeError("pikv_amd/_call is not built: build it with `python -m pikv_amd.build`")
-                _call.load(LIB_PATH)
-                _entries = _call
+                module = entry_module()
+                module.load(LIB_PATH)
+                _entries = module
     return _entries
 
 

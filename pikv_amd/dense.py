@@ -13,7 +13,7 @@ import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
 
-from . import _native
+from . import ops
 
 try:
     from torch.utils._device import DeviceContext as _DeviceContext
@@ -123,7 +123,7 @@ def ordinary_call() -> bool:
 
 def ordinary_tensor(t, device, dtype=torch.float32, align: int = 16) -> bool:
     """A dense tensor a kernel may read by its address, `align` bytes at a time (csrc/call.cpp)."""
-    return _native._call.ordinary(t, device, dtype, align)
+    return ops.ordinary_tensor(t, device, dtype, align)
 
 
 def forward_only(x) -> bool:

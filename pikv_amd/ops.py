@@ -73,12 +73,18 @@ def _refuse(t, name, dtype, ndim):
 def _need(*a, **k):
     """_need(t, name, *, dtype=None, ndim=None, optional=False): t, if it is a contiguous GPU tensor of that dtype and
     number of dimensions (or None where that may be); in csrc/call.cpp."""
-    raise N.PiKVNativeError("pikv_amd/_call is not built: build it with `python -m pikv_amd.build`")
+    N.entry_module()
+
+
+def ordinary_tensor(*a):
+    """ordinary_tensor(t, device, dtype, align): whether t is a dense tensor of that device and dtype that a kernel may read by
+    its address, `align` bytes at a time; in csrc/call.cpp."""
+    N.entry_module()
 
 
 if N._call is not None:
     N._call.setup(torch.Tensor, torch.nn.Parameter, _refuse, torch._C._has_storage if hasattr(torch._C, "_has_storage") else bool)
-    _need = N._call.need
+    _need, ordinary_tensor = N._call.need, N._call.ordinary
 
 
 def _vecf(t, name, n, device):

@@ -1,5 +1,8 @@
 """CPU checks of the typed Python entry (csrc/call.cpp): conversions, what it refuses, and the tensor checks beside it."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -151,3 +154,28 @@ def test_experts_factors_come_in_any_sequence(monkeypatch, kind):
     for (_, args), arrays in zip(seen, ((4, 5), (0, 1), (0, 1, 2))):
         for i in arrays:
             assert type(args[i]) in (list, tuple) and [type(x) in (torch.Tensor, torch.nn.Parameter) for x in args[i]] == [True] * 3
+
+
+_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _python(code):
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=_ROOT)
+
+
+def test_tensor_check_before_any_operator():
+    """dense alone sets up what its check needs."""
+    _python("import torch\nfrom pikv_amd import dense\n"
+            "assert dense.ordinary_tensor(torch.zeros(8), torch.device('cpu')) is True\n"
+            "assert dense.ordinary_tensor(torch.zeros(8)[1:], torch.device('cpu')) is False")
+
+
+def test_without_the_extension_every_way_in_says_so():
+    _python("import sys, torch\nsys.modules['pikv_amd._call'] = None\n"
+            "from pikv_amd import _native as N, dense, ops\n"
+            "for f in (lambda: dense.ordinary_tensor(torch.zeros(8), torch.device('cpu')), lambda: ops._need(torch.zeros(8), 'x'),\n"
+            "          lambda: N.call('pikv_abi_version'), lambda: N.size('pikv_evict_workspace_bytes', 1, 5)):\n"
+            "    try:\n        f()\n"
+            "    except N.PiKVNativeError as e:\n"
+            "        assert 'python -m pikv_amd.build' in str(e) and isinstance(e.__cause__, ImportError), e\n"
+            "    else:\n        raise AssertionError('no error')")
