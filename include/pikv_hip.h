@@ -85,7 +85,8 @@ extern "C" {
 
 const char* pikv_status_string(int status);
 
-/* Library/ABI version: major*1000 + minor. */
+/* Library/ABI version: major*1000 + minor, of this header and of the library. */
+#define PIKV_ABI_VERSION 1005
 int pikv_abi_version(void);
 
 /* ------------------------------------------------------------------------

@@ -148,7 +148,10 @@ def entries():
         with _lock:
             if _entries is None:
                 module = entry_module()
-                module.load(LIB_PATH)
+                try:
+                    module.load(LIB_PATH)
+                except OSError as e:
+                    raise PiKVNativeError(f"{e}: build both with `python -m pikv_amd.build`") from e
                 _entries = module
     return _entries
 

@@ -242,6 +242,9 @@ PyObject* load(PyObject*, PyObject* path) {
   if (!p) return nullptr;
   void* lib = dlopen(p, RTLD_NOW | RTLD_LOCAL);
   if (!lib) return PyErr_Format(PyExc_OSError, "%s", dlerror());
+  const auto version = reinterpret_cast<decltype(&::pikv_abi_version)>(dlsym(lib, "pikv_abi_version"));
+  if (!version || version() != PIKV_ABI_VERSION)         // its functions may have other arguments
+    return PyErr_Format(PyExc_OSError, "%s has ABI version %d, this extension was built for %d", p, version ? version() : 0, PIKV_ABI_VERSION);
   for (const Entry& e : g_entries) {
     void* s = dlsym(lib, e.name);
     if (!s) return PyErr_Format(PyExc_OSError, "%s: no symbol %s", p, e.name);

@@ -13,4 +13,4 @@ extern "C" const char* pikv_status_string(int status) {
   return "unknown status";
 }
 
-extern "C" int pikv_abi_version(void) { return 1005; }  // 1.5: + pikv_linear_tiled, pikv_evict_select_h2o, pikv_expert_combine_factors; 1.4: + pikv_quant_append (and the entry points of prefill.hip and moe.hip), pikv_cache_make_room, pikv_quant_scatter_routed
+extern "C" int pikv_abi_version(void) { return PIKV_ABI_VERSION; }  // 1.5: + pikv_linear_tiled, pikv_evict_select_h2o, pikv_expert_combine_factors; 1.4: + pikv_quant_append (and the entry points of prefill.hip and moe.hip), pikv_cache_make_room, pikv_quant_scatter_routed

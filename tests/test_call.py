@@ -179,3 +179,15 @@ def test_without_the_extension_every_way_in_says_so():
             "    except N.PiKVNativeError as e:\n"
             "        assert 'python -m pikv_amd.build' in str(e) and isinstance(e.__cause__, ImportError), e\n"
             "    else:\n        raise AssertionError('no error')")
+
+
+@pytest.mark.parametrize("body", ["int pikv_abi_version(void) { return 1004; }", "int nothing;"])
+def test_a_library_of_another_version_is_refused(monkeypatch, tmp_path, body):
+    (tmp_path / "other.c").write_text(body)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "other.so"), str(tmp_path / "other.c")], check=True)
+    monkeypatch.setattr(N, "LIB_PATH", str(tmp_path / "other.so"))
+    monkeypatch.setattr(N, "_entries", None)
+    with pytest.raises(N.PiKVNativeError, match="ABI version (1004|0)"):
+        N.entries()
+    monkeypatch.undo()
+    assert N.size("pikv_abi_version") == N.lib().pikv_abi_version() >= 1005     # ... and the one in use stays
