@@ -845,12 +845,14 @@ constexpr int kAtt8Tile = 32;    // cached tokens per step
 constexpr int kAtt8ARow = 80;    // bytes per staged A row: 32 tokens x bf16 + 16 (bank spread)
 constexpr int kAtt8PRow = 36;    // floats per query head of staged probabilities: 32 tokens + 4
 
-static size_t attend_mfma8_lds_bytes(int n_slabs, int n_q_heads, int hps) {
+static size_t attend_mfma8_lds_bytes(int n_slabs, int staged, int hps) {
   // codes [32 tokens][n_slabs*128 + 8]; scale and zero term [32][n_slabs*hps] float; A rows per
-  // wavefront [2 copies][16 rows][kAtt8ARow]; probabilities [query head][kAtt8PRow]
+  // wavefront [2 copies][16 rows][kAtt8ARow]; probabilities [staged query head][kAtt8PRow]
   return (size_t)kAtt8Tile * (n_slabs * 128 + 8) + 2 * (size_t)kAtt8Tile * n_slabs * hps * 4 +
-         4 * (size_t)2 * 16 * kAtt8ARow + (size_t)n_q_heads * kAtt8PRow * 4;
+         4 * (size_t)2 * 16 * kAtt8ARow + (size_t)staged * kAtt8PRow * 4;
 }
+// Query heads whose probabilities a block holds: at most eight of every slab, the others are other blocks or launches.
+static int attend_mfma8_staged(int n_slabs, int n_q_heads) { return n_q_heads < n_slabs * 8 ? n_q_heads : n_slabs * 8; }
 
 // HK = n_kv_heads (1..8); 2..8 query heads per kv head, at most 64 query heads.
 // Heads narrower than 128 (HPS = 128 / head_dim = 2 or 4): the kernel's kv heads are 128-dimension
@@ -1221,7 +1223,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 
 template <int SCHEME, int HPS>
 static void launch_attend_mfma8_slabs(int n_slabs, dim3 grid, hipStream_t st, const AttendArgs& a) {
-  const size_t lds = attend_mfma8_lds_bytes(n_slabs, a.n_q_heads, HPS);
+  const size_t lds = attend_mfma8_lds_bytes(n_slabs, attend_mfma8_staged(n_slabs, a.n_q_heads), HPS);
   switch (n_slabs) {
     case 1: hipLaunchKernelGGL((attend_mfma_i8_kernel<SCHEME, 1, HPS>), grid, dim3(256), lds, st, a); break;
     case 2: hipLaunchKernelGGL((attend_mfma_i8_kernel<SCHEME, 2, HPS>), grid, dim3(256), lds, st, a); break;
@@ -1271,8 +1273,7 @@ static void launch_attend_mfma8_heads(int n_slabs, int hps, dim3 grid, hipStream
     // rows of few slabs: 8, 4 or 2 neighbouring rows as one row of (up to) 8 slabs (pairs of rows of 4 slabs
     // measured the same as single rows: 322 vs 325 us at 64 caches x 32768 tokens x 16 query heads)
     const int ti = n_slabs == 1 ? 8 : n_slabs == 2 ? 4 : 2;
-    const int staged = a.n_q_heads < n_slabs * 8 ? a.n_q_heads : n_slabs * 8;   // heads of one launch
-    const size_t lds = attend_mfma8_lds_bytes(n_slabs * ti, staged * ti, 1);
+    const size_t lds = attend_mfma8_lds_bytes(n_slabs * ti, attend_mfma8_staged(n_slabs, a.n_q_heads) * ti, 1);
     if (n_slabs == 1) hipLaunchKernelGGL((attend_mfma_i8_kernel<SCHEME, 8, 1, 8>), grid, dim3(256), lds, st, a);
     else if (n_slabs == 2) hipLaunchKernelGGL((attend_mfma_i8_kernel<SCHEME, 8, 1, 4>), grid, dim3(256), lds, st, a);
     else hipLaunchKernelGGL((attend_mfma_i8_kernel<SCHEME, 6, 1, 2>), grid, dim3(256), lds, st, a);

@@ -398,6 +398,22 @@ def test_decode_attend_pieces(dev, n_caches, longest, scheme, group, heads, hq, 
     np.testing.assert_allclose(acc, np_of(pool.acc), rtol=hq * 2.0 ** -22 + 64 * 2.0 ** -23, atol=1e-12)
 
 
+@pytest.mark.parametrize("heads,hq,n_caches,longest", [(1, 1100, 1, 200), (3, 1200, 1, 130), (4, 1200, 2, 300)])
+def test_decode_attend_more_heads_than_a_block_stages(dev, heads, hq, n_caches, longest):
+    """8-bit rows under more query heads than the LDS of a compute unit has room for probabilities: a block holds eight
+    of every kv head.  Pieces of 128 tokens and more, against the public steps with the tolerance of the pieces above."""
+    r = rng(heads)
+    pool, ref = _fill_pool(dev, r, [longest] * n_caches, [longest] + [63] * (n_caches - 1), heads, 128, 128, O.Q_I8_SYM)
+    q = to_dev(O.bf16_round(r.standard_normal((n_caches, hq, 128)).astype(np.float32)), dev, "bf16")
+    out = np_of(pool.decode_attend(q, hq, now=3.0, accumulate=False))
+    scores, tmax, tsum = pool.scores(q, hq)
+    pool.h2o_accumulate(scores, tmax, tsum, now=3.0, stats_only=True)
+    want = np_of(pool.attend_values(scores, pool.head_stats, now=3.0))
+    rows = np.concatenate([ref.valid_rows(c) for c in range(n_caches)])
+    v_max = np.abs(O.dequantize_groups(ref.v_codes[rows], ref.v_scale[rows], ref.v_zero[rows], 128)).max()
+    assert np.abs(out - want).max() <= (2 * 1700 * 2.0 ** -24 + 64 * 2.0 ** -23) * v_max
+
+
 @pytest.mark.parametrize("scheme,group,heads,hq,dh", [
     (O.Q_I8_SYM, 64, 25, 25, 64),    # five blocks of 20 lanes: twelve rows per step, 16 threads without one
     (O.Q_I4_SYM, 64, 1, 71, 64),     # 2 lanes: a tile in one step, eight sets of eight heads side by side
