@@ -10,8 +10,9 @@
 // The lane with k-values 16 c + 4 quad .. + 3 feeds one of them to each of four instructions, so sums run over k in steps of 16.
 //
 // Measured, one launch against one library call a layer (us, back to back): 1000 tokens x 2048 -> 2048 + 1024 + 1024 (128 x 128,
-// 256 blocks = the chip) 125 / 143; 1000 x 512 -> 2048 21 / 56; 500 x 1536 -> 4096 52 / 66; 250 x 3072 -> 3072 56 / 57; 66 x 1536 -> 4096
-// 20 / 57 (three library calls take the host 56 us).  Against: 1000 x 3072 -> 3072 150 / 146, 4000 x 3072 -> 3072 537 / 528.  A single layer is
+// 256 blocks = the chip) 125 / 130; 1280 x 2048 -> 3072 125 / 144; 1000 x 512 -> 2048 21 / 56; 500 x 1536 -> 4096 52 / 66; 250 x 3072 -> 3072 56 / 57; 66 x 1536 -> 4096
+// 20 / 57 (three library calls take the host 56 us).  Against: 1000 x 3072 -> 3072 150 / 146, 4000 x 3072 -> 3072 537 / 528, and rounds
+// that stay half empty: 330 x 3072 -> 3072 97 / 73.  A single layer is
 // no faster than the library's (1000 x 2048 -> 2048 67 / 62).  dense.py says which calls come here.
 #include "common.hpp"
 

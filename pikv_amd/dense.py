@@ -66,19 +66,33 @@ def projections_pay(T: int, H: int, N: int) -> bool:
     return T <= 64 and H <= 3584 and H * N <= (20_000_000 if T <= 32 else 13_000_000)
 
 
+_TILES = ((128, 128, 57.0), (64, 128, 30.0), (64, 64, 16.6), (32, 64, 11.0))   # rows, columns, ns for a round of 256 and a k-value
+
+
+def _tiled_us(T: int, H: int, widths) -> float:
+    """Kernel time of linear_tiled without its start of about 5 us (tile_variant in csrc/linear.hip)."""
+    return 1e-3 * H * min(-(-(-(-T // m) * sum(-(-w // n) for w in widths)) // 256) * ns for m, n, ns in _TILES)
+
+
 def tiled_pays(T: int, H: int, widths) -> bool:
     """The same for 256 tokens and more, in LDS tiles (csrc/linear.hip).  Up to 3.5e9 multiply-adds the library's three calls are
-    bound by the host (250 x 512 x 2048 9 / 56, 1000 x 512 x 2048 21 / 56, 500 x 1536 x 4096 52 / 66); beyond, one round of 128 x 128
-    tiles that fills the chip (1000 x 2048 x 4096 125 / 143).  Outside 1000 x 3072 x 3072 150 / 146, 4000 x 3072 x 3072 537 / 528.  Fewer
-    than 256 tokens would be faster too (130 x 1024 x 3072 32 / 57), but there the library sums in another order for most widths, and
-    2e-7 of a query is 1e-5 of a probability where scores reach 100; from 256 on nearly all sums are bit for bit the library's."""
+    bound by the host, 57 us: faster while the tiles take less (250 x 512 x 2048 9 / 56, 1000 x 512 x 2048 21 / 56, 500 x 1536 x 4096 52 / 66,
+    291 x 1792 x 4096 59 / 61), behind that where they fill their rounds (100 TFLOP/s by the rule: 295 x 3840 x 3072 67 / 85, 397 x 2048 x 4096
+    68 / 74; below it 330 x 3072 x 3072 97 / 73, 539 x 3072 x 2048 96 / 83, 639 x 2304 x 2304 74 / 66, 261 x 2048 x 4608 67 / 61).  Beyond 3.5e9
+    one round of 128 x 128 tiles that fills the chip: 1280 x 2048 x 3072 125 / 144, 640 x 3072 x 6144 183 / 203, 1792 x 2560 x 2304 155 / 180,
+    896 x 3840 x 4608 229 / 267, 1000 x 2048 x 4096 125 / 130, 1024 x 4096 x 4096 245 / 244; below 87 % of it 871 x 3072 x 4096 183 / 177, outside
+    4000 x 3072 x 3072 537 / 528.  Of 171 sizes none that it takes was slower by more than half a percent.  Fewer than 256 tokens would be
+    faster too (130 x 1024 x 3072 32 / 57), but there the library sums in another order for most widths, and 2e-7 of a query is 1e-5 of a
+    probability where scores reach 100; from 256 on it was the same order, to the last bit, for nine of ten sizes measured (nearly all
+    others have layers of 256 columns, which the library splits along k)."""
     if T < 256:
         return False
     N = sum(widths)
     if T * H * N <= 3_500_000_000:
-        return True
+        us = _tiled_us(T, H, widths)
+        return us <= 55 or 2e-6 * T * H * N >= 100 * us
     tiles = -(-T // 128) * sum(-(-n // 128) for n in widths)
-    return tiles <= 256 and T * N >= 0.85 * 256 * 128 * 128
+    return tiles <= 256 and T * N >= 0.87 * 256 * 128 * 128
 
 
 def experts_tiled(T: int, H: int, E: int) -> bool:

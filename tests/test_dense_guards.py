@@ -101,3 +101,19 @@ def test_key_projection_rule_against_measured_sizes(T, H, pays):
     (8, 8192, 12288, False), (1, 8192, 1024, False)])
 def test_projection_rule_against_measured_sizes(T, H, N, pays):
     assert dense.projections_pay(T, H, N) is pays
+
+
+@pytest.mark.parametrize("T,H,widths,pays", [
+    (256, 512, (1024, 512, 512), True), (500, 1536, (2048, 1024, 1024), True), (4757, 256, (1536, 256, 256), True),
+    (291, 1792, (2048, 1024, 1024), True), (1100, 2048, (768, 384, 384), True), (295, 3840, (2048, 512, 512), True),
+    (307, 3584, (1024, 1024, 1024), True), (277, 4096, (2048, 512, 512), True), (397, 2048, (2048, 1024, 1024), True),
+    (1280, 2048, (2048, 512, 512), True), (640, 3072, (4096, 1024, 1024), True), (1792, 2560, (1536, 384, 384), True),
+    (896, 3840, (3584, 512, 512), True), (1000, 2048, (2048, 1024, 1024), True),
+    (255, 512, (1024, 512, 512), False), (300, 3072, (2048, 768, 768), False), (330, 3072, (2048, 512, 512), False),
+    (539, 3072, (1536, 256, 256), False), (639, 2304, (768, 768, 768), False), (261, 2048, (3584, 512, 512), False),
+    (276, 4096, (1536, 256, 256), False), (266, 3072, (2048, 1024, 1024), False), (337, 3328, (1024, 1024, 1024), False),
+    (871, 3072, (2048, 1024, 1024), False), (668, 3328, (3072, 1024, 1024), False), (1000, 3072, (1024, 1024, 1024), False),
+    (4000, 3072, (1024, 1024, 1024), False)])
+def test_tiled_rule_against_measured_sizes(T, H, widths, pays):
+    """Sizes where one launch for q, k and v was measured no slower than three library calls, and where it was."""
+    assert dense.tiled_pays(T, H, widths) is pays

@@ -261,6 +261,29 @@ def test_projection_size_rule(dev, monkeypatch, T, hidden, heads, kv, native):
     assert bool(calls) is native
 
 
+@pytest.mark.parametrize("T,hidden,heads,kv,native", [
+    (255, 1024, 32, 8, False), (256, 1024, 32, 8, True),
+    (1112, 2048, 16, 4, True), (1113, 2048, 16, 4, False),       # 3.5e9 multiply-adds
+    (330, 3072, 32, 8, False),                                   # ... of half empty rounds
+    (871, 3072, 32, 16, False), (892, 3072, 32, 16, True), (1024, 3072, 32, 16, True), (1025, 3072, 32, 16, False)])   # one round
+def test_tiled_projection_size_rule(dev, monkeypatch, T, hidden, heads, kv, native):
+    """Both sides of the sizes where the projections of many tokens are one launch: the modules' values to float32 sums."""
+    import torch
+    from pikv_amd import ops
+    from pikv_amd.attention import PiKVAttention
+    torch.manual_seed(T + hidden)
+    layer = PiKVAttention(hidden, heads, head_dim=64, num_kv_heads=kv, cache_size=8).to(dev).eval()
+    calls, tiled = [], ops.linear_tiled
+    monkeypatch.setattr(ops, "linear_tiled", lambda *a, **kw: calls.append(1) or tiled(*a, **kw))
+    monkeypatch.setattr(ops, "linear_group", lambda *a, **kw: calls.append(2))
+    x = torch.randn(1, T, hidden, device=dev)
+    with torch.no_grad():
+        for got, m in zip(layer._project(x), (layer.q_proj, layer.k_proj, layer.v_proj)):
+            want = m(x).view(got.shape)
+            assert torch.allclose(got, want, rtol=0, atol=16 * 2.0 ** -24 * np.sqrt(hidden) * float(want.abs().max()))
+    assert calls == [1] * native
+
+
 def test_native_prompt_attention_leaves_other_calls_alone(dev):
     """Hooks, dropout, masks, gradients, other types and forward-mode tangents keep the torch path; the two paths agree
     on what both take (float32 sums of some 200 products: 1e-5 of outputs of order one)."""
