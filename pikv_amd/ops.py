@@ -626,7 +626,16 @@ class CachePool:
         self.n_heavy = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
         self.n_recent = torch.zeros(self.n_caches, dtype=torch.int32, device=dev)
         self._budgets = torch.empty(3 * self.n_caches, dtype=torch.int32, device=dev)
-        self._row_bytes = [math.prod(p.shape[1:]) * p.element_size() for p in self.planes()]
+        self._row_bytes = self._plane_row_bytes()
+
+    def _plane_row_bytes(self):
+        return [math.prod(p.shape[1:]) * p.element_size() for p in self.planes()]
+
+    def __setstate__(self, state):
+        """A copied or unpickled pool makes its workspaces anew: their sizes, and what else is derived from the planes, are those
+        of the version that made it."""
+        self.__dict__.update((k, v) for k, v in state.items() if k not in ("_decode_ws", "_decode_ws_key", "_evict_ws"))
+        self._row_bytes = self._plane_row_bytes()
 
     # ---- checkpoint ----
     _STATE_PLANES = ("k_codes", "k_scale", "k_zero", "v_codes", "v_scale", "v_zero", "acc", "ts")

@@ -1,6 +1,8 @@
 """CPU checks of the typed Python entry (csrc/call.cpp): conversions, what it refuses, and the tensor checks beside it."""
+import copy
 import ctypes as C
 import os
+import pickle
 import subprocess
 import sys
 
@@ -121,14 +123,20 @@ def test_ordinary_tensor():
     assert seen == [False]
 
 
-@pytest.mark.parametrize("kind", [list, tuple, iter])
-def test_every_plane_of_a_compaction_has_its_row_bytes(monkeypatch, kind):
-    """The library reads as many widths as there are planes, whatever the extra ones come in."""
+def _host_pool():
+    """The host side of a pool with four planes of rows."""
     pool = object.__new__(ops.CachePool)
     pool.k_codes, pool.k_scale, pool.acc, pool.ts = torch.zeros(4, 64, dtype=torch.int8), torch.zeros(4, 2), torch.zeros(4), torch.zeros(4)
     pool.k_zero = pool.v_codes = pool.v_scale = pool.v_zero = None
     pool.row_base = pool.keep_index = pool.new_len = pool.fill = None
     pool.n_caches, pool._row_bytes = 1, [64, 8, 4, 4]
+    return pool
+
+
+@pytest.mark.parametrize("kind", [list, tuple, iter])
+def test_every_plane_of_a_compaction_has_its_row_bytes(monkeypatch, kind):
+    """The library reads as many widths as there are planes, whatever the extra ones come in."""
+    pool = _host_pool()
     seen = []
     monkeypatch.setattr(ops, "_need", lambda t, name: t)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
@@ -191,3 +199,14 @@ def test_a_library_of_another_version_is_refused(monkeypatch, tmp_path, body):
         N.entries()
     monkeypatch.undo()
     assert N.size("pikv_abi_version") == N.lib().pikv_abi_version() >= 1005     # ... and the one in use stays
+
+
+@pytest.mark.parametrize("again", [copy.copy, copy.deepcopy, lambda p: pickle.loads(pickle.dumps(p))])
+def test_a_pool_of_another_version_makes_its_workspaces_anew(again):
+    """One that another version of the package has pickled has that version's workspace sizes, and no row widths."""
+    pool = _host_pool()
+    del pool._row_bytes
+    pool._decode_ws, pool._decode_ws_key, pool._evict_ws = torch.zeros(8), (32, 700), (torch.zeros(8), 32)
+    new = again(pool)
+    assert new._row_bytes == [64, 8, 4, 4] and torch.equal(new.k_codes, pool.k_codes) and new.n_caches == 1
+    assert not {"_decode_ws", "_decode_ws_key", "_evict_ws"} & set(new.__dict__) and pool._decode_ws_key == (32, 700)
