@@ -145,11 +145,17 @@ def forward_only(x) -> bool:
     return not torch.is_grad_enabled() and x.is_cuda and ordinary_call() and ordinary_tensor(x, x.device)
 
 
+def tensor_of(m, name: str):
+    """The tensor m.<name>: a parameter (m.<name> itself looks through three tables for it), a buffer or a plain attribute."""
+    t = m._parameters.get(name)
+    return getattr(m, name, None) if t is None else t
+
+
 def linear_ok(m, n_in: int, n_out: int, device) -> bool:
     """A plain nn.Linear of this shape with a bias, as linear_group reads it."""
     if not plain(m, nn.Linear):
         return False
-    w, b = m._parameters.get("weight"), m._parameters.get("bias")    # (m.weight looks through three tables for it)
+    w, b = tensor_of(m, "weight"), tensor_of(m, "bias")
     return (w is not None and b is not None and w.shape == (n_out, n_in) and ordinary_tensor(w, device)
             and ordinary_tensor(b, device))
 

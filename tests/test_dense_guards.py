@@ -117,3 +117,21 @@ def test_projection_rule_against_measured_sizes(T, H, N, pays):
 def test_tiled_rule_against_measured_sizes(T, H, widths, pays):
     """Sizes where one launch for q, k and v was measured no slower than three library calls, and where it was."""
     assert dense.tiled_pays(T, H, widths) is pays
+
+
+@pytest.mark.parametrize("how", ["parameter", "buffer", "attribute"])
+def test_frozen_weights_are_read_like_parameters(how):
+    """Weights that were taken out of the parameters, as buffers or as plain attributes (data-parallel replicas hold theirs so)."""
+    from pikv_amd.config import config
+    from pikv_amd.moe import LoRALayer, PiKVMoE
+    lin, lora = torch.nn.Linear(8, 4), LoRALayer(config["hidden_size"], config["hidden_size"], rank=2).eval()
+    for m, names in ((lin, ("weight", "bias")), (lora, ("lora_A", "lora_B"))):
+        for n in names if how != "parameter" else ():
+            t = getattr(m, n).detach()
+            delattr(m, n)
+            m.register_buffer(n, t) if how == "buffer" else setattr(m, n, t)
+    cpu = torch.device("cpu")
+    assert dense.linear_ok(lin, 8, 4, cpu) and not dense.linear_ok(lin, 4, 8, cpu)
+    assert PiKVMoE._lora_ok(None, lora, 2, cpu) and not PiKVMoE._lora_ok(None, lora, 4, cpu)
+    lin.bias = None
+    assert not dense.linear_ok(lin, 8, 4, cpu)
