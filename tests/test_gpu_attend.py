@@ -373,6 +373,7 @@ def test_attend_block_lengths(dev, n_caches, length, scheme, heads, hq):
     (O.Q_I8_ASYM, 64, 5, 5, 64, "bf16"),     # ... twenty, 256 threads hold twelve rows
     (O.Q_I4_SYM, 32, 2, 40, 128, "bf16"),    # sets of query heads side by side, exchange format
     (O.Q_I8_SYM, 128, 1, 20, 128, "bf16"),   # ... float scores
+    (O.Q_I8_SYM, 128, 1, 128, 128, "bf16"),  # ... as many heads as there may be, eight of them staged by a block
 ])
 @pytest.mark.parametrize("n_caches,longest", [(20, 1700), (33, 1700), (90, 129), (3, 65), (130, 1025)])
 def test_decode_attend_pieces(dev, n_caches, longest, scheme, group, heads, hq, dh, qdtype):
@@ -398,20 +399,37 @@ def test_decode_attend_pieces(dev, n_caches, longest, scheme, group, heads, hq, 
     np.testing.assert_allclose(acc, np_of(pool.acc), rtol=hq * 2.0 ** -22 + 64 * 2.0 ** -23, atol=1e-12)
 
 
-@pytest.mark.parametrize("heads,hq,n_caches,longest", [(1, 1100, 1, 200), (3, 1200, 1, 130), (4, 1200, 2, 300)])
-def test_decode_attend_more_heads_than_a_block_stages(dev, heads, hq, n_caches, longest):
+@pytest.mark.parametrize("heads,hq,lens", [(4, 1200, [300, 63]), (1, 1200, [130]), (3, 1500, [257, 0, 65])])
+def test_attend_values_more_heads_than_a_block_stages(dev, heads, hq, lens):
     """8-bit rows under more query heads than the LDS of a compute unit has room for probabilities: a block holds eight
-    of every kv head.  Pieces of 128 tokens and more, against the public steps with the tolerance of the pieces above."""
+    of every kv head.  A sum of up to 300 products with weights up to 1 and nothing subtracted but the zero point's share,
+    in bf16 halves of 2^-16 each: 300 x 2^-15 of the largest value row element."""
+    import torch
     r = rng(heads)
-    pool, ref = _fill_pool(dev, r, [longest] * n_caches, [longest] + [63] * (n_caches - 1), heads, 128, 128, O.Q_I8_SYM)
-    q = to_dev(O.bf16_round(r.standard_normal((n_caches, hq, 128)).astype(np.float32)), dev, "bf16")
-    out = np_of(pool.decode_attend(q, hq, now=3.0, accumulate=False))
-    scores, tmax, tsum = pool.scores(q, hq)
-    pool.h2o_accumulate(scores, tmax, tsum, now=3.0, stats_only=True)
-    want = np_of(pool.attend_values(scores, pool.head_stats, now=3.0))
-    rows = np.concatenate([ref.valid_rows(c) for c in range(n_caches)])
-    v_max = np.abs(O.dequantize_groups(ref.v_codes[rows], ref.v_scale[rows], ref.v_zero[rows], 128)).max()
-    assert np.abs(out - want).max() <= (2 * 1700 * 2.0 ** -24 + 64 * 2.0 ** -23) * v_max
+    pool, ref = _fill_pool(dev, r, [max(lens)] * len(lens), lens, heads, 128, 128, O.Q_I8_SYM)
+    stride = (max(lens) + 63) // 64 * 64
+    p = r.random((len(lens), hq, stride)).astype(np.float32)
+    out = np_of(pool.attend_values(to_dev(p, dev)))
+    for c, L in enumerate(lens):
+        rows = ref.valid_rows(c)
+        v = O.dequantize_groups(ref.v_codes[rows], ref.v_scale[rows], ref.v_zero[rows], 128).reshape(L, heads, 128).astype(np.float64)
+        want = np.einsum("ghl,lgd->ghd", p[c, :, :L].reshape(heads, hq // heads, L).astype(np.float64), v).reshape(hq, 128)
+        assert np.abs(out[c] - want).max() <= 300 * 2.0 ** -15 * (np.abs(v).max() if L else 1.0), c
+
+
+@pytest.mark.parametrize("scheme,group,heads,hq", [(O.Q_I8_SYM, 128, 4, 28), (O.Q_I8_ASYM, 128, 8, 16), (O.Q_I4_ASYM, 32, 8, 32)])
+def test_decode_attend_queries_that_begin_between_16_bytes(dev, scheme, group, heads, hq):
+    """float32 queries at any element of a buffer: bit for bit what they give from its start."""
+    import torch
+    r = rng(hq)
+    pool, _ = _fill_pool(dev, r, [300] * 3, [300, 65, 1], heads, 128, group, scheme)
+    q = to_dev(r.standard_normal((3, hq, 128)).astype(np.float32), dev)
+    want = pool.decode_attend(q, hq, now=1.0)
+    for at in (1, 2, 3):
+        buf = torch.full((q.numel() + 4,), float("nan"), device=dev)
+        view = buf[at:at + q.numel()].view_as(q)
+        view.copy_(q)
+        assert torch.equal(pool.decode_attend(view, hq, now=1.0), want)
 
 
 @pytest.mark.parametrize("scheme,group,heads,hq,dh", [
