@@ -96,12 +96,18 @@ def tiled_pays(T: int, H: int, widths) -> bool:
 
 
 def experts_tiled(T: int, H: int, E: int) -> bool:
-    """The products of E experts [H, H] in one launch of LDS tiles: 128 x 256, 4 experts 14 us for four library calls of 34 on one
-    compute unit each; 2048 x 512, 4 experts 45 / 80.  Only where the library sums in the same order to the last bit: what the
-    experts put out is cached in codes, and the means of the caches come back in the next call.  That is from 33 tokens on but
-    for 257 to 1024 tokens of less than 384 columns (128 columns: 257 on), and for few tokens of more than 512."""
-    return (33 <= T and (T <= 256 or H >= 384 or (H >= 256 and T > 1024)) and (H <= 512 or T >= 512)
-            and T * H * H * E <= 3_500_000_000)
+    """The products of E experts [H, H] in one launch of LDS tiles: 128 x 256, 4 experts 13 us / 75 for four library calls, 1053 x 512,
+    4 experts 32 / 75, 667 x 1024, 4 experts 60 / 76; while the tiles take less time than the library's calls take the host, 18 us each
+    (outside 743 x 1536, 1 expert 52 / 36, 716 x 1536, 2 experts 84 / 71, 548 x 1280, 3 experts 70 / 62).
+
+    What the experts put out is cached in codes, and the means of the caches come back in the next call, where another order of sums
+    - 2e-7, a code in 10^4 - grows to 1e-4 of a cached row's scale.  So only sizes are taken where the library (hipBLASLt of ROCm 7, as
+    torch calls it by default) was measured to sum in the same order, to the last bit: 33 tokens on but for 257 to 1024 and more
+    than 2048 tokens of 256 columns, 257 on of 128, and fewer than 512 of more than 512; 2800 sizes up to 8192 tokens, of which 3
+    differed, all beyond what the time admits.  Another library or version may choose otherwise: no less exact, but
+    its two forms then differ by that much."""
+    same_order = (33 <= T <= 8192 and (T <= 256 or H >= 384 or H == 256 and 1024 < T <= 2048) and (H <= 512 or T >= 512))
+    return same_order and T * H * H * E <= 3_500_000_000 and _tiled_us(T, H, (H,) * E) <= 18 * E - 6
 
 
 def key_projection_pays(T: int, H: int) -> bool:

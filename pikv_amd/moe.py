@@ -252,9 +252,9 @@ class PiKVMoE(nn.Module):
                    for e, c in zip(self.experts, self.kv_caches))
 
     def _experts_forward(self, x, cached, routing_weights):
-        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]): the experts' products bit for bit
-        those of LoRAExpert.forward - in one launch where that sums in the library's order (dense.experts_tiled), by the
-        library otherwise - and the rest in four launches (the key projection of many or wide rows by the library too)."""
+        """(outputs of every expert [E, T, H], key rows [T, H], weighted sum [T, H]): the experts' products in one launch at the
+        sizes where that was measured to sum in the library's order (dense.experts_tiled), by the library otherwise, and the
+        rest in four launches (the key projection of many or wide rows by the library too)."""
         H = x.shape[-1]
         x2 = x.reshape(-1, H)
         T, E = x2.shape[0], len(self.experts)

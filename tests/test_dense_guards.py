@@ -135,3 +135,14 @@ def test_frozen_weights_are_read_like_parameters(how):
     assert PiKVMoE._lora_ok(None, lora, 2, cpu) and not PiKVMoE._lora_ok(None, lora, 4, cpu)
     lin.bias = None
     assert not dense.linear_ok(lin, 8, 4, cpu)
+
+
+@pytest.mark.parametrize("T,H,E,tiled", [
+    (33, 128, 4, True), (256, 128, 4, True), (128, 256, 4, True), (1025, 256, 4, True), (2048, 256, 8, True), (300, 384, 4, True),
+    (5900, 384, 4, True), (1053, 512, 4, True), (2280, 512, 4, True), (520, 640, 4, True), (667, 1024, 4, True), (544, 1024, 6, True),
+    (32, 128, 4, False), (257, 128, 4, False), (257, 256, 4, False), (1024, 256, 4, False), (511, 640, 4, False),     # another order
+    (2049, 256, 4, False), (3000, 256, 4, False), (6145, 512, 2, False), (3073, 1024, 1, False), (8192, 384, 8, False),
+    (743, 1536, 1, False), (633, 2048, 1, False), (716, 1536, 2, False), (548, 1280, 3, False), (1525, 1024, 1, False)])   # slower
+def test_experts_rule_against_measured_sizes(T, H, E, tiled):
+    """Sizes where the experts' products in one launch were measured faster and equal to the library's, and where not."""
+    assert dense.experts_tiled(T, H, E) is tiled

@@ -107,6 +107,38 @@ def test_tiled_experts_sum_in_the_librarys_order(dev, T, H):
         assert (T, H) in ((17, 256), (257, 256))
 
 
+@pytest.mark.parametrize("H", [128, 256, 384, 512, 640, 1024])
+def test_tiled_experts_order_at_the_edges_of_the_rule(dev, H):
+    """Both sides of every size where the rule changes, and some between, as many experts as the time admits."""
+    import torch
+    from pikv_amd import dense, ops
+    taken = 0
+    for T in (33, 64, 128, 255, 256, 257, 511, 512, 513, 700, 1000, 1023, 1024, 1025, 1500, 2047, 2048, 2049, 3000, 3333, 5000, 8192):
+        if not any(dense.experts_tiled(T, H, E) for E in (1, 2, 4)):
+            continue
+        taken += 1
+        torch.manual_seed(T)
+        x, w, b = torch.randn(T, H, device=dev), torch.randn(H, H, device=dev) * 0.05, torch.randn(H, device=dev)
+        o = torch.empty(T, H, device=dev)
+        ops.linear_tiled(x, [(w, b, o)])
+        assert torch.equal(o, torch.nn.functional.linear(x, w, b)), T
+    assert taken >= 3
+
+
+@pytest.mark.parametrize("H", [256, 512])
+@pytest.mark.parametrize("T", [33, 257, 2048])
+def test_expert_factors_sum_in_the_librarys_order(dev, T, H):
+    """The second factor at the widths and token counts in use, every rank."""
+    import torch
+    from pikv_amd import ops
+    for rank in range(1, 9):
+        torch.manual_seed(T + rank)
+        d, t, b, c, w = (torch.randn(*s, device=dev) for s in ((2, T, H), (2, T, rank), (2, rank, H), (2, H), (T, 2)))
+        want = ops.expert_combine(list(d), [torch.mm(x, y) for x, y in zip(t, b)], [0.3, 0.7], c, w)
+        got = ops.expert_combine(list(d), list(t), [0.3, 0.7], c, w, lora_b=list(b))
+        assert all(torch.equal(x, y) for x, y in zip(got, want)), rank
+
+
 @pytest.mark.parametrize("scheme,D,group", [(O.Q_I8_SYM, 272, 16), (O.Q_I8_ASYM, 256, 256), (O.Q_I4_ASYM, 1088, 32),
                                             (O.Q_I4_SYM, 64, 64)])
 @pytest.mark.parametrize("lens", [[0, 1, 63], [65, 64, 130], [5000, 4097, 2]])
