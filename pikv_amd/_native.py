@@ -128,7 +128,7 @@ try:
     from . import _call
 except ImportError as e:                 # not built, or it does not load: whoever needs it is told
     _call, _call_error = None, e
-_entries = None
+_entries = _of_checked = None
 
 
 def entry_module():
@@ -142,7 +142,7 @@ def entry_module():
 def entries():
     """The module of typed entry points (csrc/call.cpp), bound to the library that lib() loads.  Every call of this package
     goes through it; lib() remains for a ctypes caller."""
-    global _entries
+    global _entries, _of_checked
     if _entries is None:
         lib()
         with _lock:
@@ -152,13 +152,21 @@ def entries():
                     module.load(LIB_PATH)
                 except OSError as e:
                     raise PiKVNativeError(f"{e}: build both with `python -m pikv_amd.build`") from e
+                _of_checked = module.of_checked
                 _entries = module
     return _entries
 
 
 def call(name: str, *args) -> None:
-    """Call an int-status entry point and raise on a non-zero status.  Pointers: tensors, addresses, None; lists for host arrays."""
+    """Call an int-status entry point and raise on a non-zero status.  Pointers: GPU tensors, addresses, None; lists for host arrays."""
     code = getattr(_entries or entries(), name)(*args)
+    if code:
+        check(code, name)
+
+
+def launch(name: str, *args) -> None:
+    """call() for a caller that has seen that its tensors are on the GPU."""
+    code = getattr(_of_checked or entries().of_checked, name)(*args)
     if code:
         check(code, name)
 

@@ -205,11 +205,11 @@ def router_fused(x, weight, bias=None, *, top_k=2, capacity=None, expert_scale=N
         if count is not None:
             count.zero_()
         return RouterOut(probs, idx, w, slot, count, logits, capacity)
-    N.call("pikv_router_fused", x, weight, dt, bias, expert_scale,
-           expert_mask, float(temperature), float(renorm_eps), _arith(module_arithmetic),
-           T, H, E, top_k,
-           int(capacity or 0), probs, logits, idx, w, slot,
-           count, ws, ws_bytes, _stream())
+    N.launch("pikv_router_fused", x, weight, dt, bias, expert_scale,
+             expert_mask, float(temperature), float(renorm_eps), _arith(module_arithmetic),
+             T, H, E, top_k,
+             int(capacity or 0), probs, logits, idx, w, slot,
+             count, ws, ws_bytes, _stream())
     return RouterOut(probs, idx, w, slot, count, logits, capacity)
 
 
@@ -237,10 +237,10 @@ def router_tail(logits, *, top_k=2, capacity=None, logits_b=None, select=None,
         if count is not None:
             count.zero_()
         return RouterOut(probs, idx, w, slot, count, None, capacity)
-    N.call("pikv_router_tail", logits, logits_b, select, expert_scale,
-           expert_mask, float(temperature), float(renorm_eps), int(bool(use_softmax)),
-           _arith(module_arithmetic), T, E, top_k, int(capacity or 0), probs, idx, w, slot,
-           count, ws, ws_bytes, _stream())
+    N.launch("pikv_router_tail", logits, logits_b, select, expert_scale,
+             expert_mask, float(temperature), float(renorm_eps), int(bool(use_softmax)),
+             _arith(module_arithmetic), T, E, top_k, int(capacity or 0), probs, idx, w, slot,
+             count, ws, ws_bytes, _stream())
     return RouterOut(probs, idx, w, slot, count, None, capacity)
 
 
@@ -259,8 +259,8 @@ def capacity_slots(expert_idx, num_experts: int, capacity: int):
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
     if A == 0:
         return slot, count.zero_()
-    N.call("pikv_capacity_slots", expert_idx, A, num_experts, int(capacity), slot,
-           count, ws, ws_bytes, _stream())
+    N.launch("pikv_capacity_slots", expert_idx, A, num_experts, int(capacity), slot,
+             count, ws, ws_bytes, _stream())
     return slot, count
 
 
@@ -281,8 +281,8 @@ def quantize_rows(x, group: int, scheme: int):
     zero = torch.empty_like(scale) if _scheme_asym(scheme) else None
     if n == 0:
         return codes, scale, zero
-    N.call("pikv_quantize_rows", x, dt, n, D, group, scheme, 0, codes, scale,
-           zero, _stream())
+    N.launch("pikv_quantize_rows", x, dt, n, D, group, scheme, 0, codes, scale,
+             zero, _stream())
     return codes, scale, zero
 
 
@@ -301,7 +301,7 @@ def quant8_minshift(x, want_dq: bool = True):
     scale = torch.empty(n, 1, dtype=torch.float32, device=dev)
     mn = torch.empty(n, 1, dtype=torch.float32, device=dev)
     if n:
-        N.call("pikv_quant8_minshift", x, dt, n, D, codes, dq, scale, mn, _stream())
+        N.launch("pikv_quant8_minshift", x, dt, n, D, codes, dq, scale, mn, _stream())
     return dq, codes, scale, mn
 
 
@@ -330,9 +330,9 @@ def dequantize_rows(codes, scale, zero, group: int, scheme: int, out_dtype=torch
     out = torch.empty(cnt, D, dtype=out_dtype, device=codes.device)
     if cnt == 0:
         return out
-    N.call("pikv_gather_dequant", codes, scale, zero, D, group, scheme,
-           rows, row0, cnt, out, F32 if out_dtype == torch.float32 else BF16,
-           _stream())
+    N.launch("pikv_gather_dequant", codes, scale, zero, D, group, scheme,
+             rows, row0, cnt, out, F32 if out_dtype == torch.float32 else BF16,
+             _stream())
     return out
 
 
@@ -350,8 +350,8 @@ def fakequant_colblocks(x, group: int, bits: int = 8, symmetric: bool = False):
     mse = torch.zeros(nblk, dtype=torch.float32, device=dev)
     ws_bytes = N.size("pikv_fakequant_workspace_bytes", Nr, H, group)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    N.call("pikv_fakequant_colblocks", x, Nr, H, group, bits, int(bool(symmetric)),
-           out, stats, mse, ws, ws_bytes, _stream())
+    N.launch("pikv_fakequant_colblocks", x, Nr, H, group, bits, int(bool(symmetric)),
+             out, stats, mse, ws, ws_bytes, _stream())
     return out, stats, mse
 
 
@@ -372,8 +372,8 @@ def fakequant_preset(x, preset, group: int, bits: int = 8, symmetric: bool = Fal
     mse = torch.zeros(nblk, dtype=torch.float32, device=dev)
     ws_bytes = N.size("pikv_fakequant_workspace_bytes", Nr, H, group)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    N.call("pikv_fakequant_preset", x, Nr, H, group, bits, int(bool(symmetric)),
-           preset, out, mse, ws, ws_bytes, _stream())
+    N.launch("pikv_fakequant_preset", x, Nr, H, group, bits, int(bool(symmetric)),
+             preset, out, mse, ws, ws_bytes, _stream())
     return out, mse
 
 
@@ -409,9 +409,9 @@ def select_top_rows(score, seg_base, seg_len, n_keep, max_len: Optional[int] = N
         max_len = score.numel()
     ws, ws_bytes = _evict_workspace(n, int(max_len), dev)
     # H2O selection with an empty "recent" budget; the score doubles as the (unused) timestamp
-    N.call("pikv_evict_select", EVICT_H2O, score, score, seg_base, seg_len,
-           n_keep, zero, n, int(max_len), flag, index, kept, ws,
-           ws_bytes, _stream())
+    N.launch("pikv_evict_select", EVICT_H2O, score, score, seg_base, seg_len,
+             n_keep, zero, n, int(max_len), flag, index, kept, ws,
+             ws_bytes, _stream())
     return flag, index, kept
 
 
@@ -437,12 +437,12 @@ def linear_group(x, layers, rank: int = 0):
     n = len(layers)
     nb = N.size("pikv_linear_group_workspace_bytes", T, n, rank)
     ws = torch.empty(nb, dtype=torch.uint8, device=x.device) if nb else None
-    N.call("pikv_linear_group", x, T, K, n, [l["weight"] for l in layers],
-           [l["bias"] for l in layers], [l["weight"].shape[0] for l in layers],
-           [int(bool(l.get("relu"))) for l in layers], rank,
-           [l.get("lora_a") for l in layers], [l.get("lora_b") for l in layers],
-           [float(l.get("scaling", 0.0)) for l in layers],
-           [l["out"] for l in layers], ws, nb, _stream())
+    N.launch("pikv_linear_group", x, T, K, n, [l["weight"] for l in layers],
+             [l["bias"] for l in layers], [l["weight"].shape[0] for l in layers],
+             [int(bool(l.get("relu"))) for l in layers], rank,
+             [l.get("lora_a") for l in layers], [l.get("lora_b") for l in layers],
+             [float(l.get("scaling", 0.0)) for l in layers],
+             [l["out"] for l in layers], ws, nb, _stream())
 
 
 def linear_tiled(x, layers):
@@ -459,8 +459,8 @@ def linear_tiled(x, layers):
         return
     n = len(layers)
     w, b, o = zip(*layers)
-    N.call("pikv_linear_tiled", x, T, K, n, w, b, [t.shape[0] for t in w],
-           o, _stream())
+    N.launch("pikv_linear_tiled", x, T, K, n, w, b, [t.shape[0] for t in w],
+             o, _stream())
 
 
 def value_lora(mean, lora_a, lora_b, scaling):
@@ -476,8 +476,8 @@ def value_lora(mean, lora_a, lora_b, scaling):
                 or _need(b, "lora_b", dtype=torch.float32).shape != (rank, H)):
             raise ValueError("lora_a must be [H, rank], lora_b [rank, H]")
     out = torch.empty_like(mean)
-    N.call("pikv_value_lora", mean, E, H, rank, lora_a, lora_b,
-           [float(v) for v in scaling], out, _stream())
+    N.launch("pikv_value_lora", mean, E, H, rank, lora_a, lora_b,
+             [float(v) for v in scaling], out, _stream())
     return out
 
 
@@ -505,9 +505,9 @@ def expert_combine(dense, lora, scaling, add, weights, lora_b=None):
     if mix.numel():
         rest = ([float(v) for v in scaling], add, weights, T, E, H, outs, mix, _stream())
         if lora_b is None:
-            N.call("pikv_expert_combine", dense, lora, *rest)
+            N.launch("pikv_expert_combine", dense, lora, *rest)
         else:
-            N.call("pikv_expert_combine_factors", dense, lora, lora_b, rank, *rest)
+            N.launch("pikv_expert_combine_factors", dense, lora, lora_b, rank, *rest)
     return outs, mix
 
 
@@ -534,10 +534,10 @@ def adaptive_router(x_mean, selector, lb, imp, predictor, seq_len: int, top_k: i
     topk_w = torch.empty(T, top_k, dtype=torch.float32, device=dev)
     importance = torch.empty(T, dtype=torch.float32, device=dev)
     loss = torch.empty((), dtype=torch.float32, device=dev)
-    N.call("pikv_adaptive_router", x_mean, B, seq_len, H, H2, E, top_k, *selector,
-           *lb, float(temp_lb), *imp, float(temp_imp),
-           *predictor, mask, float(balance_weight), blend, probs[0], probs[1],
-           idx, topk_w, importance, loss, _stream())
+    N.launch("pikv_adaptive_router", x_mean, B, seq_len, H, H2, E, top_k, *selector,
+             *lb, float(temp_lb), *imp, float(temp_imp),
+             *predictor, mask, float(balance_weight), blend, probs[0], probs[1],
+             idx, topk_w, importance, loss, _stream())
     return probs[1], idx, topk_w, loss, importance
 
 
@@ -569,11 +569,11 @@ def prefill_attend(q, k, v, pool: Optional["CachePool"] = None, causal: bool = T
     planes = [None] * 6 if max_cached == 0 else [*pool._planes("k"), *pool._planes("v")]
     nb = N.size("pikv_prefill_attend_workspace_bytes", B, S, hkv, hq, dh, max_cached)
     ws = torch.empty(nb, dtype=torch.uint8, device=q.device) if nb else None
-    N.call("pikv_prefill_attend", q, k, v, B, S, hkv, hq, dh, int(bool(causal)),
-           float(1.0 / math.sqrt(dh) if scale_qk is None else scale_qk), *planes,
-           pool.scheme if max_cached else Q_I8_SYM, pool.group if max_cached else 0,
-           pool.row_base if max_cached else None, pool.fill if max_cached else None, max_cached,
-           out, ws, nb, _stream())
+    N.launch("pikv_prefill_attend", q, k, v, B, S, hkv, hq, dh, int(bool(causal)),
+             float(1.0 / math.sqrt(dh) if scale_qk is None else scale_qk), *planes,
+             pool.scheme if max_cached else Q_I8_SYM, pool.group if max_cached else 0,
+             pool.row_base if max_cached else None, pool.fill if max_cached else None, max_cached,
+             out, ws, nb, _stream())
     return out
 
 
@@ -718,11 +718,11 @@ class CachePool:
             raise ValueError(f"cache_id/slot must have n_src*fanout = {n_src * fanout} elements")
         if n_src == 0:
             return
-        N.call("pikv_quant_scatter", k2, v2, dt, n_src, fanout, self.D, self.group,
-               self.scheme, cache_id, slot, self.row_base, self.fill,
-               self.cap, self.n_caches, self.k_codes, self.v_codes,
-               self.k_scale, self.v_scale, self.k_zero, self.v_zero,
-               self.acc, self.ts, float(now), _stream())
+        N.launch("pikv_quant_scatter", k2, v2, dt, n_src, fanout, self.D, self.group,
+                 self.scheme, cache_id, slot, self.row_base, self.fill,
+                 self.cap, self.n_caches, self.k_codes, self.v_codes,
+                 self.k_scale, self.v_scale, self.k_zero, self.v_zero,
+                 self.acc, self.ts, float(now), _stream())
 
     def quant_scatter_routed(self, k_src, v_src, cache_id, slot, per_token: int, now: float = 0.0):
         """quant_scatter for rows that differ per cache: assignment j of token t (cache_id / slot
@@ -741,10 +741,10 @@ class CachePool:
             raise ValueError("cache_id and slot must have n * per_token elements")
         if n == 0:
             return
-        N.call("pikv_quant_scatter_routed", k_src, v_src, n, per_token, self.D, self.group, self.scheme,
-               cache_id, slot, self.row_base, self.fill, self.cap, self.n_caches,
-               self.k_codes, self.v_codes, self.k_scale, self.v_scale, self.k_zero,
-               self.v_zero, self.acc, self.ts, float(now), _stream())
+        N.launch("pikv_quant_scatter_routed", k_src, v_src, n, per_token, self.D, self.group, self.scheme,
+                 cache_id, slot, self.row_base, self.fill, self.cap, self.n_caches,
+                 self.k_codes, self.v_codes, self.k_scale, self.v_scale, self.k_zero,
+                 self.v_zero, self.acc, self.ts, float(now), _stream())
 
     def quant_gather(self, k_src, v_src, src_row_base, src_index, n_take, max_take: int,
                      src_score=None, now: float = 0.0):
@@ -774,20 +774,20 @@ class CachePool:
                 raise ValueError("src_score must have one entry per source row")
         if max_take <= 0 or k2.shape[0] == 0:
             return
-        N.call("pikv_quant_gather", k2, v2, dt, self.D, self.group, self.scheme,
-               src_row_base, src_index, n_take, int(max_take), src_score,
-               self.row_base, self.fill, self.cap, self.n_caches,
-               self.k_codes, self.v_codes, self.k_scale, self.v_scale,
-               self.k_zero, self.v_zero, self.acc, self.ts, float(now),
-               _stream())
+        N.launch("pikv_quant_gather", k2, v2, dt, self.D, self.group, self.scheme,
+                 src_row_base, src_index, n_take, int(max_take), src_score,
+                 self.row_base, self.fill, self.cap, self.n_caches,
+                 self.k_codes, self.v_codes, self.k_scale, self.v_scale,
+                 self.k_zero, self.v_zero, self.acc, self.ts, float(now),
+                 _stream())
 
     def advance(self, count, per_call_limit: int = -1):
         """fill[c] = min(fill[c] + min(count[c], limit), cap[c])."""
         count = _need(count, "count", dtype=torch.int32, ndim=1)
         if count.numel() != self.n_caches:
             raise ValueError("count must have one entry per cache")
-        N.call("pikv_cache_advance", self.fill, count, self.cap, self.n_caches,
-               int(per_call_limit), _stream())
+        N.launch("pikv_cache_advance", self.fill, count, self.cap, self.n_caches,
+                 int(per_call_limit), _stream())
 
     # ---- read path ----
     def _planes(self, which):
@@ -810,8 +810,8 @@ class CachePool:
             return out.zero_()
         nb = N.size("pikv_cache_mean_workspace_bytes", self.n_caches, self.D, self.max_cap)
         ws = torch.empty(nb, dtype=torch.uint8, device=self.device)
-        N.call("pikv_cache_mean", codes, scale, zero, self.scheme, self.group, self.D,
-               self.row_base, self.fill, self.n_caches, self.max_cap, out, ws, nb, _stream())
+        N.launch("pikv_cache_mean", codes, scale, zero, self.scheme, self.group, self.D,
+                 self.row_base, self.fill, self.n_caches, self.max_cap, out, ws, nb, _stream())
         return out
 
     def scores(self, q, n_q_heads: int, scale_qk: Optional[float] = None,
@@ -834,10 +834,10 @@ class CachePool:
         tsum = torch.empty_like(tmax)
         if scale_qk is None:
             scale_qk = 1.0 / (self.head_dim ** 0.5)
-        N.call("pikv_gather_dequant_scores", self.k_codes, self.k_scale,
-               self.k_zero, self.scheme, self.group, self.n_heads, n_q_heads, self.head_dim,
-               q, qdt, float(scale_qk), self.row_base, self.fill, self.n_caches,
-               max_len, stride, scores, tmax, tsum, _stream())
+        N.launch("pikv_gather_dequant_scores", self.k_codes, self.k_scale,
+                 self.k_zero, self.scheme, self.group, self.n_heads, n_q_heads, self.head_dim,
+                 q, qdt, float(scale_qk), self.row_base, self.fill, self.n_caches,
+                 max_len, stride, scores, tmax, tsum, _stream())
         return scores, tmax, tsum
 
     def h2o_accumulate(self, scores, tile_max, tile_sum, now: float, decay: float = 1.0,
@@ -858,10 +858,10 @@ class CachePool:
         dev = self.device
         imp = torch.zeros(nc, stride, dtype=torch.float32, device=dev) if return_importance else None
         head_stats = torch.empty(nc, hq, 2, dtype=torch.float32, device=dev)
-        N.call("pikv_h2o_accumulate", scores, tile_max, tile_sum, hq,
-               self.row_base, self.fill, nc, stride, stride, float(decay), float(now),
-               int(bool(write_probs)), None if stats_only else self.acc,
-               None if stats_only else self.ts, imp, head_stats, _stream())
+        N.launch("pikv_h2o_accumulate", scores, tile_max, tile_sum, hq,
+                 self.row_base, self.fill, nc, stride, stride, float(decay), float(now),
+                 int(bool(write_probs)), None if stats_only else self.acc,
+                 None if stats_only else self.ts, imp, head_stats, _stream())
         self.head_stats = head_stats   # (max, sum) per (cache, head): what attend_values normalises with
         return imp
 
@@ -889,11 +889,11 @@ class CachePool:
             return out
         ws_bytes = N.size("pikv_attend_workspace_bytes", nc, hq, self.head_dim, stride)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-        N.call("pikv_attend_values", scores, head_stats, stride, self.v_codes,
-               self.v_scale, self.v_zero, self.scheme, self.group, self.n_heads, hq,
-               self.head_dim, self.row_base, self.fill, nc, stride, float(decay), float(now),
-               self.acc if accumulate else None, self.ts if accumulate else None,
-               out, ws, ws_bytes, _stream())
+        N.launch("pikv_attend_values", scores, head_stats, stride, self.v_codes,
+                 self.v_scale, self.v_zero, self.scheme, self.group, self.n_heads, hq,
+                 self.head_dim, self.row_base, self.fill, nc, stride, float(decay), float(now),
+                 self.acc if accumulate else None, self.ts if accumulate else None,
+                 out, ws, ws_bytes, _stream())
         return out
 
     def decode_attend(self, q, n_q_heads: int, now: float = 0.0, scale_qk: Optional[float] = None,
@@ -922,12 +922,12 @@ class CachePool:
             self._decode_ws = torch.empty(max(nb, 256), dtype=torch.uint8, device=dev)
             self._decode_ws_key = key
         ws = self._decode_ws
-        N.call("pikv_decode_attend", self.k_codes, self.k_scale, self.k_zero,
-               self.v_codes, self.v_scale, self.v_zero, self.scheme, self.group,
-               self.n_heads, n_q_heads, self.head_dim, q, dt, float(scale_qk), self.row_base,
-               self.fill, self.n_caches, max_len, float(decay), float(now),
-               self.acc if accumulate else None, self.ts if accumulate else None,
-               out, ws, ws.numel(), _stream())
+        N.launch("pikv_decode_attend", self.k_codes, self.k_scale, self.k_zero,
+                 self.v_codes, self.v_scale, self.v_zero, self.scheme, self.group,
+                 self.n_heads, n_q_heads, self.head_dim, q, dt, float(scale_qk), self.row_base,
+                 self.fill, self.n_caches, max_len, float(decay), float(now),
+                 self.acc if accumulate else None, self.ts if accumulate else None,
+                 out, ws, ws.numel(), _stream())
         return out
 
     # ---- eviction ----
@@ -958,9 +958,9 @@ class CachePool:
         args = (self.acc, self.ts, self.row_base, self.fill, nh, nr, self.n_caches,
                 self.max_cap, self.keep_flag, self.keep_index, self.new_len, ws, ws_bytes, _stream())
         if ratios:
-            N.call("pikv_evict_select_h2o", float(heavy_ratio), float(recent_ratio), *args)
+            N.launch("pikv_evict_select_h2o", float(heavy_ratio), float(recent_ratio), *args)
         else:
-            N.call("pikv_evict_select", policy, *args)
+            N.launch("pikv_evict_select", policy, *args)
 
     def planes(self):
         ps = [self.k_codes, self.k_scale, self.k_zero, self.v_codes, self.v_scale, self.v_zero,
@@ -975,8 +975,8 @@ class CachePool:
         if len(ps) > N.MAX_PLANES:
             raise ValueError(f"at most {N.MAX_PLANES} planes")
         rbs = self._row_bytes + [math.prod(p.shape[1:]) * p.element_size() for p in extra]
-        N.call("pikv_compact_rows", ps, rbs, len(ps), self.row_base, self.keep_index,
-               self.new_len, self.fill, self.n_caches, _stream())
+        N.launch("pikv_compact_rows", ps, rbs, len(ps), self.row_base, self.keep_index,
+                 self.new_len, self.fill, self.n_caches, _stream())
 
     def make_room(self, policy: int, *, count: Optional[torch.Tensor] = None, count_all: int = 0,
                   limit: int = -1, heavy_ratio: float = 0.1, recent_ratio: float = 0.1,
@@ -996,10 +996,10 @@ class CachePool:
         if getattr(self, "_evict_ws", None) is None:
             self._evict_ws = _evict_workspace(self.n_caches, self.max_cap, self.device)
         ws, ws_bytes = self._evict_ws
-        N.call("pikv_cache_make_room", policy, count, int(count_all), int(limit), float(heavy_ratio),
-               float(recent_ratio), int(leave_room), int(append), self.acc, self.ts, self.row_base,
-               self.fill, self.cap, self.n_caches, self.max_cap, ps, rbs, len(ps), self.keep_flag,
-               self.keep_index, self.new_len, self._budgets, ws, ws_bytes, _stream())
+        N.launch("pikv_cache_make_room", policy, count, int(count_all), int(limit), float(heavy_ratio),
+                 float(recent_ratio), int(leave_room), int(append), self.acc, self.ts, self.row_base,
+                 self.fill, self.cap, self.n_caches, self.max_cap, ps, rbs, len(ps), self.keep_flag,
+                 self.keep_index, self.new_len, self._budgets, ws, ws_bytes, _stream())
 
     def append_rows(self, k_src, v_src, now: float = 0.0, advance: bool = False):
         """Quantise k_src / v_src [n_caches * rows, D] (cache-major) behind the new_len rows of every
@@ -1016,10 +1016,10 @@ class CachePool:
                 raise ValueError("v_src must match k_src")
         if rows == 0:
             return
-        N.call("pikv_quant_append", k_src, v_src if self.with_v else None, dt, rows, self.D, self.group,
-               self.scheme, self.row_base, self.new_len, self.fill if advance else None, self.cap,
-               self.n_caches, self.k_codes, self.v_codes, self.k_scale, self.v_scale, self.k_zero,
-               self.v_zero, self.acc, self.ts, float(now), _stream())
+        N.launch("pikv_quant_append", k_src, v_src if self.with_v else None, dt, rows, self.D, self.group,
+                 self.scheme, self.row_base, self.new_len, self.fill if advance else None, self.cap,
+                 self.n_caches, self.k_codes, self.v_codes, self.k_scale, self.v_scale, self.k_zero,
+                 self.v_zero, self.acc, self.ts, float(now), _stream())
 
     def evict(self, policy: int, **kw):
         self.evict_select(policy, **kw)

@@ -14,7 +14,8 @@ from pikv_amd import _native as N, dense, ops
 
 
 def test_every_entry_point_is_there():
-    assert set(N.SIGNATURES) - {"pikv_status_string"} <= set(dir(N.entries()))
+    for module in (N.entries(), N.entries().of_checked):
+        assert set(N.SIGNATURES) - {"pikv_status_string"} <= set(dir(module))
 
 
 def test_sizes_agree_with_ctypes():
@@ -77,8 +78,11 @@ def test_pointer_parameters_take_what_they_are(name):
         else:
             continue
         for w in wrong:
-            with pytest.raises((TypeError, ValueError)):       # (numpy: a strided array gives no plain buffer, a ValueError)
-                getattr(N.entries(), name)(*plain[:i], w, *plain[i + 1:])
+            # of callers that have checked their tensors everything but those is refused the same way
+            forms = [N.entries()] if isinstance(w[0] if isinstance(w, list) else w, (torch.Tensor, _Tensor)) else [N.entries(), N.entries().of_checked]
+            for f in forms:
+                with pytest.raises((TypeError, ValueError)):       # (numpy: a strided array gives no plain buffer, a ValueError)
+                    getattr(f, name)(*plain[:i], w, *plain[i + 1:])
 
 
 def test_pointer_values():
@@ -86,7 +90,7 @@ def test_pointer_values():
     # (n_caches = 0 is refused behind the null pointers: -1 null, -2 a bad size)
     for p, status in ((None, -1), (C.c_void_p(None), -1), (C.POINTER(C.c_int32)(), -1), (64, -2), (C.c_void_p(64), -2),
                       (C.cast(64, C.POINTER(C.c_int32)), -2), (_Tensor(True), -2)):
-        assert f.pikv_h2o_budget(p, 0, 0.1, 0.1, 64, 64, None) == status, p
+        assert f.pikv_h2o_budget(p, 0, 0.1, 0.1, 64, 64, None) == f.of_checked.pikv_h2o_budget(p, 0, 0.1, 0.1, 64, 64, None) == status, p
         if not isinstance(p, _Tensor):
             assert N.lib().pikv_h2o_budget(p, 0, 0.1, 0.1, 64, 64, None) == status
     # host arrays of ctypes, as the ctypes signatures take them: the width 0 is found behind them
@@ -140,7 +144,7 @@ def test_every_plane_of_a_compaction_has_its_row_bytes(monkeypatch, kind):
     seen = []
     monkeypatch.setattr(ops, "_need", lambda t, name: t)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
-    monkeypatch.setattr(N, "call", lambda name, *args: seen.append(args))
+    monkeypatch.setattr(N, "launch", lambda name, *args: seen.append(args))
     pool.compact(extra_planes=kind([torch.zeros(4, 3), torch.zeros(4, dtype=torch.int64)]))
     planes, widths, n = seen[0][:3]
     assert len(planes) == len(widths) == n == 6 and widths == [64, 8, 4, 4, 12, 8]
@@ -152,7 +156,7 @@ def test_experts_factors_come_in_any_sequence(monkeypatch, kind):
     seen = []
     monkeypatch.setattr(ops, "_need", lambda t, name, **kw: t)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
-    monkeypatch.setattr(N, "call", lambda name, *args: seen.append((name, args)))
+    monkeypatch.setattr(N, "launch", lambda name, *args: seen.append((name, args)))
     a, b, d = ([torch.ones(s) for _ in range(3)] for s in ((8, 2), (2, 8), (5, 8)))
     t = [torch.ones(5, 2) for _ in range(3)]
     ops.value_lora(torch.ones(3, 8), kind(a), kind(b), [1.0] * 3)
@@ -182,7 +186,7 @@ def test_without_the_extension_every_way_in_says_so():
     _python("import sys, torch\nsys.modules['pikv_amd._call'] = None\n"
             "from pikv_amd import _native as N, dense, ops\n"
             "for f in (lambda: dense.ordinary_tensor(torch.zeros(8), torch.device('cpu')), lambda: ops._need(torch.zeros(8), 'x'),\n"
-            "          lambda: N.call('pikv_abi_version'), lambda: N.size('pikv_evict_workspace_bytes', 1, 5)):\n"
+            "          lambda: N.call('pikv_abi_version'), lambda: N.launch('pikv_abi_version'), lambda: N.size('pikv_evict_workspace_bytes', 1, 5)):\n"
             "    try:\n        f()\n"
             "    except N.PiKVNativeError as e:\n"
             "        assert 'python -m pikv_amd.build' in str(e) and isinstance(e.__cause__, ImportError), e\n"
