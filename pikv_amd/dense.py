@@ -7,7 +7,7 @@ all go through the module's own call.
 """
 from __future__ import annotations
 
-from functools import reduce
+from functools import lru_cache, reduce
 
 import torch
 import torch.nn as nn
@@ -69,7 +69,8 @@ def projections_pay(T: int, H: int, N: int) -> bool:
 _TILES = ((128, 128, 57.0), (64, 128, 30.0), (64, 64, 16.6), (32, 64, 11.0))   # rows, columns, ns for a round of 256 and a k-value
 
 
-def _tiled_us(T: int, H: int, widths) -> float:
+@lru_cache(maxsize=1024)      # (5 us a call otherwise; a program has a few sizes)
+def _tiled_us(T: int, H: int, widths: tuple) -> float:
     """Kernel time of linear_tiled without its start of about 5 us (tile_variant in csrc/linear.hip)."""
     return 1e-3 * H * min(-(-(-(-T // m) * sum(-(-w // n) for w in widths)) // 256) * ns for m, n, ns in _TILES)
 
@@ -89,20 +90,21 @@ def tiled_pays(T: int, H: int, widths) -> bool:
         return False
     N = sum(widths)
     if T * H * N <= 3_500_000_000:
-        us = _tiled_us(T, H, widths)
+        us = _tiled_us(T, H, tuple(widths))
         return us <= 55 or 2e-6 * T * H * N >= 100 * us
     tiles = -(-T // 128) * sum(-(-n // 128) for n in widths)
     return tiles <= 256 and T * N >= 0.87 * 256 * 128 * 128
 
 
 def experts_tiled(T: int, H: int, E: int) -> bool:
-    """The products of E experts [H, H] in one launch of LDS tiles: 128 x 256, 4 experts 13 us / 75 for four library calls, 1053 x 512,
-    4 experts 32 / 75, 667 x 1024, 4 experts 60 / 76; while the tiles take less time than the library's calls take the host, 18 us each
-    (outside 743 x 1536, 1 expert 52 / 36, 716 x 1536, 2 experts 84 / 71, 548 x 1280, 3 experts 70 / 62).
+    """The products of E experts [H, H] in one launch of LDS tiles: 128 x 256, 4 experts 14 us for four library calls of 34 on one
+    compute unit each, 1053 x 512, 4 experts 32 / 75, 667 x 1024, 4 experts 60 / 76; while the tiles take less time than the
+    library's calls take the host, 18 us each (outside 743 x 1536, 1 expert 52 / 36, 716 x 1536, 2 experts 84 / 71, 548 x 1280,
+    3 experts 70 / 62).
 
     What the experts put out is cached in codes, and the means of the caches come back in the next call, where another order of sums
-    - 2e-7, a code in 10^4 - grows to 1e-4 of a cached row's scale.  So only sizes are taken where the library (hipBLASLt of ROCm 7, as
-    torch calls it by default) was measured to sum in the same order, to the last bit: 33 tokens on but for 257 to 1024 and more
+    - 2e-7, a code in 10^4 - grows to 1e-4 of a cached row's scale.  So only sizes are taken where the library (of ROCm 7, as torch
+    calls it by default) was measured to sum in the same order, to the last bit: 33 tokens on but for 257 to 1024 and more
     than 2048 tokens of 256 columns, 257 on of 128, and fewer than 512 of more than 512; 2800 sizes up to 8192 tokens, of which 3
     differed, all beyond what the time admits.  Another library or version may choose otherwise: no less exact, but
     its two forms then differ by that much."""
@@ -151,17 +153,18 @@ def forward_only(x) -> bool:
     return not torch.is_grad_enabled() and x.is_cuda and ordinary_call() and ordinary_tensor(x, x.device)
 
 
-def tensor_of(m, name: str):
-    """The tensor m.<name>: a parameter (m.<name> itself looks through three tables for it), a buffer or a plain attribute."""
-    t = m._parameters.get(name)
-    return getattr(m, name, None) if t is None else t
+def tensors_of(m, a: str, b: str):
+    """m.<a>, m.<b>: parameters (the attributes themselves look through three tables for them), buffers or plain attributes."""
+    p = m._parameters
+    ta, tb = p.get(a), p.get(b)
+    return (ta, tb) if ta is not None and tb is not None else (getattr(m, a, None), getattr(m, b, None))
 
 
 def linear_ok(m, n_in: int, n_out: int, device) -> bool:
     """A plain nn.Linear of this shape with a bias, as linear_group reads it."""
     if not plain(m, nn.Linear):
         return False
-    w, b = tensor_of(m, "weight"), tensor_of(m, "bias")
+    w, b = tensors_of(m, "weight", "bias")
     return (w is not None and b is not None and w.shape == (n_out, n_in) and ordinary_tensor(w, device)
             and ordinary_tensor(b, device))
 

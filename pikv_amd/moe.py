@@ -227,7 +227,7 @@ class PiKVMoE(nn.Module):
         if not dense.plain(m, LoRALayer):
             return False
         H = config['hidden_size']
-        a, b, drop = dense.tensor_of(m, "lora_A"), dense.tensor_of(m, "lora_B"), m._modules.get("dropout")
+        (a, b), drop = dense.tensors_of(m, "lora_A", "lora_B"), m._modules.get("dropout")
         return (a is not None and b is not None and type(m.scaling) in (int, float) and a.shape == (H, rank) and b.shape == (rank, H)
                 and dense.ordinary_tensor(a, device) and dense.ordinary_tensor(b, device)
                 and dense.plain(drop, nn.Dropout) and not (drop.training and drop.p > 0))
