@@ -320,9 +320,9 @@ static size_t attend_mfma_lds_bytes(int n_kv_heads, int n_q_heads, int nsets = 1
 // heads of a slab are the heads of those kv heads in order.  A query head is multiplied with the
 // whole slab and only the dimensions of its own kv head are written out.
 // NARROW selects that form at compile time: the kernel for heads of 128 carries none of it.
-// NSETS = 2 (up to 4 kv heads): a launch covers up to 8 query heads of every kv head as two sets of
+// NSETS = 2 (up to 4 kv heads): a block covers up to 8 query heads of every kv head as two sets of
 // four that are multiplied with the same staged tile and the same expanded codes - the V codes of a
-// cache with 5 to 8 query heads per kv head are read from memory once instead of once per launch.
+// cache with 5 to 8 query heads per kv head are read from memory once instead of once per set.
 // SPLIT (rows of a.row_slabs = groups x HK slabs): neighbouring blocks take the groups of HK slabs of
 // one token range, block index = range * groups + group; a group is a piece of HK x 64 bytes of every
 // cached row.  Rows of more than 8 slabs (e.g. 32 kv heads of 128) go as groups of 8; rows of 6, 8 or
@@ -760,7 +760,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   __syncthreads();
   if constexpr (TI > 1) {
     // the TI slabs of a kv head hold partial outputs over different tokens: added in LDS, parity by parity
-    float* ol = zl + 4 * NI * 4 * 4;   // [kv head][head of the launch: 4 * set + ro][128]
+    float* ol = zl + 4 * NI * 4 * 4;   // [kv head][head of the block: 4 * set + ro][128]
     for (int par = 0; par < TI; ++par) {
 #pragma unroll
       for (int hs = 0; hs < NI; ++hs) {
@@ -854,7 +854,7 @@ static size_t attend_mfma8_lds_bytes(int n_slabs, int staged, int hps) {
 // Query heads whose probabilities a block holds: at most eight of every slab, the others are other blocks or launches.
 static int attend_mfma8_staged(int n_slabs, int n_q_heads) { return n_q_heads < n_slabs * 8 ? n_q_heads : n_slabs * 8; }
 
-// HK = n_kv_heads (1..8); 2..8 query heads per kv head, at most 64 query heads.
+// HK = n_kv_heads (1..8); 2..8 query heads per kv head and block.
 // Heads narrower than 128 (HPS = 128 / head_dim = 2 or 4): the kernel's kv heads are 128-dimension
 // slabs of the cached row, each the stored bytes of HPS neighbouring kv heads with a scale (and
 // zero point) each; the query heads of a slab are the heads of those kv heads in order.  A query
@@ -898,11 +898,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       a.partial[((int64_t)blockIdx.x * a.n_caches + c) * a.n_q_heads * a.head_dim + idx] = 0.f;
     return;
   }
-  // a launch serves heads head_off .. head_off + rep - 1 of every kv head (more than 8 per kv head: two
-  // launches; narrow heads are launched with head_off = 0 only); the staged rows count these heads alone
+  // a block serves heads head_off .. head_off + rep - 1 of every kv head (more than 8 per kv head: blocks side by side or
+  // later launches, heads of 128 only); the staged rows count these heads alone
   const int rep_all = a.n_q_heads / HKR;
   const int rep = rep_all - head_off < 8 ? rep_all - head_off : 8;  // 1..8
-  const int nql = HKR * rep;         // staged heads: row (kv head) * rep + head of the launch
+  const int nql = HKR * rep;         // staged heads: row (kv head) * rep + head of the block
   const int rep1 = rep / HPS;        // query heads per stored kv head
   const int groups_per_row = (HKR * 128) / a.group;
   // matrix-core roles: A row / B,C column i, token group kg (tokens 8*kg .. 8*kg+7 of the tile)
@@ -1307,8 +1307,9 @@ static void launch_attend_mfma_slabs(int n_slabs, int nsets, dim3 grid, hipStrea
     default: hipLaunchKernelGGL((attend_mfma_i4_kernel<SCHEME, 8, EXCH, NARROW>), grid, dim3(256), lds, st, a); break;
   }
 }
-// All query heads of every slab: four per launch, or - up to 4 slabs - eight per launch in two sets.  A
-// later launch (same codes, next heads) adds its share to the accumulators that the first one has decayed.
+// All query heads of every slab: four to a block, or - up to 4 slabs - eight in two sets.  More are blocks side by side
+// or launches one after the other (sets_side_by_side); a later launch adds its share to the accumulators that the
+// first one has decayed.
 template <int SCHEME, bool EXCH = false>
 static void launch_attend_mfma(int n_slabs, int heads_per_slab, dim3 grid, hipStream_t st, AttendArgs a) {
   // split rows (heads of 128; whole groups of 8 slabs for more than 8 are checked by the caller): slabs per group

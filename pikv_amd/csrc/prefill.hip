@@ -22,8 +22,9 @@
 // Measured (us, back to back, before -> now; before: K of a tile loaded and waited for, queries and V in registers, 26 spilled
 // registers): 2 x 500 tokens, 16 heads of 128 over 8 kv heads 43.8 -> 35.3, over 500 cached rows of 8 bits 97 -> 81; 4 x 1000 over 1000, 32
 // heads 1216 -> 978 (101 TFLOP/s, 64 % of the products' rate); 700 over 700 rows of 4 bits 234 -> 147; 4 x 333, 32 heads of 64 50 -> 34;
-// 40 tokens 16.8 -> 10.6.  Heads of 128 take 246 registers, none spilled.  Against float64 the error is that of the torch path or
-// below (4.7e-7 and 6.2e-7).
+// 40 tokens 16.8 -> 10.6.  Heads of 128 take 246 registers, none spilled.  Error against float64 and that of the float32 torch path,
+// 2-norms, 2 x 500 tokens and the same over 500 cached rows of 8 bits: heads of 128 3.1e-7 / 3.4e-7 and 4.7e-7 / 6.2e-7, of 64 2.4e-7 / 2.8e-7
+// and 3.9e-7 / 5.7e-7; with scores eight times as large 1.2e-6 / 1.2e-6 and 1.5e-6 / 1.5e-6.
 //
 // A NaN or infinity in a V row that a query does not see reaches that query only from the query's own last tile (a
 // zero probability times it); a product over the whole score matrix spreads it to every row.
@@ -75,7 +76,7 @@ __device__ __forceinline__ int in_loop(int x) {
   return x;
 }
 
-// exp(x) for x <= 0, NaN for NaN: 2^t with t = x log2(e) in two parts.  Ten instructions; expf of any argument takes twenty,
+// exp(x) for x <= 0, NaN for NaN: 2^t with t = x log2(e) in two parts; what is below 2^-126 is 0.  Ten instructions; expf of any argument takes twenty,
 // and the matrix core and the vector unit of a SIMD do float32 in turn, not side by side (a slot of one 32 x 32 x 2 product and 16
 // multiply-adds from two wavefronts takes 145 cycles: 66 + 80).
 __device__ __forceinline__ float exp_nonpositive(float x) {

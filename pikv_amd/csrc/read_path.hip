@@ -605,7 +605,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NKV * NSET 
   const int head_dim = NARROW ? a.head_dim : 128;
   const int gshift = head_dim == 64 ? 1 : 0;          // log2 of a narrow head's groups of 32
   const int rep1 = head_dim == 64 ? rep_all >> 1 : rep_all >> 2;
-  auto owns = [&](int r, int gq) {                    // group gq of the slab belongs to the kv head of the launch's query head r
+  auto owns = [&](int r, int gq) {                    // group gq of the slab belongs to the kv head of the block's query head r
     const int ra = r + head_off;                    // ... which is head ra of the slab
     return !NARROW || (gq >> gshift) == (ra >= rep1) + (ra >= 2 * rep1) + (ra >= 3 * rep1);
   };
@@ -873,8 +873,8 @@ __global__ __launch_bounds__(256) void scores_mfma_i8_kernel(ScoreArgs a) {
   const int len = a.fill[c] < a.max_len ? a.fill[c] : a.max_len;
   const int64_t tile0 = (int64_t)blockIdx.x * a.tiles_per_block;
   if (tile0 * kTile >= len) return;  // uniform for the block
-  // a block serves heads head_off .. head_off + rep - 1 of every kv head (more than 16 per kv head: grid z
-  // launches, heads of 128 only); the staged rows are those heads, rep per kv head
+  // a block serves heads head_off .. head_off + rep - 1 of every kv head (more than 16 per kv head: blocks side by
+  // side, grid z, heads of 128 only); the staged rows are those heads, rep per kv head
   const int rep_all = a.n_q_heads / a.n_kv_heads;
   const int rep = rep_all - head_off < 16 ? rep_all - head_off : 16;
   const int lane = threadIdx.x & 63;
@@ -1542,7 +1542,7 @@ extern "C" int pikv_gather_dequant_scores(const void* k_codes, const void* k_sca
   // dimensions are served as 128-dimension slabs of two or four neighbouring kv heads
   const int hps = mfma_heads_per_slab(head_dim, n_kv_heads);
   // (float32 queries: as two bf16 limbs on the same kernel, where its operands fit)
-  // (more than 8 bf16 query heads per slab on rows of up to 4 slabs: launches of eight heads each; float32
+  // (more than 8 bf16 query heads per slab on rows of up to 4 slabs: eight to a block; float32
   // queries of such ratios stay on the vector form, which multiplies them exactly)
   const bool more_launches = hps > 0 && n_kv_heads / hps <= 4 && rep * hps > 8;
   if (!eight && group == 32 && hps > 0 && q_dtype == PIKV_F32 && rep * hps <= 8) {
