@@ -76,9 +76,9 @@ __device__ __forceinline__ int in_loop(int x) {
   return x;
 }
 
-// exp(x) for x <= 0, NaN for NaN: 2^t with t = x log2(e) in two parts; what is below 2^-126 is 0.  Ten instructions; expf of any argument takes twenty,
-// and the matrix core and the vector unit of a SIMD do float32 in turn, not side by side (a slot of one 32 x 32 x 2 product and 16
-// multiply-adds from two wavefronts takes 145 cycles: 66 + 80).
+// exp(x) for x <= 0, NaN for NaN: 2^t with t = x log2(e) in two parts; what is below 2^-126 is 0.  Ten instructions; expf of
+// any argument takes twenty, and the matrix core and the vector unit of a SIMD do float32 in turn, not side by side (a slot of one
+// 32 x 32 x 2 product and 16 multiply-adds from two wavefronts takes 145 cycles: 66 + 80).
 __device__ __forceinline__ float exp_nonpositive(float x) {
   constexpr float kLog2eHi = 0x1.715476p+0f, kLog2eLo = 0x1.4ae0cp-26f, kLn2 = 0x1.62e430p-1f;
   x = x < -120.f ? -120.f : x;           // 0 as a float32 probability
